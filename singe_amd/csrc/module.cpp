@@ -384,14 +384,6 @@ const char* const kKernelNames[kKernelCount] = {
     "singe_ragged_prefill_bf16_d48", "singe_ragged_prefill_f16_d48",
     "singe_ragged_prefill_bf16_d80", "singe_ragged_prefill_f16_d80",
     "singe_ragged_prefill_bf16_d112", "singe_ragged_prefill_f16_d112",
-    "singe_ragged_prefill_pair_bf16_d128", "singe_ragged_prefill_pair_f16_d128",
-    "singe_ragged_prefill_pair_bf16_d64", "singe_ragged_prefill_pair_f16_d64",
-    "singe_ragged_prefill_pair_bf16_d32", "singe_ragged_prefill_pair_f16_d32",
-    "singe_ragged_prefill_pair_bf16_d96", "singe_ragged_prefill_pair_f16_d96",
-    "singe_ragged_prefill_pair_bf16_d16", "singe_ragged_prefill_pair_f16_d16",
-    "singe_ragged_prefill_pair_bf16_d48", "singe_ragged_prefill_pair_f16_d48",
-    "singe_ragged_prefill_pair_bf16_d80", "singe_ragged_prefill_pair_f16_d80",
-    "singe_ragged_prefill_pair_bf16_d112", "singe_ragged_prefill_pair_f16_d112",
     "singe_attention_mfma_f32_d32_r16", "singe_attention_mfma_f32_d64_r16", "singe_attention_mfma_f32_d96_r16",
     "singe_attention_mfma_f32_d128_r16",
     "singe_attention_mfma_f32_d64_r32", "singe_attention_mfma_f32_d96_r32", "singe_attention_mfma_f32_d128_r32",
@@ -448,8 +440,7 @@ constexpr PartRun kPartRuns[] = {
     {39, 8},                      // the two-tile paged attention at head_dim 64
     {40, 8}, {41, 8},             // both at head_dim 96
     {42, 8}, {43, 8}, {44, 8}, {45, 8}, {46, 8}, {47, 8}, {48, 8}, {49, 8}, {50, 8}, {51, 8},  // and at 112, 80, 48, 32, 16
-    {3, 2}, {15, 2}, {19, 2}, {21, 2}, {23, 2}, {25, 2}, {27, 2}, {29, 2},    // packed sequences: the 32-row kernel,
-    {37, 2}, {39, 2}, {49, 2}, {41, 2}, {51, 2}, {47, 2}, {45, 2}, {43, 2},   // the two-tile kernel
+    {3, 2}, {15, 2}, {19, 2}, {21, 2}, {23, 2}, {25, 2}, {27, 2}, {29, 2},    // packed sequences
     {52, 7},                      // dense f32 attention on the matrix cores
 };
 constexpr int runs_total() {

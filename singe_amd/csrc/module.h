@@ -98,12 +98,10 @@ enum KernelId : int {
     kPagedPairD96 = kPrefillPairD96 + 8,
     // and those for 112, 80, 48, 32, 16: sixteen each, the dense eight first
     kPairOtherHeadDims = kPagedPairD96 + 8,
-    // packed sequences (ragged_kv_prefill_attention): bf16, f16 of the 32-row kernel for the head dimensions 128, 64, then as in
-    // kOtherHeadDims; then bf16, f16 of the two-tile kernel in the same order
+    // packed sequences (ragged_kv_prefill_attention): bf16, f16 for the head dimensions 128, 64, then as in kOtherHeadDims
     kRaggedPrefill = kPairOtherHeadDims + 5 * 16,
-    kRaggedPrefillPair = kRaggedPrefill + 2 * 8,
     // dense f32 attention on the matrix cores: head dimensions 32, 64, 96, 128 with 16-row tiles, then 64, 96, 128 with 32-row ones
-    kAttentionMfmaF32 = kRaggedPrefillPair + 2 * 8,
+    kAttentionMfmaF32 = kRaggedPrefill + 2 * 8,
     kKernelCount = kAttentionMfmaF32 + 7
 };
 
@@ -180,7 +178,7 @@ inline int head_dim_order(long long head_dim) {
 }
 
 // The packed-sequences kernel for a head dimension, before 1 is added for f16.
-inline int ragged_prefill_at(long long head_dim, bool pair) { return (pair ? kRaggedPrefillPair : kRaggedPrefill) + 2 * head_dim_order(head_dim); }
+inline int ragged_prefill_at(long long head_dim) { return kRaggedPrefill + 2 * head_dim_order(head_dim); }
 
 // The fused-rotation kernel for an element type, a cap and a head dimension, before the index / page form is added.
 inline int rotary_paged_attention_base(bool f16, bool softcap, long long head_dim) {

@@ -135,7 +135,9 @@ SINGE_DEVICE float begin_block(RowState& state, f32x16_t& s, unsigned int hi, fl
 //               are computed here (`next_keys` is not read), on return those of the block at `after_keys`, each
 //               read as soon as the product that used its register has been issued, a whole block before
 //               its use.  Otherwise the operands are read from `next_keys` at the start of the call.
-template <bool NEXT, bool AHEAD = false, class Half>
+//   WIDE        the weights meet the values at the precision of f32 to within 2^-18 of themselves (f16: 2^-22): each as
+//               the sum of two 16-bit values, which is two value products in place of one (split_pair).
+template <bool NEXT, bool AHEAD = false, bool WIDE = false, class Half>
 SINGE_DEVICE void finish_block(Half half, RowState& state, f32x16_t& s, float factor, float shift, const unsigned char* values,
                                const ReadOffsets& offsets, f32x16_t& next, const uint4 (&q)[kSteps], const unsigned char* next_keys,
                                uint4 (&operand)[kSteps], const unsigned char* after_keys) {
@@ -189,20 +191,33 @@ SINGE_DEVICE void finish_block(Half half, RowState& state, f32x16_t& s, float fa
     // O^T += V^T . P^T, 16 keys per MFMA: registers 8j .. 8j+7 are keys 16j + {0..3, 8..11} + 4hi.
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-        const uint4 weights = make_uint4(pack_pair(half, s[8 * j + 0], s[8 * j + 1]), pack_pair(half, s[8 * j + 2], s[8 * j + 3]),
-                                         pack_pair(half, s[8 * j + 4], s[8 * j + 5]), pack_pair(half, s[8 * j + 6], s[8 * j + 7]));
+        uint4 weights, rest;
+        if constexpr (WIDE) {
+            split_pair(half, s[8 * j + 0], s[8 * j + 1], weights.x, rest.x);
+            split_pair(half, s[8 * j + 2], s[8 * j + 3], weights.y, rest.y);
+            split_pair(half, s[8 * j + 4], s[8 * j + 5], weights.z, rest.z);
+            split_pair(half, s[8 * j + 6], s[8 * j + 7], weights.w, rest.w);
+        } else {
+            weights = make_uint4(pack_pair(half, s[8 * j + 0], s[8 * j + 1]), pack_pair(half, s[8 * j + 2], s[8 * j + 3]),
+                                 pack_pair(half, s[8 * j + 4], s[8 * j + 5]), pack_pair(half, s[8 * j + 6], s[8 * j + 7]));
+        }
 #pragma unroll
         for (int db = 0; db < kDimBlocks; ++db)
             state.out[db] = mma(half, __builtin_bit_cast(uint4, j == 0 ? first[db] : second[db]), weights, state.out[db]);
+        if constexpr (WIDE) {
+#pragma unroll
+            for (int db = 0; db < kDimBlocks; ++db)
+                state.out[db] = mma(half, __builtin_bit_cast(uint4, j == 0 ? first[db] : second[db]), rest, state.out[db]);
+        }
     }
     if constexpr (NEXT) next = upcoming;
 }
 
-template <bool NEXT, class Half>
+template <bool NEXT, bool WIDE = false, class Half>
 SINGE_DEVICE void finish_block(Half half, RowState& state, f32x16_t& s, float factor, float shift, const unsigned char* values,
                                const ReadOffsets& offsets, f32x16_t& next, const uint4 (&q)[kSteps], const unsigned char* next_keys) {
     uint4 operand[kSteps];
-    finish_block<NEXT, false>(half, state, s, factor, shift, values, offsets, next, q, next_keys, operand, next_keys);
+    finish_block<NEXT, false, WIDE>(half, state, s, factor, shift, values, offsets, next, q, next_keys, operand, next_keys);
 }
 
 // The stages of a tile's iteration, as the tile functions below take them.  The functions' pointer
@@ -229,7 +244,7 @@ SINGE_DEVICE void loads_landed() { __builtin_amdgcn_s_waitcnt(0x0F70); }  // vmc
 //   shape(scores, which)   turns the raw scores of the tile's first (which = 0) or second block into what the softmax
 //                          takes (a score cap, an added mask) before they are folded; the caller then passes the
 //                          factor that is left to apply (1 when shape did the scaling).
-template <bool AHEAD, class Half, class Issue, class Shape>
+template <bool AHEAD, bool WIDE = false, class Half, class Issue, class Shape>
 SINGE_DEVICE void fold_interior_tile(Half half, RowState& state, f32x16_t& scores, uint4 (&operand)[kSteps], const uint4 (&q)[kSteps],
                                      const ReadOffsets& offsets, unsigned int hi, float factor, const unsigned char* __restrict__ keys,
                                      const unsigned char* __restrict__ next_keys, const unsigned char* __restrict__ values,
@@ -241,21 +256,21 @@ SINGE_DEVICE void fold_interior_tile(Half half, RowState& state, f32x16_t& score
     __builtin_amdgcn_s_setprio(0);
     shape(scores, 0u);
     const float shift_even = begin_block(state, scores, hi, factor, false, [](unsigned int) { return false; });
-    finish_block<true, AHEAD>(half, state, scores, factor, shift_even, values, offsets, scores, q, keys + kBlockBytes, operand, next_keys);
+    finish_block<true, AHEAD, WIDE>(half, state, scores, factor, shift_even, values, offsets, scores, q, keys + kBlockBytes, operand, next_keys);
     __builtin_amdgcn_sched_barrier(0);  // keeps the second block's operand reads out of the first block's registers
     shape(scores, 1u);
     const float shift_odd = begin_block(state, scores, hi, factor, false, [](unsigned int) { return false; });
-    finish_block<true, AHEAD>(half, state, scores, factor, shift_odd, values + kBlockBytes, offsets, scores, q, next_keys, operand,
-                              next_keys + kBlockBytes);
+    finish_block<true, AHEAD, WIDE>(half, state, scores, factor, shift_odd, values + kBlockBytes, offsets, scores, q, next_keys, operand,
+                                    next_keys + kBlockBytes);
 }
 
-template <bool AHEAD, class Half, class Issue>
+template <bool AHEAD, bool WIDE = false, class Half, class Issue>
 SINGE_DEVICE void fold_interior_tile(Half half, RowState& state, f32x16_t& scores, uint4 (&operand)[kSteps], const uint4 (&q)[kSteps],
                                      const ReadOffsets& offsets, unsigned int hi, float factor, const unsigned char* __restrict__ keys,
                                      const unsigned char* __restrict__ next_keys, const unsigned char* __restrict__ values,
                                      unsigned char* __restrict__ key_dest, unsigned char* __restrict__ value_dest, Issue&& issue) {
-    fold_interior_tile<AHEAD>(half, state, scores, operand, q, offsets, hi, factor, keys, next_keys, values, key_dest, value_dest, issue,
-                              [](f32x16_t&, unsigned int) {});
+    fold_interior_tile<AHEAD, WIDE>(half, state, scores, operand, q, offsets, hi, factor, keys, next_keys, values, key_dest, value_dest, issue,
+                                    [](f32x16_t&, unsigned int) {});
 }
 
 // The K operands of the block at `keys`.

@@ -15,8 +15,9 @@
 //                                  fixes the V^T read pattern.
 //
 // Probabilities are rounded to bf16 for the second product and summed unrounded, like the reference's
-// tensor-core kernel (singe/src/backend/cuda/kernel_plan/source/tensor_core.rs:112-194).  The loop that
-// uses these is in prefill_blocks.hip.h.
+// tensor-core kernel (singe/src/backend/cuda/kernel_plan/source/tensor_core.rs:112-194); packed sequences, whose
+// reference keeps f32 weights, take each as the sum of two 16-bit values (split_pair).  The loop that uses these is in
+// prefill_blocks.hip.h.
 #pragma once
 
 #include "common.hip.h"
@@ -89,6 +90,24 @@ SINGE_DEVICE unsigned int pack_pair(F16, float lo, float hi) {
     return __builtin_bit_cast(unsigned int, __builtin_convertvector(both, f16x2v_t));
 }
 SINGE_DEVICE unsigned int pack_pair(float lo, float hi) { return pack_pair(Bf16{}, lo, hi); }
+
+// Two weights as two 16-bit values each: `rounded`, and in `rest` what the rounding left out, rounded in turn.  Together
+// they are within 2^-18 of a bf16 weight and 2^-22 of an f16 one.  An f16 weight is first scaled by kWideScale (no weight
+// is above 2^kMaxLag, so none overflows), without which the rest of a small weight would underflow; the accumulators then
+// hold sums that are kWideScale too large.
+template <class Half>
+constexpr float kWideScale = std::is_same<Half, F16>::value ? 512.0f : 1.0f;
+SINGE_DEVICE void split_pair(Bf16 half, float lo, float hi, unsigned int& rounded, unsigned int& rest) {
+    rounded = pack_pair(half, lo, hi);
+    rest = pack_pair(half, lo - __builtin_bit_cast(float, rounded << 16), hi - __builtin_bit_cast(float, rounded & 0xffff0000u));
+}
+SINGE_DEVICE void split_pair(F16 half, float lo, float hi, unsigned int& rounded, unsigned int& rest) {
+    lo *= kWideScale<F16>;
+    hi *= kWideScale<F16>;
+    rounded = pack_pair(half, lo, hi);
+    const f16x2v_t back = __builtin_bit_cast(f16x2v_t, rounded);
+    rest = pack_pair(half, lo - static_cast<float>(back.x), hi - static_cast<float>(back.y));
+}
 
 // D = A . B + C on the matrix core: 32 x 32 outputs, sixteen values of the contracted index per lane pair.
 SINGE_DEVICE f32x16_t mma(Bf16, uint4 a, uint4 b, f32x16_t c) {

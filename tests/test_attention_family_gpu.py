@@ -266,3 +266,45 @@ def test_packed_sequences_that_overlap_leave_the_last_owner(kv_heads, rows_per_w
         want, _ = oracle.ragged_kv_prefill_attention_f32(host(q)[:, heads_of], host(k)[:, kv_of], host(v)[:, kv_of], lens, keys, offsets,
                                                          causal=False, scale=0.125)
         close(out[:, heads_of], want, torch.bfloat16)
+
+
+def packed_reference_f64(q, k, v, lens, causal, scale):
+    """ragged_kv_prefill_attention of non-overlapping sequences in float64 on the CPU: (out, natural-log lse)."""
+    q, k, v = (x.double().cpu() for x in (q, k, v))
+    group, at = q.shape[1] // k.shape[1], 0
+    out, lse = torch.zeros_like(q), torch.zeros(q.shape[:2], dtype=torch.float64)
+    for n in lens:
+        of = slice(at, at + n)
+        rows, keys, values = (x[of].transpose(0, 1) for x in (q, k.repeat_interleave(group, 1), v.repeat_interleave(group, 1)))
+        scores = rows @ keys.transpose(1, 2).contiguous() * scale
+        if causal:
+            scores = scores.masked_fill(torch.arange(n)[None, :] > torch.arange(n)[:, None], -float("inf"))
+        lse[of] = torch.logsumexp(scores, -1).transpose(0, 1)
+        out[of] = (torch.softmax(scores, -1) @ values).transpose(0, 1)
+        at += n
+    return out, lse
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("head_dim", [128, 80, 16])
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("steepness,mean", [(1.0, 0.0), (8.0, 0.0), (3.0, 1.0)])   # flat to steep weights, values with a mean
+def test_packed_prefill_weighs_values_in_f32(dtype, head_dim, causal, steepness, mean):
+    # The weights reach the values with f32's precision, so that the output's own rounding is all the error there is:
+    # 16-bit weights, rounded as coarsely as the output, would make it about 1.4 times as large.
+    lens, heads, kv_heads = [1, 33, 64, 130, 700], 4, 2
+    tokens = sum(lens)
+    q, k, v = (normal((tokens, h, head_dim), dtype, seed) for h, seed in ((heads, 30), (kv_heads, 31), (kv_heads, 32)))
+    v = v + mean
+    out = torch.full_like(q, float("nan"))
+    lse = torch.full((tokens, heads), float("nan"), device="cuda")
+    scale = steepness * head_dim ** -0.5
+    config = A.RaggedKvPrefillAttentionConfig.contiguous(len(lens), tokens, tokens, heads, kv_heads, head_dim, causal, scale)
+    index = lambda values: torch.tensor(np.asarray(values), dtype=torch.int32, device="cuda")
+    call = A.ragged_kv_prefill_attention_bf16 if dtype == torch.bfloat16 else A.ragged_kv_prefill_attention_f16
+    call(None, out, lse, q, k, v, index(lens), index(lens), index(np.concatenate([[0], np.cumsum(lens)[:-1]])), config)
+    want, want_lse = packed_reference_f64(q, k, v, lens, causal, scale)
+    error, rounding = (out.double().cpu() - want).norm().item(), (want.to(dtype).double() - want).norm().item()
+    assert error <= 1.03 * rounding, (error, rounding)
+    # a score is head_dim products (absolute values of 0.64 on average, less than 1 in any row here) summed in f32
+    assert (lse.double().cpu() - want_lse).abs().max().item() <= head_dim * 2.0**-24 * head_dim * scale + 1e-5
