@@ -270,7 +270,7 @@ int32_t prefill(void* stream, uint16_t* out, size_t out_len, float* lse, size_t 
     args.kv_heads = static_cast<uint32_t>(c.kv_heads);
     constexpr size_t kTileRows = 32 * kDensePrefillWaves;
     args.query_tiles = static_cast<uint32_t>((c.query_len + kTileRows - 1) / kTileRows);
-    args.scale_log2e = c.scale * 1.4426950408889634074f;
+    args.scale_log2e = logit_factor(c.scale);
     args.sinks = options.sinks;
     args.key_lengths = options.key_lengths;
     const bool with_options = options.mask != nullptr || options.window >= 0 || options.softcap != 0.0f;

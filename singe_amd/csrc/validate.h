@@ -3,6 +3,9 @@
 // (ensure_len_at_least).
 #pragma once
 
+#include <cmath>
+#include <cfloat>
+
 #include <stddef.h>
 #include <stdint.h>
 
@@ -15,6 +18,14 @@ inline bool fits_i32(uint64_t value) { return value <= 0x7fffffffull; }
 
 inline bool checked_mul(size_t a, size_t b, size_t* out) { return !__builtin_mul_overflow(a, b, out); }
 inline bool checked_add(size_t a, size_t b, size_t* out) { return !__builtin_add_overflow(a, b, out); }
+
+// The factor that turns a score into a base-two logit.  The row-tile kernels hide a key by making its score -inf and apply
+// the factor afterwards, so it is never zero: a scale of zero becomes the smallest factor there is, under which every
+// visible key still weighs the same (2^(s * 2^-126) is 1 for any score below 2^100).
+inline float logit_factor(float scale) {
+    const float factor = scale * 1.4426950408889634074f;
+    return std::fabs(factor) < FLT_MIN ? std::copysign(FLT_MIN, factor) : factor;
+}
 
 inline int32_t ensure_len_at_least(const char* name, size_t actual, size_t minimum) {
     if (actual < minimum) return fail(SINGE_HIP_LENGTH_TOO_SHORT, name, minimum, actual);
