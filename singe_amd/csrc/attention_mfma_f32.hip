@@ -20,13 +20,23 @@
 // What bounds it: the f32 matrix rate (256 flop a cycle and compute unit) where a call fills the chip; below that, how
 // long a lone wave takes to walk its row tile's keys.  So a row tile's blocks are dealt out over 1, 2, 4 or 8 waves of its
 // workgroup (key_waves, chosen by the host so that the launch fills the SIMDs), which merge their states through LDS, and
-// small calls take 16-row tiles, which are twice as many.  Measured: see dense_f32_matrix in fmha_prefill.cpp, where both
+// small calls take 16-row tiles, which are twice as many.  With 32 rows at head_dim 96 and 128 a wave is alone on its SIMD,
+// so what it adds up between its products (see mma_f32) is time of its own.  Measured: see dense_f32_matrix in fmha_prefill.cpp, where both
 // are chosen.
 #include "common.hip.h"
 #include "kernel_args.h"
 
 namespace {
 
+// Sums of f32 products: a running sum of n terms of either sign carries a rounding error that grows with sqrt(n), and a
+// score's goes into its weight whole.  So a chain of products covers 4 dims of a score up to head_dim 64 (16 rows), 8 or (32
+// rows, 96 and up) 16, partial sums meeting in pairs, and 8 or 16 keys of the values: every 32-key block starts two or four
+// new sums, which are added to the running ones.  Error against float64, of the norm, and time, with one chain a score and
+// one a row's values / as it is / on the row kernels with their per-lane sums:
+//   1 x 8 x 512 x 64 causal         2.4e-7  10.3 us  /  1.20e-7  11.3 us  /  1.23e-7   38 us
+//   1 x 8 x 512 x 128 causal        3.1e-7  18.8 us  /  1.30e-7  18.8 us  /  1.34e-7   53 us
+//   4 x 12 x 1024 x 64              4.2e-7   156 us  /  1.71e-7   142 us  /  2.07e-7  1140 us
+//   4 x 12 x 1024 x 128             5.8e-7   240 us  /  1.87e-7   280 us  /  2.20e-7  1740 us
 SINGE_DEVICE f32x16_t mma_f32(float a, float b, f32x16_t c) { return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0); }
 SINGE_DEVICE f32x4_t mma_f32(float a, float b, f32x4_t c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 
@@ -75,12 +85,59 @@ SINGE_DEVICE void store_dims(float* at, const float (&value)[N]) {
     }
 }
 
+// Scores of chunks FIRST .. FIRST + COUNT - 1 (of 64 / ROWS lane groups' four dims each): chains of CHAIN products (1, 2, or
+// those of whole chunks), summed in pairs.  TIGHT: registers are short, so that the sums must not all be alive at once.
+template <int FIRST, int COUNT, int CHAIN, bool TIGHT, class Tile, int TILES, int CHUNKS>
+SINGE_DEVICE void score_chunks(Tile (&s)[TILES], const float4 (&k)[TILES][CHUNKS], const float4 (&q)[CHUNKS]) {
+    Tile zero;
+#pragma unroll
+    for (int r = 0; r < static_cast<int>(sizeof(Tile) / 4); ++r) zero[r] = 0.0f;
+    if constexpr (4 * COUNT <= CHAIN) {
+#pragma unroll
+        for (int t = FIRST; t < FIRST + COUNT; ++t) {
+#pragma unroll
+            for (int kt = 0; kt < TILES; ++kt) s[kt] = mma_f32(k[kt][t].x, q[t].x, t == FIRST ? zero : s[kt]);
+#pragma unroll
+            for (int kt = 0; kt < TILES; ++kt) s[kt] = mma_f32(k[kt][t].y, q[t].y, s[kt]);
+#pragma unroll
+            for (int kt = 0; kt < TILES; ++kt) s[kt] = mma_f32(k[kt][t].z, q[t].z, s[kt]);
+#pragma unroll
+            for (int kt = 0; kt < TILES; ++kt) s[kt] = mma_f32(k[kt][t].w, q[t].w, s[kt]);
+        }
+    } else if constexpr (COUNT > 1) {
+        Tile more[TILES];
+        score_chunks<FIRST, COUNT / 2, CHAIN, TIGHT>(s, k, q);
+        score_chunks<FIRST + COUNT / 2, COUNT - COUNT / 2, CHAIN, TIGHT>(more, k, q);
+#pragma unroll
+        for (int kt = 0; kt < TILES; ++kt) s[kt] += more[kt];
+        if constexpr (TIGHT) __builtin_amdgcn_sched_barrier(0);
+    } else {
+#pragma unroll
+        for (int kt = 0; kt < TILES; ++kt) {
+            const Tile x = mma_f32(k[kt][FIRST].x, q[FIRST].x, zero), y = mma_f32(k[kt][FIRST].y, q[FIRST].y, CHAIN > 1 ? x : zero);
+            const Tile z = mma_f32(k[kt][FIRST].z, q[FIRST].z, zero), w = mma_f32(k[kt][FIRST].w, q[FIRST].w, CHAIN > 1 ? z : zero);
+            if constexpr (CHAIN > 1) s[kt] = y + w;
+            else s[kt] = (x + y) + (z + w);
+        }
+    }
+}
+
+// The sum of values FIRST .. FIRST + COUNT - 1 of a tile, in pairs.
+template <int FIRST, int COUNT, class Tile>
+SINGE_DEVICE float tile_sum(const Tile& s) {
+    if constexpr (COUNT == 1) return s[FIRST];
+    else return tile_sum<FIRST, COUNT / 2>(s) + tile_sum<FIRST + COUNT / 2, COUNT - COUNT / 2>(s);
+}
+
 template <int D, int ROWS, int WAVES>
 SINGE_DEVICE void attention_mfma_f32_body(const PrefillF32Args& a, float* lds) {
     constexpr int kLaneGroups = 64 / ROWS;
     constexpr int kDimBlocks = D / ROWS, kChunks = D / (4 * kLaneGroups);  // ROWS-dim blocks of O^T; 16-byte chunks a lane holds of a row
     constexpr int kRegs = ROWS * ROWS / 64, kKeyTiles = 32 / ROWS;         // of a score tile; score tiles of a 32-key block
     typedef std::conditional_t<ROWS == 32, f32x16_t, f32x4_t> Tile;
+    // Products to a chain of a score, of 64 / ROWS dims each, and sums that a block's keys are dealt out to (see mma_f32).
+    constexpr int kScoreChain = ROWS == 16 ? (D <= 64 ? 1 : 2) : (D <= 64 ? 4 : 8), kValueSums = ROWS == 16 && D <= 64 ? 4 : 2;
+    constexpr bool kTight = WAVES == 8;
     const unsigned int lane = threadIdx.x & 63u;
     const unsigned int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const unsigned int column = lane % ROWS, lane_group = lane / ROWS;
@@ -121,11 +178,16 @@ SINGE_DEVICE void attention_mfma_f32_body(const PrefillF32Args& a, float* lds) {
 
     const float* const keys = a.key + batch * a.key_batch_stride + kv_head * a.key_head_stride + 4u * lane_group;
     const float* const values = a.value + batch * a.value_batch_stride + kv_head * a.value_head_stride + column * kDimBlocks;
+    // The scale stays out of the scores and goes into the exponent's multiply-add; a negative one moves its sign into Q.
+    const float factor = fabsf(a.scale_log2e), sign = a.scale_log2e < 0.0f ? -1.0f : 1.0f;
     float4 q[kChunks];
     {
         const float* at = a.query + batch * a.query_batch_stride + static_cast<size_t>(row) * a.query_sequence_stride + head * a.query_head_stride + 4u * lane_group;
 #pragma unroll
-        for (int t = 0; t < kChunks; ++t) q[t] = *reinterpret_cast<const float4*>(at + 4 * kLaneGroups * t);
+        for (int t = 0; t < kChunks; ++t) {
+            q[t] = *reinterpret_cast<const float4*>(at + 4 * kLaneGroups * t);
+            q[t].x *= sign; q[t].y *= sign; q[t].z *= sign; q[t].w *= sign;
+        }
     }
 
     Tile out[kDimBlocks];
@@ -159,26 +221,10 @@ SINGE_DEVICE void attention_mfma_f32_body(const PrefillF32Args& a, float* lds) {
                 load_dims(values + static_cast<size_t>(key) * a.value_sequence_stride, v[kt][r]);
             }
         Tile s[kKeyTiles];
+        score_chunks<0, kChunks, kScoreChain, kTight>(s, k, q);
 #pragma unroll
-        for (int kt = 0; kt < kKeyTiles; ++kt)
-#pragma unroll
-            for (int r = 0; r < kRegs; ++r) s[kt][r] = 0.0f;
-#pragma unroll
-        for (int t = 0; t < kChunks; ++t) {
-#pragma unroll
-            for (int kt = 0; kt < kKeyTiles; ++kt) s[kt] = mma_f32(k[kt][t].x, q[t].x, s[kt]);
-#pragma unroll
-            for (int kt = 0; kt < kKeyTiles; ++kt) s[kt] = mma_f32(k[kt][t].y, q[t].y, s[kt]);
-#pragma unroll
-            for (int kt = 0; kt < kKeyTiles; ++kt) s[kt] = mma_f32(k[kt][t].z, q[t].z, s[kt]);
-#pragma unroll
-            for (int kt = 0; kt < kKeyTiles; ++kt) s[kt] = mma_f32(k[kt][t].w, q[t].w, s[kt]);
-        }
+        for (int kt = 0; kt < kKeyTiles; ++kt) asm volatile("" : "+v"(s[kt]));  // (summed here, not after the loads below)
         if (block + key_waves < end_block) load_keys(block + key_waves);
-#pragma unroll
-        for (int kt = 0; kt < kKeyTiles; ++kt)
-#pragma unroll
-            for (int r = 0; r < kRegs; ++r) s[kt][r] *= a.scale_log2e;
         if (block < whole_begin || block >= whole_end) {
             asm volatile("");  // keeps this a branch: as selects it would be paid in every block
 #pragma unroll
@@ -194,7 +240,7 @@ SINGE_DEVICE void attention_mfma_f32_body(const PrefillF32Args& a, float* lds) {
         for (int kt = 0; kt < kKeyTiles; ++kt)
 #pragma unroll
             for (int r = 0; r < kRegs; ++r) most = fmaxf(most, s[kt][r]);
-        most = row_max<ROWS>(most);
+        most = row_max<ROWS>(most) * factor;
         if (__any(most > largest)) {
             const float moved = fmaxf(largest, most), base = moved == -INFINITY ? 0.0f : moved;
             const float rescale = fast_exp2(largest - base);
@@ -210,15 +256,33 @@ SINGE_DEVICE void attention_mfma_f32_body(const PrefillF32Args& a, float* lds) {
         for (int kt = 0; kt < kKeyTiles; ++kt)
 #pragma unroll
             for (int r = 0; r < kRegs; ++r) {
-                s[kt][r] = fast_exp2(s[kt][r] - base);
-                total += s[kt][r];
+                s[kt][r] = fast_exp2(fmaf(s[kt][r], factor, -base));
             }
+        if constexpr (ROWS == 16) total += tile_sum<0, kRegs>(s[0]) + tile_sum<0, kRegs>(s[kKeyTiles - 1]);
+        else total += tile_sum<0, kRegs>(s[0]);
+        constexpr int kSumKeys = kKeyTiles * kRegs / kValueSums;  // products of each of the block's sums
+        Tile ready;
 #pragma unroll
-        for (int kt = 0; kt < kKeyTiles; ++kt)
+        for (int db = 0; db < kDimBlocks; ++db) {
+            Tile part[kValueSums];
 #pragma unroll
-            for (int r = 0; r < kRegs; ++r)
+            for (int h = 0; h < kValueSums; ++h)
 #pragma unroll
-                for (int db = 0; db < kDimBlocks; ++db) out[db] = mma_f32(v[kt][r][db], s[kt][r], out[db]);
+                for (int r = 0; r < kRegs; ++r) part[h][r] = 0.0f;
+            if constexpr (kTight) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < kSumKeys; ++i)
+#pragma unroll
+                for (int h = 0; h < kValueSums; ++h) {
+                    const int at = h * kSumKeys + i, kt = at / kRegs, r = at % kRegs;
+                    part[h] = mma_f32(v[kt][r][db], s[kt][r], part[h]);
+                }
+            // (the sums are added while the next dim block's products run)
+            if (db > 0) out[db - 1] += ready;
+            if constexpr (kValueSums == 4) ready = (part[0] + part[1]) + (part[2] + part[3]);
+            else ready = part[0] + part[1];
+        }
+        out[kDimBlocks - 1] += ready;
     }
     total = row_sum<ROWS>(total);
 
@@ -228,7 +292,7 @@ SINGE_DEVICE void attention_mfma_f32_body(const PrefillF32Args& a, float* lds) {
     // A row that sees no key stays zero; its log-sum-exp is ln 0.
     auto store_lse = [&](float reference, float sum) __attribute__((always_inline)) {
         if (a.lse != nullptr && stored && lane_group == 0)
-            a.lse[(static_cast<size_t>(batch) * a.heads + head) * a.query_len + row] = sum > 0.0f ? (reference + log2f(sum)) * kLn2 : -INFINITY;
+            a.lse[(static_cast<size_t>(batch) * a.heads + head) * a.query_len + row] = sum > 0.0f ? fmaf(reference, kLn2, log2f(sum) * kLn2) : -INFINITY;
     };
     if (key_waves == 1) {
         const float inverse = total > 0.0f ? 1.0f / total : 0.0f;

@@ -166,7 +166,7 @@ bool dense_f32_matrix_takes(const PrefillF32Args& a) {
 }
 
 int32_t dense_f32_matrix(void* stream, PrefillF32Args& a) {
-    a.scale_log2e = a.scale * 1.4426950408889634074f;
+    a.scale_log2e = logit_factor(a.scale);
     // 16-row tiles where 32-row ones are too few for the chip (up to 5/8 of a tile a compute unit; at head_dim 32 always, where
     // a wave's loads and softmax weigh more than its products), and a tile's keys over as many waves as leave the SIMDs two to
     // four waves each.  Measured in us (B x H x L, causal; 16 rows with 1 / 2 / 4 / 8 waves, then 32 rows with 1 / 2 / 4 / 8):
