@@ -25,6 +25,7 @@
 // are chosen.
 #include "common.hip.h"
 #include "kernel_args.h"
+#include "row_alone.hip.h"
 
 namespace {
 
@@ -128,6 +129,19 @@ SINGE_DEVICE float tile_sum(const Tile& s) {
     if constexpr (COUNT == 1) return s[FIRST];
     else return tile_sum<FIRST, COUNT / 2>(s) + tile_sum<FIRST + COUNT / 2, COUNT - COUNT / 2>(s);
 }
+
+// A row of the problem, for row_alone.
+struct DenseF32Row {
+    const float* query_row;
+    const float* keys;    // of the batch entry and kv head
+    const float* values;
+    size_t key_stride, value_stride;
+    float* out_row;
+    SINGE_DEVICE float query(unsigned int d) const { return query_row[d]; }
+    SINGE_DEVICE float key(unsigned int k, unsigned int d) const { return keys[k * key_stride + d]; }
+    SINGE_DEVICE float value(unsigned int k, unsigned int d) const { return values[k * value_stride + d]; }
+    SINGE_DEVICE void store(unsigned int d, float value) const { out_row[d] = value; }
+};
 
 template <int D, int ROWS, int WAVES>
 SINGE_DEVICE void attention_mfma_f32_body(const PrefillF32Args& a, float* lds) {
@@ -294,9 +308,23 @@ SINGE_DEVICE void attention_mfma_f32_body(const PrefillF32Args& a, float* lds) {
         if (a.lse != nullptr && stored && lane_group == 0)
             a.lse[(static_cast<size_t>(batch) * a.heads + head) * a.query_len + row] = sum > 0.0f ? fmaf(reference, kLn2, log2f(sum) * kLn2) : -INFINITY;
     };
+    // Rows of the tile (bit r: row r) whose sums a value that is not finite has spoilt: worked out by themselves.
+    const unsigned long long spoiled = __builtin_amdgcn_ballot_w64(stored && not_finite(kRegs * kDimBlocks, [&](int i) { return out[i / kRegs][i % kRegs]; }));
+    unsigned int alone = static_cast<unsigned int>(spoiled | spoiled >> 32);
+    if constexpr (ROWS == 16) alone = (alone | alone >> 16) & 0xffffu;
+    auto redo = [&](unsigned int rows) __attribute__((always_inline)) {
+        for (; rows != 0; rows &= rows - 1u) {
+            const unsigned int own = first_row + static_cast<unsigned int>(__builtin_ctz(rows));
+            row_alone<D>(DenseF32Row{a.query + batch * a.query_batch_stride + static_cast<size_t>(own) * a.query_sequence_stride + head * a.query_head_stride,
+                                     a.key + batch * a.key_batch_stride + kv_head * a.key_head_stride,
+                                     a.value + batch * a.value_batch_stride + kv_head * a.value_head_stride, a.key_sequence_stride, a.value_sequence_stride,
+                                     a.out + batch * a.output_batch_stride + static_cast<size_t>(own) * a.output_sequence_stride + head * a.output_head_stride},
+                         lowest(own), end_of(own), a.scale_log2e);
+        }
+    };
     if (key_waves == 1) {
         const float inverse = total > 0.0f ? 1.0f / total : 0.0f;
-        if (stored) {
+        if (stored && ((alone >> column) & 1u) == 0) {
 #pragma unroll
             for (int r = 0; r < kRegs; ++r) {
                 float value[kDimBlocks];
@@ -306,6 +334,7 @@ SINGE_DEVICE void attention_mfma_f32_body(const PrefillF32Args& a, float* lds) {
             }
         }
         store_lse(largest, total);
+        redo(alone);
         return;
     }
     // The row tile's waves leave their states in LDS, and each merges and stores a share of the accumulator registers.
@@ -317,7 +346,11 @@ SINGE_DEVICE void attention_mfma_f32_body(const PrefillF32Args& a, float* lds) {
         for (int db = 0; db < kDimBlocks; ++db) mine[64 * (r * kDimBlocks + db)] = out[db][r];
     mine[64 * kRegs * kDimBlocks] = largest;
     mine[64 * (kRegs * kDimBlocks + 1)] = total;
+    unsigned int* const alone_of = reinterpret_cast<unsigned int*>(lds + WAVES * kSlot);  // a word a wave
+    if (lane == 0) alone_of[row_wave * key_waves + key_wave] = alone;
     __syncthreads();
+    for (unsigned int w = 0; w < key_waves; ++w) alone |= alone_of[row_wave * key_waves + w];
+    alone = __builtin_amdgcn_readfirstlane(alone);
     const float* const tile = lds + row_wave * key_waves * kSlot + lane;
     float reference = -INFINITY;
     for (unsigned int w = 0; w < key_waves; ++w) reference = fmaxf(reference, tile[w * kSlot + 64 * kRegs * kDimBlocks]);
@@ -336,9 +369,13 @@ SINGE_DEVICE void attention_mfma_f32_body(const PrefillF32Args& a, float* lds) {
         }
 #pragma unroll
         for (int db = 0; db < kDimBlocks; ++db) value[db] *= inverse;
-        if (stored) store(static_cast<int>(r), value);
+        if (stored && ((alone >> column) & 1u) == 0) store(static_cast<int>(r), value);
     }
     if (key_wave == 0) store_lse(reference, sum);
+    // (row r of the tile falls to wave r % key_waves)
+    unsigned int share = 0;
+    for (unsigned int r = key_wave; r < ROWS; r += key_waves) share |= 1u << r;
+    redo(alone & share);
 }
 
 }  // namespace
@@ -346,7 +383,7 @@ SINGE_DEVICE void attention_mfma_f32_body(const PrefillF32Args& a, float* lds) {
 // From head_dim 96 on a 32-row wave needs more than half a SIMD's registers: four waves a workgroup, one a SIMD.
 #define SINGE_ATTENTION_MFMA_F32_KERNEL(DIM, ROWS, WAVES)                                                                 \
     extern "C" __global__ __launch_bounds__(64 * WAVES, WAVES / 4) void singe_attention_mfma_f32_d##DIM##_r##ROWS(PrefillF32Args args) { \
-        __shared__ float lds[WAVES * (ROWS * DIM + 128)];                                                                 \
+        __shared__ float lds[WAVES * (ROWS * DIM + 128 + 1)];                                                                 \
         attention_mfma_f32_body<DIM, ROWS, WAVES>(args, lds);                                                             \
     }
 

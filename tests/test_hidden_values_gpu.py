@@ -36,7 +36,7 @@ def visible_only(q, k, v, first, end, scale):
 def same(out, want, dtype):
     out = out.double().cpu()
     finite = want.isfinite()
-    assert (out[finite] - want[finite]).abs().max().item() <= TOL[dtype]
+    assert ((out[finite] - want[finite]).abs() <= TOL[dtype]).all()
     assert (out.isnan() == want.isnan()).all() and (out[want.isinf()] == want[want.isinf()]).all()
 
 
@@ -62,3 +62,27 @@ def test_packed(dtype, dim, causal, bad):
     first = [start for start, n in zip(offsets, lens) for _ in range(n)]
     end = [start + (i + 1 if causal else n) for start, n in zip(offsets, lens) for i in range(n)]
     same(out, visible_only(q, k, v, first, end, scale), dtype)
+
+
+@pytest.mark.parametrize("dim", [32, 64, 96, 128])
+@pytest.mark.parametrize("batch,heads,length,window", [
+    (1, 6, 200, 0), (1, 6, 200, 17),       # 16-row tiles, whose keys several waves share
+    (14, 64, 65, 0), (14, 64, 65, 9),      # 32-row tiles, two waves a tile
+    (70, 64, 30, 0),                       # 32-row tiles from head_dim 64 on, a wave a tile
+])
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("bad", [INF, NAN])
+def test_dense_f32(dim, batch, heads, length, window, causal, bad):
+    scale = dim ** -0.5
+    q, k, v = (draw(seed, batch, length, h, dim) for seed, h in ((1, heads), (2, heads // 2), (3, heads // 2)))
+    v[:, length // 2, 0, 3] = bad           # inside a block that the rows before it share
+    v[:, length - 1, -1, dim - 1] = -bad    # the last key, which the keys past it re-read
+    k[:, length // 2 + 3, -1] = NAN
+    out = torch.full_like(q, 7.0).cuda()
+    config = A.FmhaPrefillConfig.contiguous(batch, length, length, heads, heads // 2, dim, scale, causal)
+    A.softcapped_window_attention_f32(None, out, q.cuda(), k.cuda(), v.cuda(), A.SoftcappedWindowAttentionConfig(config, window, None))
+    first = [max(0, i - window) if window else 0 for i in range(length)]
+    end = [min(length, i + 1 if causal else i + window + 1 if window else length) for i in range(length)]
+    for b, of in ((0, slice(0, 2)), (batch - 1, slice(heads - 2, heads))):
+        kv = slice(of.start // 2, of.start // 2 + 1)
+        same(out[b, :, of], visible_only(q[b, :, of], k[b, :, kv], v[b, :, kv], first, end, scale), torch.float32)
