@@ -20,7 +20,8 @@
 // What bounds it: the f32 matrix rate (256 flop a cycle and compute unit) where a call fills the chip; below that, how
 // long a lone wave takes to walk its row tile's keys.  So a row tile's blocks are dealt out over 1, 2, 4 or 8 waves of its
 // workgroup (key_waves, chosen by the host so that the launch fills the SIMDs), which merge their states through LDS, and
-// small calls take 16-row tiles, which are twice as many.  With 32 rows at head_dim 96 and 128 a wave is alone on its SIMD,
+// small calls take 16-row tiles, which are twice as many, and fewer of them to a workgroup (row_waves) while compute units
+// would be idle: waves on one SIMD take turns at its matrix core.  With 32 rows at head_dim 96 and 128 a wave is alone on its SIMD,
 // so what it adds up between its products (see mma_f32) is time of its own.  Measured: see dense_f32_matrix in fmha_prefill.cpp, where both
 // are chosen.
 #include "common.hip.h"
@@ -150,14 +151,14 @@ SINGE_DEVICE void attention_mfma_f32_body(const PrefillF32Args& a, float* lds) {
     constexpr int kRegs = ROWS * ROWS / 64, kKeyTiles = 32 / ROWS;         // of a score tile; score tiles of a 32-key block
     typedef std::conditional_t<ROWS == 32, f32x16_t, f32x4_t> Tile;
     // Products to a chain of a score, of 64 / ROWS dims each, and sums that a block's keys are dealt out to (see mma_f32).
-    constexpr int kScoreChain = ROWS == 16 ? (D <= 64 ? 1 : 2) : (D <= 64 ? 4 : 8), kValueSums = ROWS == 16 && D <= 64 ? 4 : 2;
+    constexpr int kScoreChain = ROWS == 16 ? (D <= 64 ? 1 : 2) : (D <= 64 ? 4 : 8), kValueSums = ROWS == 16 && D == 64 ? 4 : 2;
     constexpr bool kTight = WAVES == 8;
     const unsigned int lane = threadIdx.x & 63u;
     const unsigned int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const unsigned int column = lane % ROWS, lane_group = lane / ROWS;
     // Row of an accumulator tile (key of a score tile, dim block of an output tile) that register r holds.
     auto tile_row = [&](int r) __attribute__((always_inline)) { return ROWS == 32 ? 8u * (r >> 2) + 4u * lane_group + (r & 3) : 4u * lane_group + r; };
-    const unsigned int key_waves = a.key_waves, row_waves = WAVES / key_waves;
+    const unsigned int key_waves = a.key_waves, row_waves = a.row_waves;
     const unsigned int key_wave = wave % key_waves, row_wave = wave / key_waves;
 
     // Workgroup -> (batch, head), row tiles: heads side by side (neighbouring workgroups go to different XCDs, and with a

@@ -81,6 +81,19 @@ int32_t validate_call(const SingeFmhaPrefillConfig& c, const void* out, size_t o
     return 0;
 }
 
+// Small calls without shared heads that the row kernel (a workgroup per (batch, query, kv head)) is done with first: a
+// matrix-core wave's one or two blocks take it as long however few rows there are.  Kernel times in us, row / matrix-core
+// kernel (batch x heads x queries x keys):
+//   head_dim 128   1 x 1 x 64 x 64 6.0 / 7.0    1 x 1 x 200 x 200 9.6 / 11.9   1 x 1 x 512 x 512 18.4 / 19.1
+//                  1 x 8 x 64 x 64 7.1 / 7.2    1 x 8 x 100 x 100 10.9 / 9.0   1 x 1 x 64 x 4096 105 / 94
+//   head_dim 64    1 x 1 x 16 x 16 4.0 / 4.2    1 x 1 x 100 x 100  6.1 / 6.0   1 x 8 x 64 x 64 5.7 / 5.6
+// With heads that share their keys the row kernel takes longer the more there are (1 x 8 over 2 x 64 x 64 x 1024: 73 / 32).
+bool rows_f32_is_faster(const PrefillF32Args& a) {
+    if (a.heads != a.kv_heads) return false;
+    const uint64_t rows = static_cast<uint64_t>(a.batch) * a.heads * a.query_len;
+    return (a.head_dim == 128 && rows <= 512 && a.key_len <= 1024) || (a.head_dim == 64 && rows <= 192 && a.key_len <= 64);
+}
+
 int32_t prefill_f32(void* stream, float* out, size_t out_len, float* lse, size_t lse_len, bool with_lse, const float* query,
                     size_t query_len, const float* key, size_t key_len, const float* value, size_t value_len,
                     const SingeFmhaPrefillConfig* config, size_t window_size, bool has_soft_cap, float soft_cap,
@@ -122,7 +135,7 @@ int32_t prefill_f32(void* stream, float* out, size_t out_len, float* lse, size_t
     args.has_soft_cap = has_soft_cap ? 1u : 0u;
     args.soft_cap = soft_cap;
     args.scale = c.scale;
-    if (!has_soft_cap && dense_f32_matrix_takes(args)) {
+    if (!has_soft_cap && !rows_f32_is_faster(args) && dense_f32_matrix_takes(args)) {
         if (window_size > 0) args.look_back = args.look_ahead = static_cast<uint32_t>(window_size);
         if (c.causal) args.look_ahead = 0;
         return dense_f32_matrix(stream, args);
@@ -177,15 +190,18 @@ int32_t dense_f32_matrix(void* stream, PrefillF32Args& a) {
     //                 4 x 8 x 512     91 / 54 / 41 / 47     77 / 45 / 38
     //                 4 x 12 x 1024  185 / 177 / 187 / 213  151 / 149 / 164;  not causal 379 / 301 / 319 / 361  301 / 241 / 260
     //   head_dim 32   4 x 12 x 1024   66 / 48 / 48 / 50    104 / 90 / 64 / 56
-    const uint64_t pairs = static_cast<uint64_t>(a.batch) * a.heads, blocks = (static_cast<uint64_t>(a.key_len) + 31) / 32;
-    const uint32_t rows = a.head_dim == 32 || pairs * ((static_cast<uint64_t>(a.query_len) + 31) / 32) * 8 <= 5ull * compute_units() ? 16 : 32;
+    // A wave without a block of its own costs nothing: 7 blocks on 8 waves take 12.1 us, on 4 waves 18.8 (1 x 8 x 200 x 128).
+    const uint64_t pairs = static_cast<uint64_t>(a.batch) * a.heads, blocks = (static_cast<uint64_t>(a.key_len) + 31) / 32, units = compute_units();
+    const uint32_t rows = a.head_dim == 32 || pairs * ((static_cast<uint64_t>(a.query_len) + 31) / 32) * 8 <= 5 * units ? 16 : 32;
     const uint32_t waves = rows == 16 || a.head_dim <= 64 ? 8 : 4;  // of a workgroup
-    const uint64_t tiles = (static_cast<uint64_t>(a.query_len) + rows - 1) / rows, most = (rows == 16 ? 32ull : 2ull * waves) * compute_units();
+    const uint64_t tiles = (static_cast<uint64_t>(a.query_len) + rows - 1) / rows, most = (rows == 16 ? 32 : 2 * waves) * units;
     a.key_waves = 1;
-    while (a.key_waves < waves && pairs * tiles * a.key_waves < most && 2ull * a.key_waves <= blocks) a.key_waves *= 2;
-    const uint64_t groups = (tiles + waves / a.key_waves - 1) / (waves / a.key_waves);
+    while (a.key_waves < waves && pairs * tiles * a.key_waves < most && a.key_waves < blocks) a.key_waves *= 2;
+    a.row_waves = waves / a.key_waves;
+    while (a.row_waves > 1 && pairs * ((tiles + a.row_waves - 1) / a.row_waves) < units) a.row_waves /= 2;
+    const uint64_t groups = (tiles + a.row_waves - 1) / a.row_waves;
     const int kernel = kAttentionMfmaF32 + static_cast<int>(rows == 16 ? a.head_dim / 32 - 1 : a.head_dim / 32 + 2);
-    return launch(static_cast<KernelId>(kernel), static_cast<unsigned>(pairs * groups), 1, 1, 64 * waves, stream, a);
+    return launch(static_cast<KernelId>(kernel), static_cast<unsigned>(pairs * groups), 1, 1, 64 * a.key_waves * a.row_waves, stream, a);
 }
 
 }  // namespace singe_hip

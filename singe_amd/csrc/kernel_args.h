@@ -133,6 +133,7 @@ struct PrefillF32Args {
     uint32_t look_back = 0xffffffffu, look_ahead = 0xffffffffu;
     const int32_t* key_lengths = nullptr;
     uint32_t key_waves = 1;
+    uint32_t row_waves = 1;         // row tiles of a workgroup, which has key_waves * row_waves waves
 };
 
 struct PagedAttentionArgs {
