@@ -234,56 +234,57 @@ SINGE_DEVICE void fmha_prefill_tile(const PrefillArgs& a, unsigned char* lds, un
     auto fold = [&](unsigned int block, f32x16_t& s, const unsigned char* values) __attribute__((always_inline)) {
         const unsigned int key0 = block * 32u;
         if constexpr (OPTIONS) {
-            // A window alone leaves the scores as they are: their scale stays in the exponent's multiply-add, and only the
-            // blocks that the window's or the mask's edge crosses for some row of the wave look at their keys one by one.
-            if (a.mask == nullptr && a.cap_log2e == 0.0f) {
-                const bool edge = (CAUSAL && key0 + 31u > first_row) || key0 + 32u > key_len || key0 < last_low;
-                const float shift = begin_block(state, s, hi, factor, edge, [&](unsigned int key_in_block) { return key0 + key_in_block - my_low >= my_span; });
-                finish_block<false>(half, state, s, factor, shift, values, offsets, s, q, values);
-                return;
-            }
-            // Scores in their final units (base-two logits): scaled, capped (singe/src/backend/cpu/normalization/
-            // attention.rs:255-262: the cap, then the mask), the mask added.  Register r of lane (query, hi) is key
-            // key0 + 8 (r / 4) + 4 hi + (r % 4).
-            const bool capped = a.cap_log2e != 0.0f;
-            const float to_units = capped ? a.cap_scale : factor;
-            const uint16_t* mask_row = nullptr;
-            if (a.mask != nullptr)
-                mask_row = a.mask + batch * a.mask_strides[0] + head * a.mask_strides[1] + static_cast<size_t>(query_valid ? my_query : 0) * a.mask_strides[2];
-            // The lane's keys come in four runs of four; a run inside the keys is one 8-byte load when the host found
-            // every mask row to start on an 8-byte boundary with its keys side by side.
-            uint16_t mask_bits[16];
-            if (mask_row != nullptr) {
+            // Only the blocks that the window's or the causal mask's edge crosses for some row of the wave look at their keys
+            // one by one.  A window alone leaves the scores as they are: their scale stays in the exponent's multiply-add.
+            // (One fold after the branch, whatever is left to apply: a fold in either branch is two more copies of it in
+            // each of the loops below, which at head_dim 128 spilt 70 registers and cost masks, caps and windows alike.)
+            const bool edge = (CAUSAL && key0 + 31u > first_row) || key0 + 32u > key_len || key0 < last_low;
+            float left = factor;
+            if (a.mask != nullptr || a.cap_log2e != 0.0f) {
+                // Scores in their final units (base-two logits): scaled, capped (singe/src/backend/cpu/normalization/
+                // attention.rs:255-262: the cap, then the mask), the mask added.  Register r of lane (query, hi) is key
+                // key0 + 8 (r / 4) + 4 hi + (r % 4).
+                left = 1.0f;
+                const bool capped = a.cap_log2e != 0.0f;
+                const float to_units = capped ? a.cap_scale : factor;
+                const uint16_t* mask_row = nullptr;
+                if (a.mask != nullptr)
+                    mask_row = a.mask + batch * a.mask_strides[0] + head * a.mask_strides[1] + static_cast<size_t>(query_valid ? my_query : 0) * a.mask_strides[2];
+                // The lane's keys come in four runs of four; a run inside the keys is one 8-byte load when the host found
+                // every mask row to start on an 8-byte boundary with its keys side by side.
+                uint16_t mask_bits[16];
+                if (mask_row != nullptr) {
 #pragma unroll
-                for (int run = 0; run < 4; ++run) {
-                    const unsigned int key = key0 + 8u * run + 4u * hi;
-                    if (a.mask_packed && key + 3u < key_len) {
-                        const uint2 four = *reinterpret_cast<const uint2*>(mask_row + key);
-                        mask_bits[4 * run + 0] = static_cast<uint16_t>(four.x);
-                        mask_bits[4 * run + 1] = static_cast<uint16_t>(four.x >> 16);
-                        mask_bits[4 * run + 2] = static_cast<uint16_t>(four.y);
-                        mask_bits[4 * run + 3] = static_cast<uint16_t>(four.y >> 16);
-                    } else {
+                    for (int run = 0; run < 4; ++run) {
+                        const unsigned int key = key0 + 8u * run + 4u * hi;
+                        if (a.mask_packed && key + 3u < key_len) {
+                            const uint2 four = *reinterpret_cast<const uint2*>(mask_row + key);
+                            mask_bits[4 * run + 0] = static_cast<uint16_t>(four.x);
+                            mask_bits[4 * run + 1] = static_cast<uint16_t>(four.x >> 16);
+                            mask_bits[4 * run + 2] = static_cast<uint16_t>(four.y);
+                            mask_bits[4 * run + 3] = static_cast<uint16_t>(four.y >> 16);
+                        } else {
 #pragma unroll
-                        for (int i = 0; i < 4; ++i)
-                            mask_bits[4 * run + i] = mask_row[static_cast<size_t>(key + i < key_len ? key + i : 0) * a.mask_strides[3]];
+                            for (int i = 0; i < 4; ++i)
+                                mask_bits[4 * run + i] = mask_row[static_cast<size_t>(key + i < key_len ? key + i : 0) * a.mask_strides[3]];
+                        }
                     }
                 }
-            }
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                float x = s[r] * to_units;
-                if (capped) x = fast_tanh(x) * a.cap_log2e;
-                if (mask_row != nullptr) {
-                    float extra;
-                    if constexpr (std::is_same_v<Half, F16>) extra = static_cast<float>(__builtin_bit_cast(_Float16, mask_bits[r]));
-                    else extra = __builtin_bit_cast(float, static_cast<unsigned int>(mask_bits[r]) << 16);
-                    x += extra * kLog2e;
+                for (int r = 0; r < 16; ++r) {
+                    float x = s[r] * to_units;
+                    if (capped) x = fast_tanh(x) * a.cap_log2e;
+                    if (mask_row != nullptr) {
+                        float extra;
+                        if constexpr (std::is_same_v<Half, F16>) extra = static_cast<float>(__builtin_bit_cast(_Float16, mask_bits[r]));
+                        else extra = __builtin_bit_cast(float, static_cast<unsigned int>(mask_bits[r]) << 16);
+                        x += extra * kLog2e;
+                    }
+                    s[r] = x;
                 }
-                s[r] = x;
             }
-            const float shift = begin_block(state, s, hi, 1.0f, true, [&](unsigned int key_in_block) { return key0 + key_in_block - my_low >= my_span; });
-            finish_block<false>(half, state, s, 1.0f, shift, values, offsets, s, q, values);
+            const float shift = begin_block(state, s, hi, left, edge, [&](unsigned int key_in_block) { return key0 + key_in_block - my_low >= my_span; });
+            finish_block<false>(half, state, s, left, shift, values, offsets, s, q, values);
             return;
         }
         const bool edge = (CAUSAL && key0 + 31u > first_row) || key0 + 32u > key_len;

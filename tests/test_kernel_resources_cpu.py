@@ -18,6 +18,9 @@ BUILDS = [
     ("latent_attention_mfma.hip", [], [r"singe_paged_mla_attention_(bf16|f16)_(l512_p64|any)"]),
     ("fmha_prefill_pair.hip", [], [r"singe_fmha_prefill_pair_.*"]),
     ("paged_attention_pair.hip", [], [r"singe_(rotary_)?paged_attention_pair_.*"]),
+    ("fmha_prefill.hip", [], [r"singe_fmha_prefill_(bf16|f16)_d128_(causal|full)(_options)?"]),
+    ("paged_attention.hip", [], [r"singe_ragged_prefill_(bf16|f16)_d128"]),
+    ("attention_mfma_f32.hip", [], [r"singe_attention_mfma_f32_d\d+_r\d+"]),
     ("paged_decode.hip", [], [r"singe_paged_decode_(bf16|f16)_d128_g1_b16", r"singe_paged_decode_f8kv_wide(_relaxed)?_d128_b16",
                               r"singe_paged_decode_(bf16|f16)_wide_d128_b16"]),
 ]
