@@ -354,9 +354,21 @@ bool dense_prefill_packs_heads(const SingeFmhaPrefillConfig& c) {
     return !c.causal && c.kv_heads > 0 && c.heads > c.kv_heads && c.heads % c.kv_heads == 0 && c.query_len * (c.heads / c.kv_heads) <= kTileRows;
 }
 
-// One tile a workgroup where pairs would not fill the chip's two workgroups a compute unit, and shares of the keys only
-// where even single tiles leave half the compute units idle (a launch of one query tile a head, a decode step, keeps the
-// count it asks attention_key_splits for).  Pairs against single tiles with 1 / 2 / 3 / 4 shares, us with the host's part:
+// One tile a workgroup where pairs would not fill the chip's two workgroups a compute unit.  Shares of the keys as
+// attention_key_splits counts them where even single tiles leave half the compute units idle, and for a launch of one query
+// tile a head (a decode step); none where there are more tiles than compute units; in between two, if the rows see so many
+// keys that a workgroup's walk over them outweighs the merge: 1536 under the causal mask, whose last tile alone walks them
+// all, 4096 without it.  (In between, one share took up to 1.3 times as long as pairs with their shares: 1 x 8 x 2500.)
+// Pairs, with the shares they were cut into before single tiles, against single tiles with 1 / 2 / 4 shares, us:
+//   head_dim 128, causal    1 x 8 x 2500 (160 tiles)   46  54 / 42 / 35     1 x 16 x 2000 (256)  49  45 / 42 / 45
+//                           1 x 20 x 1024 (160)        36  26 / 29 / 33     1 x 20 x 1536 (240)  46  38 / 36 / 44
+//                           1 x 32 x 1024 (256)        38  27 / 32 / 40     1 x 24 x 2000 (384)  71  52 / 54 / 65
+//   head_dim 96, causal     1 x 8 x 2500 (160)         39  51 / 39 / 31     1 x 12 x 2000 (192)  37  42 / 36 / 35
+//   head_dim 64, causal     1 x 8 x 2500 (160)         36  39 / 30 / 26     1 x 16 x 2000 (256)  36  32 / 31 / 30
+//   head_dim 128, queries x keys without a mask   64 heads x 512 x 2048 (256)   73  48 / 53 / 65
+//                           64 x 512 x 16384   369  358 / 295 / 305         80 x 512 x 16384 (320) 507 428 / 448 / 408
+//   head_dim 64, no mask    64 x 512 x 2048 (256)      49  33 / 33 / 39     20 x 1024 x 8192 (160) 111 114 / 77 / 70
+// Pairs against single tiles with 1 / 2 / 3 / 4 shares, us with the host's part:
 //   8 x 6 heads x 1500, head_dim 64, ragged keys       59 / 57 / 63        42 / 50 / 54 / 57
 //   8 x 12 heads x 600, head_dim 64, ragged keys       29 / 33 / 38        17 / 32 / 34 / 39
 //   1 x 32 heads x 773, head_dim 128, causal           31 / 32 / 34        23 / 30 / 34 / 35
@@ -370,9 +382,15 @@ DenseShares dense_prefill_shares(const SingeFmhaPrefillConfig& c) {
     const uint64_t query_tiles = (c.query_len + kTileRows - 1) / kTileRows, units = compute_units();
     const uint64_t rows = static_cast<uint64_t>(c.batch) * (dense_prefill_packs_heads(c) ? c.kv_heads : c.heads);
     uint64_t tiles = rows * query_tiles;
+    uint32_t most = 0xffffffffu;
     const bool single = rows * ((query_tiles + 1) / 2) < 2 * units;
-    if (query_tiles > 1 && 2 * tiles > units && tiles < 2 * units) tiles = 2 * units;  // (counts as a full chip)
-    return {single, attention_key_splits(single ? tiles : rows * ((query_tiles + 1) / 2), c.key_len)};
+    if (query_tiles > 1 && 2 * tiles > units && tiles < 2 * units) {
+        const uint64_t seen = c.causal && c.query_len < c.key_len ? c.query_len : c.key_len;
+        if (tiles <= units && seen >= (c.causal ? 1536 : 4096)) most = 2;
+        else tiles = 2 * units;  // (counts as a full chip)
+    }
+    const uint32_t splits = attention_key_splits(single ? tiles : rows * ((query_tiles + 1) / 2), c.key_len);
+    return {single, splits < most ? splits : most};
 }
 
 uint32_t dense_prefill_splits(const SingeFmhaPrefillConfig& c) { return dense_prefill_shares(c).splits; }

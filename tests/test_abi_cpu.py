@@ -445,3 +445,25 @@ def test_dense_family_validation_order_needs_no_device():
     assert through(8, cache, _native.PagedKvAttentionConfigC(sliding._c(), 0, 11, 4, 128, 128))[0] == 1
     packed = _native.PackedQkvAttentionConfigC(sliding._c(), 0, 10, 1 << 40)
     assert named(lib.singe_hip_sliding_window_attention_packed_qkv_f32(None, fake, 640, fake, 5000, ctypes.byref(packed))) == (2, "qkv")
+
+
+@pytest.mark.parametrize("batch,heads,query_len,key_len,head_dim,causal,shares", [
+    (1, 8, 2500, 2500, 128, 1, 2),      # 160 tiles, long rows: two shares
+    (1, 8, 2500, 2500, 96, 1, 2),
+    (1, 16, 2000, 2000, 128, 1, 2),     # 256 tiles, one a compute unit
+    (1, 32, 773, 773, 128, 1, 1),       # 224 tiles, short rows: none
+    (1, 11, 1535, 1535, 64, 1, 1),      # either side of 1536 keys
+    (1, 11, 1536, 1536, 64, 1, 2),
+    (1, 80, 200, 100000, 128, 1, 1),    # causal rows see no more keys than there are queries
+    (1, 48, 512, 4095, 64, 0, 1),       # either side of 4096 without a mask
+    (1, 48, 512, 4096, 64, 0, 2),
+    (1, 24, 2000, 2000, 128, 1, 1),     # 384 tiles: more than compute units
+    (1, 8, 2000, 2000, 128, 1, 4),      # 128 tiles, half the compute units: as many as the keys allow
+    (1, 8, 1, 4096, 128, 0, 8),         # a decode step
+])
+def test_dense_key_shares(batch, heads, query_len, key_len, head_dim, causal, shares):
+    # (without a device the library counts on 256 compute units)
+    problem = _native.AttentionProblemC(batch, heads, heads, query_len, key_len, head_dim, head_dim, (ctypes.c_int64 * 4)(0, 0, 0, 0), 1, causal,
+                                        0, 0, 0, 0.0, 0.0, 0)
+    wanted = shares * batch * heads * query_len * (head_dim + 1) * 4 if shares > 1 else 0   # shares x rows x (values + log-sum-exp) of f32
+    assert _native.lib().singe_hip_scaled_dot_product_attention_scratch_bytes(ctypes.byref(problem)) == wanted
