@@ -467,3 +467,24 @@ def test_dense_key_shares(batch, heads, query_len, key_len, head_dim, causal, sh
                                         0, 0, 0, 0.0, 0.0, 0)
     wanted = shares * batch * heads * query_len * (head_dim + 1) * 4 if shares > 1 else 0   # shares x rows x (values + log-sum-exp) of f32
     assert _native.lib().singe_hip_scaled_dot_product_attention_scratch_bytes(ctypes.byref(problem)) == wanted
+
+
+@pytest.mark.parametrize("heads,kv_heads,head_dim,chunks,chunk,decoding,rows", [
+    (64, 8, 128, 2, 512, 62, 32),     # few chunks beside many decoding sequences
+    (64, 8, 128, 2, 512, 56, 64),     # 33 whole 256-row tiles: either side of 9/16 of one a sequence
+    (64, 8, 128, 2, 512, 57, 32),
+    (64, 8, 64, 1, 1025, 62, 32),     # either side of 1024 tokens more than sequences
+    (64, 8, 64, 1, 1026, 62, 64),
+    (64, 8, 32, 2, 512, 62, 64),      # narrow heads: 256-row tiles
+    (28, 4, 64, 1, 4096, 126, 64),    # a long chunk: 256-row tiles, however many sequences decode beside it
+    (32, 8, 64, 1, 2048, 65, 64),
+    (64, 8, 128, 64, 32, 0, 64),      # many short chunks
+    (8, 8, 128, 1, 512, 62, 32),      # too few tiles for the chip
+])
+def test_paged_attention_row_tiles(heads, kv_heads, head_dim, chunks, chunk, decoding, rows):
+    # (without a device the library counts on 256 compute units)
+    tokens, sequences = chunks * chunk + decoding, chunks + decoding
+    fields = dict(tokens=tokens, heads=heads, kv_heads=kv_heads, head_dim=head_dim, page_size=16, sequences=sequences, cache_pages=20000,
+                  page_table=20000, index_type=0, causal=1, has_scale=0, has_window=0, has_softcap=0, scale=0.0, softcap=0.0, window=0)
+    problem = _native.PagedAttentionProblemC(*fields.values())
+    assert _native.lib().singe_hip_paged_attention_rows_per_wave(ctypes.byref(problem)) == rows

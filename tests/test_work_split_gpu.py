@@ -74,8 +74,12 @@ def test_windows_at_block_edges(window, dim, length, causal, sinks):
 
 @pytest.mark.parametrize("chunks,chunk,decoding", [
     (2, 512, 62),   # half a whole 256-row tile a sequence: 128-row tiles
-    (4, 256, 21),   # 32 tiles, 25 sequences (5 / 4 and a bit): the last on 256-row tiles
-    (4, 256, 22),   # 26 sequences: the first on 128-row tiles
+    (4, 256, 21),   # 32 tiles, 25 sequences: 256-row tiles
+    (4, 256, 22),
+    (2, 512, 56),   # 33 tiles, 58 sequences (9 / 16 and a bit): the last on 256-row tiles
+    (2, 512, 57),   # 59 sequences: the first on 128-row tiles
+    (1, 1025, 62),  # 1024 tokens more than sequences: still 128-row tiles
+    (1, 1026, 62),  # 1025: 256-row tiles
 ])
 def test_mixed_steps_either_side_of_the_tile_choice(chunks, chunk, decoding):
     heads, kv_heads, dim, page = 64, 8, 128, 16
