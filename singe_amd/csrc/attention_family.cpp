@@ -257,7 +257,7 @@ int32_t ragged_kv_prefill(void* stream, int32_t data_type, void* out, size_t out
     const char* names[] = {"out", "lse", "query", "key", "value", "actual_seq_lens_q", "actual_seq_lens_kv", "actual_seq_offsets"};
     if (int32_t s = null_check(pointers, names, 8)) return s;
     if (c.head_dim > 256) return fail(SINGE_HIP_UNSUPPORTED_WIDTH, op, c.head_dim, 0);
-    if (data_type != SINGE_HIP_F32 && ragged_prefill_takes(c.kv_heads, c.head_dim, out, query, key, value))
+    if (data_type != SINGE_HIP_F32 && ragged_prefill_takes(c.total_query_tokens, c.batch, c.heads, c.kv_heads, c.head_dim, out, query, key, value))
         return ragged_prefill_matrix(data_type == SINGE_HIP_F16, stream, query, key, value, lens_q, lens_kv, offsets, out, lse,
                                      c.total_query_tokens, c.total_kv_tokens, c.batch, c.heads, c.kv_heads, c.head_dim, c.causal != 0, c.scale);
     DenseGeneralOperands o;

@@ -66,9 +66,10 @@ SINGE_DEVICE bool locate(const PagedAttentionArgs& a, unsigned int& unit, unsign
         const unsigned int pair = xcd + 8u * (within / kBand);
         if (pair >= a.kv_heads * bands) return false;
         const unsigned int kv_head = pair % a.kv_heads;
-        unsigned int entry = (pair / a.kv_heads) * kBand + within % kBand;
+        // (overlapping sequences can have more row tiles in all than 32 bits count)
+        std::conditional_t<FORM == kPacked, unsigned long long, unsigned int> entry = (pair / a.kv_heads) * kBand + within % kBand;
         if (entry >= a.row_tiles) return false;
-        if constexpr (FORM == kPacked) entry += round * a.row_tiles;
+        if constexpr (FORM == kPacked) entry += static_cast<unsigned long long>(round) * a.row_tiles;
         more = true;
         const unsigned int lane = threadIdx.x & 63u, groups = a.heads / a.kv_heads;
         auto tiles_of = [&](unsigned int s) __attribute__((always_inline)) {
@@ -87,12 +88,12 @@ SINGE_DEVICE bool locate(const PagedAttentionArgs& a, unsigned int& unit, unsign
             if constexpr (FORM == kPacked) more = __ballot(before + mine > (round + 1u) * a.row_tiles) != 0;
             const unsigned int owner = static_cast<unsigned int>(__builtin_ctzll(holds));
             unit = owner * a.kv_heads + kv_head;
-            row_tile = entry - __shfl(before, owner, 64);
+            row_tile = static_cast<unsigned int>(entry) - __shfl(before, owner, 64);
             // (packed prompts see as many keys as they have tokens before them: their last tiles are the long ones)
             if constexpr (FORM == kPacked) row_tile = __shfl(mine, owner, 64) - 1u - row_tile;
             return true;
         }
-        unsigned int base = 0;
+        // (from here on `entry` counts from the first row tile of the sequences looked at)
         for (unsigned int first = 0; first < a.sequences; first += 64u) {
             const unsigned int s = first + lane;
             const unsigned int mine = s < a.sequences ? tiles_of(s) : 0u;
@@ -103,15 +104,15 @@ SINGE_DEVICE bool locate(const PagedAttentionArgs& a, unsigned int& unit, unsign
                 if (lane >= static_cast<unsigned int>(step)) through += below;
             }
             const unsigned int total = __shfl(through, 63, 64);
-            if (entry < base + total) {
-                const unsigned long long holds = __ballot(entry < base + through);  // first lane whose range reaches the entry
+            if (entry < total) {
+                const unsigned long long holds = __ballot(entry < through);  // first lane whose range reaches the entry
                 const unsigned int owner = static_cast<unsigned int>(__builtin_ctzll(holds));
                 const unsigned int owner_through = __shfl(through, owner, 64), owner_mine = __shfl(mine, owner, 64);
                 unit = (first + owner) * a.kv_heads + kv_head;
-                row_tile = entry - (base + owner_through - owner_mine);
+                row_tile = static_cast<unsigned int>(entry) - (owner_through - owner_mine);
                 return true;
             }
-            base += total;
+            entry -= total;
         }
         return false;
     }

@@ -110,7 +110,8 @@ namespace singe_hip {
 bool dense_f32_matrix_takes(const PrefillF32Args& args);
 int32_t dense_f32_matrix(void* stream, PrefillF32Args& args);
 // paged_attention.cpp: ragged_kv_prefill_attention of 16-bit tensors on the matrix cores, and whether they take a call.
-bool ragged_prefill_takes(uint64_t kv_heads, uint64_t head_dim, const void* out, const void* query, const void* key, const void* value);
+bool ragged_prefill_takes(uint64_t tokens, uint64_t sequences, uint64_t heads, uint64_t kv_heads, uint64_t head_dim, const void* out,
+                          const void* query, const void* key, const void* value);
 int32_t ragged_prefill_matrix(bool f16, void* stream, const void* query, const void* key, const void* value, const int32_t* query_lengths,
                               const int32_t* key_lengths, const int32_t* offsets, void* output, float* lse, uint64_t tokens,
                               uint64_t kv_tokens, uint64_t sequences, uint64_t heads, uint64_t kv_heads, uint64_t head_dim, bool causal,

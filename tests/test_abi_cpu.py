@@ -488,3 +488,15 @@ def test_paged_attention_row_tiles(heads, kv_heads, head_dim, chunks, chunk, dec
                   page_table=20000, index_type=0, causal=1, has_scale=0, has_window=0, has_softcap=0, scale=0.0, softcap=0.0, window=0)
     problem = _native.PagedAttentionProblemC(*fields.values())
     assert _native.lib().singe_hip_paged_attention_rows_per_wave(ctypes.byref(problem)) == rows
+
+
+@pytest.mark.parametrize("tokens,heads,kv_heads,batch", [
+    (2**31 - 1, 64, 1, 1),         # 2^37 rows to the one kv head: more than the packed kernel's 32-bit row counts hold
+    (2**29, 64, 4, 3),             # 2^33
+])
+def test_packed_prefill_leaves_row_counts_beyond_32_bits_to_the_row_kernel(tokens, heads, kv_heads, batch):
+    # which refuses these for their number of workgroups, before anything is launched or read
+    config = A.RaggedKvPrefillAttentionConfig.contiguous(batch, tokens, 16, heads, kv_heads, 16, True, 0.25)._c()
+    address, many = 1 << 20, 2**60
+    arguments = [address if i % 2 == 0 else many for i in range(16)]
+    assert _native.lib().singe_hip_ragged_kv_prefill_attention_bf16(None, *arguments, ctypes.byref(config)) == 8
