@@ -220,7 +220,7 @@ def test_family_validation_on_the_device():
     (8, 2, [1, 63, 64, 65, 16, 33]),                    # 128-row tiles: ends of key tiles and of sixteen-key groups
     (3, 1, [1] * 70 + [130, 2]),                        # more than 64 sequences, rows that no power of two divides
     (32, 16, [255, 257, 300, 1, 128, 511, 640]),        # MHA-like: two heads a kv head
-    (64, 64, [1537]),                                   # 256-row tiles on the two-tile kernel, one row past a tile
+    (64, 64, [1537]),                                   # one row past a tile
 ])
 def test_packed_prefill_on_the_matrix_cores(dtype, head_dim, causal, heads, kv_heads, lens):
     tokens = sum(lens)
@@ -245,7 +245,7 @@ def test_packed_prefill_on_the_matrix_cores(dtype, head_dim, causal, heads, kv_h
 
 
 @pytest.mark.parametrize("kv_heads", [1, 16])
-@pytest.mark.parametrize("rows_per_wave", [32, 64])      # 128-row tiles, 256-row tiles
+@pytest.mark.parametrize("rows_per_wave", [32, 64])      # (the paged op's choice of tiles, which packed sequences do not share)
 def test_packed_sequences_that_overlap_leave_the_last_owner(kv_heads, rows_per_wave):
     # Three sequences over the same tokens: more row tiles than the token count says, and the last owner's rows stand.
     heads, head_dim, tokens = kv_heads * 2, 64, 2100
@@ -263,9 +263,10 @@ def test_packed_sequences_that_overlap_leave_the_last_owner(kv_heads, rows_per_w
         _native.lib().singe_hip_set_paged_attention_rows_per_wave(0)
     for of in {0, kv_heads - 1}:
         heads_of, kv_of = slice(2 * of, 2 * of + 2), slice(of, of + 1)
-        want, _ = oracle.ragged_kv_prefill_attention_f32(host(q)[:, heads_of], host(k)[:, kv_of], host(v)[:, kv_of], lens, keys, offsets,
-                                                         causal=False, scale=0.125)
+        want, want_lse = oracle.ragged_kv_prefill_attention_f32(host(q)[:, heads_of], host(k)[:, kv_of], host(v)[:, kv_of], lens, keys, offsets,
+                                                                causal=False, scale=0.125)
         close(out[:, heads_of], want, torch.bfloat16)
+        assert np.abs(lse.cpu().numpy()[:, heads_of] - want_lse).max() <= 1e-4   # an f32 sum, the same keys on both sides
 
 
 def packed_reference_f64(q, k, v, lens, causal, scale):

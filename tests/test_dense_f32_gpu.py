@@ -150,3 +150,37 @@ def test_matrix_core_sums_are_as_exact_as_the_row_kernels(dim, batch, heads, len
         scores = scores.masked_fill(torch.ones(length, length).triu(1).bool(), -float("inf"))
     want = torch.softmax(scores, -1) @ v
     assert ((out - want).norm() / want.norm()).item() <= bound
+
+
+@pytest.mark.parametrize("dim", [64, 96, 128])
+@pytest.mark.parametrize("batch,heads,lq,lk,causal,window", [
+    (32, 64, 33, 70, True, 0),       # a wave a tile (two at head_dim 64: 4096 tiles and more are one), a last tile of one row
+    (64, 64, 63, 45, False, 0),
+    (90, 64, 20, 31, False, 0),      # a single block of keys
+    (6, 32, 33, 100, True, 0),       # four waves a tile, a block each
+    (6, 32, 33, 257, False, 0),      # eight waves a tile at head_dim 64, four above; a last block of one key
+    (6, 32, 40, 321, False, 90),
+    (3, 64, 31, 200, False, 0),      # seven blocks: one of eight waves without any
+])
+def test_thirty_two_row_tiles_and_their_waves(dim, batch, heads, lq, lk, causal, window):
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(dim + lq)
+    q, k, v = (torch.randn((batch, h, n, dim), generator=gen, device="cuda") for h, n in ((heads, lq), (heads // 2, lk), (heads // 2, lk)))
+    out = torch.full_like(q, float("nan"))
+    config = A.bhsd_config(batch, heads, heads // 2, lq, lk, dim, dim ** -0.5, causal)
+    lse = None
+    if window:
+        A.softcapped_window_attention_f32(None, out, q, k, v, A.SoftcappedWindowAttentionConfig(config, window, None))
+    else:
+        lse = torch.full((batch, heads, lq), float("nan"), device="cuda")
+        A.fmha_prefill_lse_f32(None, out, lse, q, k, v, config)
+    assert not out.isnan().any()
+    i, j = torch.arange(lq)[:, None], torch.arange(lk)[None, :]
+    hidden = (j > i if causal else torch.zeros((lq, lk), dtype=torch.bool)) | ((i - j).abs() > window if window else False)
+    for b, h in ((0, 0), (0, heads - 1), (batch // 2, 5), (batch - 1, 0), (batch - 1, heads - 1)):
+        rows, keys, values = q[b, h].double().cpu(), k[b, h // 2].double().cpu(), v[b, h // 2].double().cpu()
+        scores = (rows @ keys.T * dim ** -0.5).masked_fill(hidden, -float("inf"))
+        want = torch.softmax(scores, -1) @ values
+        assert (out[b, h].double().cpu() - want).abs().max().item() <= 1e-5   # f32 sums of values up to about 4
+        if lse is not None:
+            assert (lse[b, h].double().cpu() - torch.logsumexp(scores, -1)).abs().max().item() <= 1e-5
