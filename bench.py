@@ -679,7 +679,7 @@ def dense_f32_section(with_cpu=True):
                     "(BASELINE config 1, the accuracy anchor)",
         "value": stats["mean_ms"] * 1e3, "unit": "us", "us_per_step_median": stats["median_ms"] * 1e3,
         "algorithmic_flops": 4 * dim * heads * (seq * (seq + 1) // 2), "algorithmic_bytes": 4 * batch * heads * seq * dim * 4,
-        "kernel": "singe_fmha_prefill_rows_f32_d64", **timing_fields(stats),
+        "kernel": "singe_attention_mfma_f32_d64_r16", **timing_fields(stats),
     }
     if with_cpu:
         result["cpu_baseline"] = dense_f32_cpu_baseline(q, k, v)

@@ -480,7 +480,9 @@ SINGE_HIP_API void singe_hip_set_paged_attention_splits(uint32_t splits);
 /* Packed rows a wave of the bf16 / f16 paged attention kernels takes, as singe_hip_set_dense_prefill_rows_per_wave: 32,
  * 64 (only calls at a head_dim that is a multiple of 16 up to 128 with a page size that is a power of two of at least 16 keys and a positive scale,
  * without a softcap, a window or key splits have that form, with or without the fused query rotation; others keep
- * 32), or 0 (the default): 64 where the call has that form and its 256-row tiles still fill the chip. */
+ * 32), or 0 (the default): 64 where the call has that form and its 256-row tiles still fill the chip, unless it is a step
+ * of few new tokens beside many sequences that decode (head_dim 64 up, at most 1024 tokens more than sequences, at most
+ * 9/16 of a whole 256-row tile a sequence).  Packed prefill (singe_hip_ragged_kv_prefill_attention_*) does not look at it. */
 SINGE_HIP_API void singe_hip_set_paged_attention_rows_per_wave(uint32_t rows);
 /* What a bf16 / f16 call of this problem takes when it is given scratch: 32 or 64 rows a wave,
  * 0 when the head dimension has no matrix-core build. */

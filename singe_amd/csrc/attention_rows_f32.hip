@@ -18,7 +18,8 @@
 // taken four at a time to bound registers (a group of more than four re-reads the slice from L2).
 //
 // The same loop serves the dense f32 prefill ops at these head dimensions where attention_mfma_f32.hip does not (a score cap,
-// unaligned rows, head dimensions other than 32, 64 and 128: fmha_prefill_f32, fmha_prefill_lse_f32,
+// unaligned rows, head dimensions other than 32, 64 and 128, and calls of so few rows that this loop is done first:
+// fmha_prefill_f32, fmha_prefill_lse_f32,
 // softcapped_window_attention_f32) and the f32 forms of the two block-table ops, paged_kv_decode_attention_f32 and
 // paged_kv_prefill_attention_f32 (singe-kernel/src/cpu/attention.rs:1172-1341; launch API
 // singe-kernel/src/cuda/attention/paged.rs): only where the rows come from and where the result goes differ.

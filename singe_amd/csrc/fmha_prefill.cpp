@@ -182,14 +182,15 @@ int32_t dense_f32_matrix(void* stream, PrefillF32Args& a) {
     a.scale_log2e = logit_factor(a.scale);
     // 16-row tiles where 32-row ones are too few for the chip (up to 5/8 of a tile a compute unit; at head_dim 32 always, where
     // a wave's loads and softmax weigh more than its products), and a tile's keys over as many waves as leave the SIMDs two to
-    // four waves each.  Measured in us (B x H x L, causal; 16 rows with 1 / 2 / 4 / 8 waves, then 32 rows with 1 / 2 / 4 / 8):
-    //   head_dim 64   1 x 8 x 512     44 / 27 / 17 / 11     72 / 44 / 26 / 17     (the row kernel below: 38)
-    //                 1 x 12 x 1024   85 / 47 / 29 / 31    146 / 82 / 46 / 29
-    //                 4 x 12 x 1024   86 / 86 / 98 / 111   150 / 84 / 86 / 96
-    //   head_dim 128  1 x 8 x 512     90 / 53 / 31 / 19     77 / 44 / 26 (four waves a workgroup)
-    //                 4 x 8 x 512     91 / 54 / 41 / 47     77 / 45 / 38
-    //                 4 x 12 x 1024  185 / 177 / 187 / 213  151 / 149 / 164;  not causal 379 / 301 / 319 / 361  301 / 241 / 260
-    //   head_dim 32   4 x 12 x 1024   66 / 48 / 48 / 50    104 / 90 / 64 / 56
+    // four waves each.  Kernel times in us (B x H x L, causal; 16 rows with 1 / 2 / 4 / 8 waves, then 32 rows with 1 / 2 / 4 / 8):
+    //   head_dim 64   1 x 8 x 512     30 / 18 / 12 / 12     45 / 27 / 17 / 18     (the row kernel: 38)
+    //                 1 x 12 x 1024   67 / 40 / 34 / 36     87 / 58 / 37 / 32
+    //                 4 x 12 x 1024   97 / 98 / 111 / 129  116 / 89 / 92 / 102
+    //   head_dim 128  1 x 8 x 512     48 / 27 / 18 / 19     84 / 47 / 29 (four waves a workgroup)
+    //                 4 x 8 x 512     53 / 54 / 45 / 52     88 / 52 / 44
+    //                 4 x 12 x 1024  169 / 174 / 198 / 232 178 / 172 / 188;  not causal 341 / 280 / 319 / 375  355 / 283 / 303
+    //   head_dim 96   4 x 12 x 1024  132 / 135 / 150 / 177 141 / 137 / 150
+    //   head_dim 32   4 x 12 x 1024   68 / 50 / 52 / 55
     // A wave without a block of its own costs nothing: 7 blocks on 8 waves take 12.1 us, on 4 waves 18.8 (1 x 8 x 200 x 128).
     const uint64_t pairs = static_cast<uint64_t>(a.batch) * a.heads, blocks = (static_cast<uint64_t>(a.key_len) + 31) / 32, units = compute_units();
     const uint32_t rows = a.head_dim == 32 || pairs * ((static_cast<uint64_t>(a.query_len) + 31) / 32) * 8 <= 5 * units ? 16 : 32;

@@ -17,8 +17,9 @@
 // its keys side by side, which keeps its K/V in that XCD's L2.  Small launches take one tile to a workgroup
 // instead, the longest first (`single_tiles`).
 #include "kernel_args.h"
-// Up to head_dim 64 an LDS row is 128 bytes: 40 KiB a workgroup, so a compute unit holds four of them instead of two,
-// and every lane of a tile's loads fetches something.
+// Up to head_dim 64 an LDS row is 128 bytes: 40 KiB a workgroup, so a compute unit holds as many as its registers allow
+// instead of two (four at head_dim 16 and 32, three at 48 and 64, with or without the options), and every lane of a tile's
+// loads fetches something.
 #if defined(SINGE_HEAD_DIM) && SINGE_HEAD_DIM <= 64
 #define SINGE_PREFILL_ROW_BYTES 128
 #endif
