@@ -309,8 +309,9 @@ SINGE_DEVICE void attention_mfma_f32_body(const PrefillF32Args& a, float* lds) {
         if (a.lse != nullptr && stored && lane_group == 0)
             a.lse[(static_cast<size_t>(batch) * a.heads + head) * a.query_len + row] = sum > 0.0f ? fmaf(reference, kLn2, log2f(sum) * kLn2) : -INFINITY;
     };
-    // Rows of the tile (bit r: row r) whose sums a value that is not finite has spoilt: worked out by themselves.
-    const unsigned long long spoiled = __builtin_amdgcn_ballot_w64(stored && not_finite(kRegs * kDimBlocks, [&](int i) { return out[i / kRegs][i % kRegs]; }));
+    // Rows of the tile (bit r: row r) whose sums a value that is not finite has spoilt: worked out by themselves.  (Where the
+    // weights' sum is NaN, so is the score of a key the row sees, and every output of it either way.)
+    const unsigned long long spoiled = __builtin_amdgcn_ballot_w64(stored && total == total && not_finite(kRegs * kDimBlocks, [&](int i) { return out[i / kRegs][i % kRegs]; }));
     unsigned int alone = static_cast<unsigned int>(spoiled | spoiled >> 32);
     if constexpr (ROWS == 16) alone = (alone | alone >> 16) & 0xffffu;
     auto redo = [&](unsigned int rows) __attribute__((always_inline)) {

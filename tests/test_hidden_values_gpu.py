@@ -9,6 +9,7 @@ import math
 import pytest
 import torch
 
+from singe_amd import neural
 from singe_amd.kernel import attention as A
 
 pytestmark = pytest.mark.gpu
@@ -86,3 +87,23 @@ def test_dense_f32(dim, batch, heads, length, window, causal, bad):
     for b, of in ((0, slice(0, 2)), (batch - 1, slice(heads - 2, heads))):
         kv = slice(of.start // 2, of.start // 2 + 1)
         same(out[b, :, of], visible_only(q[b, :, of], k[b, :, kv], v[b, :, kv], first, end, scale), torch.float32)
+
+
+@pytest.mark.parametrize("dim", [64, 128])
+@pytest.mark.parametrize("lengths", [None, [70, 150]])
+@pytest.mark.parametrize("bad", [INF, NAN])
+def test_dense_f32_of_the_tensor_surface(dim, lengths, bad):
+    # scaled_dot_product_attention of f32 tensors: a window, and keys past a batch entry's own count
+    batch, heads, length, window = 2, 8, 150, 40
+    q, k, v = (draw(seed, batch, h, length, dim) for seed, h in ((4, heads), (5, heads), (6, heads)))
+    v[:, 0, 60, 1] = bad
+    if lengths is None:
+        out = neural.attend(q.cuda(), k.cuda(), v.cuda(), None, None, neural.AttentionOptions(causal=True, window=window))
+    else:
+        v[0, :, lengths[0]:] = bad
+        out = neural.attend_padded(q.cuda(), k.cuda(), v.cuda(), torch.tensor(lengths, dtype=torch.int32, device="cuda"))
+    for b in range(batch):
+        first = [max(0, i + 1 - window) if lengths is None else 0 for i in range(length)]
+        end = [i + 1 if lengths is None else lengths[b] for i in range(length)]
+        rows = [t[b].transpose(0, 1) for t in (q, k, v)]
+        same(out[b].transpose(0, 1), visible_only(*rows, first, end, dim ** -0.5), torch.float32)
