@@ -310,6 +310,15 @@ struct GeneralPagedArgs {
 };
 
 // singe_paged_mla_attention_general_*: contiguous operands of one element type.
+// What the matrix-core latent kernel leaves for the merge about a unit (128 rows of a sequence at most).
+struct alignas(16) LatentUnit {
+    uint64_t first_row;   // its first row of [tokens, heads]
+    uint64_t first_slot;  // its first partial row; share s of row r is `first_slot + s * rows + r`
+    uint32_t rows;        // 0: nothing to merge
+    uint32_t shares;
+    uint32_t unused[2];
+};
+
 struct LatentAttentionArgs {
     const void* latent_queries;      // [tokens, heads, latent_dim]
     const void* positional_queries;  // [tokens, heads, position_dim]
@@ -326,14 +335,19 @@ struct LatentAttentionArgs {
     uint32_t row_blocks;             // workgroups per sequence (4 rows each; 128 each on the matrix-core kernel)
     uint32_t causal, wide_index;
     float scale;
-    // Matrix-core kernel with key splits (splits > 1): each of a row tile's `splits` workgroups leaves its rows
-    // normalised in partial_out [splits, tokens, heads, latent_dim] with a base-two log-sum-exp in partial_lse
-    // [splits, tokens, heads] (-inf and zeros for a share without keys); singe_paged_mla_attention_combine_* merges.
+    // Matrix-core kernel with key splits: each workgroup that shares a unit (a row tile) leaves its rows normalised in
+    // partial_out [slots, 512] with a base-two log-sum-exp in partial_lse [slots] (-inf and zeros for a share without
+    // keys), the unit's first one a record in units [unit_slots]; singe_paged_mla_attention_combine_* merges.  `splits` > 1:
+    // that many shares of every unit; `share_budget` > 0: shares of one length for all units, as many workgroups.
     uint32_t splits;
     int32_t page_shift;              // log2(page_size) when that is a power of two, else -1 (matrix-core kernel)
     float* partial_out;
     float* partial_lse;
     uint32_t unit_band;              // matrix-core kernel: neighbouring units (row tiles) that go to one XCD together
+    uint32_t share_budget;
+    uint32_t unit_slots;
+    uint64_t slots;
+    LatentUnit* units;               // null without splits
 };
 
 // singe_rotary_cache_write_*: contiguous operands of one element type; angles may be f32.

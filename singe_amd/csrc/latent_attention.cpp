@@ -27,33 +27,47 @@ bool on_matrix_cores(const SingePagedMlaAttentionProblem& p) {
 bool built_shape(const SingePagedMlaAttentionProblem& p) { return p.latent_dim == 512 && p.position_dim == 64; }
 
 // Key splits for a problem: the row tiles of a decode step or a short chunk (one workgroup each, one workgroup to a
-// compute unit) leave most of the chip idle, so each tile's keys are shared out until there is about one workgroup
-// per compute unit: 64 shares at most (the merge keeps a share's weight per lane), and no more than leave a share
-// four key tiles of a sequence of average length (the page table bounds the keys from above).  The count of live
-// tiles is not known on the host (it depends on the offsets on the device): every sequence has at least one, and
-// together they hold at least tokens * heads / 128.
-// 0 = chosen by problem size (singe_hip_set_paged_mla_attention_splits).
+// compute unit) leave most of the chip idle, so their keys are shared out until there is about one workgroup per
+// compute unit.  The kernel chooses the shares (place_balanced: it sees the sequences' lengths): their length is the
+// same for all sequences, four key tiles at least, and a row tile has 64 at most (the merge keeps a share's weight per
+// lane).  The count of live tiles is not known on the host (it depends on the offsets on the device): every sequence
+// has at least one, and together they hold at least tokens * heads / 128.  Calls whose sequences hold less than two
+// such shares on average (the page table bounds the keys from above) are not split.
+// Or a count of shares fixed by the caller, the same for every row tile: 0 = chosen as above
+// (singe_hip_set_paged_mla_attention_splits).
 std::atomic<uint32_t> g_latent_splits{0};
 
-uint32_t latent_splits(const SingePagedMlaAttentionProblem& p) {
-    if (!on_matrix_cores(p) || p.tokens <= 0 || p.heads <= 0 || p.sequences <= 0) return 1;
-    if (const uint32_t fixed = effective_count(thread_options().paged_mla_attention_splits, g_latent_splits.load(std::memory_order_relaxed)))
-        return fixed;
-    const uint64_t packed = (static_cast<uint64_t>(p.tokens) * p.heads + 127) / 128;
-    const uint64_t workgroups = packed > static_cast<uint64_t>(p.sequences) ? packed : static_cast<uint64_t>(p.sequences);
-    const uint64_t wanted = compute_units();
-    if (workgroups >= wanted) return 1;
-    const uint64_t mean_keys = static_cast<uint64_t>(p.page_table > 0 ? p.page_table : 0) * static_cast<uint64_t>(p.page_size) / static_cast<uint64_t>(p.sequences);
-    const uint64_t worth = mean_keys / (4 * 32);
-    uint64_t splits = wanted / workgroups;
-    if (splits > 64) splits = 64;
-    if (splits > worth) splits = worth;
-    return static_cast<uint32_t>(splits < 1 ? 1 : splits);
-}
+struct Shares {
+    uint32_t fixed = 1;    // shares of every row tile
+    uint32_t budget = 0;   // workgroups to share all row tiles' keys out to (0: `fixed`)
+    uint64_t slots = 0;    // partial rows
+    uint64_t units = 0;    // row tiles, an upper bound
+    bool any() const { return fixed > 1 || budget > 0; }
+    // partial rows, their log-sum-exps, the units' records (each on a 16-byte boundary)
+    size_t records_at() const { return (static_cast<size_t>(slots) * (512 + 1) * sizeof(float) + 15) / 16 * 16; }
+    size_t bytes() const { return any() ? records_at() + static_cast<size_t>(units) * sizeof(LatentUnit) : 0; }
+};
 
-size_t latent_scratch_bytes(const SingePagedMlaAttentionProblem& p, uint32_t splits) {
-    if (splits <= 1) return 0;
-    return static_cast<size_t>(splits) * static_cast<size_t>(p.tokens) * static_cast<size_t>(p.heads) * (512 + 1) * sizeof(float);
+Shares latent_shares(const SingePagedMlaAttentionProblem& p) {
+    Shares shares;
+    if (!on_matrix_cores(p) || p.tokens <= 0 || p.heads <= 0 || p.sequences <= 0) return shares;
+    const uint64_t rows = static_cast<uint64_t>(p.tokens) * static_cast<uint64_t>(p.heads), packed = (rows + 127) / 128;
+    const uint64_t sequences = static_cast<uint64_t>(p.sequences);
+    shares.units = packed + sequences;
+    if (const uint32_t fixed = effective_count(thread_options().paged_mla_attention_splits, g_latent_splits.load(std::memory_order_relaxed))) {
+        shares.fixed = fixed;
+        shares.slots = fixed * rows;
+        return shares;
+    }
+    const uint64_t workgroups = packed > sequences ? packed : sequences;
+    const uint64_t wanted = compute_units();
+    const uint64_t mean_keys = static_cast<uint64_t>(p.page_table > 0 ? p.page_table : 0) * static_cast<uint64_t>(p.page_size) / sequences;
+    if (workgroups >= wanted || mean_keys < 2 * 4 * 32 || sequences > 256) return shares;
+    shares.budget = static_cast<uint32_t>(wanted > shares.units ? wanted : shares.units);
+    // A workgroup leaves 128 partial rows at most, a row 64 of them.
+    const uint64_t by_workgroup = shares.budget * (rows < 128 ? rows : 128), by_row = 64 * rows;
+    shares.slots = by_workgroup < by_row ? by_workgroup : by_row;
+    return shares;
 }
 
 int32_t paged_mla_attention(void* stream, const void* latent_queries, const void* positional_queries, const void* latent_cache,
@@ -120,6 +134,10 @@ int32_t paged_mla_attention(void* stream, const void* latent_queries, const void
     const uint64_t blocks = row_blocks + static_cast<uint64_t>(p.sequences);
     if (blocks > 0x7fffffffull || row_blocks > 0xffffffffull) return fail(SINGE_HIP_UNSUPPORTED_CONFIGURATION, "too many workgroups");
     args.splits = 1;
+    args.share_budget = 0;
+    args.slots = 0;
+    args.unit_slots = 0;
+    args.units = nullptr;
     args.page_shift = -1;
     for (int shift = 0; shift < 31; ++shift)
         if (p.page_size == (int64_t{1} << shift)) args.page_shift = shift;
@@ -129,29 +147,34 @@ int32_t paged_mla_attention(void* stream, const void* latent_queries, const void
     if (tiles) {
         // Key splits, when the caller lent scratch for them: the attention kernel leaves partials, a second kernel
         // merges them.
-        uint32_t splits = scratch != nullptr ? latent_splits(p) : 1;
-        if (splits > 1 && (scratch_bytes < latent_scratch_bytes(p, splits) || blocks * splits > 0x7fffffffull || blocks * 32 > 0x7fffffffull))
-            splits = 1;
-        if (splits > 1) {
+        Shares shares = scratch != nullptr ? latent_shares(p) : Shares{};
+        if (shares.any() && (scratch_bytes < shares.bytes() || blocks * shares.fixed > 0x7fffffffull || blocks * 32 > 0x7fffffffull))
+            shares = Shares{};
+        const bool split = shares.any();
+        if (split) {
             if (reinterpret_cast<uintptr_t>(scratch) % 16 != 0) return fail(SINGE_HIP_INVALID_ARGUMENT, "scratch alignment");
-            args.splits = splits;
+            args.splits = shares.fixed;
+            args.share_budget = shares.budget;
+            args.slots = shares.slots;
+            args.unit_slots = static_cast<uint32_t>(blocks);
             args.partial_out = static_cast<float*>(scratch);
-            args.partial_lse = args.partial_out + static_cast<size_t>(splits) * p.tokens * p.heads * 512;
+            args.partial_lse = args.partial_out + static_cast<size_t>(shares.slots) * 512;
+            args.units = reinterpret_cast<LatentUnit*>(static_cast<unsigned char*>(scratch) + shares.records_at());
         }
         // Without splits, units go to the XCDs in bands of neighbours (see the kernel): as wide as leaves every XCD
         // something to do, 32 (an XCD's compute units, each of which holds one workgroup) at most.  The width follows
         // the units that are surely live (the count of blocks is an upper bound: up to one per sequence more), and the
-        // grid covers whole rounds of eight bands.  With splits the grid is the units times their shares.
+        // grid covers whole rounds of eight bands.  With splits the grid is the units times their shares, or the budget.
         const uint64_t surely_live = row_blocks > static_cast<uint64_t>(p.sequences) ? row_blocks : static_cast<uint64_t>(p.sequences);
         const uint64_t band = surely_live >= 256 ? 32 : (surely_live + 7) / 8;
         const uint64_t rounds = (blocks + 8 * band - 1) / (8 * band);
         args.unit_band = static_cast<uint32_t>(band);
-        const uint64_t grid = splits > 1 ? blocks * splits : rounds * 8 * band;
+        const uint64_t grid = shares.budget > 0 ? shares.budget : split ? blocks * shares.fixed : rounds * 8 * band;
         if (grid > 0x7fffffffull) return fail(SINGE_HIP_UNSUPPORTED_CONFIGURATION, "too many workgroups");
         const bool bf16 = p.data_type == SINGE_HIP_BF16, built = built_shape(p);
         const KernelId tiles_kernel = built ? (bf16 ? kLatentTilesBf16 : kLatentTilesF16) : (bf16 ? kLatentTilesAnyBf16 : kLatentTilesAnyF16);
         const int32_t launched = launch(tiles_kernel, static_cast<unsigned>(grid), 1, 1, 512, stream, args);
-        if (launched != 0 || splits == 1) return launched;
+        if (launched != 0 || !split) return launched;
         // The merge: 32 workgroups of four waves to a unit, a wave to a row.
         const KernelId merge = built ? (bf16 ? kLatentCombineBf16 : kLatentCombineF16) : (bf16 ? kLatentCombineAnyBf16 : kLatentCombineAnyF16);
         return launch(merge, static_cast<unsigned>(blocks * 32), 1, 1, 256, stream, args);
@@ -177,7 +200,7 @@ extern "C" void singe_hip_set_paged_mla_attention_splits(uint32_t splits) {
 
 extern "C" size_t singe_hip_paged_mla_attention_scratch_bytes(const SingePagedMlaAttentionProblem* problem) {
     if (problem == nullptr) return 0;
-    return latent_scratch_bytes(*problem, latent_splits(*problem));
+    return latent_shares(*problem).bytes();
 }
 
 extern "C" int32_t singe_hip_paged_mla_attention_scratch(void* stream, const void* latent_queries, const void* positional_queries,

@@ -52,7 +52,9 @@ constexpr int kStageBytes = kLatentTileBytes + kPositionalTileBytes;
 // wave registers for the operands in flight.
 constexpr int kParkedSteps = 8;
 constexpr int kParkedBytes = kParkedSteps * 1024 * kWaves;
-constexpr int kLdsBytes = 2 * kStageBytes + kParkedBytes;
+// Where the workgroup's partial rows go waits behind that for the end of the loop, which has no register for it.
+constexpr int kSlotAt = 2 * kStageBytes + kParkedBytes;
+constexpr int kLdsBytes = kSlotAt + 16;
 constexpr int kLatentSteps = kLatent / 32, kSteps = (kLatent + kPositional) / 32;
 constexpr int kDimBlocks = kLatent / 16;
 
@@ -148,6 +150,134 @@ SINGE_DEVICE bool find_unit(const LatentAttentionArgs& a, unsigned int unit, uns
     return false;
 }
 
+// Sum and maximum over a wave's 64 lanes, in every lane: four rotations inside the rows of sixteen, two swaps across.
+template <class Join>
+SINGE_DEVICE unsigned int across_wave(unsigned int value, Join join) {
+    value = join(value, static_cast<unsigned int>(__builtin_amdgcn_update_dpp(0, static_cast<int>(value), 0x128, 0xF, 0xF, false)));
+    value = join(value, static_cast<unsigned int>(__builtin_amdgcn_update_dpp(0, static_cast<int>(value), 0x124, 0xF, 0xF, false)));
+    value = join(value, static_cast<unsigned int>(__builtin_amdgcn_update_dpp(0, static_cast<int>(value), 0x122, 0xF, 0xF, false)));
+    value = join(value, static_cast<unsigned int>(__builtin_amdgcn_update_dpp(0, static_cast<int>(value), 0x121, 0xF, 0xF, false)));
+    float a, b;
+    swap_with_self<16>(as_float(static_cast<int>(value)), a, b);
+    value = join(static_cast<unsigned int>(as_int(a)), static_cast<unsigned int>(as_int(b)));
+    swap_with_self<32>(as_float(static_cast<int>(value)), a, b);
+    return join(static_cast<unsigned int>(as_int(a)), static_cast<unsigned int>(as_int(b)));
+}
+
+// What of a problem a workgroup takes: share `share` of `shares` of the key tiles of a unit (a row tile of a sequence).
+// Shares are `share_tiles` long, or (0) the unit's tiles over the shares.  Partial rows of a unit start at `first_slot`,
+// its shares one after the other.
+struct Placement {
+    unsigned int sequence, row_tile, unit, share, shares, share_tiles;
+    unsigned long long first_slot;
+};
+
+// Shares of one length for every unit (a.share_budget workgroups, or one a unit where there are more units).  A compute
+// unit holds one workgroup, so a decode step takes as long as its longest share, and with an equal *count* of shares
+// that was a fourth of the longest sequence: 64 sequences of 1024 to 8192 keys under 128 heads 64 tiles of 32 keys,
+// where 36 would be an even deal; the length found here is 41 (kernel 139 -> 110 us, whole op 148.6 -> 125.6 us; 128
+// such sequences 266 -> 239 us, 64 under 16 heads 109 -> 90 us, sequences of one length as before).  It is the smallest under
+// which the shares of all units fit the budget, and every wave finds it for itself: the sequences' key tiles and row
+// tiles sit in the lanes' registers (the host takes this path up to 64 * kShareChunks sequences), the length lies
+// between tiles / budget and tiles / (budget - units), and a step of the search between them (four here) is a division
+// a lane and a sum over the wave.
+// Returns false for a workgroup past the last share; `units` is how many there are.
+constexpr int kShareChunks = 4;
+constexpr unsigned int kMostShares = 64;      // of a unit: the merge keeps a share's weight a lane
+constexpr unsigned int kLeastShareTiles = 4;  // a workgroup's start and its way out cost about as much
+template <int FORM>
+SINGE_DEVICE bool place_balanced(const LatentAttentionArgs& a, unsigned int workgroup, Placement& place, unsigned int& units) {
+    const unsigned int lane = threadIdx.x & 63u;
+    auto add = [](unsigned int x, unsigned int y) { return x + y; };
+    auto larger = [](unsigned int x, unsigned int y) { return x > y ? x : y; };
+    unsigned int unit_count[kShareChunks], tile_count[kShareChunks], row_count[kShareChunks];
+#pragma unroll
+    for (int c = 0; c < kShareChunks; ++c) {
+        const unsigned int s = 64u * c + lane;
+        unit_count[c] = tile_count[c] = row_count[c] = 0;
+        if (s < a.sequences) {
+            // (as find_unit counts units; the sequence's own checks come later, counts that make no sense are held to their buffers)
+            long long count = read_index<FORM>(a.query_offsets, s + 1) - read_index<FORM>(a.query_offsets, s);
+            long long pages = read_index<FORM>(a.page_offsets, s + 1) - read_index<FORM>(a.page_offsets, s);
+            long long last = read_index<FORM>(a.last_page_lengths, s);
+            count = count < 0 ? 0 : count > static_cast<long long>(a.tokens) ? static_cast<long long>(a.tokens) : count;
+            pages = pages < 0 ? 0 : pages > static_cast<long long>(a.page_table) ? static_cast<long long>(a.page_table) : pages;
+            last = last < 0 ? 0 : last > static_cast<long long>(a.page_size) ? static_cast<long long>(a.page_size) : last;
+            const long long keys = pages == 0 ? 0 : (pages - 1) * a.page_size + last;
+            row_count[c] = static_cast<unsigned int>(count) * a.heads;  // (tokens * heads is at most 128 rows a unit of the budget here)
+            unit_count[c] = row_count[c] == 0 ? 1u : (row_count[c] + kRows - 1) / kRows;
+            tile_count[c] = static_cast<unsigned int>((keys + kKeys - 1) / kKeys);
+        }
+    }
+    unsigned int mine_units = 0, mine_longest = 0;
+    float mine_tiles = 0.0f;  // (bounds of the search only: a relative error of 2^-24 a term, allowed for below)
+#pragma unroll
+    for (int c = 0; c < kShareChunks; ++c) {
+        mine_units += unit_count[c];
+        mine_longest = larger(mine_longest, tile_count[c]);
+        mine_tiles += static_cast<float>(unit_count[c]) * static_cast<float>(tile_count[c]);
+    }
+    units = across_wave(mine_units, add);
+    const unsigned int longest = across_wave(mine_longest, larger);
+    float all_tiles = mine_tiles;
+#pragma unroll
+    for (int step = 32; step >= 1; step >>= 1) all_tiles += __shfl_xor(all_tiles, step, 64);
+    // sum of units * ceil(tiles / length) is at least all tiles / length and at most that and the units
+    const unsigned int budget = larger(a.share_budget, units), least = larger(kLeastShareTiles, (longest + kMostShares - 1) / kMostShares);
+    unsigned int low = larger(least, static_cast<unsigned int>(0.9999f * all_tiles / static_cast<float>(budget))), high = larger(least, longest);
+    if (budget > units) {
+        const float enough = 1.0001f * all_tiles / static_cast<float>(budget - units) + 1.0f;
+        if (enough < static_cast<float>(high)) high = larger(least, static_cast<unsigned int>(enough) + 1u);
+    }
+    low = low < high ? low : high;
+    auto shares_of = [&](unsigned int tiles, unsigned int length) __attribute__((always_inline)) {
+        return tiles <= length ? 1u : (tiles + length - 1u) / length;
+    };
+    while (low < high) {
+        const unsigned int length = (low + high) / 2u;
+        unsigned int mine = 0;
+#pragma unroll
+        for (int c = 0; c < kShareChunks; ++c)
+            if (64u * c < a.sequences) mine += unit_count[c] * shares_of(tile_count[c], length);
+        if (across_wave(mine, add) <= budget) high = length;
+        else low = length + 1u;
+    }
+    const unsigned int length = __builtin_amdgcn_readfirstlane(high);
+    // The owner of the workgroup: inclusive prefix sums of workgroups, units and partial rows over the sequences.
+    unsigned int workgroups_before = 0, units_before = 0, slots_before = 0;
+#pragma unroll
+    for (int c = 0; c < kShareChunks; ++c) {
+        if (64u * c >= a.sequences) break;
+        const unsigned int shares = shares_of(tile_count[c], length);
+        unsigned int groups = unit_count[c] * shares, tiles = unit_count[c], slots = row_count[c] * shares;
+        const unsigned int own_groups = groups, own_tiles = tiles, own_slots = slots;
+#pragma unroll
+        for (int step = 1; step < 64; step <<= 1) {
+            const unsigned int g = __shfl_up(groups, step, 64), t = __shfl_up(tiles, step, 64), r = __shfl_up(slots, step, 64);
+            if (lane >= static_cast<unsigned int>(step)) groups += g, tiles += t, slots += r;
+        }
+        const unsigned int total = __builtin_amdgcn_readfirstlane(__shfl(groups, 63, 64));
+        if (workgroup < workgroups_before + total) {
+            const unsigned long long holds = __ballot(workgroup < workgroups_before + groups);
+            const unsigned int owner = static_cast<unsigned int>(__builtin_ctzll(holds));
+            const unsigned int within = workgroup - (workgroups_before + __shfl(groups - own_groups, owner, 64));
+            place.shares = __builtin_amdgcn_readfirstlane(__shfl(shares, owner, 64));
+            place.sequence = __builtin_amdgcn_readfirstlane(64u * c + owner);
+            place.row_tile = __builtin_amdgcn_readfirstlane(within / place.shares);
+            place.share = __builtin_amdgcn_readfirstlane(within % place.shares);
+            place.unit = __builtin_amdgcn_readfirstlane(units_before + __shfl(tiles - own_tiles, owner, 64) + place.row_tile);
+            // A unit's rows before the last are whole tiles.
+            place.first_slot = __builtin_amdgcn_readfirstlane(slots_before + __shfl(slots - own_slots, owner, 64) + place.shares * place.row_tile * kRows);
+            place.share_tiles = length;
+            return true;
+        }
+        workgroups_before += total;
+        units_before += __shfl(tiles, 63, 64);
+        slots_before += __shfl(slots, 63, 64);
+    }
+    return false;
+}
+
 // What a wave needs to know of the keys it loads for one tile: its four latent rows (wave-uniform) and, for waves
 // 0-3, each lane's positional row.
 template <int FORM>
@@ -181,27 +311,60 @@ SINGE_DEVICE void latent_tile_rows(const LatentAttentionArgs& a, unsigned char* 
     // With key splits the units are few and their shares read different keys: the shares of a unit are neighbouring
     // workgroups and so go round the XCDs, which keeps every XCD busy however few units there are (and share s of
     // every unit still meets the same few XCDs when the count of shares is a power of two).
-    unsigned int split = 0, unit;
-    if (splits > 1) {
-        split = blockIdx.x % splits;
-        unit = blockIdx.x / splits;
+    Placement place;
+    bool found;
+    if (a.share_budget != 0) {
+        unsigned int units;
+        found = place_balanced<FORM>(a, blockIdx.x, place, units);
+        if (blockIdx.x == 0)  // the merge's grid covers a.unit_slots units: those past the last have no rows
+            for (unsigned int at = units + threadIdx.x; at < a.unit_slots; at += 64u * kWaves) a.units[at] = LatentUnit{};
     } else {
-        const unsigned int xcd = blockIdx.x & 7u, within = blockIdx.x >> 3;
-        unit = ((within / a.unit_band) * 8u + xcd) * a.unit_band + within % a.unit_band;
+        place.share_tiles = 0;
+        place.shares = splits;
+        if (splits > 1) {
+            place.share = blockIdx.x % splits;
+            place.unit = blockIdx.x / splits;
+        } else {
+            const unsigned int xcd = blockIdx.x & 7u, within = blockIdx.x >> 3;
+            place.share = 0;
+            place.unit = ((within / a.unit_band) * 8u + xcd) * a.unit_band + within % a.unit_band;
+        }
+        found = find_unit<FORM>(a, place.unit, place.sequence, place.row_tile);
+        if (!found && splits > 1 && place.share == 0 && threadIdx.x == 0) a.units[place.unit] = LatentUnit{};
     }
-    unsigned int sequence, row_tile;
-    if (!find_unit<FORM>(a, unit, sequence, row_tile)) return;
-    sequence = __builtin_amdgcn_readfirstlane(sequence);
-    row_tile = __builtin_amdgcn_readfirstlane(row_tile);
+    if (!found) return;
+    // (the same for every lane, which the compiler has lost sight of by here)
+    const unsigned int sequence = __builtin_amdgcn_readfirstlane(place.sequence), row_tile = __builtin_amdgcn_readfirstlane(place.row_tile);
+    const unsigned int split = __builtin_amdgcn_readfirstlane(place.share), unit_shares = __builtin_amdgcn_readfirstlane(place.shares);
+    const unsigned int share_tiles = __builtin_amdgcn_readfirstlane(place.share_tiles);
     const SequenceSpan span = load_span<FORM>(sequence, a.query_offsets, a.page_offsets, a.last_page_lengths, nullptr, a.tokens,
                                               a.page_table, a.page_size);
+    const unsigned long long rows = static_cast<unsigned long long>(span.queries) * a.heads;  // (none where the span is not valid)
+    const unsigned long long first_row = static_cast<unsigned long long>(row_tile) * kRows;
+    const unsigned int unit_rows = first_row >= rows ? 0u : rows - first_row < kRows ? static_cast<unsigned int>(rows - first_row) : kRows;
+    if (a.share_budget == 0) place.first_slot = (static_cast<unsigned long long>(span.query_start) * a.heads + first_row) * splits;
+    // A unit that is not shared out is stored as it is.  (Sequences whose offsets make sense never need more slots than
+    // there are; ones that overlap because others run backwards may, and those others report it.)
+    const bool shared = unit_shares > 1, fits = !shared || place.first_slot + static_cast<unsigned long long>(unit_rows) * unit_shares <= a.slots;
+    if (a.units != nullptr && split == 0 && threadIdx.x == 0 && place.unit < a.unit_slots) {
+        LatentUnit unit = {};
+        if (shared && span.valid && fits) {
+            unit.first_row = static_cast<unsigned long long>(span.query_start) * a.heads + first_row;
+            unit.first_slot = place.first_slot;
+            unit.rows = unit_rows;
+            unit.shares = unit_shares;
+        }
+        a.units[place.unit] = unit;
+    }
     if (!span.valid) {
         if (threadIdx.x == 0) report_index_error(a.status);
         return;
     }
-    const unsigned long long rows = static_cast<unsigned long long>(span.queries) * a.heads;
-    const unsigned long long first_row = static_cast<unsigned long long>(row_tile) * kRows;
-    if (first_row >= rows) return;
+    if (unit_rows == 0 || !fits) return;
+    // (every wave writes the same words, so that none has to wait for another's)
+    if (lane == 0)
+        *reinterpret_cast<ulonglong2*>(lds + kSlotAt) =
+            make_ulonglong2(shared ? place.first_slot + static_cast<unsigned long long>(split) * unit_rows : ~0ull, 0);
     const unsigned int keys = span.keys;
 
     // Queries are the sequence's last tokens, with the CPU path's saturating position (attention.rs:619-627).
@@ -225,8 +388,8 @@ SINGE_DEVICE void latent_tile_rows(const LatentAttentionArgs& a, unsigned char* 
     }
     // With key splits this workgroup takes one share of the tiles; a share may be empty.
     unsigned int first_tile = 0, tiles = (key_end + kKeys - 1) / kKeys;
-    if (splits > 1) {
-        const unsigned int share = (tiles + splits - 1) / splits;
+    if (shared) {
+        const unsigned int share = share_tiles != 0 ? share_tiles : (tiles + splits - 1) / splits;
         first_tile = split * share;
         tiles = tiles < first_tile + share ? tiles : first_tile + share;
     }
@@ -534,8 +697,9 @@ SINGE_DEVICE void latent_tile_rows(const LatentAttentionArgs& a, unsigned char* 
     // Normalise and store; a row that sees no key stays zero and has a log-sum-exp of -inf.
     const float sum = across_groups_sum(running_sum);
     const float inverse = sum > 0.0f ? 1.0f / sum : 0.0f;
-    if (row_valid && splits > 1) {
-        const size_t slot = static_cast<size_t>(split) * a.tokens * a.heads + flat;
+    const unsigned long long share_slot = *reinterpret_cast<const unsigned long long*>(lds + kSlotAt);
+    if (row_valid && share_slot != ~0ull) {
+        const size_t slot = static_cast<size_t>(share_slot) + 16u * wave + column;
         float* row = a.partial_out + slot * kLatent + 4u * g;
 #pragma unroll
         for (int db = 0; db < kDimBlocks; ++db)
@@ -566,21 +730,17 @@ SINGE_DEVICE void latent_tile_rows(const LatentAttentionArgs& a, unsigned char* 
 // are asked for four at a time.
 constexpr unsigned int kCombineBlocks = kRows / 4;
 
-template <class Half, int FORM, bool ANY>
+template <class Half, bool ANY>
 SINGE_DEVICE void latent_combine_rows(const LatentAttentionArgs& a) {
     const unsigned int wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
-    // Workgroups map to (sequence, row tile) as in the attention kernel, so only rows that kernel wrote are read.
-    unsigned int sequence, row_tile;
-    if (!find_unit<FORM>(a, blockIdx.x / kCombineBlocks, sequence, row_tile)) return;
-    const SequenceSpan span = load_span<FORM>(sequence, a.query_offsets, a.page_offsets, a.last_page_lengths, nullptr, a.tokens,
-                                              a.page_table, a.page_size);
-    if (!span.valid) return;  // the attention kernel has reported it
-    const unsigned long long rows = static_cast<unsigned long long>(span.queries) * a.heads;
-    const size_t rows_total = static_cast<size_t>(a.tokens) * a.heads;
-    const unsigned long long local = static_cast<unsigned long long>(row_tile) * kRows + 4u * (blockIdx.x % kCombineBlocks) + wave;
-    if (local >= rows) return;
-    const size_t row = (static_cast<size_t>(span.query_start) + local / a.heads) * a.heads + local % a.heads;
-    const float mine = lane < a.splits ? a.partial_lse[lane * rows_total + row] : -INFINITY;
+    // The attention kernel has left a record of every unit: where its rows and its partial rows are and how many of
+    // either (no rows where there is nothing to merge).
+    const LatentUnit unit = a.units[blockIdx.x / kCombineBlocks];
+    const unsigned int local = 4u * (blockIdx.x % kCombineBlocks) + wave, splits = unit.shares;
+    if (local >= unit.rows) return;
+    const size_t row = static_cast<size_t>(unit.first_row) + local;
+    const size_t first_slot = static_cast<size_t>(unit.first_slot) + local;
+    const float mine = lane < splits ? a.partial_lse[first_slot + static_cast<size_t>(lane) * unit.rows] : -INFINITY;
     float largest = mine;
 #pragma unroll
     for (int step = 32; step >= 1; step >>= 1) largest = fmaxf(largest, __shfl_xor(largest, step, 64));
@@ -590,8 +750,8 @@ SINGE_DEVICE void latent_combine_rows(const LatentAttentionArgs& a) {
 #pragma unroll
     for (int step = 32; step >= 1; step >>= 1) total += __shfl_xor(total, step, 64);
     float acc[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-    const float* part = a.partial_out + row * kLatent + 8u * lane;
-    const size_t share_stride = rows_total * kLatent;
+    const float* part = a.partial_out + first_slot * kLatent + 8u * lane;
+    const size_t share_stride = static_cast<size_t>(unit.rows) * kLatent;
     auto fold = [&](float w, const float4& low, const float4& high) __attribute__((always_inline)) {
         acc[0] = fmaf(w, low.x, acc[0]); acc[1] = fmaf(w, low.y, acc[1]);
         acc[2] = fmaf(w, low.z, acc[2]); acc[3] = fmaf(w, low.w, acc[3]);
@@ -599,7 +759,7 @@ SINGE_DEVICE void latent_combine_rows(const LatentAttentionArgs& a) {
         acc[6] = fmaf(w, high.z, acc[6]); acc[7] = fmaf(w, high.w, acc[7]);
     };
     unsigned int s = 0;
-    for (; s + 4 <= a.splits; s += 4) {
+    for (; s + 4 <= splits; s += 4) {
         float4 low[4], high[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -610,7 +770,7 @@ SINGE_DEVICE void latent_combine_rows(const LatentAttentionArgs& a) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) fold(__shfl(weight, s + i, 64), low[i], high[i]);
     }
-    for (; s < a.splits; ++s) {
+    for (; s < splits; ++s) {
         const float* from = part + s * share_stride;
         fold(__shfl(weight, s, 64), *reinterpret_cast<const float4*>(from), *reinterpret_cast<const float4*>(from + 4));
     }
@@ -649,10 +809,7 @@ SINGE_DEVICE void latent_tile_body(const LatentAttentionArgs& a, unsigned char* 
 
 #define SINGE_LATENT_COMBINE_KERNEL(NAME, HALF, ANY)                                             \
     extern "C" __global__ __launch_bounds__(256) void NAME(LatentAttentionArgs args) {          \
-        if (args.wide_index)                                                                    \
-            latent_mfma::latent_combine_rows<prefill::HALF, kCsrI64, ANY>(args);                \
-        else                                                                                    \
-            latent_mfma::latent_combine_rows<prefill::HALF, kCsrI32, ANY>(args);                \
+        latent_mfma::latent_combine_rows<prefill::HALF, ANY>(args);                             \
     }
 
 SINGE_LATENT_COMBINE_KERNEL(singe_paged_mla_attention_combine_bf16, Bf16, false)

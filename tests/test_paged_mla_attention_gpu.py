@@ -399,3 +399,68 @@ def random_latent_case(seed):
 @pytest.mark.parametrize("seed", range(24))
 def test_random_shapes_over_pages_of_whole_tiles_and_others(seed):
     random_latent_case(seed)
+
+
+@pytest.mark.parametrize("index_dtype", [torch.int32, torch.int64])
+@pytest.mark.parametrize("count,heads,low,high,queries", [
+    (1, 16, 300, 300, 3),       # one unit, shared out as far as four tiles a share go
+    (64, 128, 1, 1100, 1),      # a wave's lanes are full: sequences from one key to nine shares
+    (65, 16, 0, 900, 2),        # one sequence in the second chunk of lanes, some without keys
+    (129, 16, 40, 700, 1),      # three chunks
+    (200, 24, 0, 700, 6),       # four chunks, two units to some sequences, more units than a share each leaves room for
+    (12, 128, 500, 1500, 3),    # several units to every sequence
+])
+def test_shares_of_one_length_over_unequal_sequences(count, heads, low, high, queries, index_dtype):
+    """The shares the kernel deals out by itself, whose number differs from sequence to sequence: against the CPU, and the
+    rows of sequences that are not shared out bit for bit those of the unsplit kernel."""
+    rng = np.random.default_rng(count + heads)
+    keys = [int(n) for n in rng.integers(low, high + 1, size=count)]
+    counts = [int(n) for n in rng.integers(0 if count > 1 else queries, queries + 1, size=count)]
+    counts[0] = queries
+    page_size = 32
+    query_offsets, page_offsets, last, needed = [0], [0], [], 0
+    for wanted, held in zip(counts, keys):
+        query_offsets.append(query_offsets[-1] + wanted)
+        pages = (held + page_size - 1) // page_size
+        needed += pages
+        page_offsets.append(needed)
+        last.append(0 if held == 0 else held - (pages - 1) * page_size)
+    table = [int(page) for page in rng.permutation(needed + 1)[:needed]]
+    tokens = query_offsets[-1]
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(count)
+    rand = lambda *shape: torch.randn(shape, generator=gen, device="cuda").to(torch.bfloat16)
+    device = [rand(tokens, heads, 512), rand(tokens, heads, 64), rand(needed + 1, page_size, 512), rand(needed + 1, page_size, 64)]
+    index = lambda entries: torch.tensor(entries, dtype=index_dtype, device="cuda")
+    paging = neural.Paging(index(query_offsets), index(page_offsets), index(table), index(last))
+    options = neural.AttentionOptions(causal=True)
+    whole, whole_lse = neural.paged_mla_attention(*device, paging, options, scratch=False)
+    out, lse = neural.paged_mla_attention(*device, paging, options)
+    torch.cuda.synchronize()
+    status, want, want_lse = oracle.paged_mla_attention(*[tensor.float().cpu().numpy() for tensor in device], query_offsets, page_offsets, table,
+                                                        last, causal=True, threads=8)
+    assert status == 0
+    got, got_lse = out.float().cpu().numpy(), lse.cpu().numpy()
+    gap = np.abs(got - want)
+    assert gap.max() <= 2e-2 and gap.mean() <= 2e-3, (gap.max(), gap.mean())
+    empty = np.isneginf(want_lse)
+    assert np.array_equal(np.isneginf(got_lse), empty) and not got[empty].any()
+    assert np.abs(got_lse[~empty] - want_lse[~empty]).max(initial=0.0) <= 5e-3
+    for sequence, held in enumerate(keys):
+        if held <= 4 * 32:  # a share is four tiles of 32 keys at least
+            rows = slice(query_offsets[sequence], query_offsets[sequence + 1])
+            assert torch.equal(out[rows], whole[rows]) and torch.equal(lse[rows], whole_lse[rows]), sequence
+
+
+def test_offsets_that_run_backwards_are_reported_by_a_shared_out_step():
+    """Sequences 0 and 2 both claim every token because sequence 1 runs backwards: reported, nothing out of bounds (the
+    partial rows such sequences would need are more than there are)."""
+    heads, page_size, pages, tokens = 128, 64, 64, 64
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(1)
+    rand = lambda *shape: torch.randn(shape, generator=gen, device="cuda").to(torch.bfloat16)
+    device = [rand(tokens, heads, 512), rand(tokens, heads, 64), rand(pages, page_size, 512), rand(pages, page_size, 64)]
+    index = lambda entries: torch.tensor(entries, dtype=torch.int32, device="cuda")
+    paging = neural.Paging(index([0, tokens, 0, tokens]), index([0, pages, pages, 2 * pages]), index(list(range(pages)) * 2), index([64, 0, 64]))
+    with pytest.raises(error.IndexOutOfBounds):
+        neural.paged_mla_attention(*device, paging, neural.AttentionOptions(causal=True))
