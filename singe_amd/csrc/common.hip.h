@@ -118,3 +118,20 @@ SINGE_DEVICE float fast_log2(float x) { return __builtin_amdgcn_logf(x); }
 // tanh(x) = 1 - 2 / (e^(2x) + 1): one exponential and one reciprocal; exact at both infinities, absolute error
 // about 1e-7 near zero (the subtraction), which a capped score multiplies by the cap.
 SINGE_DEVICE float fast_tanh(float x) { return 1.0f - 2.0f * __builtin_amdgcn_rcpf(fast_exp2(x * (2.0f * kLog2e)) + 1.0f); }
+
+// One direct-to-LDS load: every active lane's 16 bytes at `shared_base` (the same for every lane, kept in scalar
+// registers) + `lane_offset` go to the byte address `lds_byte_address` + 16 * lane of LDS.  Written as text so that the
+// compiler keeps counting its own LDS reads and loads as usual (it makes every LDS read after the built-in form wait for
+// all of them, and the first one for the load itself): the caller waits for these loads itself.  M0 carries the LDS
+// address; it is read when the load issues, so the statement puts back what M0 held.
+SINGE_DEVICE void load_16_to_lds(const unsigned char* shared_base, unsigned int lane_offset, unsigned int lds_byte_address) {
+    const unsigned int base = __builtin_amdgcn_readfirstlane(lds_byte_address);
+    const unsigned long long bits = reinterpret_cast<unsigned long long>(shared_base);
+    // (the built-in returns an int: through unsigned int first, or a low word with its top bit set would fill the high word)
+    const unsigned int low_word = __builtin_amdgcn_readfirstlane(static_cast<unsigned int>(bits));
+    const unsigned int high_word = __builtin_amdgcn_readfirstlane(static_cast<unsigned int>(bits >> 32));
+    const unsigned long long scalar = static_cast<unsigned long long>(low_word) | (static_cast<unsigned long long>(high_word) << 32);
+    unsigned int kept;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %3\n\ts_mov_b32 m0, %0"
+                 : "=&s"(kept) : "s"(base), "v"(lane_offset), "s"(scalar) : "memory");
+}

@@ -95,19 +95,6 @@ SINGE_DEVICE void load_to_lds(const unsigned char* shared_base, unsigned int lan
                  : "=&s"(kept) : "s"(base), "v"(lane_offset), "s"(scalar) : "memory");
 }
 
-// The same with the destination as the byte address in LDS that M0 takes (a pointer into LDS costs a null test and a
-// select on its way there).
-SINGE_DEVICE void load_to_lds(const unsigned char* shared_base, unsigned int lane_offset, unsigned int lds_byte_address) {
-    const unsigned int base = __builtin_amdgcn_readfirstlane(lds_byte_address);
-    const unsigned long long bits = reinterpret_cast<unsigned long long>(shared_base);
-    const unsigned int low_word = __builtin_amdgcn_readfirstlane(static_cast<unsigned int>(bits));
-    const unsigned int high_word = __builtin_amdgcn_readfirstlane(static_cast<unsigned int>(bits >> 32));
-    const unsigned long long scalar = static_cast<unsigned long long>(low_word) | (static_cast<unsigned long long>(high_word) << 32);
-    unsigned int kept;
-    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %3\n\ts_mov_b32 m0, %0"
-                 : "=&s"(kept) : "s"(base), "v"(lane_offset), "s"(scalar) : "memory");
-}
-
 // Where the chunk permutation of a latent row puts things: see the header comment.
 SINGE_DEVICE unsigned int chunk_flip(unsigned int key) {
     const unsigned int pair = (key & 3u) | ((((key >> 2) ^ (key >> 3)) & 1u) << 2);
@@ -498,12 +485,12 @@ SINGE_DEVICE void latent_tile_rows(const LatentAttentionArgs& a, unsigned char* 
             if (piece < 4) {
                 const unsigned int row = wave + 8u * piece, kept = row < from.last ? row : from.last;
                 if (!ANY || lane_chunk[piece & 1] < 16u * latent_chunks)
-                    load_to_lds(from.latent + kept * latent_row_bytes, lane_chunk[piece & 1], lds_start + stage_at + row * kLatentRowBytes);
+                    load_16_to_lds(from.latent + kept * latent_row_bytes, lane_chunk[piece & 1], lds_start + stage_at + row * kLatentRowBytes);
             } else if (wave < 4) {
                 const unsigned int kept = positional_row < from.last ? positional_row : from.last;
                 if (!ANY || positional_chunk < 16u * positional_chunks)
-                    load_to_lds(from.positional, kept * positional_row_bytes + positional_chunk,
-                                lds_start + stage_at + kLatentTileBytes + 8u * wave * kPositionalRowBytes);
+                    load_16_to_lds(from.positional, kept * positional_row_bytes + positional_chunk,
+                                   lds_start + stage_at + kLatentTileBytes + 8u * wave * kPositionalRowBytes);
             }
             return;
         }

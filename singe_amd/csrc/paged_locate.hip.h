@@ -51,6 +51,105 @@ SINGE_DEVICE unsigned int entries_before_longest_first(const PagedAttentionArgs&
     return before;
 }
 
+// a.alternate (at most 64 * kAlternateChunks sequences, some of which decode beside others that bring row tiles): the
+// compact list takes the sequences of at most sixteen packed rows by themselves, longest first, and alternates runs of
+// them with runs of the others' row tiles, as many of either as an XCD's compute units hold one of.  The first bring the
+// cache from memory with the matrix cores all but idle (paged_narrow.hip.h), the others use the matrix cores on keys that
+// the XCD's L2 holds; side by side on a compute unit they take little from each other, and a long sequence that starts last
+// would run on by itself.  (Lengths are compared up to 4095 pages.  Sequences whose offsets make no sense come first of
+// all, so that one is in the grid however many tiles the others claim.)
+// Finds the entry's sequence and row tile; false past the list's end.
+constexpr int kAlternateChunks = 4;
+template <int FORM, unsigned int ROWS>
+SINGE_DEVICE bool locate_alternating(const PagedAttentionArgs& a, unsigned int entry, unsigned int& sequence, unsigned int& row_tile) {
+    const unsigned int lane = threadIdx.x & 63u, groups = a.heads / a.kv_heads;
+    constexpr unsigned int kMostHeld = 4095u, kHeldBits = 13u;
+    unsigned long long narrow[kAlternateChunks];
+    unsigned int held[kAlternateChunks], tiles[kAlternateChunks], through[kAlternateChunks];  // tiles: of wide sequences, and their inclusive prefix sums
+    unsigned int narrow_count = 0, wide_count = 0;
+#pragma unroll
+    for (int c = 0; c < kAlternateChunks; ++c) {
+        narrow[c] = 0;
+        held[c] = tiles[c] = through[c] = 0;
+        if (64u * c >= a.sequences) continue;
+        const unsigned int s = 64u * c + lane;
+        bool is_narrow = false;
+        if (s < a.sequences) {
+            const long long count = read_index<FORM>(a.query_offsets, s + 1) - read_index<FORM>(a.query_offsets, s);
+            const long long pages = read_index<FORM>(a.page_offsets, s + 1) - read_index<FORM>(a.page_offsets, s);
+            const bool bad = count < 0 || count > static_cast<long long>(a.tokens);
+            const unsigned long long rows = bad ? 0ull : static_cast<unsigned long long>(count) * groups;
+            is_narrow = rows <= 16u;
+            held[c] = bad ? 2u * kMostHeld + 1u : pages < 0 ? 0u : pages > static_cast<long long>(kMostHeld) ? kMostHeld : static_cast<unsigned int>(pages);
+            tiles[c] = is_narrow ? 0u : static_cast<unsigned int>((rows + ROWS - 1) / ROWS);
+        }
+        narrow[c] = __ballot(is_narrow);
+        narrow_count += static_cast<unsigned int>(__builtin_popcountll(narrow[c]));
+        through[c] = tiles[c];
+#pragma unroll
+        for (int step = 1; step < 64; step <<= 1) {
+            const unsigned int below = __shfl_up(through[c], step, 64);
+            if (lane >= static_cast<unsigned int>(step)) through[c] += below;
+        }
+        wide_count += __builtin_amdgcn_readlane(through[c], 63);
+    }
+    const unsigned int run = a.kv_heads >= 256u ? 1u : 256u / a.kv_heads;
+    const unsigned int narrow_runs = narrow_count / run, wide_runs = wide_count / run, pairs = narrow_runs < wide_runs ? narrow_runs : wide_runs;
+    bool takes_narrow;
+    unsigned int index;
+    if (entry < 2u * run * pairs) {
+        const unsigned int within = entry % (2u * run);
+        takes_narrow = within >= run;
+        index = entry / (2u * run) * run + (takes_narrow ? within - run : within);
+    } else {
+        const unsigned int rest = entry - 2u * run * pairs, wide_left = wide_count - run * pairs;
+        takes_narrow = rest >= wide_left;
+        index = run * pairs + (takes_narrow ? rest - wide_left : rest);
+    }
+    if (takes_narrow) {
+        if (index >= narrow_count) return false;
+        // The index-th longest: bit by bit from the top, keep the candidates that have the bit where enough of them do.
+#pragma unroll 1
+        for (int bit = kHeldBits - 1; bit >= 0; --bit) {
+            unsigned long long with[kAlternateChunks];
+            unsigned int count = 0;
+#pragma unroll
+            for (int c = 0; c < kAlternateChunks; ++c) {
+                with[c] = narrow[c] == 0 ? 0ull : __ballot((held[c] >> bit & 1u) != 0u) & narrow[c];
+                count += static_cast<unsigned int>(__builtin_popcountll(with[c]));
+            }
+            const bool enough = index < count;
+            if (!enough) index -= count;
+#pragma unroll
+            for (int c = 0; c < kAlternateChunks; ++c) narrow[c] = enough ? with[c] : narrow[c] & ~with[c];
+        }
+#pragma unroll
+        for (int c = 0; c < kAlternateChunks; ++c) {
+            const unsigned int here = static_cast<unsigned int>(__builtin_popcountll(narrow[c]));
+            if (index < here) {
+                const bool mine = (narrow[c] >> lane & 1ull) != 0 && static_cast<unsigned int>(__builtin_popcountll(narrow[c] & ((1ull << lane) - 1ull))) == index;
+                sequence = 64u * c + static_cast<unsigned int>(__builtin_ctzll(__ballot(mine)));
+                row_tile = 0;
+                return true;
+            }
+            index -= here;
+        }
+        return false;
+    }
+#pragma unroll
+    for (int c = 0; c < kAlternateChunks; ++c) {
+        const unsigned int total = __builtin_amdgcn_readlane(through[c], 63);
+        if (index < total) {
+            const unsigned int owner = static_cast<unsigned int>(__builtin_ctzll(__ballot(index < through[c])));
+            sequence = 64u * c + owner;
+            row_tile = index - (__builtin_amdgcn_readlane(through[c], owner) - __builtin_amdgcn_readlane(tiles[c], owner));
+            return true;
+        }
+        index -= total;
+    }
+    return false;
+}
+
 // kPacked only: packed sequences may overlap, and their row tiles can then outnumber the list the grid was sized for.
 // Workgroups come back for another `round` of entries as long as `more` says there may be one.
 template <int FORM, unsigned int ROWS>
@@ -71,6 +170,14 @@ SINGE_DEVICE bool locate(const PagedAttentionArgs& a, unsigned int& unit, unsign
         if (entry >= a.row_tiles) return false;
         if constexpr (FORM == kPacked) entry += static_cast<unsigned long long>(round) * a.row_tiles;
         more = true;
+        if constexpr (FORM == kCsrI32 || FORM == kCsrI64) {
+            if (a.alternate != 0) {
+                unsigned int sequence;
+                if (!locate_alternating<FORM, ROWS>(a, entry, sequence, row_tile)) return false;
+                unit = sequence * a.kv_heads + kv_head;
+                return true;
+            }
+        }
         const unsigned int lane = threadIdx.x & 63u, groups = a.heads / a.kv_heads;
         auto tiles_of = [&](unsigned int s) __attribute__((always_inline)) {
             long long count;

@@ -464,3 +464,51 @@ def test_pages_beyond_two_and_four_gib_of_a_cache_read_the_same_as_the_first_pag
     torch.cuda.synchronize()
     assert torch.equal(far, near) and torch.equal(far_lse, near_lse)
     assert far.float().abs().max().item() > 0.1
+
+
+NARROW = [(1, 1), (2, 15), (1, 16), (2, 17), (1, 63), (2, 64), (1, 65), (2, 0), (0, 40), (2, 1), (1, 129), (2, 1000)]
+
+
+@pytest.mark.parametrize("options", OPTIONS + [neural.AttentionOptions(causal=True, scale=-0.07, window=33)])
+@pytest.mark.parametrize("heads,kv_heads,page_size,dim,index_dtype", [
+    (8, 1, 16, 128, torch.int64), (12, 3, 32, 64, torch.int32), (6, 6, 64, 96, torch.int64), (16, 2, 16, 32, torch.int32), (14, 2, 128, 128, torch.int32)])
+def test_sequences_of_at_most_sixteen_rows_beside_a_chunk(heads, kv_heads, page_size, dim, index_dtype, options):
+    """Groups of sixteen keys dealt to four waves: keys either side of a group's, a turn's and a page's end, sequences with
+    fewer groups than waves, one to sixteen rows, without queries or keys, beside a chunk that fills row tiles."""
+    run_case(NARROW + [(150, 400)], heads, kv_heads, page_size, options, index_dtype=index_dtype, seed=dim + heads, dim=dim)
+
+
+@pytest.mark.parametrize("heads,kv_heads,splits", [(8, 1, 0), (8, 1, 3), (4, 2, 1)])
+def test_sequences_of_at_most_sixteen_rows_over_many_keys(heads, kv_heads, splits):
+    # a wave looks 64 groups' page ids up at a time: 64 turns are 4096 keys
+    _native.lib().singe_hip_set_paged_attention_splits(splits)
+    try:
+        run_case([(1, 4095), (2, 4096), (1, 4160), (1, 8300), (40, 100)], heads, kv_heads, 16, neural.AttentionOptions(causal=True), seed=splits)
+    finally:
+        _native.lib().singe_hip_set_paged_attention_splits(0)
+
+
+@pytest.mark.parametrize("index_dtype", [torch.int32, torch.int64])
+@pytest.mark.parametrize("heads,kv_heads,decoding,chunks", [(8, 1, 60, 2), (16, 2, 100, 12), (6, 3, 230, 20), (32, 32, 40, 3), (64, 8, 66, 4)])
+def test_decoding_sequences_and_row_tiles_take_turns_in_the_grid(heads, kv_heads, decoding, chunks, index_dtype):
+    """Long enough on average that the list of row tiles alternates runs of either: more sequences than a wave has lanes,
+    fewer of either than a run, every sequence attended."""
+    rng = np.random.default_rng(heads + decoding)
+    sequences = [(1, int(n)) for n in rng.integers(300, 1500, size=decoding)]
+    sequences += [(int(q), int(q) + int(n)) for q, n in zip(rng.integers(17, 90, size=chunks), rng.integers(0, 900, size=chunks))]
+    order = rng.permutation(len(sequences))
+    run_case([sequences[i] for i in order], heads, kv_heads, 16, neural.AttentionOptions(causal=True), index_dtype=index_dtype, seed=decoding)
+
+
+def test_offsets_that_run_backwards_are_reported_from_a_list_that_takes_turns():
+    heads, kv_heads, page_size, pages = 16, 2, 16, 80
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(2)
+    rand = lambda *shape: torch.randn(shape, generator=gen, device="cuda").to(torch.bfloat16)
+    index = lambda values: torch.tensor(values, dtype=torch.int32, device="cuda")
+    # sequence 1 runs backwards, and the tokens are claimed three times over
+    paging = neural.Paging(index([0, 300, 0, 300] + list(range(240, 301)) + [0, 300]), index([pages * i for i in range(67)]),
+                           index([i % pages for i in range(66 * pages)]), index([16] * 66))
+    with pytest.raises(error.IndexOutOfBounds):
+        neural.paged_attention(rand(300, heads, 128), rand(pages, page_size, kv_heads, 128), rand(pages, page_size, kv_heads, 128), paging,
+                               neural.AttentionOptions(causal=True))
