@@ -481,12 +481,32 @@ SINGE_HIP_API void singe_hip_set_paged_attention_splits(uint32_t splits);
  * 64 (only calls at a head_dim that is a multiple of 16 up to 128 with a page size that is a power of two of at least 16 keys and a positive scale,
  * without a softcap, a window or key splits have that form, with or without the fused query rotation; others keep
  * 32), or 0 (the default): 64 where the call has that form and its 256-row tiles still fill the chip, unless it is a step
- * of few new tokens beside many sequences that decode (head_dim 64 up, at most 1024 tokens more than sequences, at most
- * 9/16 of a whole 256-row tile a sequence).  Packed prefill (singe_hip_ragged_kv_prefill_attention_*) does not look at it. */
+ * of chunks beside many sequences that decode (head_dim 64 up; the line, which depends on the keys a sequence has on
+ * average, stands at two_tiles_a_wave in csrc/paged_attention.cpp).  Packed prefill (singe_hip_ragged_kv_prefill_attention_*) does not look at it. */
 SINGE_HIP_API void singe_hip_set_paged_attention_rows_per_wave(uint32_t rows);
 /* What a bf16 / f16 call of this problem takes when it is given scratch: 32 or 64 rows a wave,
  * 0 when the head dimension has no matrix-core build. */
 SINGE_HIP_API uint32_t singe_hip_paged_attention_rows_per_wave(const SingePagedAttentionProblem* problem);
+/* singe_hip_paged_attention_scratch_* for an output that holds nothing yet: the rows of tokens that no valid sequence owns
+ * are written too, zeros with a log-sum-exp of -inf, where the others leave them as they are.  data_type SINGE_HIP_BF16 or
+ * SINGE_HIP_F16 at a head_dim that is a multiple of 16 up to 128 and at least one sequence; SINGE_HIP_UNSUPPORTED_WIDTH
+ * otherwise.  `scratch` may be null. */
+SINGE_HIP_API int32_t singe_hip_paged_attention_every_row(
+    int32_t data_type,
+    void* stream,
+    const void* query_rows,
+    const void* key_cache,
+    const void* value_cache,
+    const void* query_offsets,
+    const void* page_offsets,
+    const void* pages,
+    const void* last_page_lengths,
+    void* output,
+    float* lse,
+    uint32_t* status,
+    void* scratch,
+    size_t scratch_bytes,
+    const SingePagedAttentionProblem* problem);
 SINGE_HIP_API int32_t singe_hip_paged_attention_scratch_bf16(
     void* stream,
     const uint16_t* query_rows,
@@ -973,6 +993,25 @@ SINGE_HIP_API int32_t singe_hip_paged_mla_attention(
  * most 64); it changes what ..._scratch_bytes returns. */
 SINGE_HIP_API size_t singe_hip_paged_mla_attention_scratch_bytes(const SingePagedMlaAttentionProblem* problem);
 SINGE_HIP_API void singe_hip_set_paged_mla_attention_splits(uint32_t splits);
+/* singe_hip_paged_mla_attention_scratch for an output that holds nothing yet: the rows of tokens that no valid sequence
+ * owns are written too, zeros with a log-sum-exp of -inf, where the others leave them as they are.  For the shapes on the
+ * matrix cores and at least one sequence; SINGE_HIP_UNSUPPORTED_WIDTH otherwise.  `scratch` may be null. */
+SINGE_HIP_API int32_t singe_hip_paged_mla_attention_every_row(
+    void* stream,
+    const void* latent_queries,
+    const void* positional_queries,
+    const void* latent_cache,
+    const void* positional_cache,
+    const void* query_offsets,
+    const void* page_offsets,
+    const void* pages,
+    const void* last_page_lengths,
+    void* output,
+    float* lse,
+    uint32_t* status,
+    void* scratch,
+    size_t scratch_bytes,
+    const SingePagedMlaAttentionProblem* problem);
 SINGE_HIP_API int32_t singe_hip_paged_mla_attention_scratch(
     void* stream,
     const void* latent_queries,

@@ -330,6 +330,8 @@ def bind(path: str) -> ctypes.CDLL:
     handle.singe_hip_rotary_paged_attention_f16.restype = i32
     handle.singe_hip_paged_attention_scratch_bf16.argtypes = [c_void] * 12 + [ctypes.c_size_t, ctypes.POINTER(PagedAttentionProblemC)]
     handle.singe_hip_paged_attention_scratch_bf16.restype = i32
+    handle.singe_hip_paged_attention_every_row.argtypes = [i32] + [c_void] * 12 + [ctypes.c_size_t, ctypes.POINTER(PagedAttentionProblemC)]
+    handle.singe_hip_paged_attention_every_row.restype = i32
     handle.singe_hip_paged_attention_scratch_bytes.argtypes = [ctypes.POINTER(PagedAttentionProblemC)]
     handle.singe_hip_paged_attention_scratch_bytes.restype = ctypes.c_size_t
     handle.singe_hip_set_paged_attention_splits.argtypes = [ctypes.c_uint32]
@@ -338,6 +340,8 @@ def bind(path: str) -> ctypes.CDLL:
     handle.singe_hip_paged_mla_attention.restype = i32
     handle.singe_hip_paged_mla_attention_scratch.argtypes = [c_void] * 13 + [c_size, ctypes.POINTER(PagedMlaAttentionProblemC)]
     handle.singe_hip_paged_mla_attention_scratch.restype = i32
+    handle.singe_hip_paged_mla_attention_every_row.argtypes = handle.singe_hip_paged_mla_attention_scratch.argtypes
+    handle.singe_hip_paged_mla_attention_every_row.restype = i32
     handle.singe_hip_paged_mla_attention_scratch_bytes.argtypes = [ctypes.POINTER(PagedMlaAttentionProblemC)]
     handle.singe_hip_paged_mla_attention_scratch_bytes.restype = ctypes.c_size_t
     handle.singe_hip_set_paged_mla_attention_splits.argtypes = [ctypes.c_uint32]

@@ -178,6 +178,8 @@ struct PagedAttentionArgs {
     uint32_t table_type = 0;                  // SingeElement of cos and sin
     uint32_t has_query_norm = 0;              // RMS norm over the head dimension before the rotation
     float query_eps = 0.0f;
+    // Workgroups from this one on clear the rows of tokens that no valid sequence owns (clear_unowned_tokens); 0: none do.
+    uint32_t clear_from = 0;
 };
 
 // singe_mfma_ceiling_*: the register-only product loop.
@@ -349,6 +351,7 @@ struct LatentAttentionArgs {
     uint32_t unit_slots;
     uint64_t slots;
     LatentUnit* units;               // null without splits
+    uint32_t clear_from;             // matrix-core kernel: workgroups from this one on clear the rows of tokens no valid sequence owns; 0: none do
 };
 
 // singe_rotary_cache_write_*: contiguous operands of one element type; angles may be f32.

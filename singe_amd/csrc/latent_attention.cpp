@@ -73,9 +73,11 @@ Shares latent_shares(const SingePagedMlaAttentionProblem& p) {
 int32_t paged_mla_attention(void* stream, const void* latent_queries, const void* positional_queries, const void* latent_cache,
                             const void* positional_cache, const void* query_offsets, const void* page_offsets, const void* pages,
                             const void* last_page_lengths, void* output, float* lse, uint32_t* status, void* scratch,
-                            size_t scratch_bytes, const SingePagedMlaAttentionProblem* problem) {
+                            size_t scratch_bytes, const SingePagedMlaAttentionProblem* problem, bool every_row = false) {
     if (problem == nullptr) return fail(SINGE_HIP_NULL_POINTER, "problem");
     const SingePagedMlaAttentionProblem& p = *problem;
+    if (every_row && (!on_matrix_cores(p) || p.sequences <= 0))
+        return fail(SINGE_HIP_UNSUPPORTED_WIDTH, "paged_mla_attention_every_row", static_cast<uint64_t>(p.latent_dim));
     // paged_mla_attention_problem: a page holds at least one key and the latent width is positive; the
     // positional width may be zero.
     if (p.tokens < 0 || p.heads < 0 || p.latent_dim <= 0 || p.position_dim < 0 || p.page_size <= 0 || p.sequences < 0 ||
@@ -136,6 +138,7 @@ int32_t paged_mla_attention(void* stream, const void* latent_queries, const void
     args.splits = 1;
     args.share_budget = 0;
     args.slots = 0;
+    args.clear_from = 0;
     args.unit_slots = 0;
     args.units = nullptr;
     args.page_shift = -1;
@@ -169,7 +172,11 @@ int32_t paged_mla_attention(void* stream, const void* latent_queries, const void
         const uint64_t band = surely_live >= 256 ? 32 : (surely_live + 7) / 8;
         const uint64_t rounds = (blocks + 8 * band - 1) / (8 * band);
         args.unit_band = static_cast<uint32_t>(band);
-        const uint64_t grid = shares.budget > 0 ? shares.budget : split ? blocks * shares.fixed : rounds * 8 * band;
+        uint64_t grid = shares.budget > 0 ? shares.budget : split ? blocks * shares.fixed : rounds * 8 * band;
+        if (every_row) {  // one workgroup more for 512 tokens
+            args.clear_from = static_cast<uint32_t>(grid);
+            grid += (static_cast<uint64_t>(p.tokens) + 511) / 512;
+        }
         if (grid > 0x7fffffffull) return fail(SINGE_HIP_UNSUPPORTED_CONFIGURATION, "too many workgroups");
         const bool bf16 = p.data_type == SINGE_HIP_BF16, built = built_shape(p);
         const KernelId tiles_kernel = built ? (bf16 ? kLatentTilesBf16 : kLatentTilesF16) : (bf16 ? kLatentTilesAnyBf16 : kLatentTilesAnyF16);
@@ -211,4 +218,14 @@ extern "C" int32_t singe_hip_paged_mla_attention_scratch(void* stream, const voi
                                                          const SingePagedMlaAttentionProblem* problem) {
     return paged_mla_attention(stream, latent_queries, positional_queries, latent_cache, positional_cache, query_offsets, page_offsets,
                                pages, last_page_lengths, output, lse, status, scratch, scratch_bytes, problem);
+}
+
+extern "C" int32_t singe_hip_paged_mla_attention_every_row(void* stream, const void* latent_queries, const void* positional_queries,
+                                                           const void* latent_cache, const void* positional_cache,
+                                                           const void* query_offsets, const void* page_offsets, const void* pages,
+                                                           const void* last_page_lengths, void* output, float* lse, uint32_t* status,
+                                                           void* scratch, size_t scratch_bytes,
+                                                           const SingePagedMlaAttentionProblem* problem) {
+    return paged_mla_attention(stream, latent_queries, positional_queries, latent_cache, positional_cache, query_offsets, page_offsets,
+                               pages, last_page_lengths, output, lse, status, scratch, scratch_bytes, problem, true);
 }

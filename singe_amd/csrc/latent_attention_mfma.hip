@@ -776,6 +776,18 @@ SINGE_DEVICE void latent_combine_rows(const LatentAttentionArgs& a) {
 
 template <class Half, bool ANY>
 SINGE_DEVICE void latent_tile_body(const LatentAttentionArgs& a, unsigned char* lds) {
+    if (a.clear_from != 0 && blockIdx.x >= a.clear_from) {
+        constexpr unsigned int kThreads = 64u * kWaves;
+        unsigned int* owned = reinterpret_cast<unsigned int*>(lds);
+        const unsigned int first = kThreads * (blockIdx.x - a.clear_from), token_bytes = a.heads * a.latent_dim * 2u;
+        if (a.wide_index)
+            clear_unowned_tokens<kCsrI64, kThreads>(owned, first, a.query_offsets, a.page_offsets, a.last_page_lengths, a.tokens, a.sequences,
+                                                    a.page_table, a.page_size, a.output, token_bytes, a.lse, a.heads);
+        else
+            clear_unowned_tokens<kCsrI32, kThreads>(owned, first, a.query_offsets, a.page_offsets, a.last_page_lengths, a.tokens, a.sequences,
+                                                    a.page_table, a.page_size, a.output, token_bytes, a.lse, a.heads);
+        return;
+    }
     const bool in_page = a.page_shift >= 5;  // a power of two of at least a tile's 32 keys
     if (a.wide_index) {
         if (in_page) latent_tile_rows<Half, kCsrI64, ANY, true>(a, lds);

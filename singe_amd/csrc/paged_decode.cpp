@@ -316,7 +316,7 @@ int32_t launch_paged_decode(const SingePagedKvDecodeAttentionConfig& c, const Pa
     CombineArgs combine;
     combine.out = l.out;
     combine.lse = l.lse;
-    combine.row_lengths = l.row_starts != nullptr ? l.actual_seq_lens : nullptr;
+    combine.row_lengths = l.row_starts != nullptr && !l.every_row ? l.actual_seq_lens : nullptr;  // (such rows have no keys)
     combine.partial_out = args.partial_out;
     combine.partial_lse = args.partial_lse;
     combine.meta = args.meta;

@@ -104,6 +104,45 @@ SINGE_DEVICE SequenceSpan load_span(unsigned int sequence, const void* query_off
     return span;
 }
 
+// The rows of the `THREADS` tokens from `first` on that no valid sequence owns: zeros and a log-sum-exp of -inf, for callers
+// whose output holds nothing yet.  One workgroup of THREADS; `owned` is THREADS / 32 + 1 words of LDS.  Where a sequence's
+// query offsets make no sense, the others may claim tokens more than once and some of their row tiles may lie outside the
+// grid: then every token is cleared (the status word says so, and what the rows hold besides is not defined).
+template <int FORM, unsigned int THREADS>
+SINGE_DEVICE void clear_unowned_tokens(unsigned int* owned, unsigned int first, const void* query_offsets, const void* page_offsets,
+                                       const void* last_page_lengths, unsigned int tokens, unsigned int sequences, unsigned int page_table,
+                                       unsigned int page_size, void* output, unsigned int token_bytes, float* lse, unsigned int heads) {
+    constexpr unsigned int kWords = THREADS / 32u;
+    const unsigned int tid = threadIdx.x;
+    if (tid <= kWords) owned[tid] = 0u;
+    __syncthreads();
+    for (unsigned int s = tid; s < sequences; s += THREADS) {
+        const SequenceSpan span = load_span<FORM>(s, query_offsets, page_offsets, last_page_lengths, nullptr, tokens, page_table, page_size);
+        const long long count = read_index<FORM>(query_offsets, s + 1) - span.query_start;
+        if (span.query_start < 0 || count < 0 || span.query_start + count > static_cast<long long>(tokens)) atomicOr(&owned[kWords], 1u);
+        if (!span.valid || span.queries == 0) continue;
+        const long long from = span.query_start - static_cast<long long>(first), until = from + span.queries;
+        const unsigned int low = from < 0 ? 0u : from > static_cast<long long>(THREADS) ? THREADS : static_cast<unsigned int>(from);
+        const unsigned int high = until < 0 ? 0u : until > static_cast<long long>(THREADS) ? THREADS : static_cast<unsigned int>(until);
+        for (unsigned int word = low / 32u; word * 32u < high; ++word) {
+            const unsigned int begin = word * 32u < low ? low - word * 32u : 0u, end = high - word * 32u < 32u ? high - word * 32u : 32u;
+            if (begin < end) atomicOr(&owned[word], (end == 32u ? ~0u : (1u << end) - 1u) & ~((1u << begin) - 1u));
+        }
+    }
+    __syncthreads();
+    const bool everything = owned[kWords] != 0u;
+    for (unsigned int word = 0; word < kWords; ++word) {
+        for (unsigned int left = everything ? ~0u : ~owned[word]; left != 0u; left &= left - 1u) {
+            const unsigned int token = first + word * 32u + static_cast<unsigned int>(__builtin_ctz(left));
+            if (token >= tokens) return;
+            unsigned char* row = static_cast<unsigned char*>(output) + static_cast<size_t>(token) * token_bytes;
+            for (unsigned int at = tid * 8u; at < token_bytes; at += THREADS * 8u) *reinterpret_cast<uint2*>(row + at) = make_uint2(0u, 0u);
+            if (lse != nullptr)
+                for (unsigned int head = tid; head < heads; head += THREADS) lse[static_cast<size_t>(token) * heads + head] = -INFINITY;
+        }
+    }
+}
+
 // Packed sequences may overlap, and then the last one that owns a token writes its rows, as the CPU loop's later writes
 // win.  Whether any sequence after `sequence` reaches into its `queries` tokens (the same answer in every lane) ...
 SINGE_DEVICE bool later_sequence_overlaps(const void* offsets, const void* query_lengths, unsigned int sequences, unsigned int sequence,

@@ -87,6 +87,7 @@ struct PagedDecodeLaunch {
     const uint32_t* row_starts = nullptr;
     const uint32_t* row_begins = nullptr;  // with row_starts: keys at the front of each row that a window hides, or null
     float* lse = nullptr;
+    bool every_row = false;  // with row_starts: rows that belong to no sequence become zeros with a log-sum-exp of -inf instead of being left alone
 };
 int32_t launch_paged_decode(const SingePagedKvDecodeAttentionConfig& config, const PagedDecodeLaunch& launch);
 size_t paged_decode_workspace_bytes(const SingePagedKvDecodeAttentionConfig& config);

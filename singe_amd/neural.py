@@ -268,34 +268,38 @@ def paged_attention(query: torch.Tensor, key_cache: torch.Tensor, value_cache: t
         if not tensor.is_cuda or not tensor.is_contiguous():
             raise error.InvalidArgument("paged attention index tensors must be contiguous device tensors")
     problem = _problem(query, key_cache, value_cache, paging, options)
-    output = torch.zeros_like(query)
-    lse = torch.full(query.shape[:2], float("-inf"), device=query.device, dtype=torch.float32)
+    # The matrix-core kernels write every row, those of tokens that no sequence owns included; the others leave such rows
+    # alone, so their outputs are filled first.
+    sixteen_bit = query.dtype in (torch.bfloat16, torch.float16)
+    every_row = sixteen_bit and query.shape[2] % 16 == 0 and query.shape[2] <= 128 and problem.sequences > 0
+    if every_row:
+        output = torch.empty_like(query)
+        lse = torch.empty(query.shape[:2], device=query.device, dtype=torch.float32)
+    else:
+        output = torch.zeros_like(query)
+        lse = torch.full(query.shape[:2], float("-inf"), device=query.device, dtype=torch.float32)
     if status is None:
         status = torch.zeros(1, device=query.device, dtype=torch.int32)
     handle = int((stream or torch.cuda.current_stream()).cuda_stream)
-    entry = {torch.bfloat16: _native.lib().singe_hip_paged_attention_bf16,
-             torch.float32: _native.lib().singe_hip_paged_attention_f32,
-             torch.float64: _native.lib().singe_hip_paged_attention_f64,
-             torch.float16: _native.lib().singe_hip_paged_attention_f16}[query.dtype]
-    # bf16 calls with few query rows (decoding) share a row tile's keys out over several workgroups, given
+    # 16-bit calls with few query rows (decoding) share a row tile's keys out over several workgroups, given
     # scratch: ``scratch`` is a uint8 device tensor, True for this module's own per-device buffer (calls on
     # different streams must then not overlap), or False for none.
     wanted = 0
-    if query.dtype in (torch.bfloat16, torch.float16) and scratch is not False:
+    if sixteen_bit and scratch is not False:
         wanted = int(_native.lib().singe_hip_paged_attention_scratch_bytes(ctypes.byref(problem)))
-    if wanted > 0:
-        lent = _scratch_for(query.device, wanted) if scratch is True else scratch
-        with_scratch = (_native.lib().singe_hip_paged_attention_scratch_bf16 if query.dtype == torch.bfloat16
-                        else _native.lib().singe_hip_paged_attention_scratch_f16)
-        code = with_scratch(
-            handle, query.data_ptr(), key_cache.data_ptr(), value_cache.data_ptr(), paging.query_offsets.data_ptr(),
-            paging.page_offsets.data_ptr(), paging.pages.data_ptr(), paging.last_page_lengths.data_ptr(),
-            output.data_ptr(), lse.data_ptr(), status.data_ptr(), lent.data_ptr(), lent.numel(), ctypes.byref(problem))
+    lent = None if wanted == 0 else _scratch_for(query.device, wanted) if scratch is True else scratch
+    operands = (handle, query.data_ptr(), key_cache.data_ptr(), value_cache.data_ptr(), paging.query_offsets.data_ptr(),
+                paging.page_offsets.data_ptr(), paging.pages.data_ptr(), paging.last_page_lengths.data_ptr(), output.data_ptr(),
+                lse.data_ptr(), status.data_ptr())
+    scratch_operands = (0, 0) if lent is None else (lent.data_ptr(), lent.numel())
+    if every_row:
+        code = _native.lib().singe_hip_paged_attention_every_row(_ATTENTION_TYPES[query.dtype], *operands, *scratch_operands, ctypes.byref(problem))
     else:
-        code = entry(
-            handle, query.data_ptr(), key_cache.data_ptr(), value_cache.data_ptr(), paging.query_offsets.data_ptr(),
-            paging.page_offsets.data_ptr(), paging.pages.data_ptr(), paging.last_page_lengths.data_ptr(),
-            output.data_ptr(), lse.data_ptr(), status.data_ptr(), ctypes.byref(problem))
+        entry = {torch.bfloat16: _native.lib().singe_hip_paged_attention_bf16,
+                 torch.float32: _native.lib().singe_hip_paged_attention_f32,
+                 torch.float64: _native.lib().singe_hip_paged_attention_f64,
+                 torch.float16: _native.lib().singe_hip_paged_attention_f16}[query.dtype]
+        code = entry(*operands, ctypes.byref(problem))
     _native.check(code, "paged_attention")
     if check and int(status.item()) == STATUS_INDEX_OUT_OF_BOUNDS:
         raise error.IndexOutOfBounds("paged attention paging value outside its buffers")
@@ -342,23 +346,26 @@ def paged_mla_attention(query: torch.Tensor, query_positions: torch.Tensor, late
         tokens, heads, latent, positional, page_size, sequences, pages, paging.pages.numel(), _DATA_TYPES[query.dtype],
         1 if paging.pages.dtype == torch.int64 else 0, 1 if options.causal else 0, 1 if options.scale is not None else 0,
         options.scale if options.scale is not None else 0.0)
-    output = torch.zeros_like(query)
-    lse = torch.full((tokens, heads), float("-inf"), device=query.device, dtype=torch.float32)
+    # (the widths on the matrix cores, whose kernels write every row: see paged_attention)
+    every_row = (query.dtype in (torch.bfloat16, torch.float16) and latent <= 512 and latent % 32 == 0 and positional <= 64
+                 and positional % 8 == 0 and (latent + positional) % 16 == 0 and sequences > 0)
+    if every_row:
+        output = torch.empty_like(query)
+        lse = torch.empty((tokens, heads), device=query.device, dtype=torch.float32)
+    else:
+        output = torch.zeros_like(query)
+        lse = torch.full((tokens, heads), float("-inf"), device=query.device, dtype=torch.float32)
     if status is None:
         status = torch.zeros(1, device=query.device, dtype=torch.int32)
     handle = int((stream or torch.cuda.current_stream()).cuda_stream)
     wanted = 0 if scratch is False else int(_native.lib().singe_hip_paged_mla_attention_scratch_bytes(ctypes.byref(problem)))
-    if wanted > 0:
-        lent = _scratch_for(query.device, wanted) if scratch is True else scratch
-        code = _native.lib().singe_hip_paged_mla_attention_scratch(
-            handle, query.data_ptr(), query_positions.data_ptr(), latent_cache.data_ptr(), position_cache.data_ptr(),
-            paging.query_offsets.data_ptr(), paging.page_offsets.data_ptr(), paging.pages.data_ptr(), paging.last_page_lengths.data_ptr(),
-            output.data_ptr(), lse.data_ptr(), status.data_ptr(), lent.data_ptr(), lent.numel(), ctypes.byref(problem))
-    else:
-        code = _native.lib().singe_hip_paged_mla_attention(
-            handle, query.data_ptr(), query_positions.data_ptr(), latent_cache.data_ptr(), position_cache.data_ptr(),
-            paging.query_offsets.data_ptr(), paging.page_offsets.data_ptr(), paging.pages.data_ptr(), paging.last_page_lengths.data_ptr(),
-            output.data_ptr(), lse.data_ptr(), status.data_ptr(), ctypes.byref(problem))
+    lent = None if wanted == 0 else _scratch_for(query.device, wanted) if scratch is True else scratch
+    entry = _native.lib().singe_hip_paged_mla_attention_every_row if every_row else _native.lib().singe_hip_paged_mla_attention_scratch
+    code = entry(
+        handle, query.data_ptr(), query_positions.data_ptr(), latent_cache.data_ptr(), position_cache.data_ptr(),
+        paging.query_offsets.data_ptr(), paging.page_offsets.data_ptr(), paging.pages.data_ptr(), paging.last_page_lengths.data_ptr(),
+        output.data_ptr(), lse.data_ptr(), status.data_ptr(), 0 if lent is None else lent.data_ptr(), 0 if lent is None else lent.numel(),
+        ctypes.byref(problem))
     _native.check(code, "paged_mla_attention")
     if check and int(status.item()) == STATUS_INDEX_OUT_OF_BOUNDS:
         raise error.IndexOutOfBounds("paged mla attention paging value outside its buffers")

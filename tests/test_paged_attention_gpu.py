@@ -512,3 +512,44 @@ def test_offsets_that_run_backwards_are_reported_from_a_list_that_takes_turns():
     with pytest.raises(error.IndexOutOfBounds):
         neural.paged_attention(rand(300, heads, 128), rand(pages, page_size, kv_heads, 128), rand(pages, page_size, kv_heads, 128), paging,
                                neural.AttentionOptions(causal=True))
+
+
+def poison(*shapes):
+    """Blocks of NaN given back to the allocator: what an output that nothing wrote would hold."""
+    blocks = [torch.full(shape, float("nan"), device="cuda", dtype=dtype) for shape, dtype in shapes]
+    torch.cuda.synchronize()
+    del blocks
+
+
+@pytest.mark.parametrize("index_dtype", [torch.int32, torch.int64])
+@pytest.mark.parametrize("case", ["row tiles", "shares", "two tiles a wave", "decode", "many keys"])
+def test_tokens_no_sequence_owns_are_zero_with_a_log_sum_exp_of_minus_infinity(case, index_dtype):
+    heads, kv_heads, page_size = 8, 2, 16
+    tokens, owned = {"decode": (40, [(5, 1), (9, 1), (10, 0), (10, 1)]), "many keys": (300, [(33, 1), (40, 200)])}.get(
+        case, (700, [(3, 7), (10, 0), (10, 255), (265, 1), (266, 200)]))
+    keys = [4000 if case == "many keys" else 90 + 10 * s for s in range(len(owned))]
+    if case == "decode":  # a token a sequence at most, sequences without tokens after them
+        owned, keys = owned + [(11, 0)] * 40, keys + [20] * 40
+    pages = [(k + page_size - 1) // page_size for k in keys]
+    offsets = [start for start, _ in owned] + [owned[-1][0] + owned[-1][1]]
+    # (sequences are consecutive: the gap after one goes to the next, so only the front and the back are unowned)
+    mine = torch.zeros(tokens, dtype=torch.bool, device="cuda")
+    mine[offsets[0]:offsets[-1]] = True
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(3)
+    rand = lambda *shape: torch.randn(shape, generator=gen, device="cuda").to(torch.bfloat16)
+    index = lambda values: torch.tensor([int(v) for v in values], dtype=index_dtype, device="cuda")
+    paging = neural.Paging(index(offsets), index(np.concatenate([[0], np.cumsum(pages)])), index(np.arange(sum(pages))),
+                           index([k - (n - 1) * page_size for k, n in zip(keys, pages)]))
+    q, kc, vc = rand(tokens, heads, 128), rand(sum(pages), page_size, kv_heads, 128), rand(sum(pages), page_size, kv_heads, 128)
+    _native.lib().singe_hip_set_paged_attention_splits(3 if case == "shares" else 0)
+    _native.lib().singe_hip_set_paged_attention_rows_per_wave(64 if case == "two tiles a wave" else 0)
+    try:
+        poison(((tokens, heads, 128), torch.bfloat16), ((tokens, heads), torch.float32))
+        out, lse = neural.paged_attention(q, kc, vc, paging, neural.AttentionOptions(causal=True))
+    finally:
+        _native.lib().singe_hip_set_paged_attention_splits(0)
+        _native.lib().singe_hip_set_paged_attention_rows_per_wave(0)
+    assert not out[~mine].any() and torch.isneginf(lse[~mine]).all()
+    assert torch.isfinite(out[mine].float()).all() and torch.isfinite(lse[mine]).all()
+    assert (out[mine].float().abs().amax(dim=-1) > 0).all()

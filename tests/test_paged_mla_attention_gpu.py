@@ -464,3 +464,30 @@ def test_offsets_that_run_backwards_are_reported_by_a_shared_out_step():
     paging = neural.Paging(index([0, tokens, 0, tokens]), index([0, pages, pages, 2 * pages]), index(list(range(pages)) * 2), index([64, 0, 64]))
     with pytest.raises(error.IndexOutOfBounds):
         neural.paged_mla_attention(*device, paging, neural.AttentionOptions(causal=True))
+
+
+@pytest.mark.parametrize("index_dtype", [torch.int32, torch.int64])
+@pytest.mark.parametrize("keys,splits", [(100, 0), (2000, 0), (2000, 3)])
+def test_tokens_no_sequence_owns_are_zero_with_a_log_sum_exp_of_minus_infinity(keys, splits, index_dtype):
+    from singe_amd import _native
+    heads, page_size, tokens, offsets = 16, 32, 700, [5, 6, 6, 40]
+    pages = (keys + page_size - 1) // page_size
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(4)
+    rand = lambda *shape: torch.randn(shape, generator=gen, device="cuda").to(torch.bfloat16)
+    index = lambda entries: torch.tensor(entries, dtype=index_dtype, device="cuda")
+    paging = neural.Paging(index(offsets), index([0, pages, 2 * pages, 3 * pages]), index(list(range(3 * pages))),
+                           index([keys - (pages - 1) * page_size] * 3))
+    operands = [rand(tokens, heads, 512), rand(tokens, heads, 64), rand(3 * pages, page_size, 512), rand(3 * pages, page_size, 64)]
+    _native.lib().singe_hip_set_paged_mla_attention_splits(splits)
+    try:
+        blocks = [torch.full((tokens, heads, 512), float("nan"), device="cuda", dtype=torch.bfloat16), torch.full((tokens, heads), float("nan"), device="cuda")]
+        torch.cuda.synchronize()
+        del blocks  # (what an output that nothing wrote would hold)
+        out, lse = neural.paged_mla_attention(*operands, paging, neural.AttentionOptions(causal=True))
+    finally:
+        _native.lib().singe_hip_set_paged_mla_attention_splits(0)
+    mine = torch.zeros(tokens, dtype=torch.bool, device="cuda")
+    mine[5:40] = True
+    assert not out[~mine].any() and torch.isneginf(lse[~mine]).all()
+    assert torch.isfinite(out[mine].float()).all() and torch.isfinite(lse[mine]).all()
