@@ -500,3 +500,20 @@ def test_packed_prefill_leaves_row_counts_beyond_32_bits_to_the_row_kernel(token
     address, many = 1 << 20, 2**60
     arguments = [address if i % 2 == 0 else many for i in range(16)]
     assert _native.lib().singe_hip_ragged_kv_prefill_attention_bf16(None, *arguments, ctypes.byref(config)) == 8
+
+
+@pytest.mark.parametrize("chunks,chunk,decoding,keys,rows", [
+    (2, 512, 32, 2112, 32),           # less than a whole 256-row tile a sequence, sequences of 1024 to 4096 keys
+    (2, 512, 30, 2112, 64),           # 32 whole tiles, 32 sequences
+    (2, 512, 32, 1023, 64),           # either side of 1024 and 4096 keys
+    (2, 512, 32, 4097, 64),
+    (1, 2049, 80, 2112, 32),          # either side of 2048 tokens more than sequences
+    (1, 2050, 80, 2112, 64),
+])
+def test_paged_attention_row_tiles_by_the_keys_a_sequence_has(chunks, chunk, decoding, keys, rows):
+    tokens, sequences = chunks * chunk + decoding, chunks + decoding
+    fields = dict(tokens=tokens, heads=64, kv_heads=8, head_dim=128, page_size=16, sequences=sequences, cache_pages=20000,
+                  page_table=-(-keys * sequences // 16), index_type=0, causal=1, has_scale=0, has_window=0, has_softcap=0, scale=0.0, softcap=0.0,
+                  window=0)
+    problem = _native.PagedAttentionProblemC(*fields.values())
+    assert _native.lib().singe_hip_paged_attention_rows_per_wave(ctypes.byref(problem)) == rows
