@@ -318,9 +318,9 @@ typedef struct SingeFmhaPrefillConfig {
 /* Tuning knob of the dense bf16 / f16 prefill at the multiples of 16 up to 128: the query rows a wave takes.  32: four waves share a
  * compute unit's SIMDs two by two, 128 rows a workgroup.  64: a wave has a SIMD to itself and folds every key block
  * into two 32-row tiles, 256 rows a workgroup; only calls without a mask, a window, a cap or key splits (sinks and
- * key lengths are taken) with a positive scale have this form, others keep 32.  0 (the default): 64 where the call has that form,
- * its 256-row tiles still fill the chip and the head dimension is one the form is faster at (64 and up; 48 without
- * the causal mask).  Results are the same up to the order in which a row's
+ * key lengths are taken) with a positive scale have this form, others keep 32.  0 (the default): 64 where the call has that form and
+ * measured faster in it: enough workgroups, in whole rounds of the chip, and long rows (above head_dim 64; at 48 and 64 only
+ * without the causal mask; the line stands at two_tiles_a_wave in csrc/fmha_prefill.cpp).  Results are the same up to the order in which a row's
  * reference point moves.  The counterpart of AttentionParameters::{warps, min_blocks}
  * (singe/src/backend/cuda/kernel_plan/source/parameters.rs:21-57). */
 SINGE_HIP_API void singe_hip_set_dense_prefill_rows_per_wave(uint32_t rows);

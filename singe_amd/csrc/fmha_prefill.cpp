@@ -209,19 +209,36 @@ int32_t dense_f32_matrix(void* stream, PrefillF32Args& a) {
 
 namespace {
 
-// Whether a call without options runs on the kernel that gives a wave two 32-row tiles: a head_dim that is a multiple of 16 up to 128, a positive
-// scale, no heads packed into one tile, and (unless the knob says 64) 256-row tiles that still fill the chip.
+// Whether a call without options runs on the kernel that gives a wave two 32-row tiles: a head_dim that is a multiple of 16
+// up to 128, a positive scale, no heads packed into one tile, and (unless the knob says 64) where it is the faster one:
+// enough of its workgroups (pairs of 256-row tiles, one to a compute unit) in whole rounds of the chip, and enough keys to
+// each that the ends of a tile do not weigh.  32-row / two-tile kernel, us, batch * heads x length (workgroups; equal
+// query and key counts, a seventh of the shapes timed):
+//   head_dim 128, causal  128 x 600 (256) 35 / 41    256 x 768 (512) 65 / 85     256 x 1280 (768)  141 / 151   96 x 1536 (288) 101 / 112
+//                         64 x 1536 (192) 71 / 56    128 x 1536 (384) 102 / 113  256 x 1536 (768)  186 / 185   64 x 1792 (256)  81 / 67
+//                         64 x 2048 (256) 81 / 77    64 x 2560 (320) 149 / 155   128 x 2048 (512)  156 / 151   32 x 3072 (192) 111 / 87
+//                         64 x 3072 (384) 183 / 183  128 x 3072 (768) 326 / 298  128 x 4096 (1024) 558 / 506
+//   head_dim 128, full    128 x 768 (256) 53 / 54    256 x 768 (512) 97 / 103    256 x 1024 (512)  149 / 142   96 x 1280 (288)  90 / 110
+//                         64 x 1280 (192) 76 / 68    32 x 2560 (160) 137 / 117   32 x 2048 (128)    73 / 97    128 x 4096       1037 / 918
+//   head_dim 96           causal 64 x 1536 64 / 50, 128 x 1536 91 / 99, 128 x 4096 479 / 425; full 96 x 1280 78 / 97, 128 x 4096 880 / 770
+//   head_dim 64, causal   96 x 1536 (288) 54 / 83    128 x 1024 (256) 32 / 38    256 x 1280 (768)   80 / 112   128 x 4096 (1024) 332 / 346
+//   head_dim 64, full     128 x 1280 (384) 75 / 105  128 x 2048 (512) 175 / 170  256 x 2048 (1024) 322 / 327   64 x 4096 (512)   337 / 310
+// (Up to 64 the 32-row kernel holds three workgroups a compute unit and the softmax's vector instructions bound both: two or
+// three waves a SIMD share them out better than one.)
 bool two_tiles_a_wave(const SingeFmhaPrefillConfig& c) {
     const uint32_t wanted = g_rows_per_wave.load(std::memory_order_relaxed);
     if (wanted == 32 || !has_pair_build(static_cast<long long>(c.head_dim)) || c.key_len == 0 || !(c.scale > 0.0f) || dense_prefill_packs_heads(c))
         return false;
-    const uint64_t rows = (static_cast<uint64_t>(c.batch) * c.heads + 7) / 8 * 8, pair_tiles = (c.query_len + 255) / 256;
     if (wanted == 64) return true;
-    // Measured against the 32-row kernel at batch 4 x 32 heads x 4096: faster from head_dim 64 up (1.02 - 1.14 x), at 48
-    // without the causal mask only (1.09 x; 0.97 x with it), slower at 32 and 16 under the mask, where the softmax's vector
-    // instructions bound both kernels and two waves a SIMD share them out better than one.
-    if (c.head_dim < 48 || (c.head_dim == 48 && c.causal)) return false;
-    return rows * ((pair_tiles + 1) / 2) >= compute_units();
+    const uint64_t rows = (static_cast<uint64_t>(c.batch) * c.heads + 7) / 8 * 8, pair_tiles = (c.query_len + 255) / 256;
+    const uint64_t units = compute_units(), workgroups = rows * ((pair_tiles + 1) / 2), rounds = (workgroups + units - 1) / units;
+    const uint64_t seen = c.causal && c.query_len < c.key_len ? c.query_len : c.key_len;
+    const uint64_t share = 100 * workgroups / (rounds * units);  // of the rounds' places that a workgroup takes, in percent
+    if (c.head_dim < 48) return false;
+    if (c.head_dim <= 64) return !c.causal && seen >= 4096 && workgroups >= units && share >= 90;
+    if (4 * workgroups < 3 * units) return !c.causal && seen >= 2560 && 8 * workgroups >= 5 * units;
+    if (!c.causal) return seen >= 900 && !(rounds == 2 && 4 * workgroups < 5 * units && seen < 1536);
+    return seen >= 3072 || (seen >= 2048 && share >= 70) || (seen >= 1536 && (rounds == 1 || share >= 95));
 }
 
 int32_t prefill(void* stream, uint16_t* out, size_t out_len, float* lse, size_t lse_len, bool with_lse,

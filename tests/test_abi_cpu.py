@@ -517,3 +517,30 @@ def test_paged_attention_row_tiles_by_the_keys_a_sequence_has(chunks, chunk, dec
                   window=0)
     problem = _native.PagedAttentionProblemC(*fields.values())
     assert _native.lib().singe_hip_paged_attention_rows_per_wave(ctypes.byref(problem)) == rows
+
+
+@pytest.mark.parametrize("batch,heads,head_dim,query_len,key_len,causal,rows", [
+    (4, 32, 128, 4096, 4096, 1, 64),    # whole rounds of long rows
+    (4, 32, 128, 1024, 1024, 1, 32),    # short causal rows
+    (2, 32, 128, 1535, 1535, 1, 32),    # either side of 1536 keys, less than a round
+    (2, 32, 128, 1536, 1536, 1, 64),
+    (4, 32, 128, 1536, 1536, 1, 32),    # one and a half rounds
+    (4, 32, 128, 2048, 2048, 1, 64),
+    (2, 32, 128, 2560, 2560, 1, 32),    # one and a quarter
+    (1, 32, 128, 3072, 3072, 1, 64),    # three quarters of a round
+    (1, 31, 128, 2048, 2048, 1, 32),    # half of one
+    (4, 32, 128, 899, 899, 0, 32),      # either side of 900 keys without a mask
+    (4, 32, 128, 900, 900, 0, 64),
+    (4, 32, 128, 1024, 899, 0, 32),
+    (3, 32, 96, 1280, 1280, 0, 32),     # a little more than a round
+    (3, 32, 96, 1536, 1536, 0, 64),
+    (1, 32, 128, 2560, 2560, 0, 64),
+    (4, 32, 64, 4096, 4096, 1, 32),     # narrow heads
+    (4, 32, 64, 4096, 4096, 0, 64),
+    (4, 32, 64, 2048, 2048, 0, 32),
+    (4, 32, 32, 4096, 4096, 0, 32),
+])
+def test_dense_prefill_rows_per_wave(batch, heads, head_dim, query_len, key_len, causal, rows):
+    # (without a device the library counts on 256 compute units)
+    config = A.FmhaPrefillConfig.contiguous(batch, query_len, key_len, heads, heads, head_dim, 0.125, bool(causal))
+    assert _native.lib().singe_hip_dense_prefill_rows_per_wave(ctypes.byref(config._c())) == rows
