@@ -67,7 +67,7 @@ SINGE_DEVICE void fmha_prefill_tile(const PrefillArgs& a, unsigned char* lds, un
     const unsigned int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const unsigned int column = lane & 31, hi = lane >> 5;
 
-    // (packed_heads: `bh` counts (batch, kv head) pairs and the rows of the one tile are (query, head of the group) pairs.)
+    // (packed_heads: `bh` counts (batch, kv head) pairs and the rows of the tiles are (query, head of the group) pairs.)
     const bool packed = a.packed_heads != 0;
     const unsigned int group = a.heads / a.kv_heads;
     const unsigned int batch = packed ? bh / a.kv_heads : bh / a.heads;
@@ -86,6 +86,16 @@ SINGE_DEVICE void fmha_prefill_tile(const PrefillArgs& a, unsigned char* lds, un
     const unsigned int my_query = packed ? my_row / group : my_row;
     const unsigned int head = packed ? kv_head * group + my_row % group : bh % a.heads;
     const bool query_valid = my_query < a.query_len;
+    // The queries of rows of this tile, for what masks and windows look at.  Rows are queries, but for the packed rows of a
+    // window (packed_heads == 2); packed rows without a mask to apply have one tile and nobody asks.
+    unsigned int tile_query = query_tile * kRows, tile_last_query = tile_query + kRows - 1u, wave_query = first_row, wave_last_query = first_row + 31u;
+    if (OPTIONS && packed) {
+        asm volatile("s_nop 0");  // (kept a branch: the divisions of the others' rows would cost every tile 0.3 us)
+        tile_query /= group;
+        tile_last_query /= group;
+        wave_query /= group;
+        wave_last_query /= group;
+    }
 
     const uint16_t* q_base = a.query + batch * a.query_batch_stride + head * a.query_head_stride;
     const unsigned char* const k_bytes = reinterpret_cast<const unsigned char*>(a.key + batch * a.key_batch_stride + kv_head * a.key_head_stride);
@@ -113,20 +123,20 @@ SINGE_DEVICE void fmha_prefill_tile(const PrefillArgs& a, unsigned char* lds, un
     // block wholly after the wave's last query contributes nothing.
     unsigned int key_end = key_len;
     if (CAUSAL) {
-        const unsigned int reach = query_tile * kRows + kRows;
+        const unsigned int reach = tile_last_query + 1u;
         key_end = key_end < reach ? key_end : reach;
     }
     unsigned int tiles = (key_end + kKeyTile - 1) / kKeyTile;
     unsigned int wave_blocks = (key_end + 31u) / 32u;
     if (CAUSAL) {
-        const unsigned int seen = (first_row + 31u) / 32u + 1u;
+        const unsigned int seen = wave_last_query / 32u + 1u;
         wave_blocks = wave_blocks < seen ? wave_blocks : seen;
     }
     // The first tile any row of the workgroup can see: 0, or with a window the tile of the first key the
     // workgroup's first row still sees (later rows see later keys).
     unsigned int first_tile = 0;
     if (OPTIONS && a.window >= 0) {
-        const unsigned long long low = static_cast<unsigned long long>(query_tile) * kRows + 1u;
+        const unsigned long long low = static_cast<unsigned long long>(tile_query) + 1u;
         const unsigned long long window = static_cast<unsigned long long>(a.window);
         if (low > window) first_tile = static_cast<unsigned int>((low - window) / kKeyTile);
         first_tile = first_tile < tiles ? first_tile : tiles;
@@ -152,9 +162,8 @@ SINGE_DEVICE void fmha_prefill_tile(const PrefillArgs& a, unsigned char* lds, un
                 return query >= window ? query - static_cast<unsigned int>(window) + 1u : 0u;
             };
             my_low = low(my_query);
-            // (packed rows: neighbouring rows share a query, and the tile's first row has its lowest)
-            last_low = low(packed ? (first_row + 31u) / group : first_row + 31u);
-            const unsigned int first_block = low(packed ? first_row / group : first_row) / 32u;
+            last_low = low(wave_last_query);
+            const unsigned int first_block = low(wave_query) / 32u;
             wave_first_block = wave_first_block > first_block ? wave_first_block : first_block;
         }
         my_span = my_end > my_low ? my_end - my_low : 0u;
@@ -239,7 +248,7 @@ SINGE_DEVICE void fmha_prefill_tile(const PrefillArgs& a, unsigned char* lds, un
             // one by one.  A window alone leaves the scores as they are: their scale stays in the exponent's multiply-add.
             // (One fold after the branch, whatever is left to apply: a fold in either branch is two more copies of it in
             // each of the loops below, which at head_dim 128 spilt 70 registers and cost masks, caps and windows alike.)
-            const bool edge = (CAUSAL && key0 + 31u > first_row) || key0 + 32u > key_len || key0 < last_low;
+            const bool edge = (CAUSAL && key0 + 31u > wave_query) || key0 + 32u > key_len || key0 < last_low;
             float left = factor;
             if (a.mask != nullptr || a.cap_log2e != 0.0f) {
                 // Scores in their final units (base-two logits): scaled, capped (singe/src/backend/cpu/normalization/
@@ -326,7 +335,7 @@ SINGE_DEVICE void fmha_prefill_tile(const PrefillArgs& a, unsigned char* lds, un
     // first for every wave (the mask's edge and the end of the keys are the last tiles a wave works on).
     unsigned int interior_tiles = wave_blocks > 2 ? (wave_blocks - 1) / 2 : 0;  // tiles t with 2 t + 2 < wave_blocks
     if (CAUSAL) {
-        const unsigned int unmasked = (first_row + 1) / kKeyTile;  // tiles t with 64 t + 63 <= first_row
+        const unsigned int unmasked = (wave_query + 1) / kKeyTile;  // tiles t with 64 t + 63 <= the wave's first query
         interior_tiles = interior_tiles < unmasked ? interior_tiles : unmasked;
     }
     {
@@ -341,8 +350,8 @@ SINGE_DEVICE void fmha_prefill_tile(const PrefillArgs& a, unsigned char* lds, un
     if (OPTIONS) {
         if (a.mask != nullptr) interior_tiles = 0;
         if (a.window >= 0) {
-            // Tile t lies inside every row's window when 64 t + window > first_row + 31.
-            const unsigned long long past = static_cast<unsigned long long>(first_row) + 32u, window = static_cast<unsigned long long>(a.window);
+            // Tile t lies inside every row's window when 64 t + window is past the wave's last query.
+            const unsigned long long past = static_cast<unsigned long long>(wave_last_query) + 1u, window = static_cast<unsigned long long>(a.window);
             if (past > window) {
                 const unsigned long long whole = (past - window + kKeyTile - 1) / kKeyTile;
                 inner_begin = whole < tiles ? static_cast<unsigned int>(whole) : tiles;
@@ -434,12 +443,23 @@ template <bool CAUSAL, class Half, int WAVES, bool OPTIONS = false>
 SINGE_DEVICE void fmha_prefill_body(const PrefillArgs& a, unsigned char* lds) {
     const unsigned int xcd = blockIdx.x & 7u;
     unsigned int within = blockIdx.x >> 3;
-    const unsigned int split = within % a.splits;  // the shares of a query tile are neighbours
-    within /= a.splits;
-    const unsigned int pairs = a.single_tiles != 0 ? a.query_tiles : (a.query_tiles + 1u) / 2u;
-    const unsigned int bh = (within / pairs) * 8u + xcd;
-    if (bh >= a.batch * (a.packed_heads != 0 ? a.kv_heads : a.heads)) return;
-    const unsigned int heavy = a.query_tiles - 1u - within % pairs, light = a.single_tiles != 0 ? heavy : within % pairs;
+    unsigned int split = 0, bh, heavy, light;
+    if (CAUSAL && OPTIONS && a.packed_heads == 2) {
+        // The tiles of all (batch, kv head) pairs, the longest first, go to the XCDs in runs of eight neighbours, whose
+        // windows overlap: a pair's tiles on one XCD would leave the others idle where there are few pairs.
+        const unsigned int at = ((within / 8u) * 8u + xcd) * 8u + within % 8u;
+        bh = at / a.query_tiles;
+        if (bh >= a.batch * a.kv_heads) return;
+        heavy = light = a.query_tiles - 1u - at % a.query_tiles;
+    } else {
+        split = within % a.splits;  // the shares of a query tile are neighbours
+        within /= a.splits;
+        const unsigned int pairs = a.single_tiles != 0 ? a.query_tiles : (a.query_tiles + 1u) / 2u;
+        bh = (within / pairs) * 8u + xcd;
+        if (bh >= a.batch * (a.packed_heads != 0 ? a.kv_heads : a.heads)) return;
+        heavy = a.query_tiles - 1u - within % pairs;
+        light = a.single_tiles != 0 ? heavy : within % pairs;
+    }
     fmha_prefill_tile<CAUSAL, Half, WAVES, OPTIONS>(a, lds, bh, heavy, split);
     if (light != heavy) fmha_prefill_tile<CAUSAL, Half, WAVES, OPTIONS>(a, lds, bh, light, split);
 }

@@ -98,7 +98,8 @@ struct PrefillArgs {
     // Few query rows under grouped heads (a decode step through the dense op, no causal mask): with packed_heads != 0
     // a workgroup takes a (batch, kv head) pair and its tile's row r is query r / group of head kv_head * group +
     // r % group (group = heads / kv_heads, query_len * group at most the tile's rows), so the kv head's keys and values
-    // are fetched once for all of its query heads.
+    // are fetched once for all of its query heads.  2: the rows of a causal call with a window, in as many tiles as they
+    // fill (query_tiles), each in a workgroup of its own.
     uint32_t packed_heads = 0;
     // With single_tiles != 0 a workgroup takes one query tile instead of two (32-row kernels).
     uint32_t single_tiles = 0;

@@ -421,3 +421,31 @@ def test_sinks_on_the_two_tile_kernel(dim, dtype):
         close(host(out), want, dtype)
     finally:
         _native.lib().singe_hip_set_dense_prefill_rows_per_wave(0)
+
+
+@pytest.mark.parametrize("options", [dict(window=1), dict(window=31), dict(window=32, sinks=True), dict(window=33, softcap=4.0), dict(window=128, sinks=True),
+                                     dict(window=299), dict(window=300), dict(window=0), dict(window=70, scale=-0.1)])
+@pytest.mark.parametrize("batch,heads,kv_heads,query_len,key_len,dim,dtype", [
+    (1, 8, 1, 300, 300, 64, torch.bfloat16),    # sixteen queries a tile: whole tiles and a last one of part of a query's heads
+    (2, 14, 2, 129, 129, 128, torch.float16),   # a group that does not divide a tile's rows
+    (1, 4, 2, 300, 170, 96, torch.bfloat16),    # more queries than keys
+    (3, 6, 2, 65, 300, 48, torch.float16),      # more keys than queries, more pairs than XCDs
+    (1, 64, 2, 9, 40, 64, torch.bfloat16),      # more rows a query than a wave has
+])
+def test_causal_windows_over_grouped_heads_share_tiles(batch, heads, kv_heads, query_len, key_len, dim, dtype, options):
+    options = dict(options)
+    sinks = None
+    q, k, v = tensors((batch, heads, query_len, dim), (batch, kv_heads, key_len, dim), (batch, kv_heads, key_len, dim), dtype, heads + dim)
+    if options.pop("sinks", False):
+        sinks = torch.linspace(-2.0, 2.0, heads, device="cuda").to(dtype)
+    out = neural.attend(q, k, v, None, sinks, neural.AttentionOptions(causal=True, **options))
+    want = oracle.scaled_dot_product_attention_f32(host(q), host(k), host(v), causal=True, threads=8,
+                                                   sinks=None if sinks is None else host(sinks), **options)
+    close(host(out), want, dtype)
+    lengths = torch.tensor([key_len - 7 * b for b in range(batch)], device="cuda", dtype=torch.int32)
+    padded = neural.attend_padded(q, k, v, lengths, neural.AttentionOptions(causal=True, **options))
+    for b in range(batch):
+        n = int(lengths[b])
+        want = oracle.scaled_dot_product_attention_f32(host(q[b:b + 1]), host(k[b:b + 1, :, :n]), host(v[b:b + 1, :, :n]), causal=True, threads=8,
+                                                       **options)
+        close(host(padded[b:b + 1]), want, dtype)
