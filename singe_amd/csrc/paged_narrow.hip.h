@@ -246,7 +246,7 @@ SINGE_DEVICE void narrow_rows(const PagedAttentionArgs& a, unsigned char* lds, c
                     if (key >= keys || (causal && key > my_position) || (windowed && key + window <= my_position)) x[r] = -INFINITY;
                 }
             }
-            const float largest = across_groups_max(max2(max2(x[0], x[1]), max2(x[2], x[3]))) * factor;
+            const float largest = across_groups_max(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3]))) * factor;  // (not max2: nothing would wait for the products)
             if (__any(largest > reference + kMaxLag || (reference == -INFINITY && largest != -INFINITY))) {
                 const float moved = fmaxf(reference, largest), base = moved == -INFINITY ? 0.0f : moved;
                 const float rescale = fast_exp2(reference - base);

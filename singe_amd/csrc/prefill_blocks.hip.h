@@ -70,7 +70,10 @@ SINGE_DEVICE ReadOffsets read_offsets(unsigned int lane) {
 }
 
 // Scores of the wave's 32 queries against the 32 keys of the block at `keys` (LDS byte address of the
-// block's first row).  The products run on while the caller does other work.
+// block's first row).  The row maximum reads them in assembly (max3), in front of which the compiler does not wait for a
+// matrix instruction's result as it does for its own readers: the wait (11 issue cycles at least) is written out here.
+// Without it a block whose scores are folded right after they are made, with no mask to apply, took a stale maximum, and
+// scores that outgrew the reference point by more than 2^127 (f16: 2^16) made NaN rows.
 template <class Half>
 SINGE_DEVICE void score_block(Half half, f32x16_t& scores, const uint4 (&q)[kSteps], const unsigned char* keys, const ReadOffsets& offsets) {
     f32x16_t s;
@@ -82,6 +85,7 @@ SINGE_DEVICE void score_block(Half half, f32x16_t& scores, const uint4 (&q)[kSte
 #pragma unroll
     for (int step = 0; step < kSteps; ++step)
         s = mma(half, operand[step], q[step], s);
+    asm volatile("s_nop 7\n\ts_nop 7" : "+v"(s));
     scores = s;
 }
 

@@ -449,3 +449,20 @@ def test_causal_windows_over_grouped_heads_share_tiles(batch, heads, kv_heads, q
         want = oracle.scaled_dot_product_attention_f32(host(q[b:b + 1]), host(k[b:b + 1, :, :n]), host(v[b:b + 1, :, :n]), causal=True, threads=8,
                                                        **options)
         close(host(padded[b:b + 1]), want, dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("heads,length", [(4, 700), (4, 2000), (1, 90)])
+def test_scores_that_outgrow_a_share_s_reference_point(heads, length, causal, dtype):
+    """Scores that grow by thousands from key to key, over shares of a tile's keys and tails of one block: a row maximum that
+    is read before the matrix core has written it makes weights that do not fit their type, and NaN rows."""
+    magnitude = 30.0
+    q, k, v = tensors((1, heads, length, 128), (1, heads, length, 128), (1, heads, length, 128), torch.float32, 17)
+    q, k = q * magnitude, k * magnitude
+    k[..., 0] += torch.linspace(0, 40 * magnitude, length, device="cuda")
+    q[..., 0] = magnitude
+    q, k, v = q.to(dtype), k.to(dtype), v.to(dtype)
+    out = neural.scaled_dot_product_attention(q, k, v, causal=causal)
+    want = oracle.scaled_dot_product_attention_f32(host(q), host(k), host(v), causal=causal, threads=8)
+    close(host(out), want, dtype)
