@@ -334,6 +334,16 @@ int32_t prefill(void* stream, uint16_t* out, size_t out_len, float* lse, size_t 
     // (the merge counts rows in 32 bits)
     if (splits > 1 && static_cast<uint64_t>(c.batch) * c.heads * c.query_len > 0xffffffffull) splits = 1;
     if (splits > 1 && (options.scratch_bytes < dense_prefill_scratch_bytes(c, splits) || groups * splits > 0x7fffffffull)) splits = 1;
+    // Two sets of waves to a tile instead, each on one half of its keys, where a tile a compute unit is all there is and its
+    // keys are worth it (and, up to half as many tiles, no more shares could be lent for).  One set / two, us, f16 and bf16 alike:
+    //   head_dim 128, causal  32 heads x 300 (96 tiles) 11.6 / 12.1   x 512 (128) 16.6 / 16.0   x 773 (224) 22.5 / 20.4   x 1024 (256) 27.9 / 24.3
+    //                         x 1500 (384) 44.9 / 45.4                16 x 2048 (256) 46.7 / 36.9 (two shares 42)         8 x 4096 (256) 85.5 / 63.8
+    //   head_dim 128, full    32 x 1024 (256) 29.1 / 26.1             32 x 1500 (384) 49.9 / 59.8  8 x 4096 (256) 89.3 / 76.4
+    //   head_dim 64           causal 32 x 1024 (256) 19.8 / 16.6, 8 x 4096 (256) 60.6 / 43.4; full 64 x 512 (256) 12.9 / 11.6, 8 x 4096 63.1 / 47.8
+    const uint64_t query_tiles = static_cast<uint64_t>(c.batch) * c.heads * args.query_tiles, seen = c.causal && c.query_len < c.key_len ? c.query_len : c.key_len;
+    const bool halves = !with_options && args.packed_heads == 0 && args.single_tiles != 0 && query_tiles <= compute_units() && seen >= 512 &&
+                        (splits == 1 || 2 * query_tiles > compute_units());
+    if (halves) splits = 1;
     args.splits = splits;
     if (splits > 1) {
         const size_t row_count = static_cast<size_t>(c.batch) * c.heads * c.query_len;
@@ -365,6 +375,10 @@ int32_t prefill(void* stream, uint16_t* out, size_t out_len, float* lse, size_t 
             args.query_tiles = static_cast<uint32_t>(tiles);
             groups = (all + 63) / 64 * 64;
         }
+    }
+    if (halves) {
+        const int kernel = prefill_halves_at(head_dim) + (c.causal ? 0 : 1) + (f16 ? 2 : 0);
+        return launch(static_cast<KernelId>(kernel), static_cast<unsigned>(groups), 1, 1, 128 * kDensePrefillWaves, stream, args);
     }
     const KernelId kernel = static_cast<KernelId>((f16 ? kPrefillCausalF16 : kPrefillCausal) + (c.causal ? 0 : 1) + (with_options ? 4 : 0));
     if (int32_t status = launch(at_head_dim(kernel, head_dim), static_cast<unsigned>(groups), 1, 1, 64 * kDensePrefillWaves, stream, args))

@@ -55,13 +55,18 @@ SINGE_DEVICE void fold_window_tile(Half half, f32x16_t& scores, const uint4 (&q)
 // One 128-row query tile of (batch, head) pair `bh`.
 // OPTIONS: the dense op's additive mask, window and score cap, applied block by block to the scaled scores; every
 // tile then takes the masked path.
-template <bool CAUSAL, class Half, int WAVES, bool OPTIONS>
+// HALVES == 2: the tile has two sets of waves and of LDS stages (`lds` is the first one's), which walk one half of its keys
+// each and meet at the end.
+template <bool CAUSAL, class Half, int WAVES, bool OPTIONS, int HALVES = 1>
 SINGE_DEVICE void fmha_prefill_tile(const PrefillArgs& a, unsigned char* lds, unsigned int bh, unsigned int query_tile, unsigned int split) {
     constexpr unsigned int kRows = 32u * WAVES;        // query rows of the workgroup
     constexpr unsigned int kWaveLoadRows = 1024u / kRowBytes;      // key rows one load instruction brings in
     constexpr unsigned int kLoadRows = kWaveLoadRows * WAVES;      // and one of every wave
     constexpr unsigned int kLoads = kKeyTile / kLoadRows;
-    const unsigned int tid = threadIdx.x, lane = tid & 63;
+    static_assert(HALVES == 1 || (HALVES == 2 && WAVES == 4 && !OPTIONS), "two halves of four waves");
+    const unsigned int set = HALVES == 1 ? 0u : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+    const unsigned int tid = HALVES == 1 ? threadIdx.x : threadIdx.x & 255u, lane = tid & 63;
+    lds += set * kStagedLdsBytes;
     // The wave index is the same in all lanes; saying so keeps everything derived from it (which blocks
     // are live, whether a block is on the mask's edge, LDS bases) in scalar registers and scalar branches.
     const unsigned int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -150,6 +155,15 @@ SINGE_DEVICE void fmha_prefill_tile(const PrefillArgs& a, unsigned char* lds, un
         wave_blocks = wave_blocks < 2u * tiles ? wave_blocks : 2u * tiles;
     }
 
+    unsigned int half_tiles = 0;
+    if constexpr (HALVES == 2) {
+        half_tiles = (tiles + 1u) / 2u;  // (of either set; the second one's may be one fewer, and it then waits at a barrier more)
+        first_tile = set * half_tiles;
+        tiles = tiles < first_tile + half_tiles ? tiles : first_tile + half_tiles;
+        first_tile = first_tile < tiles ? first_tile : tiles;
+        wave_blocks = wave_blocks < 2u * tiles ? wave_blocks : 2u * tiles;
+    }
+
     // With options: the keys this lane's row sees, [my_low, my_low + my_span), the first key that every row of the wave sees
     // (last_low: the last row's) and the first block that any row of it does.
     unsigned int my_low = 0, my_span = 0, last_low = 0, wave_first_block = 2u * first_tile;
@@ -220,7 +234,7 @@ SINGE_DEVICE void fmha_prefill_tile(const PrefillArgs& a, unsigned char* lds, un
 
     RowState state;
     reset(state);
-    if (a.sinks != nullptr && split == 0) {
+    if (a.sinks != nullptr && split == 0 && set == 0) {
         // The head's sink: a score that is always there and weighs no value.  The row starts with it as its reference
         // point and a sum of one (held by one of the row's two lanes).
         const uint16_t bits = a.sinks[head];
@@ -403,6 +417,33 @@ SINGE_DEVICE void fmha_prefill_tile(const PrefillArgs& a, unsigned char* lds, un
         leave();
     }
 
+    if constexpr (HALVES == 2) {
+        // The second set's state goes through its own stages, which nobody reads any more after as many barriers as tiles;
+        // lane l of wave w finds that of the same rows and dims, since either set's waves have the tile's rows.
+        for (unsigned int done = tiles - first_tile; done < half_tiles; ++done) __syncthreads();
+        constexpr unsigned int kWords = (16u * kDimBlocks + 2u) * 64u;  // of a wave
+        static_assert(4u * kWords * 4u <= static_cast<unsigned int>(kStagedLdsBytes), "a set's state fits its stages");
+        float* const other = reinterpret_cast<float*>(lds + (set == 0 ? kStagedLdsBytes : 0)) + wave * kWords + lane;
+        if (set == 1) {
+#pragma unroll
+            for (int db = 0; db < kDimBlocks; ++db)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) other[64 * (16 * db + r)] = state.out[db][r];
+            other[64 * 16 * kDimBlocks] = state.reference;
+            other[64 * (16 * kDimBlocks + 1)] = state.running_sum;
+        }
+        __syncthreads();
+        if (set == 1) return;
+        const float reference = other[64 * 16 * kDimBlocks], largest = fmaxf(state.reference, reference);
+        const float mine = state.reference == -INFINITY ? 0.0f : fast_exp2(state.reference - largest);
+        const float theirs = reference == -INFINITY ? 0.0f : fast_exp2(reference - largest);
+        state.running_sum = fmaf(state.running_sum, mine, theirs * other[64 * (16 * kDimBlocks + 1)]);
+        state.reference = largest;
+#pragma unroll
+        for (int db = 0; db < kDimBlocks; ++db)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) state.out[db][r] = fmaf(state.out[db][r], mine, theirs * other[64 * (16 * db + r)]);
+    }
     // Normalise and store.  Lane (query, hi) holds dims 32db + 8(r / 4) + 4hi + (r % 4).
     const float sum = swap32_sum(state.running_sum);
     const float inverse = sum > 0.0f ? 1.0f / sum : 0.0f;
@@ -439,7 +480,7 @@ SINGE_DEVICE void fmha_prefill_tile(const PrefillArgs& a, unsigned char* lds, un
 }
 
 // Workgroup id -> (batch * heads + head, pair of query tiles): see the header comment.
-template <bool CAUSAL, class Half, int WAVES, bool OPTIONS = false>
+template <bool CAUSAL, class Half, int WAVES, bool OPTIONS = false, int HALVES = 1>
 SINGE_DEVICE void fmha_prefill_body(const PrefillArgs& a, unsigned char* lds) {
     const unsigned int xcd = blockIdx.x & 7u;
     unsigned int within = blockIdx.x >> 3;
@@ -460,8 +501,8 @@ SINGE_DEVICE void fmha_prefill_body(const PrefillArgs& a, unsigned char* lds) {
         heavy = a.query_tiles - 1u - within % pairs;
         light = a.single_tiles != 0 ? heavy : within % pairs;
     }
-    fmha_prefill_tile<CAUSAL, Half, WAVES, OPTIONS>(a, lds, bh, heavy, split);
-    if (light != heavy) fmha_prefill_tile<CAUSAL, Half, WAVES, OPTIONS>(a, lds, bh, light, split);
+    fmha_prefill_tile<CAUSAL, Half, WAVES, OPTIONS, HALVES>(a, lds, bh, heavy, split);
+    if (HALVES == 1 && light != heavy) fmha_prefill_tile<CAUSAL, Half, WAVES, OPTIONS, HALVES>(a, lds, bh, light, split);
 }
 
 // Merges the key splits of a row: each share's rows weigh 2^(lse - largest) over the sum of those (the reference's
@@ -538,6 +579,15 @@ SINGE_DEVICE void fmha_prefill_combine_body(const PrefillArgs& a) {
         fmha_prefill_body<CAUSAL, prefill::HALF, kDenseWaves, true>(args, prefill_lds);             \
     }
 
+// Two sets of four waves to a tile, for launches that leave compute units with one tile or none: its keys are walked from two
+// places at once.  Bound by the longest tile's walk (the two sets meet at one barrier a tile, which costs some of what half
+// the walk gains): 1 x 32 / 8 heads x 773 x 128, f16, causal 22.5 -> 20.4 us, 16 heads x 2048 46.7 -> 36.9 us.
+#define SINGE_FMHA_PREFILL_HALVES_KERNEL(NAME, CAUSAL, HALF)                                       \
+    extern "C" __global__ __launch_bounds__(128 * kDenseWaves, 2) void NAME(PrefillArgs args) {      \
+        __shared__ __attribute__((aligned(1024))) unsigned char prefill_lds[2 * kStagedLdsBytes];    \
+        fmha_prefill_body<CAUSAL, prefill::HALF, kDenseWaves, false, 2>(args, prefill_lds);         \
+    }
+
 // Names carry the head dimension of the build: singe_fmha_prefill_bf16_d128_causal, ..._d64_causal.
 #define SINGE_PASTE3_(a, b, c) a##b##c
 #define SINGE_PASTE3(a, b, c) SINGE_PASTE3_(a, b, c)
@@ -551,5 +601,9 @@ SINGE_FMHA_PREFILL_KERNEL(SINGE_PREFILL_NAME(bf16, _causal), true, Bf16)
 SINGE_FMHA_PREFILL_KERNEL(SINGE_PREFILL_NAME(bf16, _full), false, Bf16)
 SINGE_FMHA_PREFILL_KERNEL(SINGE_PREFILL_NAME(f16, _causal), true, F16)
 SINGE_FMHA_PREFILL_KERNEL(SINGE_PREFILL_NAME(f16, _full), false, F16)
+SINGE_FMHA_PREFILL_HALVES_KERNEL(SINGE_PREFILL_NAME(bf16, _causal_halves), true, Bf16)
+SINGE_FMHA_PREFILL_HALVES_KERNEL(SINGE_PREFILL_NAME(bf16, _full_halves), false, Bf16)
+SINGE_FMHA_PREFILL_HALVES_KERNEL(SINGE_PREFILL_NAME(f16, _causal_halves), true, F16)
+SINGE_FMHA_PREFILL_HALVES_KERNEL(SINGE_PREFILL_NAME(f16, _full_halves), false, F16)
 extern "C" __global__ __launch_bounds__(256) void SINGE_PREFILL_NAME(bf16, _combine)(PrefillArgs args) { fmha_prefill_combine_body<prefill::Bf16>(args); }
 extern "C" __global__ __launch_bounds__(256) void SINGE_PREFILL_NAME(f16, _combine)(PrefillArgs args) { fmha_prefill_combine_body<prefill::F16>(args); }

@@ -387,6 +387,22 @@ const char* const kKernelNames[kKernelCount] = {
     "singe_attention_mfma_f32_d32_r16", "singe_attention_mfma_f32_d64_r16", "singe_attention_mfma_f32_d96_r16",
     "singe_attention_mfma_f32_d128_r16",
     "singe_attention_mfma_f32_d64_r32", "singe_attention_mfma_f32_d96_r32", "singe_attention_mfma_f32_d128_r32",
+    "singe_fmha_prefill_bf16_d128_causal_halves", "singe_fmha_prefill_bf16_d128_full_halves",
+    "singe_fmha_prefill_f16_d128_causal_halves", "singe_fmha_prefill_f16_d128_full_halves",
+    "singe_fmha_prefill_bf16_d64_causal_halves", "singe_fmha_prefill_bf16_d64_full_halves",
+    "singe_fmha_prefill_f16_d64_causal_halves", "singe_fmha_prefill_f16_d64_full_halves",
+    "singe_fmha_prefill_bf16_d32_causal_halves", "singe_fmha_prefill_bf16_d32_full_halves",
+    "singe_fmha_prefill_f16_d32_causal_halves", "singe_fmha_prefill_f16_d32_full_halves",
+    "singe_fmha_prefill_bf16_d96_causal_halves", "singe_fmha_prefill_bf16_d96_full_halves",
+    "singe_fmha_prefill_f16_d96_causal_halves", "singe_fmha_prefill_f16_d96_full_halves",
+    "singe_fmha_prefill_bf16_d16_causal_halves", "singe_fmha_prefill_bf16_d16_full_halves",
+    "singe_fmha_prefill_f16_d16_causal_halves", "singe_fmha_prefill_f16_d16_full_halves",
+    "singe_fmha_prefill_bf16_d48_causal_halves", "singe_fmha_prefill_bf16_d48_full_halves",
+    "singe_fmha_prefill_f16_d48_causal_halves", "singe_fmha_prefill_f16_d48_full_halves",
+    "singe_fmha_prefill_bf16_d80_causal_halves", "singe_fmha_prefill_bf16_d80_full_halves",
+    "singe_fmha_prefill_f16_d80_causal_halves", "singe_fmha_prefill_f16_d80_full_halves",
+    "singe_fmha_prefill_bf16_d112_causal_halves", "singe_fmha_prefill_bf16_d112_full_halves",
+    "singe_fmha_prefill_f16_d112_causal_halves", "singe_fmha_prefill_f16_d112_full_halves",
 };
 
 // The code object is built in parts, one per kernel source (so they compile side by side and a process loads only
@@ -442,6 +458,7 @@ constexpr PartRun kPartRuns[] = {
     {42, 8}, {43, 8}, {44, 8}, {45, 8}, {46, 8}, {47, 8}, {48, 8}, {49, 8}, {50, 8}, {51, 8},  // and at 112, 80, 48, 32, 16
     {3, 2}, {15, 2}, {19, 2}, {21, 2}, {23, 2}, {25, 2}, {27, 2}, {29, 2},    // packed sequences
     {52, 7},                      // dense f32 attention on the matrix cores
+    {1, 4}, {14, 4}, {18, 4}, {20, 4}, {22, 4}, {24, 4}, {26, 4}, {28, 4},    // the dense prefill with two sets of waves to a tile
 };
 constexpr int runs_total() {
     int total = 0;

@@ -102,7 +102,10 @@ enum KernelId : int {
     kRaggedPrefill = kPairOtherHeadDims + 5 * 16,
     // dense f32 attention on the matrix cores: head dimensions 32, 64, 96, 128 with 16-row tiles, then 64, 96, 128 with 32-row ones
     kAttentionMfmaF32 = kRaggedPrefill + 2 * 8,
-    kKernelCount = kAttentionMfmaF32 + 7
+    // the dense prefill with two sets of waves to a tile (no options), four to a head dimension in kRaggedPrefill's order:
+    // + (no causal mask) + 2 * f16
+    kPrefillHalves = kAttentionMfmaF32 + 7,
+    kKernelCount = kPrefillHalves + 4 * 8
 };
 
 // The two-tile kernels (fmha_prefill_pair.hip, paged_attention_pair.hip) have a build for every multiple of 16 up to 128.
@@ -176,6 +179,9 @@ inline KernelId prefill_combine_at(long long head_dim) {
 inline int head_dim_order(long long head_dim) {
     return head_dim == 128 ? 0 : head_dim == 64 ? 1 : 2 + (other_head_dim_bank(head_dim) - kOtherHeadDims) / (10 + (kSplitKReduce - kPagedAttentionI32));
 }
+
+// The dense prefill with two sets of waves to a tile for a head dimension, before 1 without the causal mask and 2 for f16.
+inline int prefill_halves_at(long long head_dim) { return kPrefillHalves + 4 * head_dim_order(head_dim); }
 
 // The packed-sequences kernel for a head dimension, before 1 is added for f16.
 inline int ragged_prefill_at(long long head_dim) { return kRaggedPrefill + 2 * head_dim_order(head_dim); }

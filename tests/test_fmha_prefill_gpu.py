@@ -292,3 +292,20 @@ def test_two_tiles_a_wave_head_major_layout(two_tiles_a_wave, causal, dim):
     want, want_lse = oracle.fmha_prefill_lse_f32(rows(q), rows(k), rows(v), batch=batch, query_len=query_len, key_len=key_len,
                                                  heads=heads, kv_heads=kv_heads, head_dim=dim, scale=scale, causal=causal, threads=8)
     check(rows(out), lse.cpu().numpy(), want, want_lse, f"two tiles, head-major layout, head_dim {dim}, causal={causal}")
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("batch,query_len,key_len,heads,kv_heads,dim", [
+    (1, 512, 512, 6, 6, 128),     # a diagonal tile in the second half
+    (1, 520, 577, 4, 2, 64),      # last tiles that are not whole: one row, one key
+    (2, 100, 513, 3, 1, 96),      # an odd count of key tiles: the sets' halves differ by one
+    (1, 640, 512, 2, 1, 48),      # rows past the last key under the mask
+    (1, 1000, 1000, 5, 5, 128),
+    (1, 130, 4100, 2, 2, 16),
+    (1, 600, 700, 2, 1, 112),
+])
+def test_two_sets_of_waves_to_a_tile_match_oracle(batch, query_len, key_len, heads, kv_heads, dim, causal):
+    """Launches of no more tiles than compute units over at least 512 keys: either half of the keys has waves of its own."""
+    q, k, v = make(batch, query_len, key_len, heads, kv_heads, seed=query_len + 3 * key_len, dim=dim)
+    got, lse, want, want_lse = run(q, k, v, causal)
+    check(got, lse, want, want_lse, f"two sets of waves: {query_len} x {key_len}, {dim}, causal={causal}")
