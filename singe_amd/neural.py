@@ -12,6 +12,7 @@ from dataclasses import dataclass
 import torch
 
 from . import _native, error
+from .kernel.attention import _stream_handle
 
 STATUS_INDEX_OUT_OF_BOUNDS = 1  # singe/src/backend/kernel_lowering/mod.rs:40-61
 
@@ -159,7 +160,7 @@ def _attend_all_ordered(query, key, value, mask, sinks, key_lengths, options, *,
         options.scale if options.scale is not None else 0.0, options.softcap if options.softcap is not None else 0.0,
         options.window if options.window is not None else 0)
     output = torch.empty((batch, heads, query_len, value_dim), device=query.device, dtype=query.dtype)
-    handle = int((stream or torch.cuda.current_stream()).cuda_stream)
+    handle = _stream_handle(stream)
     pointer = lambda tensor: tensor.data_ptr() if tensor is not None else None
     # A decode-shaped call (few query rows, many keys) shares its keys out over several workgroups, on this module's
     # per-device scratch (calls on different streams must then not overlap), as the reference's plan splits them
@@ -280,7 +281,7 @@ def paged_attention(query: torch.Tensor, key_cache: torch.Tensor, value_cache: t
         lse = torch.full(query.shape[:2], float("-inf"), device=query.device, dtype=torch.float32)
     if status is None:
         status = torch.zeros(1, device=query.device, dtype=torch.int32)
-    handle = int((stream or torch.cuda.current_stream()).cuda_stream)
+    handle = _stream_handle(stream)
     # 16-bit calls with few query rows (decoding) share a row tile's keys out over several workgroups, given
     # scratch: ``scratch`` is a uint8 device tensor, True for this module's own per-device buffer (calls on
     # different streams must then not overlap), or False for none.
@@ -357,7 +358,7 @@ def paged_mla_attention(query: torch.Tensor, query_positions: torch.Tensor, late
         lse = torch.full((tokens, heads), float("-inf"), device=query.device, dtype=torch.float32)
     if status is None:
         status = torch.zeros(1, device=query.device, dtype=torch.int32)
-    handle = int((stream or torch.cuda.current_stream()).cuda_stream)
+    handle = _stream_handle(stream)
     wanted = 0 if scratch is False else int(_native.lib().singe_hip_paged_mla_attention_scratch_bytes(ctypes.byref(problem)))
     lent = None if wanted == 0 else _scratch_for(query.device, wanted) if scratch is True else scratch
     entry = _native.lib().singe_hip_paged_mla_attention_every_row if every_row else _native.lib().singe_hip_paged_mla_attention_scratch
@@ -408,7 +409,7 @@ def rotary_paged_attention(query: torch.Tensor, key_cache: torch.Tensor, value_c
     lse = torch.full(query.shape[:2], float("-inf"), device=query.device, dtype=torch.float32)
     if status is None:
         status = torch.zeros(1, device=query.device, dtype=torch.int32)
-    handle = int((stream or torch.cuda.current_stream()).cuda_stream)
+    handle = _stream_handle(stream)
     entry = _native.lib().singe_hip_rotary_paged_attention_bf16 if query.dtype == torch.bfloat16 else _native.lib().singe_hip_rotary_paged_attention_f16
     code = entry(
         handle, query.data_ptr(), key_cache.data_ptr(), value_cache.data_ptr(), paging.query_offsets.data_ptr(),
@@ -471,7 +472,7 @@ def rotary_cache_write(query, key, value, cos, sin, pages, slots, key_cache, val
     if status is None:
         status = torch.zeros(1, device=key.device, dtype=torch.int32)
     pointer = lambda tensor: tensor.data_ptr() if tensor is not None else None
-    handle = int((stream or torch.cuda.current_stream()).cuda_stream)
+    handle = _stream_handle(stream)
     code = _native.lib().singe_hip_rotary_cache_write(
         handle, pointer(query), key.data_ptr(), value.data_ptr(), cos.data_ptr(), sin.data_ptr(), pages.contiguous().data_ptr(),
         slots.contiguous().data_ptr(), pointer(weights[0]), pointer(weights[1]), pointer(query_out), key_cache.data_ptr(),
@@ -503,7 +504,7 @@ def paging_indices(paging: Paging, *, tokens: int, page_size: int, cache_pages: 
         status = torch.zeros(1, device=device, dtype=torch.int32)
     problem = _native.PagingIndicesProblemC(sequences, tokens, paging.pages.numel(), page_size, cache_pages, width, row_elements,
                                             1 if paging.pages.dtype == torch.int64 else 0)
-    handle = int((stream or torch.cuda.current_stream()).cuda_stream)
+    handle = _stream_handle(stream)
     code = _native.lib().singe_hip_paging_indices(
         handle, paging.query_offsets.data_ptr(), paging.page_offsets.data_ptr(), paging.pages.data_ptr(),
         paging.last_page_lengths.data_ptr(), packed.data_ptr(), query_lengths.data_ptr(), key_lengths.data_ptr(), table.data_ptr(),
