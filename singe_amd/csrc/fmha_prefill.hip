@@ -116,13 +116,10 @@ SINGE_DEVICE void fmha_prefill_tile(const PrefillArgs& a, unsigned char* lds, un
     {
         const uint16_t* row = q_base + static_cast<size_t>(query_valid ? my_query : 0) * a.query_sequence_stride + 8 * hi;
 #pragma unroll
-        for (int s = 0; s < kSteps; ++s) {
-            uint4 bits = *reinterpret_cast<const uint4*>(row + 16 * s);
-            if (!query_valid) bits = make_uint4(0, 0, 0, 0);
-            bits.x ^= flip; bits.y ^= flip; bits.z ^= flip; bits.w ^= flip;
-            q[s] = bits;
-        }
+        for (int s = 0; s < kSteps; ++s) q[s] = *reinterpret_cast<const uint4*>(row + 16 * s);
     }
+    const bool has_sink = a.sinks != nullptr && split == 0 && set == 0;
+    const uint16_t sink_bits = *(has_sink ? a.sinks + head : a.query);  // (some word without one: a load in a branch is waited for there)
 
     // Keys this workgroup must visit, and the blocks of them this wave folds: under the causal mask a
     // block wholly after the wave's last query contributes nothing.
@@ -232,20 +229,7 @@ SINGE_DEVICE void fmha_prefill_tile(const PrefillArgs& a, unsigned char* lds, un
         load_tile(v_bytes, value_stride_bytes, value_lane, value_chunk, value_lane_live, tile, stage);
     };
 
-    RowState state;
-    reset(state);
-    if (a.sinks != nullptr && split == 0 && set == 0) {
-        // The head's sink: a score that is always there and weighs no value.  The row starts with it as its reference
-        // point and a sum of one (held by one of the row's two lanes).
-        const uint16_t bits = a.sinks[head];
-        float sink;
-        if constexpr (std::is_same_v<Half, F16>) sink = static_cast<float>(__builtin_bit_cast(_Float16, bits));
-        else sink = __builtin_bit_cast(float, static_cast<unsigned int>(bits) << 16);
-        state.reference = sink * kLog2e;
-        state.running_sum = hi == 0 && state.reference != -INFINITY ? 1.0f : 0.0f;
-    }
     const ReadOffsets offsets = read_offsets(lane);
-
     if (first_tile < tiles) {
         load_keys(first_tile, lds);
         load_values(first_tile, lds + kValueBase);
@@ -253,6 +237,26 @@ SINGE_DEVICE void fmha_prefill_tile(const PrefillArgs& a, unsigned char* lds, un
     if (first_tile + 1 < tiles) load_keys(first_tile + 1, lds + kTileBytes);
     loads_landed();
     __syncthreads();
+
+    // What was asked for before the tiles is first touched here, so that its round trip to memory is the tiles' own.  (Rows
+    // past the end zeroed where they are loaded were a branch and a wait a load, and the sink's word another one: 64 / 8
+    // heads x 8192 x 64, window 128, sinks 64.7 us so, 61.1 as it is; 1 x 32 / 8 heads x 773 x 128 19.76 and 19.61.)
+#pragma unroll
+    for (int s = 0; s < kSteps; ++s) {
+        if (!query_valid) q[s] = make_uint4(0, 0, 0, 0);
+        q[s].x ^= flip; q[s].y ^= flip; q[s].z ^= flip; q[s].w ^= flip;
+    }
+    RowState state;
+    reset(state);
+    if (has_sink) {
+        // The head's sink: a score that is always there and weighs no value.  The row starts with it as its reference
+        // point and a sum of one (held by one of the row's two lanes).
+        float sink;
+        if constexpr (std::is_same_v<Half, F16>) sink = static_cast<float>(__builtin_bit_cast(_Float16, sink_bits));
+        else sink = __builtin_bit_cast(float, static_cast<unsigned int>(sink_bits) << 16);
+        state.reference = sink * kLog2e;
+        state.running_sum = hi == 0 && state.reference != -INFINITY ? 1.0f : 0.0f;
+    }
 
     // Folds block `block` (scores in `s`, values at `values`) with the mask's edges applied.
     auto fold = [&](unsigned int block, f32x16_t& s, const unsigned char* values) __attribute__((always_inline)) {
