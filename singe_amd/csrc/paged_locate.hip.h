@@ -26,13 +26,40 @@ constexpr unsigned int kNoPage = 0xFFFFFFFFu;  // a table entry outside the cach
 // finds its entry by a prefix sum over the sequences' query counts, 64 sequences at a time.  The list is cut into
 // bands of 32 entries; (band, kv head) pairs go round the XCDs, so a band's tiles for one kv head are neighbours on
 // one XCD and walk their keys side by side.
+// Whether a CSR sequence's query offsets make no sense (its own checks report it).  Such a sequence has one entry, and a list
+// that holds one is taken in sequence order whatever the call asked for: the sequences before the first of them follow one
+// another inside [0, tokens] and fit the grid, and it comes next, so the error is reported however many row tiles the
+// sequences after it claim.  (Those may then lie past the grid; a sequence of which any row tile does is not attended.)
+template <int FORM>
+SINGE_DEVICE bool bad_queries(long long start, long long end, unsigned int tokens) {
+    if constexpr (has_lengths(FORM)) return false;
+    return start < 0 || end < start || end > static_cast<long long>(tokens);
+}
+
+// Entries of sequence `s` in the list; `bad` as above.
+template <int FORM, unsigned int ROWS>
+SINGE_DEVICE unsigned int row_tiles_of(const void* query_offsets, const void* query_lengths, unsigned int tokens, unsigned int groups,
+                                       unsigned int s, bool& bad) {
+    long long count;
+    bad = false;
+    if constexpr (has_lengths(FORM)) {
+        count = read_index<FORM>(query_lengths, s);
+        count = count < 0 ? 0 : count > static_cast<long long>(tokens) ? static_cast<long long>(tokens) : count;
+    } else {
+        const long long start = read_index<FORM>(query_offsets, s), end = read_index<FORM>(query_offsets, s + 1);
+        bad = bad_queries<FORM>(start, end, tokens);
+        count = bad ? 0 : end - start;
+    }
+    const unsigned long long tiles = (static_cast<unsigned long long>(count) * groups + ROWS - 1) / ROWS;
+    return tiles == 0 ? 1u : static_cast<unsigned int>(tiles);
+}
+
 // a.longest_first (at most 64 sequences, several row tiles each: chunks of a prefill): the compact list takes the
 // sequences longest first (by pages held, ties by index), so that the workgroups with the most keys to walk start
 // first and the short ones fill the chip's last round.  Lane s learns how many list entries come before sequence s's
-// own (`mine` of them) in that order; any values give some order, and a sequence's own checks report the ones that
-// make no sense.  (Decode-shaped calls keep the sequences' own order: their workgroups are short, and the two loads
-// and the ranking in front of everything else cost them more than the order gains: 62 -> 70 us on the decode
-// benchmark's shape.)
+// own (`mine` of them) in that order.  (Decode-shaped calls keep the sequences' own order: their workgroups are short,
+// and the two loads and the ranking in front of everything else cost them more than the order gains: 62 -> 70 us on the
+// decode benchmark's shape.)
 template <int FORM>
 SINGE_DEVICE unsigned int entries_before_longest_first(const PagedAttentionArgs& a, unsigned int mine) {
     const unsigned int s = threadIdx.x & 63u;
@@ -56,17 +83,19 @@ SINGE_DEVICE unsigned int entries_before_longest_first(const PagedAttentionArgs&
 // them with runs of the others' row tiles, as many of either as an XCD's compute units hold one of.  The first bring the
 // cache from memory with the matrix cores all but idle (paged_narrow.hip.h), the others use the matrix cores on keys that
 // the XCD's L2 holds; side by side on a compute unit they take little from each other, and a long sequence that starts last
-// would run on by itself.  (Lengths are compared up to 4095 pages.  Sequences whose offsets make no sense come first of
-// all, so that one is in the grid however many tiles the others claim.)
-// Finds the entry's sequence and row tile; false past the list's end.
+// would run on by itself.  (Lengths are compared up to 4095 pages.)
+// Finds the entry's sequence and row tile; kPastList past the list's end, kInOrder where offsets make no sense and the list
+// is taken in sequence order.
+enum class Alternating { kFound, kPastList, kInOrder };
 constexpr int kAlternateChunks = 4;
 template <int FORM, unsigned int ROWS>
-SINGE_DEVICE bool locate_alternating(const PagedAttentionArgs& a, unsigned int entry, unsigned int& sequence, unsigned int& row_tile) {
+SINGE_DEVICE Alternating locate_alternating(const PagedAttentionArgs& a, unsigned int entry, unsigned int& sequence, unsigned int& row_tile) {
     const unsigned int lane = threadIdx.x & 63u, groups = a.heads / a.kv_heads;
-    constexpr unsigned int kMostHeld = 4095u, kHeldBits = 13u;
+    constexpr unsigned int kMostHeld = 4095u, kHeldBits = 12u;
     unsigned long long narrow[kAlternateChunks];
     unsigned int held[kAlternateChunks], tiles[kAlternateChunks], through[kAlternateChunks];  // tiles: of wide sequences, and their inclusive prefix sums
     unsigned int narrow_count = 0, wide_count = 0;
+    bool any_bad = false;
 #pragma unroll
     for (int c = 0; c < kAlternateChunks; ++c) {
         narrow[c] = 0;
@@ -75,12 +104,13 @@ SINGE_DEVICE bool locate_alternating(const PagedAttentionArgs& a, unsigned int e
         const unsigned int s = 64u * c + lane;
         bool is_narrow = false;
         if (s < a.sequences) {
-            const long long count = read_index<FORM>(a.query_offsets, s + 1) - read_index<FORM>(a.query_offsets, s);
+            const long long start = read_index<FORM>(a.query_offsets, s), end = read_index<FORM>(a.query_offsets, s + 1);
             const long long pages = read_index<FORM>(a.page_offsets, s + 1) - read_index<FORM>(a.page_offsets, s);
-            const bool bad = count < 0 || count > static_cast<long long>(a.tokens);
-            const unsigned long long rows = bad ? 0ull : static_cast<unsigned long long>(count) * groups;
+            const bool bad = bad_queries<FORM>(start, end, a.tokens);
+            any_bad |= bad;
+            const unsigned long long rows = bad ? 0ull : static_cast<unsigned long long>(end - start) * groups;
             is_narrow = rows <= 16u;
-            held[c] = bad ? 2u * kMostHeld + 1u : pages < 0 ? 0u : pages > static_cast<long long>(kMostHeld) ? kMostHeld : static_cast<unsigned int>(pages);
+            held[c] = pages < 0 ? 0u : pages > static_cast<long long>(kMostHeld) ? kMostHeld : static_cast<unsigned int>(pages);
             tiles[c] = is_narrow ? 0u : static_cast<unsigned int>((rows + ROWS - 1) / ROWS);
         }
         narrow[c] = __ballot(is_narrow);
@@ -93,6 +123,7 @@ SINGE_DEVICE bool locate_alternating(const PagedAttentionArgs& a, unsigned int e
         }
         wide_count += __builtin_amdgcn_readlane(through[c], 63);
     }
+    if (__any(any_bad)) return Alternating::kInOrder;
     const unsigned int run = a.kv_heads >= 256u ? 1u : 256u / a.kv_heads;
     const unsigned int narrow_runs = narrow_count / run, wide_runs = wide_count / run, pairs = narrow_runs < wide_runs ? narrow_runs : wide_runs;
     bool takes_narrow;
@@ -107,7 +138,7 @@ SINGE_DEVICE bool locate_alternating(const PagedAttentionArgs& a, unsigned int e
         index = run * pairs + (takes_narrow ? rest - wide_left : rest);
     }
     if (takes_narrow) {
-        if (index >= narrow_count) return false;
+        if (index >= narrow_count) return Alternating::kPastList;
         // The index-th longest: bit by bit from the top, keep the candidates that have the bit where enough of them do.
 #pragma unroll 1
         for (int bit = kHeldBits - 1; bit >= 0; --bit) {
@@ -130,11 +161,11 @@ SINGE_DEVICE bool locate_alternating(const PagedAttentionArgs& a, unsigned int e
                 const bool mine = (narrow[c] >> lane & 1ull) != 0 && static_cast<unsigned int>(__builtin_popcountll(narrow[c] & ((1ull << lane) - 1ull))) == index;
                 sequence = 64u * c + static_cast<unsigned int>(__builtin_ctzll(__ballot(mine)));
                 row_tile = 0;
-                return true;
+                return Alternating::kFound;
             }
             index -= here;
         }
-        return false;
+        return Alternating::kPastList;
     }
 #pragma unroll
     for (int c = 0; c < kAlternateChunks; ++c) {
@@ -143,11 +174,11 @@ SINGE_DEVICE bool locate_alternating(const PagedAttentionArgs& a, unsigned int e
             const unsigned int owner = static_cast<unsigned int>(__builtin_ctzll(__ballot(index < through[c])));
             sequence = 64u * c + owner;
             row_tile = index - (__builtin_amdgcn_readlane(through[c], owner) - __builtin_amdgcn_readlane(tiles[c], owner));
-            return true;
+            return Alternating::kFound;
         }
         index -= total;
     }
-    return false;
+    return Alternating::kPastList;
 }
 
 // kPacked only: packed sequences may overlap, and their row tiles can then outnumber the list the grid was sized for.
@@ -173,22 +204,22 @@ SINGE_DEVICE bool locate(const PagedAttentionArgs& a, unsigned int& unit, unsign
         if constexpr (FORM == kCsrI32 || FORM == kCsrI64) {
             if (a.alternate != 0) {
                 unsigned int sequence;
-                if (!locate_alternating<FORM, ROWS>(a, entry, sequence, row_tile)) return false;
-                unit = sequence * a.kv_heads + kv_head;
-                return true;
+                const Alternating found = locate_alternating<FORM, ROWS>(a, entry, sequence, row_tile);
+                if (found == Alternating::kPastList) return false;
+                if (found == Alternating::kFound) {
+                    unit = sequence * a.kv_heads + kv_head;
+                    return true;
+                }
             }
         }
         const unsigned int lane = threadIdx.x & 63u, groups = a.heads / a.kv_heads;
-        auto tiles_of = [&](unsigned int s) __attribute__((always_inline)) {
-            long long count;
-            if constexpr (has_lengths(FORM)) count = read_index<FORM>(a.query_lengths, s);
-            else count = read_index<FORM>(a.query_offsets, s + 1) - read_index<FORM>(a.query_offsets, s);
-            count = count < 0 ? 0 : count > static_cast<long long>(a.tokens) ? static_cast<long long>(a.tokens) : count;
-            const unsigned long long tiles = (static_cast<unsigned long long>(count) * groups + ROWS - 1) / ROWS;
-            return tiles == 0 ? 1u : static_cast<unsigned int>(tiles);
+        auto tiles_of = [&](unsigned int s, bool& bad) __attribute__((always_inline)) {
+            return row_tiles_of<FORM, ROWS>(a.query_offsets, a.query_lengths, a.tokens, groups, s, bad);
         };
-        if (a.longest_first != 0) {
-            const unsigned int mine = lane < a.sequences ? tiles_of(lane) : 0u;
+        bool bad = false;
+        const unsigned int first_mine = a.longest_first != 0 && lane < a.sequences ? tiles_of(lane, bad) : 0u;
+        if (a.longest_first != 0 && !__any(bad)) {
+            const unsigned int mine = first_mine;
             const unsigned int before = entries_before_longest_first<FORM>(a, mine);
             const unsigned long long holds = __ballot(entry >= before && entry - before < mine);
             if (holds == 0) return false;
@@ -200,10 +231,11 @@ SINGE_DEVICE bool locate(const PagedAttentionArgs& a, unsigned int& unit, unsign
             if constexpr (FORM == kPacked) row_tile = __shfl(mine, owner, 64) - 1u - row_tile;
             return true;
         }
-        // (from here on `entry` counts from the first row tile of the sequences looked at)
+        // (from here on `entry` counts from the first row tile of the sequences looked at, `left` what the list holds from there)
+        unsigned int left = a.row_tiles;
         for (unsigned int first = 0; first < a.sequences; first += 64u) {
             const unsigned int s = first + lane;
-            const unsigned int mine = s < a.sequences ? tiles_of(s) : 0u;
+            const unsigned int mine = s < a.sequences ? tiles_of(s, bad) : 0u;
             unsigned int through = mine;  // inclusive prefix sum over the wave
 #pragma unroll
             for (int step = 1; step < 64; step <<= 1) {
@@ -215,11 +247,13 @@ SINGE_DEVICE bool locate(const PagedAttentionArgs& a, unsigned int& unit, unsign
                 const unsigned long long holds = __ballot(entry < through);  // first lane whose range reaches the entry
                 const unsigned int owner = static_cast<unsigned int>(__builtin_ctzll(holds));
                 const unsigned int owner_through = __shfl(through, owner, 64), owner_mine = __shfl(mine, owner, 64);
+                if (!has_lengths(FORM) && owner_through > left) return false;  // (only behind offsets that make no sense)
                 unit = (first + owner) * a.kv_heads + kv_head;
                 row_tile = static_cast<unsigned int>(entry) - (owner_through - owner_mine);
                 return true;
             }
             entry -= total;
+            left -= total;
         }
         return false;
     }

@@ -521,6 +521,43 @@ def poison(*shapes):
     del blocks
 
 
+def run_backwards(heads, kv_heads, tokens, offsets, page_counts, rows_per_wave=0):
+    """The outputs, the status word and what the call needs again, for sequences whose query offsets need not make sense."""
+    page_size, cache_pages = 16, 50
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(tokens + len(offsets))
+    rand = lambda *shape: torch.randn(shape, generator=gen, device="cuda").to(torch.bfloat16)
+    index = lambda values: torch.tensor([int(v) for v in values], dtype=torch.int32, device="cuda")
+    ends = np.concatenate([[0], np.cumsum(page_counts)])
+    paging = neural.Paging(index(offsets), index(ends), index(np.arange(ends[-1]) % cache_pages), index([page_size] * len(page_counts)))
+    q, kc, vc = rand(tokens, heads, 128), rand(cache_pages, page_size, kv_heads, 128), rand(cache_pages, page_size, kv_heads, 128)
+    status = torch.zeros(1, dtype=torch.int32, device="cuda")
+    _native.lib().singe_hip_set_paged_attention_rows_per_wave(rows_per_wave)
+    try:
+        poison(((tokens, heads, 128), torch.bfloat16), ((tokens, heads), torch.float32))
+        out, lse = neural.paged_attention(q, kc, vc, paging, neural.AttentionOptions(causal=True), status=status, check=False)
+    finally:
+        _native.lib().singe_hip_set_paged_attention_rows_per_wave(0)
+    return out, lse, int(status.item()), (q, kc, vc, paging)
+
+
+# Sequences that claim the same tokens over and over, between them ones that run backwards: more row tiles than the grid holds in
+# front of the first of those, were they taken in any order but their own.
+BACKWARDS = {
+    "fewer decoding sequences than a run": (8, 1, 1000, [0, 1000] * 35 + [0], [40] * 70),
+    "a handful of sequences": (16, 2, 300, [0, 300] * 6, [40] * 11),
+    "longest first": (16, 2, 1000, [0, 1000] * 6, [40, 1] * 5 + [40]),
+    "past the last token": (16, 2, 1000, [0, 500, 1001, 1000, 200, 1000, 0, 1000], [40, 1, 1, 40, 40, 1, 40]),
+    "before the first token": (16, 2, 1000, [-1000, 0, 1000, 0, 1000, 0, 1000], [1, 40, 1, 40, 1, 40]),
+}
+
+
+@pytest.mark.parametrize("rows_per_wave", [32, 64])
+@pytest.mark.parametrize("case", BACKWARDS)
+def test_offsets_that_make_no_sense_are_reported_however_many_row_tiles_are_claimed(case, rows_per_wave):
+    assert run_backwards(*BACKWARDS[case], rows_per_wave=rows_per_wave)[2] == neural.STATUS_INDEX_OUT_OF_BOUNDS
+
+
 @pytest.mark.parametrize("index_dtype", [torch.int32, torch.int64])
 @pytest.mark.parametrize("case", ["row tiles", "shares", "two tiles a wave", "decode", "many keys"])
 def test_tokens_no_sequence_owns_are_zero_with_a_log_sum_exp_of_minus_infinity(case, index_dtype):
