@@ -488,7 +488,9 @@ SINGE_HIP_API void singe_hip_set_paged_attention_rows_per_wave(uint32_t rows);
  * 0 when the head dimension has no matrix-core build. */
 SINGE_HIP_API uint32_t singe_hip_paged_attention_rows_per_wave(const SingePagedAttentionProblem* problem);
 /* singe_hip_paged_attention_scratch_* for an output that holds nothing yet: the rows of tokens that no valid sequence owns
- * are written too, zeros with a log-sum-exp of -inf, where the others leave them as they are.  data_type SINGE_HIP_BF16 or
+ * are written too, zeros with a log-sum-exp of -inf, where the others leave them as they are.  Sequences before the first whose
+ * query offsets make no sense are attended as ever, those after it whole or not at all; rows of tokens that two of them claim
+ * are written, and not defined; the status word says that there is such a sequence.  data_type SINGE_HIP_BF16 or
  * SINGE_HIP_F16 at a head_dim that is a multiple of 16 up to 128 and at least one sequence; SINGE_HIP_UNSUPPORTED_WIDTH
  * otherwise.  `scratch` may be null. */
 SINGE_HIP_API int32_t singe_hip_paged_attention_every_row(
@@ -994,7 +996,8 @@ SINGE_HIP_API int32_t singe_hip_paged_mla_attention(
 SINGE_HIP_API size_t singe_hip_paged_mla_attention_scratch_bytes(const SingePagedMlaAttentionProblem* problem);
 SINGE_HIP_API void singe_hip_set_paged_mla_attention_splits(uint32_t splits);
 /* singe_hip_paged_mla_attention_scratch for an output that holds nothing yet: the rows of tokens that no valid sequence
- * owns are written too, zeros with a log-sum-exp of -inf, where the others leave them as they are.  For the shapes on the
+ * owns are written too, zeros with a log-sum-exp of -inf, where the others leave them as they are (and, as there, sequences after
+ * one whose query offsets make no sense are attended whole or not at all).  For the shapes on the
  * matrix cores and at least one sequence; SINGE_HIP_UNSUPPORTED_WIDTH otherwise.  `scratch` may be null. */
 SINGE_HIP_API int32_t singe_hip_paged_mla_attention_every_row(
     void* stream,

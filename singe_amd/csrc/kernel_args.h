@@ -179,7 +179,7 @@ struct PagedAttentionArgs {
     uint32_t table_type = 0;                  // SingeElement of cos and sin
     uint32_t has_query_norm = 0;              // RMS norm over the head dimension before the rotation
     float query_eps = 0.0f;
-    // Workgroups from this one on clear the rows of tokens that no valid sequence owns (clear_unowned_tokens); 0: none do.
+    // Workgroups from this one on clear the rows of tokens that no attended sequence owns (clear_unowned_tokens); 0: none do.
     uint32_t clear_from = 0;
 };
 
@@ -317,10 +317,10 @@ struct GeneralPagedArgs {
 // What the matrix-core latent kernel leaves for the merge about a unit (128 rows of a sequence at most).
 struct alignas(16) LatentUnit {
     uint64_t first_row;   // its first row of [tokens, heads]
-    uint64_t first_slot;  // its first partial row; share s of row r is `first_slot + s * rows + r`
+    uint64_t first_slot;  // its first partial row; share s of row r is `first_slot + s * share_stride + r`
+    uint64_t share_stride;
     uint32_t rows;        // 0: nothing to merge
     uint32_t shares;
-    uint32_t unused[2];
 };
 
 struct LatentAttentionArgs {
@@ -349,10 +349,10 @@ struct LatentAttentionArgs {
     float* partial_lse;
     uint32_t unit_band;              // matrix-core kernel: neighbouring units (row tiles) that go to one XCD together
     uint32_t share_budget;
-    uint32_t unit_slots;
+    uint32_t unit_slots;             // matrix-core kernel: the units that all sequences' offsets can make, and the records
     uint64_t slots;
     LatentUnit* units;               // null without splits
-    uint32_t clear_from;             // matrix-core kernel: workgroups from this one on clear the rows of tokens no valid sequence owns; 0: none do
+    uint32_t clear_from;             // matrix-core kernel: workgroups from this one on clear the rows of tokens no attended sequence owns; 0: none do
 };
 
 // singe_rotary_cache_write_*: contiguous operands of one element type; angles may be f32.

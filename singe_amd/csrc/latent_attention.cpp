@@ -139,7 +139,7 @@ int32_t paged_mla_attention(void* stream, const void* latent_queries, const void
     args.share_budget = 0;
     args.slots = 0;
     args.clear_from = 0;
-    args.unit_slots = 0;
+    args.unit_slots = static_cast<uint32_t>(blocks);
     args.units = nullptr;
     args.page_shift = -1;
     for (int shift = 0; shift < 31; ++shift)
@@ -159,7 +159,6 @@ int32_t paged_mla_attention(void* stream, const void* latent_queries, const void
             args.splits = shares.fixed;
             args.share_budget = shares.budget;
             args.slots = shares.slots;
-            args.unit_slots = static_cast<uint32_t>(blocks);
             args.partial_out = static_cast<float*>(scratch);
             args.partial_lse = args.partial_out + static_cast<size_t>(shares.slots) * 512;
             args.units = reinterpret_cast<LatentUnit*>(static_cast<unsigned char*>(scratch) + shares.records_at());

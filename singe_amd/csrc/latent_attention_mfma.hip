@@ -103,20 +103,16 @@ SINGE_DEVICE unsigned int chunk_flip(unsigned int key) {
 
 // Workgroup units map to (sequence, row tile) in sequence order: sequence s owns max(1, ceil(rows_s / 128)) units (one
 // even without rows, so that its paging values are checked), which every wave finds for itself by a prefix sum over
-// the query offsets, 64 sequences at a time.  Returns false for a unit past the last sequence's.
+// the query offsets, 64 sequences at a time.  Returns false for a unit past the last sequence's, and for one of a sequence
+// that has a unit past a.unit_slots (only behind offsets that make no sense: see bad_queries).
 template <int FORM>
 SINGE_DEVICE bool find_unit(const LatentAttentionArgs& a, unsigned int unit, unsigned int& sequence, unsigned int& row_tile) {
     const unsigned int lane = threadIdx.x & 63u;
     unsigned int base = 0;
     for (unsigned int first = 0; first < a.sequences; first += 64u) {
         const unsigned int s = first + lane;
-        unsigned int mine = 0;
-        if (s < a.sequences) {
-            long long count = read_index<FORM>(a.query_offsets, s + 1) - read_index<FORM>(a.query_offsets, s);
-            count = count < 0 ? 0 : count > static_cast<long long>(a.tokens) ? static_cast<long long>(a.tokens) : count;
-            const unsigned long long tiles = (static_cast<unsigned long long>(count) * a.heads + kRows - 1) / kRows;
-            mine = tiles == 0 ? 1u : static_cast<unsigned int>(tiles);
-        }
+        bool bad;
+        const unsigned int mine = s < a.sequences ? row_tiles_of<FORM, kRows>(a.query_offsets, nullptr, a.tokens, a.heads, s, bad) : 0u;
         unsigned int through = mine;  // inclusive prefix sum over the wave
 #pragma unroll
         for (int step = 1; step < 64; step <<= 1) {
@@ -128,6 +124,7 @@ SINGE_DEVICE bool find_unit(const LatentAttentionArgs& a, unsigned int unit, uns
             const unsigned long long holds = __ballot(unit < base + through);  // first lane whose range reaches the unit
             const unsigned int owner = static_cast<unsigned int>(__builtin_ctzll(holds));
             const unsigned int owner_through = __shfl(through, owner, 64), owner_mine = __shfl(mine, owner, 64);
+            if (base + owner_through > a.unit_slots) return false;
             sequence = first + owner;
             row_tile = unit - (base + owner_through - owner_mine);
             return true;
@@ -152,8 +149,9 @@ SINGE_DEVICE unsigned int across_wave(unsigned int value, Join join) {
 }
 
 // What of a problem a workgroup takes: share `share` of `shares` of the key tiles of a unit (a row tile of a sequence).
-// Shares are `share_tiles` long, or (0) the unit's tiles over the shares.  Partial rows of a unit start at `first_slot`,
-// its shares one after the other.
+// Shares are `share_tiles` long, or (0) the unit's tiles over the shares.  Partial rows of a unit start at `first_slot`, its
+// shares one after the other; with a fixed count of shares a row has the slot of its index in each share's [tokens, heads], so
+// that sequences which claim the same tokens (behind offsets that make no sense) disturb those tokens' rows alone.
 struct Placement {
     unsigned int sequence, row_tile, unit, share, shares, share_tiles;
     unsigned long long first_slot;
@@ -167,8 +165,9 @@ struct Placement {
 // which the shares of all units fit the budget, and every wave finds it for itself: the sequences' key tiles and row
 // tiles sit in the lanes' registers (the host takes this path up to 64 * kShareChunks sequences), the length lies
 // between tiles / budget and tiles / (budget - units), and a step of the search between them (four here) is a division
-// a lane and a sum over the wave.
-// Returns false for a workgroup past the last share; `units` is how many there are.
+// a lane and a sum over the wave.  A step with a sequence whose query offsets make no sense is not shared out: its units
+// are as many workgroups, none of which leaves the merge anything to do.
+// Returns false for a workgroup past the last share; `units` is how many leave a record for the merge.
 constexpr int kShareChunks = 4;
 constexpr unsigned int kMostShares = 64;      // of a unit: the merge keeps a share's weight a lane
 constexpr unsigned int kLeastShareTiles = 4;  // a workgroup's start and its way out cost about as much
@@ -178,23 +177,34 @@ SINGE_DEVICE bool place_balanced(const LatentAttentionArgs& a, unsigned int work
     auto add = [](unsigned int x, unsigned int y) { return x + y; };
     auto larger = [](unsigned int x, unsigned int y) { return x > y ? x : y; };
     unsigned int unit_count[kShareChunks], tile_count[kShareChunks], row_count[kShareChunks];
+    bool any_bad = false;
 #pragma unroll
     for (int c = 0; c < kShareChunks; ++c) {
         const unsigned int s = 64u * c + lane;
         unit_count[c] = tile_count[c] = row_count[c] = 0;
         if (s < a.sequences) {
-            // (as find_unit counts units; the sequence's own checks come later, counts that make no sense are held to their buffers)
-            long long count = read_index<FORM>(a.query_offsets, s + 1) - read_index<FORM>(a.query_offsets, s);
+            // (as find_unit counts units; the sequence's own checks come later, pages that make no sense are held to their buffers)
+            const long long start = read_index<FORM>(a.query_offsets, s), end = read_index<FORM>(a.query_offsets, s + 1);
+            const bool bad = bad_queries<FORM>(start, end, a.tokens);
+            any_bad |= bad;
             long long pages = read_index<FORM>(a.page_offsets, s + 1) - read_index<FORM>(a.page_offsets, s);
             long long last = read_index<FORM>(a.last_page_lengths, s);
-            count = count < 0 ? 0 : count > static_cast<long long>(a.tokens) ? static_cast<long long>(a.tokens) : count;
             pages = pages < 0 ? 0 : pages > static_cast<long long>(a.page_table) ? static_cast<long long>(a.page_table) : pages;
             last = last < 0 ? 0 : last > static_cast<long long>(a.page_size) ? static_cast<long long>(a.page_size) : last;
             const long long keys = pages == 0 ? 0 : (pages - 1) * a.page_size + last;
-            row_count[c] = static_cast<unsigned int>(count) * a.heads;  // (tokens * heads is at most 128 rows a unit of the budget here)
+            row_count[c] = bad ? 0u : static_cast<unsigned int>(end - start) * a.heads;  // (tokens * heads is at most 128 rows a unit of the budget here)
             unit_count[c] = row_count[c] == 0 ? 1u : (row_count[c] + kRows - 1) / kRows;
             tile_count[c] = static_cast<unsigned int>((keys + kKeys - 1) / kKeys);
         }
+    }
+    if (__any(any_bad)) {
+        units = 0;
+        place.share = 0;
+        place.shares = 1;
+        place.share_tiles = 0;
+        place.first_slot = 0;
+        place.unit = workgroup;
+        return find_unit<FORM>(a, workgroup, place.sequence, place.row_tile);
     }
     unsigned int mine_units = 0, mine_longest = 0;
     float mine_tiles = 0.0f;  // (bounds of the search only: a relative error of 2^-24 a term, allowed for below)
@@ -329,15 +339,18 @@ SINGE_DEVICE void latent_tile_rows(const LatentAttentionArgs& a, unsigned char* 
     const unsigned long long rows = static_cast<unsigned long long>(span.queries) * a.heads;  // (none where the span is not valid)
     const unsigned long long first_row = static_cast<unsigned long long>(row_tile) * kRows;
     const unsigned int unit_rows = first_row >= rows ? 0u : rows - first_row < kRows ? static_cast<unsigned int>(rows - first_row) : kRows;
-    if (a.share_budget == 0) place.first_slot = (static_cast<unsigned long long>(span.query_start) * a.heads + first_row) * splits;
-    // A unit that is not shared out is stored as it is.  (Sequences whose offsets make sense never need more slots than
-    // there are; ones that overlap because others run backwards may, and those others report it.)
-    const bool shared = unit_shares > 1, fits = !shared || place.first_slot + static_cast<unsigned long long>(unit_rows) * unit_shares <= a.slots;
+    unsigned long long share_stride = unit_rows;
+    if (a.share_budget == 0) {
+        place.first_slot = static_cast<unsigned long long>(span.query_start) * a.heads + first_row;
+        share_stride = static_cast<unsigned long long>(a.tokens) * a.heads;
+    }
+    const bool shared = unit_shares > 1;  // (a unit that is not is stored as it is)
     if (a.units != nullptr && split == 0 && threadIdx.x == 0 && place.unit < a.unit_slots) {
         LatentUnit unit = {};
-        if (shared && span.valid && fits) {
+        if (shared && span.valid) {
             unit.first_row = static_cast<unsigned long long>(span.query_start) * a.heads + first_row;
             unit.first_slot = place.first_slot;
+            unit.share_stride = share_stride;
             unit.rows = unit_rows;
             unit.shares = unit_shares;
         }
@@ -347,11 +360,11 @@ SINGE_DEVICE void latent_tile_rows(const LatentAttentionArgs& a, unsigned char* 
         if (threadIdx.x == 0) report_index_error(a.status);
         return;
     }
-    if (unit_rows == 0 || !fits) return;
+    if (unit_rows == 0) return;
     // (every wave writes the same words, so that none has to wait for another's)
     if (lane == 0)
         *reinterpret_cast<ulonglong2*>(lds + kSlotAt) =
-            make_ulonglong2(shared ? place.first_slot + static_cast<unsigned long long>(split) * unit_rows : ~0ull, 0);
+            make_ulonglong2(shared ? place.first_slot + static_cast<unsigned long long>(split) * share_stride : ~0ull, 0);
     const unsigned int keys = span.keys;
 
     // Queries are the sequence's last tokens, with the CPU path's saturating position (attention.rs:619-627).
@@ -741,7 +754,7 @@ SINGE_DEVICE void latent_combine_rows(const LatentAttentionArgs& a) {
     if (local >= unit.rows) return;
     const size_t row = static_cast<size_t>(unit.first_row) + local;
     const size_t first_slot = static_cast<size_t>(unit.first_slot) + local;
-    const float mine = lane < splits ? a.partial_lse[first_slot + static_cast<size_t>(lane) * unit.rows] : -INFINITY;
+    const float mine = lane < splits ? a.partial_lse[first_slot + static_cast<size_t>(lane) * unit.share_stride] : -INFINITY;
     float largest = mine;
 #pragma unroll
     for (int step = 32; step >= 1; step >>= 1) largest = fmaxf(largest, __shfl_xor(largest, step, 64));
@@ -752,7 +765,7 @@ SINGE_DEVICE void latent_combine_rows(const LatentAttentionArgs& a) {
     for (int step = 32; step >= 1; step >>= 1) total += __shfl_xor(total, step, 64);
     float acc[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
     const float* part = a.partial_out + first_slot * kLatent + 8u * lane;
-    const size_t share_stride = static_cast<size_t>(unit.rows) * kLatent;
+    const size_t share_stride = static_cast<size_t>(unit.share_stride) * kLatent;
     auto fold = [&](float w, const float4& low, const float4& high) __attribute__((always_inline)) {
         acc[0] = fmaf(w, low.x, acc[0]); acc[1] = fmaf(w, low.y, acc[1]);
         acc[2] = fmaf(w, low.z, acc[2]); acc[3] = fmaf(w, low.w, acc[3]);
@@ -795,11 +808,11 @@ SINGE_DEVICE void latent_tile_body(const LatentAttentionArgs& a, unsigned char* 
         unsigned int* owned = reinterpret_cast<unsigned int*>(lds);
         const unsigned int first = kThreads * (blockIdx.x - a.clear_from), token_bytes = a.heads * a.latent_dim * 2u;
         if (a.wide_index)
-            clear_unowned_tokens<kCsrI64, kThreads>(owned, first, a.query_offsets, a.page_offsets, a.last_page_lengths, a.tokens, a.sequences,
-                                                    a.page_table, a.page_size, a.output, token_bytes, a.lse, a.heads);
+            clear_unowned_tokens<kCsrI64, kThreads, kRows>(owned, first, a.query_offsets, a.page_offsets, a.last_page_lengths, a.tokens, a.sequences,
+                                                           a.page_table, a.page_size, a.heads, a.unit_slots, a.output, token_bytes, a.lse, a.heads, a.status);
         else
-            clear_unowned_tokens<kCsrI32, kThreads>(owned, first, a.query_offsets, a.page_offsets, a.last_page_lengths, a.tokens, a.sequences,
-                                                    a.page_table, a.page_size, a.output, token_bytes, a.lse, a.heads);
+            clear_unowned_tokens<kCsrI32, kThreads, kRows>(owned, first, a.query_offsets, a.page_offsets, a.last_page_lengths, a.tokens, a.sequences,
+                                                           a.page_table, a.page_size, a.heads, a.unit_slots, a.output, token_bytes, a.lse, a.heads, a.status);
         return;
     }
     const bool in_page = a.page_shift >= 5;  // a power of two of at least a tile's 32 keys

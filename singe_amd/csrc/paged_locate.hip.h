@@ -26,34 +26,6 @@ constexpr unsigned int kNoPage = 0xFFFFFFFFu;  // a table entry outside the cach
 // finds its entry by a prefix sum over the sequences' query counts, 64 sequences at a time.  The list is cut into
 // bands of 32 entries; (band, kv head) pairs go round the XCDs, so a band's tiles for one kv head are neighbours on
 // one XCD and walk their keys side by side.
-// Whether a CSR sequence's query offsets make no sense (its own checks report it).  Such a sequence has one entry, and a list
-// that holds one is taken in sequence order whatever the call asked for: the sequences before the first of them follow one
-// another inside [0, tokens] and fit the grid, and it comes next, so the error is reported however many row tiles the
-// sequences after it claim.  (Those may then lie past the grid; a sequence of which any row tile does is not attended.)
-template <int FORM>
-SINGE_DEVICE bool bad_queries(long long start, long long end, unsigned int tokens) {
-    if constexpr (has_lengths(FORM)) return false;
-    return start < 0 || end < start || end > static_cast<long long>(tokens);
-}
-
-// Entries of sequence `s` in the list; `bad` as above.
-template <int FORM, unsigned int ROWS>
-SINGE_DEVICE unsigned int row_tiles_of(const void* query_offsets, const void* query_lengths, unsigned int tokens, unsigned int groups,
-                                       unsigned int s, bool& bad) {
-    long long count;
-    bad = false;
-    if constexpr (has_lengths(FORM)) {
-        count = read_index<FORM>(query_lengths, s);
-        count = count < 0 ? 0 : count > static_cast<long long>(tokens) ? static_cast<long long>(tokens) : count;
-    } else {
-        const long long start = read_index<FORM>(query_offsets, s), end = read_index<FORM>(query_offsets, s + 1);
-        bad = bad_queries<FORM>(start, end, tokens);
-        count = bad ? 0 : end - start;
-    }
-    const unsigned long long tiles = (static_cast<unsigned long long>(count) * groups + ROWS - 1) / ROWS;
-    return tiles == 0 ? 1u : static_cast<unsigned int>(tiles);
-}
-
 // a.longest_first (at most 64 sequences, several row tiles each: chunks of a prefill): the compact list takes the
 // sequences longest first (by pages held, ties by index), so that the workgroups with the most keys to walk start
 // first and the short ones fill the chip's last round.  Lane s learns how many list entries come before sequence s's
@@ -247,7 +219,7 @@ SINGE_DEVICE bool locate(const PagedAttentionArgs& a, unsigned int& unit, unsign
                 const unsigned long long holds = __ballot(entry < through);  // first lane whose range reaches the entry
                 const unsigned int owner = static_cast<unsigned int>(__builtin_ctzll(holds));
                 const unsigned int owner_through = __shfl(through, owner, 64), owner_mine = __shfl(mine, owner, 64);
-                if (!has_lengths(FORM) && owner_through > left) return false;  // (only behind offsets that make no sense)
+                if (!has_lengths(FORM) && owner_through > left) return false;  // (only behind offsets that make no sense: see bad_queries)
                 unit = (first + owner) * a.kv_heads + kv_head;
                 row_tile = static_cast<unsigned int>(entry) - (owner_through - owner_mine);
                 return true;

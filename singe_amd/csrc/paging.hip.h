@@ -104,23 +104,51 @@ SINGE_DEVICE SequenceSpan load_span(unsigned int sequence, const void* query_off
     return span;
 }
 
-// The rows of the `THREADS` tokens from `first` on that no valid sequence owns: zeros and a log-sum-exp of -inf, for callers
-// whose output holds nothing yet.  One workgroup of THREADS; `owned` is THREADS / 32 + 1 words of LDS.  Where a sequence's
-// query offsets make no sense, the others may claim tokens more than once and some of their row tiles may lie outside the
-// grid: then every token is cleared (the status word says so, and what the rows hold besides is not defined).
-template <int FORM, unsigned int THREADS>
+// Whether a CSR sequence's query offsets make no sense (its own checks report it).  Such a sequence has one entry, and a list
+// that holds one is taken in sequence order whatever the call asked for: the sequences before the first of them follow one
+// another inside [0, tokens] and fit the grid, and it comes next, so the error is reported however many row tiles the
+// sequences after it claim.  (Those may then lie past the grid; a sequence of which any row tile does is not attended.)
+template <int FORM>
+SINGE_DEVICE bool bad_queries(long long start, long long end, unsigned int tokens) {
+    if constexpr (has_lengths(FORM)) return false;
+    return start < 0 || end < start || end > static_cast<long long>(tokens);
+}
+
+// Entries of sequence `s` in the list; `bad` as above.
+template <int FORM, unsigned int ROWS>
+SINGE_DEVICE unsigned int row_tiles_of(const void* query_offsets, const void* query_lengths, unsigned int tokens, unsigned int groups,
+                                       unsigned int s, bool& bad) {
+    long long count;
+    bad = false;
+    if constexpr (has_lengths(FORM)) {
+        count = read_index<FORM>(query_lengths, s);
+        count = count < 0 ? 0 : count > static_cast<long long>(tokens) ? static_cast<long long>(tokens) : count;
+    } else {
+        const long long start = read_index<FORM>(query_offsets, s), end = read_index<FORM>(query_offsets, s + 1);
+        bad = bad_queries<FORM>(start, end, tokens);
+        count = bad ? 0 : end - start;
+    }
+    const unsigned long long tiles = (static_cast<unsigned long long>(count) * groups + ROWS - 1) / ROWS;
+    return tiles == 0 ? 1u : static_cast<unsigned int>(tiles);
+}
+
+// The rows of the `THREADS` tokens from `first` on that no attended sequence owns: zeros and a log-sum-exp of -inf, for
+// callers whose output holds nothing yet.  One workgroup of THREADS; `owned` is THREADS / 32 + 1 words of LDS.  No row is
+// written here and by an attention workgroup as well: behind a sequence whose query offsets make no sense others may claim
+// more entries of the list than the grid has (`limit`; ROWS rows of `groups` to a token each), and those are left out here by
+// the rule by which they are not attended.
+template <int FORM, unsigned int THREADS, unsigned int ROWS>
 SINGE_DEVICE void clear_unowned_tokens(unsigned int* owned, unsigned int first, const void* query_offsets, const void* page_offsets,
                                        const void* last_page_lengths, unsigned int tokens, unsigned int sequences, unsigned int page_table,
-                                       unsigned int page_size, void* output, unsigned int token_bytes, float* lse, unsigned int heads) {
+                                       unsigned int page_size, unsigned int groups, unsigned int limit, void* output, unsigned int token_bytes,
+                                       float* lse, unsigned int heads, unsigned int* status) {
     constexpr unsigned int kWords = THREADS / 32u;
     const unsigned int tid = threadIdx.x;
-    if (tid <= kWords) owned[tid] = 0u;
-    __syncthreads();
-    for (unsigned int s = tid; s < sequences; s += THREADS) {
-        const SequenceSpan span = load_span<FORM>(s, query_offsets, page_offsets, last_page_lengths, nullptr, tokens, page_table, page_size);
-        const long long count = read_index<FORM>(query_offsets, s + 1) - span.query_start;
-        if (span.query_start < 0 || count < 0 || span.query_start + count > static_cast<long long>(tokens)) atomicOr(&owned[kWords], 1u);
-        if (!span.valid || span.queries == 0) continue;
+    auto span_of = [&](unsigned int s) __attribute__((always_inline)) {
+        return load_span<FORM>(s, query_offsets, page_offsets, last_page_lengths, nullptr, tokens, page_table, page_size);
+    };
+    auto mark = [&](const SequenceSpan& span) __attribute__((always_inline)) {
+        if (!span.valid || span.queries == 0) return;
         const long long from = span.query_start - static_cast<long long>(first), until = from + span.queries;
         const unsigned int low = from < 0 ? 0u : from > static_cast<long long>(THREADS) ? THREADS : static_cast<unsigned int>(from);
         const unsigned int high = until < 0 ? 0u : until > static_cast<long long>(THREADS) ? THREADS : static_cast<unsigned int>(until);
@@ -128,11 +156,40 @@ SINGE_DEVICE void clear_unowned_tokens(unsigned int* owned, unsigned int first, 
             const unsigned int begin = word * 32u < low ? low - word * 32u : 0u, end = high - word * 32u < 32u ? high - word * 32u : 32u;
             if (begin < end) atomicOr(&owned[word], (end == 32u ? ~0u : (1u << end) - 1u) & ~((1u << begin) - 1u));
         }
+    };
+    if (tid <= kWords) owned[tid] = 0u;
+    __syncthreads();
+    for (unsigned int s = tid; s < sequences; s += THREADS) {
+        const SequenceSpan span = span_of(s);
+        if (bad_queries<FORM>(span.query_start, read_index<FORM>(query_offsets, s + 1), tokens)) atomicOr(&owned[kWords], 1u);
+        mark(span);
     }
     __syncthreads();
-    const bool everything = owned[kWords] != 0u;
+    if (owned[kWords] != 0u) {
+        if (tid == 0) report_index_error(status);
+        if (tid < kWords) owned[tid] = 0u;
+        __syncthreads();
+        if (tid < 64u) {
+            unsigned int left = limit;
+            for (unsigned int chunk = 0; chunk < sequences; chunk += 64u) {
+                const unsigned int s = chunk + tid;
+                bool bad;
+                unsigned int through = s < sequences ? row_tiles_of<FORM, ROWS>(query_offsets, nullptr, tokens, groups, s, bad) : 0u;
+#pragma unroll
+                for (int step = 1; step < 64; step <<= 1) {
+                    const unsigned int below = __shfl_up(through, step, 64);
+                    if (tid >= static_cast<unsigned int>(step)) through += below;
+                }
+                if (s < sequences && through <= left) mark(span_of(s));
+                const unsigned int total = __shfl(through, 63, 64);
+                if (total > left) break;
+                left -= total;
+            }
+        }
+        __syncthreads();
+    }
     for (unsigned int word = 0; word < kWords; ++word) {
-        for (unsigned int left = everything ? ~0u : ~owned[word]; left != 0u; left &= left - 1u) {
+        for (unsigned int left = ~owned[word]; left != 0u; left &= left - 1u) {
             const unsigned int token = first + word * 32u + static_cast<unsigned int>(__builtin_ctz(left));
             if (token >= tokens) return;
             unsigned char* row = static_cast<unsigned char*>(output) + static_cast<size_t>(token) * token_bytes;

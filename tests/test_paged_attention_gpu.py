@@ -521,24 +521,54 @@ def poison(*shapes):
     del blocks
 
 
-def run_backwards(heads, kv_heads, tokens, offsets, page_counts, rows_per_wave=0):
-    """The outputs, the status word and what the call needs again, for sequences whose query offsets need not make sense."""
+def run_with_faults(heads, kv_heads, tokens, offsets, page_offsets, last, rows_per_wave=0, splits=0, index_dtype=torch.int32):
+    """The outputs over poisoned memory, the status word and the operands, for sequences whose paging need not make sense."""
     page_size, cache_pages = 16, 50
     gen = torch.Generator(device="cuda")
     gen.manual_seed(tokens + len(offsets))
     rand = lambda *shape: torch.randn(shape, generator=gen, device="cuda").to(torch.bfloat16)
-    index = lambda values: torch.tensor([int(v) for v in values], dtype=torch.int32, device="cuda")
-    ends = np.concatenate([[0], np.cumsum(page_counts)])
-    paging = neural.Paging(index(offsets), index(ends), index(np.arange(ends[-1]) % cache_pages), index([page_size] * len(page_counts)))
+    index = lambda values: torch.tensor([int(v) for v in values], dtype=index_dtype, device="cuda")
     q, kc, vc = rand(tokens, heads, 128), rand(cache_pages, page_size, kv_heads, 128), rand(cache_pages, page_size, kv_heads, 128)
+    pages = [(7 * i + 3) % cache_pages for i in range(max(page_offsets))]
     status = torch.zeros(1, dtype=torch.int32, device="cuda")
     _native.lib().singe_hip_set_paged_attention_rows_per_wave(rows_per_wave)
+    _native.lib().singe_hip_set_paged_attention_splits(splits)
     try:
         poison(((tokens, heads, 128), torch.bfloat16), ((tokens, heads), torch.float32))
-        out, lse = neural.paged_attention(q, kc, vc, paging, neural.AttentionOptions(causal=True), status=status, check=False)
+        out, lse = neural.paged_attention(q, kc, vc, neural.Paging(index(offsets), index(page_offsets), index(pages), index(last)),
+                                          neural.AttentionOptions(causal=True), status=status, check=False)
     finally:
         _native.lib().singe_hip_set_paged_attention_rows_per_wave(0)
-    return out, lse, int(status.item()), (q, kc, vc, paging)
+        _native.lib().singe_hip_set_paged_attention_splits(0)
+
+    def alone(s):
+        mine = pages[page_offsets[s]:page_offsets[s + 1]]
+        return neural.paged_attention(q[offsets[s]:offsets[s + 1]].contiguous(), kc, vc,
+                                      neural.Paging(index([0, offsets[s + 1] - offsets[s]]), index([0, len(mine)]), index(mine), index([last[s]])),
+                                      neural.AttentionOptions(causal=True))
+
+    return out, lse, int(status.item()), alone
+
+
+def check_rows_are_whole(tokens, offsets, valid, out, lse, alone, attended):
+    """Every row is that of a valid sequence that has its token, or zeros with a log-sum-exp of -inf: the latter where there is
+    no such sequence, the former where `attended` says that its sequence is attended.  Tokens that two sequences claim have rows
+    of either, head by head and share by share."""
+    zero = ~out.any(dim=-1).any(dim=-1) & torch.isneginf(lse).all(dim=-1)
+    right, claims, needed = zero.clone(), torch.zeros_like(zero, dtype=torch.int32), torch.zeros_like(zero)
+    for s in np.flatnonzero(valid):
+        rows = slice(offsets[s], offsets[s + 1])
+        if offsets[s] == offsets[s + 1]:
+            continue
+        want, want_lse = alone(s)
+        right[rows] |= ((out[rows].float() - want.float()).abs().amax(dim=(1, 2)) <= MAX_ABS) & ((lse[rows] - want_lse).abs().amax(dim=1) <= LSE_ABS)
+        claims[rows] += 1
+        needed[rows] |= bool(attended[s])
+    assert torch.isfinite(out.float()).all() and not torch.isnan(lse).any()
+    right |= claims > 1
+    assert right.all(), torch.nonzero(~right).flatten().tolist()[:8]
+    assert zero[claims == 0].all()
+    assert not zero[needed].any()
 
 
 # Sequences that claim the same tokens over and over, between them ones that run backwards: more row tiles than the grid holds in
@@ -555,7 +585,49 @@ BACKWARDS = {
 @pytest.mark.parametrize("rows_per_wave", [32, 64])
 @pytest.mark.parametrize("case", BACKWARDS)
 def test_offsets_that_make_no_sense_are_reported_however_many_row_tiles_are_claimed(case, rows_per_wave):
-    assert run_backwards(*BACKWARDS[case], rows_per_wave=rows_per_wave)[2] == neural.STATUS_INDEX_OUT_OF_BOUNDS
+    heads, kv_heads, tokens, offsets, page_counts = BACKWARDS[case]
+    ends = np.concatenate([[0], np.cumsum(page_counts)]).tolist()
+    out, lse, status, alone = run_with_faults(heads, kv_heads, tokens, offsets, ends, [16] * len(page_counts), rows_per_wave)
+    assert status == neural.STATUS_INDEX_OUT_OF_BOUNDS
+    valid = [0 <= start <= end <= tokens for start, end in zip(offsets, offsets[1:])]
+    first_bad = valid.index(False)
+    check_rows_are_whole(tokens, offsets, valid, out, lse, alone, [s < first_bad for s in range(len(valid))])
+
+
+# (query tokens, pages held) of the sequences, the rows a wave, the key shares; tokens before the first and after the last one
+ROUTES = {
+    "row tiles, longest first": ([(200, 30), (330, 50), (150, 12), (200, 40), (64, 20)], 32, 1),
+    "row tiles and decoding sequences in turns": ([(1, 40 + s) for s in range(12)] + [(200, 60)] + [(1, 70), (2, 50)], 32, 1),
+    "row tiles in order": ([(1, 3), (2, 5), (90, 9), (1, 6), (40, 4)], 32, 1),
+    "one row tile a sequence": ([(1, 3), (2, 5), (9, 9), (1, 6), (4, 4)], 32, 1),
+    "shares": ([(1, 40), (60, 45), (30, 50), (1, 60), (40, 44)], 32, 3),
+    "two tiles a wave": ([(200, 30), (330, 50), (150, 12), (200, 40), (64, 20)], 64, 1),
+    "decode": ([(1, 5 + s % 7) for s in range(40)] + [(0, 2)] * 20, 0, 0),
+    "decode over many keys": ([(1, 1500), (1, 1400), (1, 1600), (1, 1500), (1, 900)] + [(0, 1)] * 20, 0, 0),
+}
+
+
+@pytest.mark.parametrize("index_dtype", [torch.int32, torch.int64])
+@pytest.mark.parametrize("fault", ["query offsets", "page offsets", "last page length"])
+@pytest.mark.parametrize("route", ROUTES)
+def test_a_sequence_that_is_refused_leaves_the_others_whole_and_its_own_rows_zero(route, fault, index_dtype):
+    sequences, rows_per_wave, splits = ROUTES[route]
+    offsets = (5 + np.concatenate([[0], np.cumsum([queries for queries, _ in sequences])])).tolist()
+    page_offsets = np.concatenate([[0], np.cumsum([pages for _, pages in sequences])]).tolist()
+    last = [9] * len(sequences)
+    tokens, bad = offsets[-1] + (9 if splits != 0 or rows_per_wave != 0 else 0), 2
+    if fault == "query offsets":
+        offsets[bad + 1] = offsets[bad] - 1
+    elif fault == "page offsets":
+        page_offsets[bad + 1] = page_offsets[bad] - 1
+    else:
+        last[bad] = 17
+    out, lse, status, alone = run_with_faults(8, 2, tokens, offsets, page_offsets, last, rows_per_wave, 0 if splits == 1 else splits, index_dtype)
+    assert status == neural.STATUS_INDEX_OUT_OF_BOUNDS
+    valid = [s != bad for s in range(len(sequences))]
+    # (the decode kernels look a token's sequence up by bisection, which offsets that run backwards lead astray)
+    attended = [s < bad or fault != "query offsets" or not route.startswith("decode") for s in range(len(sequences))]
+    check_rows_are_whole(tokens, offsets, valid, out, lse, alone, attended)
 
 
 @pytest.mark.parametrize("index_dtype", [torch.int32, torch.int64])

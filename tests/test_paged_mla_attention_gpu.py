@@ -491,3 +491,53 @@ def test_tokens_no_sequence_owns_are_zero_with_a_log_sum_exp_of_minus_infinity(k
     mine[5:40] = True
     assert not out[~mine].any() and torch.isneginf(lse[~mine]).all()
     assert torch.isfinite(out[mine].float()).all() and torch.isfinite(lse[mine]).all()
+
+
+@pytest.mark.parametrize("index_dtype", [torch.int32, torch.int64])
+@pytest.mark.parametrize("fault", ["query offsets", "claimed over and over", "page offsets", "last page length"])
+@pytest.mark.parametrize("splits", [0, 1, 3])
+def test_a_sequence_that_is_refused_leaves_the_others_whole_and_its_own_rows_zero(splits, fault, index_dtype):
+    from singe_amd import _native
+    heads, page_size, tokens, cache_pages = 32, 64, 60, 40
+    offsets, page_offsets, last, bad = [4, 14, 18, 30, 31, 52], [0, 30, 62, 90, 130, 165], [33] * 5, 2
+    if fault == "query offsets":
+        offsets[bad + 1] = offsets[bad] - 1
+    elif fault == "claimed over and over":
+        offsets, page_offsets, last, bad = [0, 60, 0, 60, 0, 60, 0, 60], [0, 30, 31, 62, 63, 100, 101, 140], [33] * 7, 1
+    elif fault == "page offsets":
+        page_offsets[bad + 1] = page_offsets[bad] - 1
+    else:
+        last[bad] = 65
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(9)
+    rand = lambda *shape: torch.randn(shape, generator=gen, device="cuda").to(torch.bfloat16)
+    index = lambda entries: torch.tensor(entries, dtype=index_dtype, device="cuda")
+    q, positions, cache, position_cache = rand(tokens, heads, 512), rand(tokens, heads, 64), rand(cache_pages, page_size, 512), rand(cache_pages, page_size, 64)
+    pages = [(7 * i + 3) % cache_pages for i in range(max(page_offsets))]
+    status = torch.zeros(1, dtype=torch.int32, device="cuda")
+    _native.lib().singe_hip_set_paged_mla_attention_splits(splits)
+    try:
+        blocks = [torch.full((tokens, heads, 512), float("nan"), device="cuda", dtype=torch.bfloat16), torch.full((tokens, heads), float("nan"), device="cuda")]
+        torch.cuda.synchronize()
+        del blocks  # (what an output that nothing wrote would hold)
+        out, lse = neural.paged_mla_attention(q, positions, cache, position_cache, neural.Paging(index(offsets), index(page_offsets), index(pages), index(last)),
+                                              neural.AttentionOptions(causal=True), status=status, check=False)
+    finally:
+        _native.lib().singe_hip_set_paged_mla_attention_splits(0)
+    assert int(status.item()) == neural.STATUS_INDEX_OUT_OF_BOUNDS
+    zero = ~out.any(dim=-1).any(dim=-1) & torch.isneginf(lse).all(dim=-1)
+    right, claims, needed = zero.clone(), torch.zeros_like(zero, dtype=torch.int32), torch.zeros_like(zero)
+    for s in range(len(last)):
+        if s == bad or offsets[s + 1] < offsets[s]:
+            continue
+        mine, rows = pages[page_offsets[s]:page_offsets[s + 1]], slice(offsets[s], offsets[s + 1])
+        want, want_lse = neural.paged_mla_attention(q[rows].contiguous(), positions[rows].contiguous(), cache, position_cache,
+                                                    neural.Paging(index([0, offsets[s + 1] - offsets[s]]), index([0, len(mine)]), index(mine), index([last[s]])),
+                                                    neural.AttentionOptions(causal=True))
+        right[rows] |= ((out[rows].float() - want.float()).abs().amax(dim=(1, 2)) <= 2e-2) & ((lse[rows] - want_lse).abs().amax(dim=1) <= 5e-3)
+        claims[rows] += 1
+        needed[rows] |= s < bad or fault != "claimed over and over"
+    assert torch.isfinite(out.float()).all() and not torch.isnan(lse).any()
+    right |= claims > 1  # (rows of either sequence, share by share)
+    assert right.all(), torch.nonzero(~right).flatten().tolist()[:8]
+    assert zero[claims == 0].all() and not zero[needed].any()
