@@ -161,10 +161,16 @@ size_t hand_over(const std::string& key, char* buffer, size_t capacity) {
 
 namespace singe_hip {
 
-uint32_t attention_key_splits(uint64_t workgroups, uint64_t keys) {
+static uint64_t split_below() {
     const SingeHipThreadOptions& own = thread_options();
     const uint64_t installed = g_split_below_plus_one.load(std::memory_order_relaxed);
-    const uint64_t below = own.has_split_below_blocks ? own.split_below_blocks : installed == 0 ? default_split_below() : installed - 1;
+    return own.has_split_below_blocks ? own.split_below_blocks : installed == 0 ? default_split_below() : installed - 1;
+}
+
+bool split_below_is_default() { return split_below() == default_split_below(); }
+
+uint32_t attention_key_splits(uint64_t workgroups, uint64_t keys) {
+    const uint64_t below = split_below();
     if (below == 0 || workgroups == 0 || workgroups >= below || keys <= kShareTiles * kKeyTile) return 1;
     uint64_t wanted = (2 * below + workgroups - 1) / workgroups;
     const uint64_t chunks = (keys + kShareTiles * kKeyTile - 1) / (kShareTiles * kKeyTile);

@@ -95,6 +95,8 @@ size_t paged_decode_workspace_bytes(const SingePagedKvDecodeAttentionConfig& con
 // attention_parameters.cpp: the shares a launch of `workgroups` workgroups over at most `keys` keys splits its keys
 // into under the installed AttentionParameters (1 = no split).
 uint32_t attention_key_splits(uint64_t workgroups, uint64_t keys);
+// Whether this thread's calls follow the default split_below_blocks: nobody has asked for another number of shares.
+bool split_below_is_default();
 
 // general_attention.cpp: the one-wave-per-row kernels behind entry points of other files, for head dimensions the
 // matrix-core kernels are not built for.  Block-table prefill (query_lengths given) or decode (query_lengths null).

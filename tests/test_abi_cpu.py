@@ -177,6 +177,26 @@ def test_paged_attention_scratch_query_needs_no_device():
     assert lib.singe_hip_paged_attention_scratch_bytes(None) == 0
 
 
+@pytest.mark.parametrize("heads,kv_heads,dim,sequences,chunk,decoding,keys,shares", [
+    (16, 2, 128, 1, 64, 0, 16384, 16), (16, 2, 128, 1, 128, 0, 16384, 8), (16, 2, 128, 1, 256, 0, 16384, 4), (16, 2, 128, 4, 256, 0, 16384, 2),
+    (64, 8, 128, 1, 64, 0, 16384, 16), (64, 8, 128, 1, 256, 0, 16384, 4), (32, 8, 128, 1, 128, 0, 16384, 16), (28, 4, 128, 1, 64, 0, 16384, 16), (28, 4, 128, 1, 256, 0, 16384, 4), (28, 4, 128, 2, 256, 0, 16384, 2),
+    (28, 4, 128, 4, 256, 0, 16384, 2), (64, 8, 128, 1, 64, 0, 1024, 2),           # (two shares of eight key tiles are all there is)
+    (16, 2, 128, 1, 1024, 20, 2112, 2), (16, 2, 128, 1, 64, 62, 2112, 4), (64, 8, 128, 1, 256, 32, 2112, 2)])
+def test_key_shares_of_chunks_fill_the_chip_and_no_more(heads, kv_heads, dim, sequences, chunk, decoding, keys, shares):
+    lib, both, tokens = _native.lib(), sequences + decoding, sequences * chunk + decoding
+    problem = _native.PagedAttentionProblemC(tokens, heads, kv_heads, dim, 16, both, 100000, both * keys // 16, 0, 1, 0, 0, 0, 0.0, 0.0, 0)
+    row = tokens * heads * (dim + 1) * 4
+    assert lib.singe_hip_paged_attention_scratch_bytes(ctypes.byref(problem)) == shares * row
+    own = _native.ThreadOptionsC(-1, 0, 0, 0, True, 1024)  # a caller's own number of workgroups is taken at its word
+    lib.singe_hip_set_thread_options(ctypes.byref(own))
+    try:
+        tiles = kv_heads * (heads // kv_heads * tokens // 128 + both)
+        wanted = min(-(-2 * 1024 // tiles), -(-keys // 512), 64)
+        assert lib.singe_hip_paged_attention_scratch_bytes(ctypes.byref(problem)) == (wanted * row if wanted > 1 else 0)
+    finally:
+        lib.singe_hip_set_thread_options(None)
+
+
 def test_paged_mla_attention_validation():
     lib = _native.lib()
     fake = 0x1000
