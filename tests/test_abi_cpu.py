@@ -539,6 +539,20 @@ def test_paged_attention_row_tiles_by_the_keys_a_sequence_has(chunks, chunk, dec
     assert _native.lib().singe_hip_paged_attention_rows_per_wave(ctypes.byref(problem)) == rows
 
 
+@pytest.mark.parametrize("heads,kv_heads,head_dim,chunks,chunk,decoding,rows", [
+    (64, 8, 96, 2, 512, 40, 32),      # past 9/16 of a whole 256-row tile a sequence, where the 128-row kernel has a loop for few rows
+    (64, 8, 80, 2, 512, 40, 64),      # ... and where it has none
+    (64, 8, 112, 2, 512, 40, 64),
+    (68, 4, 128, 2, 512, 100, 64),    # ... or the rows of a token are more than the loop takes
+    (64, 4, 128, 2, 512, 100, 32),
+    (64, 8, 80, 2, 512, 62, 32),
+])
+def test_paged_attention_row_tiles_by_the_loop_for_few_rows(heads, kv_heads, head_dim, chunks, chunk, decoding, rows):
+    tokens, sequences = chunks * chunk + decoding, chunks + decoding
+    problem = _native.PagedAttentionProblemC(tokens, heads, kv_heads, head_dim, 16, sequences, 20000, 132 * sequences, 0, 1, 0, 0, 0, 0.0, 0.0, 0)
+    assert _native.lib().singe_hip_paged_attention_rows_per_wave(ctypes.byref(problem)) == rows
+
+
 @pytest.mark.parametrize("batch,heads,head_dim,query_len,key_len,causal,rows", [
     (4, 32, 128, 4096, 4096, 1, 64),    # whole rounds of long rows
     (4, 32, 128, 1024, 1024, 1, 32),    # short causal rows
