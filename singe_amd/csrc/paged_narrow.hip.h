@@ -130,7 +130,6 @@ SINGE_DEVICE void narrow_rows(const PagedAttentionArgs& a, unsigned char* lds, c
     // A slot is filled by four instructions, four rows each: lane l of instruction i brings what belongs at chunk place
     // l % 16 of row 4 i + l / 16 (K keeps chunk c of a row at c ^ row, V at c ^ 4 (row & 3)).
     const unsigned int load_row = lane >> 4, place = lane & 15u;
-    const size_t page_bytes = static_cast<size_t>(a.page_size) * a.kv_heads * kGlobalRowBytes;
     const unsigned int head_bytes = kv_head * kGlobalRowBytes, slot_bytes = a.kv_heads * kGlobalRowBytes;
     unsigned int key_chunk_of[4], value_chunk_of[4], key_offset[4], value_offset[4];  // of instruction i: the lane's chunk, and its place behind the group's first row
 #pragma unroll
@@ -162,8 +161,8 @@ SINGE_DEVICE void narrow_rows(const PagedAttentionArgs& a, unsigned char* lds, c
     auto bring = [&](auto is_value, unsigned int t, unsigned int page, unsigned int slot) __attribute__((always_inline)) {
         constexpr bool kValue = decltype(is_value)::value;
         const unsigned int key0 = key_of(t);
-        const unsigned char* base = reinterpret_cast<const unsigned char*>(kValue ? a.value_cache : a.key_cache) + page * page_bytes +
-                                    ((key0 & (a.page_size - 1u)) * slot_bytes + head_bytes);
+        const unsigned char* base = reinterpret_cast<const unsigned char*>(kValue ? a.value_cache : a.key_cache) +
+                                    (static_cast<size_t>(page) * a.page_size + (key0 & (a.page_size - 1u))) * slot_bytes + head_bytes;
         const unsigned int dest = lds_start + slot * kNarrowSlotBytes;
         if (key0 + kNarrowKeys <= keys) {
             narrow_load(base, kValue ? value_offset : key_offset, kValue ? value_chunk_of : key_chunk_of, dest);

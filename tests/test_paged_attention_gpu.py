@@ -466,6 +466,29 @@ def test_pages_beyond_two_and_four_gib_of_a_cache_read_the_same_as_the_first_pag
     assert far.float().abs().max().item() > 0.1
 
 
+@pytest.mark.parametrize("page_size,near_page", [(1 << 20, 512), ((1 << 20) + 3, 515)])
+@pytest.mark.parametrize("queries", [2, 40])
+def test_places_beyond_four_gib_of_one_page_read_the_same_as_near_its_start(queries, page_size, near_page):
+    # One page of 5.4 GB (20 kv heads x 128: 5 KiB a key): its last keys, all that the window leaves, lie past byte 2^32 of it.
+    # The same keys at the end of a small page must give the same bits.
+    heads, kv_heads, window = 40, 20, 200
+    keys, skipped = page_size - 5, page_size - near_page
+    assert skipped % 64 == 0
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(queries)
+    rand = lambda *shape: torch.randn(shape, generator=gen, device="cuda").to(torch.bfloat16)
+    q, small_k, small_v = rand(queries, heads, 128), rand(1, near_page, kv_heads, 128), rand(1, near_page, kv_heads, 128)
+    big_k, big_v = (torch.zeros((1, page_size, kv_heads, 128), device="cuda", dtype=torch.bfloat16) for _ in range(2))
+    big_k[:, skipped:], big_v[:, skipped:] = small_k, small_v
+    index = lambda *values: torch.tensor(values, dtype=torch.int32, device="cuda")
+    options = neural.AttentionOptions(causal=True, window=window)
+    far, far_lse = neural.paged_attention(q, big_k, big_v, neural.Paging(index(0, queries), index(0, 1), index(0), index(keys)), options)
+    near, near_lse = neural.paged_attention(q, small_k, small_v, neural.Paging(index(0, queries), index(0, 1), index(0), index(keys - skipped)), options)
+    torch.cuda.synchronize()
+    assert torch.equal(far, near) and torch.equal(far_lse, near_lse)
+    assert far.float().abs().max().item() > 0.1
+
+
 NARROW = [(1, 1), (2, 15), (1, 16), (2, 17), (1, 63), (2, 64), (1, 65), (2, 0), (0, 40), (2, 1), (1, 129), (2, 1000)]
 
 
