@@ -76,8 +76,6 @@ int32_t paged_mla_attention(void* stream, const void* latent_queries, const void
                             size_t scratch_bytes, const SingePagedMlaAttentionProblem* problem, bool every_row = false) {
     if (problem == nullptr) return fail(SINGE_HIP_NULL_POINTER, "problem");
     const SingePagedMlaAttentionProblem& p = *problem;
-    if (every_row && (!on_matrix_cores(p) || p.sequences <= 0))
-        return fail(SINGE_HIP_UNSUPPORTED_WIDTH, "paged_mla_attention_every_row", static_cast<uint64_t>(p.latent_dim));
     // paged_mla_attention_problem: a page holds at least one key and the latent width is positive; the
     // positional width may be zero.
     if (p.tokens < 0 || p.heads < 0 || p.latent_dim <= 0 || p.position_dim < 0 || p.page_size <= 0 || p.sequences < 0 ||
@@ -93,6 +91,8 @@ int32_t paged_mla_attention(void* stream, const void* latent_queries, const void
         if (!fits_i32(static_cast<uint64_t>(extent))) return fail(SINGE_HIP_LENGTH_EXCEEDS_I32, "problem");
     if (p.latent_dim > 512) return fail(SINGE_HIP_UNSUPPORTED_WIDTH, "paged_mla_attention", static_cast<uint64_t>(p.latent_dim));
     if (p.position_dim > 128) return fail(SINGE_HIP_UNSUPPORTED_WIDTH, "paged_mla_attention", static_cast<uint64_t>(p.position_dim));
+    if (every_row && (!on_matrix_cores(p) || p.sequences <= 0))
+        return fail(SINGE_HIP_UNSUPPORTED_WIDTH, "paged_mla_attention_every_row", static_cast<uint64_t>(p.latent_dim));
     if (p.tokens == 0 || p.heads == 0 || p.sequences == 0) return 0;  // nothing to attend
     const void* pointers[] = {latent_queries, latent_cache, query_offsets, page_offsets, last_page_lengths, output};
     const char* names[] = {"latent_queries", "latent_cache", "query_offsets", "page_offsets", "last_page_lengths", "output"};

@@ -578,3 +578,22 @@ def test_dense_prefill_rows_per_wave(batch, heads, head_dim, query_len, key_len,
     # (without a device the library counts on 256 compute units)
     config = A.FmhaPrefillConfig.contiguous(batch, query_len, key_len, heads, heads, head_dim, 0.125, bool(causal))
     assert _native.lib().singe_hip_dense_prefill_rows_per_wave(ctypes.byref(config._c())) == rows
+
+
+@pytest.mark.parametrize("fields,status", [
+    (dict(head_dim=0), 9),         # a problem that makes no sense is refused as the other entry points refuse it
+    (dict(page_size=0), 9),
+    (dict(head_dim=24), 5),        # one that does, at a width without a matrix-core build
+    (dict(sequences=0), 5),
+    (dict(tokens=0), 0),
+])
+def test_every_row_refuses_what_makes_no_sense_before_what_it_has_no_build_for(fields, status):
+    lib = _native.lib()
+    known = dict(tokens=4, heads=8, kv_heads=2, head_dim=64, page_size=16, sequences=2, cache_pages=4, page_table=4, index_type=0, causal=1,
+                 has_scale=0, has_window=0, has_softcap=0, scale=0.0, softcap=0.0, window=0)
+    problem = _native.PagedAttentionProblemC(*{**known, **fields}.values())
+    assert lib.singe_hip_paged_attention_every_row(1, None, *[0x1000] * 10, None, 0, ctypes.byref(problem)) == status
+    if status != 5 or "sequences" in fields:
+        latent = _native.PagedMlaAttentionProblemC(fields.get("tokens", 4), 8, fields.get("head_dim", 512), 64, fields.get("page_size", 16),
+                                                   fields.get("sequences", 2), 4, 4, 1, 0, 1, 0, 0.0)
+        assert lib.singe_hip_paged_mla_attention_every_row(None, *[0x1000] * 11, None, 0, ctypes.byref(latent)) == status
