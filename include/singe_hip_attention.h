@@ -698,8 +698,8 @@ SINGE_HIP_API int32_t singe_hip_scaled_dot_product_attention(
  * (batch, head) and cannot fill the chip; given scratch, bf16 / f16 calls at a head_dim that is a multiple of 16 up to
  * 128 share the keys of a
  * query tile out over several workgroups, each leaving a normalised f32 partial and its base-two log-sum-exp, and a
- * second kernel merges them (sinks join the first share).  ..._scratch_bytes says how much the problem wants (0: it
- * would not split, by SingeAttentionParameters.split_below_blocks and the key count); with a null or smaller buffer,
+ * second kernel merges them (sinks join the first share).  ..._scratch_bytes says how much the problem wants at most, with
+ * a mask or without (0: it would not split, by SingeAttentionParameters.split_below_blocks and the key count); with a null or smaller buffer,
  * and for every other type and width, the call is singe_hip_scaled_dot_product_attention.  The scratch holds nothing
  * between calls; calls that share it must not overlap. */
 SINGE_HIP_API size_t singe_hip_scaled_dot_product_attention_scratch_bytes(const SingeAttentionProblem* problem);

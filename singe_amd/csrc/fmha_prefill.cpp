@@ -335,14 +335,15 @@ int32_t prefill(void* stream, uint16_t* out, size_t out_len, float* lse, size_t 
     if (splits > 1 && static_cast<uint64_t>(c.batch) * c.heads * c.query_len > 0xffffffffull) splits = 1;
     if (splits > 1 && (options.scratch_bytes < dense_prefill_scratch_bytes(c, splits) || groups * splits > 0x7fffffffull)) splits = 1;
     // Two sets of waves to a tile instead, each on one half of its keys, where a tile a compute unit is all there is and its
-    // keys are worth it (and, up to half as many tiles, no more shares could be lent for).  One set / two, us, f16 and bf16 alike:
+    // keys are worth it (and, up to half as many tiles, no more shares could be lent for; a caller's own split_below_blocks
+    // that asks for shares gets them).  One set / two, us, f16 and bf16 alike:
     //   head_dim 128, causal  32 heads x 300 (96 tiles) 11.6 / 12.1   x 512 (128) 16.6 / 16.0   x 773 (224) 22.5 / 20.4   x 1024 (256) 27.9 / 24.3
     //                         x 1500 (384) 44.9 / 45.4                16 x 2048 (256) 46.7 / 36.9 (two shares 42)         8 x 4096 (256) 85.5 / 63.8
     //   head_dim 128, full    32 x 1024 (256) 29.1 / 26.1             32 x 1500 (384) 49.9 / 59.8  8 x 4096 (256) 89.3 / 76.4
     //   head_dim 64           causal 32 x 1024 (256) 19.8 / 16.6, 8 x 4096 (256) 60.6 / 43.4; full 64 x 512 (256) 12.9 / 11.6, 8 x 4096 63.1 / 47.8
     const uint64_t query_tiles = static_cast<uint64_t>(c.batch) * c.heads * args.query_tiles, seen = c.causal && c.query_len < c.key_len ? c.query_len : c.key_len;
     const bool halves = !with_options && args.packed_heads == 0 && args.single_tiles != 0 && query_tiles <= compute_units() && seen >= 512 &&
-                        (splits == 1 || 2 * query_tiles > compute_units());
+                        (splits == 1 || (2 * query_tiles > compute_units() && split_below_is_default()));
     if (halves) splits = 1;
     args.splits = splits;
     if (splits > 1) {
@@ -405,6 +406,9 @@ bool dense_prefill_packs_heads(const SingeFmhaPrefillConfig& c) {
 // tile a head (a decode step); none where there are more tiles than compute units; in between two, if the rows see so many
 // keys that a workgroup's walk over them outweighs the merge: 1536 under the causal mask, whose last tile alone walks them
 // all, 4096 without it.  (In between, one share took up to 1.3 times as long as pairs with their shares: 1 x 8 x 2500.)
+// (Those two are for calls with a mask, a window or a cap: the others walk a tile's keys from two places at once instead, on
+// two sets of waves, see `halves`, and leave the scratch alone.  The scratch is sized for both: a mask is the launch's, not the
+// problem's.)
 // Pairs, with the shares they were cut into before single tiles, against single tiles with 1 / 2 / 4 shares, us:
 //   head_dim 128, causal    1 x 8 x 2500 (160 tiles)   46  54 / 42 / 35     1 x 16 x 2000 (256)  49  45 / 42 / 45
 //                           1 x 20 x 1024 (160)        36  26 / 29 / 33     1 x 20 x 1536 (240)  46  38 / 36 / 44

@@ -181,3 +181,27 @@ def test_grouped_heads_of_a_decode_shaped_dense_call_share_a_tile(heads, kv_head
                                                                        softcap=20.0, threads=8), dtype)
         close(host(padded), oracle.scaled_dot_product_attention_f32(host(q), host(k), host(v), key_lengths=[key_len, 700], window=900,
                                                                     threads=8), dtype)
+
+
+@pytest.mark.parametrize("heads, length", [(8, 2500), (16, 2048)])
+def test_a_callers_own_split_below_blocks_gets_its_shares_where_the_default_takes_two_sets_of_waves(heads, length):
+    """More query tiles than half the compute units and no more than there are: by default one launch that leaves the
+    scratch alone, under a caller's own threshold the shares that it asks for."""
+    units = torch.cuda.get_device_properties(0).multi_processor_count
+    q, k, v = tensors((1, heads, length, 128), (1, heads, length, 128), (1, heads, length, 128), torch.bfloat16, length)
+    want = oracle.scaled_dot_product_attention_f32(host(q), host(k), host(v), causal=True, threads=8)
+    problem = _native.AttentionProblemC(1, heads, heads, length, length, 128, 128, (ctypes.c_int64 * 4)(0, 0, 0, 0), neural._DATA_TYPES[q.dtype],
+                                        1, 0, 0, 0, 0.0, 0.0, 0)
+    for below, shares in ((None, 0), (4 * units, 2)):
+        neural.set_attention_parameters(None if below is None else neural.AttentionParameters(split_below_blocks=below))
+        try:
+            need = int(_native.lib().singe_hip_scaled_dot_product_attention_scratch_bytes(ctypes.byref(problem)))
+            scratch, out = torch.full((need,), 0x5A, dtype=torch.uint8, device="cuda"), torch.empty_like(q)
+            _native.check(_native.lib().singe_hip_scaled_dot_product_attention_scratch(
+                int(torch.cuda.current_stream().cuda_stream), q.data_ptr(), k.data_ptr(), v.data_ptr(), None, None, None, out.data_ptr(),
+                scratch.data_ptr(), need, ctypes.byref(problem)), "attention")
+        finally:
+            neural.set_attention_parameters(None)
+        close(host(out), want, torch.bfloat16)
+        written = need // 4 - int((scratch.view(torch.int32) == 0x5A5A5A5A).sum().item())
+        assert written >= shares * heads * length * 128 if shares else written == 0
