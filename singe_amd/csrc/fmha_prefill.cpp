@@ -366,15 +366,24 @@ int32_t prefill(void* stream, uint16_t* out, size_t out_len, float* lse, size_t 
         return launch(pair, static_cast<unsigned>(pair_groups), 1, 1, 256, stream, args);
     }
     // Under a causal window grouped heads share tiles: 128 rows are then 128 / group queries, whose windows overlap almost
-    // whole, and a tile walks window + 128 / group keys instead of window + 128.  64 / 8 heads x 64, 1 x 8192, window
-    // 128: 75 -> 64 us (61 since the queries' loads are waited for with the tiles'); 64 / 8 x 128, 2 x 1122, window 142: 59 -> 41; 16 / 2 x 128, 2 x 5943, window 1310: 177 -> 143.
+    // whole, and a tile walks window + 128 / group keys instead of window + 128.  Not two heads under a window of three
+    // quarters of the rows and more, where that saves next to nothing and a workgroup gives up the pair of a long and a short
+    // tile.  Each head's own tiles / shared ones, us:
+    //   64 / 8 heads x 64    1 x 8192, window 128   69 / 57    512  117 / 100   2048  319 / 282   4096  537 / 463   8191  623 / 608
+    //   64 / 8 x 128         1 x 2048, window 128   39 / 32    512   57 / 50    1024   78 / 71    1536   79 / 77    2047   80 / 78
+    //   32 / 8 x 128         8 x 4096, window 128  266 / 236   512  423 / 388   2048  928 / 865   3072 1061 / 1037  4095 1094 / 1094
+    //   12 / 4 x 96          4 x 2048, window 128   29 / 25    512   40 / 38    1024   56 / 51    1536   66 / 52    2047   72 / 54
+    //   32 / 16 x 64         2 x 2048, window 128   24 / 21    512   36 / 32    1024   49 / 43    1536   49 / 51    2047   50 / 52
+    //   32 / 16 x 128        4 x 4096, window 128  139 / 130   1024 311 / 297   2048  478 / 440   3072  532 / 530   4095  549 / 558
     const uint64_t group = c.heads / c.kv_heads, packed_rows = static_cast<uint64_t>(c.query_len) * group;
-    if (c.causal && window >= 0 && options.mask == nullptr && splits == 1 && group > 1 && args.packed_heads == 0 && packed_rows <= 0x7fffff00ull) {
-        const uint64_t tiles = (packed_rows + kTileRows - 1) / kTileRows, all = static_cast<uint64_t>(c.batch) * c.kv_heads * tiles;
-        if (all <= 0x7fffff00ull) {
+    if (c.causal && window >= 0 && options.mask == nullptr && splits == 1 && group > 1 && args.packed_heads == 0 && packed_rows <= 0x7fffff00ull &&
+        (group > 2 || 4 * static_cast<uint64_t>(window) < 3 * static_cast<uint64_t>(c.query_len))) {
+        // (runs of eight tiles, whole rounds of the XCDs: see fmha_prefill_body)
+        const uint64_t tiles = (packed_rows + kTileRows - 1) / kTileRows, runs = static_cast<uint64_t>(c.batch) * c.kv_heads * ((tiles + 7) / 8);
+        if (runs <= 0x7fffff0ull) {
             args.packed_heads = 2;
             args.query_tiles = static_cast<uint32_t>(tiles);
-            groups = (all + 63) / 64 * 64;
+            groups = (runs + 7) / 8 * 64;
         }
     }
     if (halves) {

@@ -490,12 +490,16 @@ SINGE_DEVICE void fmha_prefill_body(const PrefillArgs& a, unsigned char* lds) {
     unsigned int within = blockIdx.x >> 3;
     unsigned int split = 0, bh, heavy, light;
     if (CAUSAL && OPTIONS && a.packed_heads == 2) {
-        // The tiles of all (batch, kv head) pairs, the longest first, go to the XCDs in runs of eight neighbours, whose
-        // windows overlap: a pair's tiles on one XCD would leave the others idle where there are few pairs.
-        const unsigned int at = ((within / 8u) * 8u + xcd) * 8u + within % 8u;
-        bh = at / a.query_tiles;
-        if (bh >= a.batch * a.kv_heads) return;
-        heavy = light = a.query_tiles - 1u - at % a.query_tiles;
+        // Runs of eight neighbouring tiles, whose windows overlap, go to the XCDs: the last run of every (batch, kv head) pair,
+        // then the one before it of every pair, ..., so that the longest start first and a pair stays on its XCD.  Where the
+        // pairs are no multiple of the XCDs those take every other round the other way about (or the first of them would
+        // have the longer runs of every round).
+        const unsigned int pairs = a.batch * a.kv_heads, round = within / 8u;
+        const unsigned int run = round * 8u + (pairs % 8u != 0u && round % 2u != 0u ? 7u - xcd : xcd);
+        const unsigned int back = run / pairs * 8u + within % 8u;
+        if (back >= a.query_tiles) return;
+        bh = run % pairs;
+        heavy = light = a.query_tiles - 1u - back;
     } else {
         split = within % a.splits;  // the shares of a query tile are neighbours
         within /= a.splits;

@@ -451,6 +451,20 @@ def test_causal_windows_over_grouped_heads_share_tiles(batch, heads, kv_heads, q
         close(host(padded[b:b + 1]), want, dtype)
 
 
+@pytest.mark.parametrize("batch,heads,kv_heads,length,window", [
+    (1, 32, 8, 256, 40),      # as many pairs as XCDs, one run of eight tiles each
+    (2, 16, 4, 257, 200),     # ... and a second run of one tile
+    (4, 12, 3, 700, 699),     # twelve pairs of seventeen tiles: every other round the other way about
+    (1, 9, 3, 1000, 128),     # fewer pairs than XCDs over several rounds
+    (1, 16, 8, 400, 299),     # two heads a kv head, either side of three quarters of the rows
+    (1, 16, 8, 400, 300),
+])
+def test_runs_of_row_tiles_under_a_causal_window_cover_every_row(batch, heads, kv_heads, length, window):
+    q, k, v = tensors((batch, heads, length, 64), (batch, kv_heads, length, 64), (batch, kv_heads, length, 64), torch.bfloat16, length)
+    out = neural.attend(q, k, v, None, None, neural.AttentionOptions(causal=True, window=window))
+    close(host(out), oracle.scaled_dot_product_attention_f32(host(q), host(k), host(v), causal=True, window=window, threads=8), torch.bfloat16)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("heads,length", [(4, 700), (4, 2000), (1, 90)])
