@@ -225,6 +225,20 @@ namespace {
 //   head_dim 64, full     128 x 1280 (384) 75 / 105  128 x 2048 (512) 175 / 170  256 x 2048 (1024) 322 / 327   64 x 4096 (512)   337 / 310
 // (Up to 64 the 32-row kernel holds three workgroups a compute unit and the softmax's vector instructions bound both: two or
 // three waves a SIMD share them out better than one.)
+// Where the two lengths differ, in the same units, batch * heads x queries x keys:
+//   a causal row past the last key sees them all, so that tiles are as even as without the mask
+//     head_dim 128          128 x 4096 x 1024 (1024) 278 / 267    64 x 4096 x 1500 (512) 189 / 176    64 x 2048 x 700 (256) 54 / 56
+//     head_dim 64           64 x 4096 x 1500 (512) 137 / 129      32 x 8192 x 2048 (512) 187 / 158    (64 x 4096 x 4096 (512) 179 / 172)
+//   few keys without the mask: only for a round of full tiles, 2048 queries and up
+//     head_dim 128          64 x 2048 x 512 (256) 47 / 45         32 x 4096 x 800 (256) 65 / 60       256 x 1024 x 512 (512) 90 / 91
+//     head_dim 96           64 x 2048 x 860 (256) 59 / 56         64 x 4096 x 300 (512) 57 / 64       128 x 2048 x 512 (512) 76 / 77
+//   one 256-row tile to a head takes its keys from memory once, two 128-row tiles of a workgroup twice
+//     head_dim 48           512 x 160 x 1024 (512) 73 / 51        1024 x 256 x 512 (1024) 82 / 68     256 x 256 x 512 (256) 18 / 19
+//     head_dim 64           1024 x 256 x 2048 (1024) 263 / 206    512 x 256 x 1024 (512) 55 / 55      1024 x 256 x 512 (1024) 64 / 67
+//     head_dim 80           512 x 256 x 1024 (512) 89 / 67        1024 x 160 x 512 (1024) 92 / 79     1024 x 256 x 1024, causal 55 / 67
+// Narrow heads without the mask in two rounds: 64 x 3500 (448) 279 / 256 at head_dim 64, 272 / 251 at 48; of short rows, whose last
+// tiles are not whole, 256 x 700 x 3000 (512) 172 / 226.  What the lines cost: 6 % for 128 x 2048 (512) there (172 / 162, on the
+// 32-row kernel), 5 % and less for the other shapes timed either side of them.
 bool two_tiles_a_wave(const SingeFmhaPrefillConfig& c) {
     const uint32_t wanted = g_rows_per_wave.load(std::memory_order_relaxed);
     if (wanted == 32 || !has_pair_build(static_cast<long long>(c.head_dim)) || c.key_len == 0 || !(c.scale > 0.0f) || dense_prefill_packs_heads(c))
@@ -235,9 +249,17 @@ bool two_tiles_a_wave(const SingeFmhaPrefillConfig& c) {
     const uint64_t seen = c.causal && c.query_len < c.key_len ? c.query_len : c.key_len;
     const uint64_t share = 100 * workgroups / (rounds * units);  // of the rounds' places that a workgroup takes, in percent
     if (c.head_dim < 48) return false;
-    if (c.head_dim <= 64) return !c.causal && seen >= 4096 && workgroups >= units && share >= 90;
+    if (!c.causal && pair_tiles == 1 && c.query_len > 128 && workgroups >= 2 * units && seen >= (c.head_dim == 64 ? 2048 : 512)) return true;
+    const bool two_whole_rounds = rounds == 2 && share >= 85;
+    if (c.head_dim <= 64) {
+        if (c.causal) return c.head_dim == 64 && two_whole_rounds && share >= 95 && c.query_len >= 4096 && seen >= 1000;
+        return (seen >= 4096 && workgroups >= units && share >= 90) || (two_whole_rounds && seen >= 3000 && c.query_len >= 3000);
+    }
     if (4 * workgroups < 3 * units) return !c.causal && seen >= 2560 && 8 * workgroups >= 5 * units;
-    if (!c.causal) return seen >= 900 && !(rounds == 2 && 4 * workgroups < 5 * units && seen < 1536);
+    if (!c.causal)
+        return (seen >= 900 && !(rounds == 2 && 4 * workgroups < 5 * units && seen < 1536)) ||
+               (rounds == 1 && share >= 95 && c.query_len >= 2048 && seen >= 512);
+    if (2 * c.query_len >= 5 * c.key_len && c.key_len >= 1024 && share >= 90) return true;
     return seen >= 3072 || (seen >= 2048 && share >= 70) || (seen >= 1536 && (rounds == 1 || share >= 95));
 }
 

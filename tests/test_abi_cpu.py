@@ -580,6 +580,37 @@ def test_dense_prefill_rows_per_wave(batch, heads, head_dim, query_len, key_len,
     assert _native.lib().singe_hip_dense_prefill_rows_per_wave(ctypes.byref(config._c())) == rows
 
 
+@pytest.mark.parametrize("batch,heads,head_dim,query_len,key_len,causal,rows", [
+    (2, 32, 128, 4096, 1600, 1, 64),    # most causal rows see all keys
+    (2, 32, 128, 4096, 1650, 1, 64),    # (either side of two and a half times as many queries as keys, 1536 keys and up)
+    (2, 32, 128, 4096, 1535, 1, 64),
+    (1, 64, 128, 2559, 1024, 1, 32),
+    (4, 32, 128, 4096, 1023, 1, 32),    # either side of 1024 keys
+    (4, 32, 128, 4096, 1024, 1, 64),
+    (2, 32, 96, 2048, 512, 0, 64),      # one round of full tiles over few keys
+    (2, 32, 96, 2048, 511, 0, 32),
+    (4, 32, 96, 2048, 512, 0, 32),      # ... two
+    (16, 32, 48, 256, 512, 0, 64),      # one 256-row tile to a head
+    (16, 32, 48, 128, 512, 0, 32),      # ... one 128-row tile
+    (16, 32, 48, 257, 512, 0, 32),
+    (16, 32, 48, 256, 511, 0, 32),
+    (15, 32, 80, 256, 512, 0, 32),      # ... less than two to a compute unit
+    (16, 32, 80, 256, 512, 1, 32),
+    (16, 32, 64, 256, 2047, 0, 32),
+    (16, 32, 64, 256, 2048, 0, 64),
+    (2, 32, 64, 4096, 4096, 1, 64),     # narrow heads in two whole rounds
+    (2, 32, 64, 4096, 999, 1, 32),
+    (2, 32, 48, 4096, 4096, 1, 32),
+    (2, 32, 48, 3500, 3500, 0, 64),
+    (2, 32, 64, 3072, 3072, 0, 32),     # one and a half
+    (2, 32, 64, 3500, 2999, 0, 32),
+    (8, 32, 64, 700, 3000, 0, 32),      # short rows, the last tile of each not whole
+])
+def test_dense_prefill_rows_per_wave_of_unequal_lengths_and_narrow_heads(batch, heads, head_dim, query_len, key_len, causal, rows):
+    config = A.FmhaPrefillConfig.contiguous(batch, query_len, key_len, heads, heads, head_dim, 0.125, bool(causal))
+    assert _native.lib().singe_hip_dense_prefill_rows_per_wave(ctypes.byref(config._c())) == rows
+
+
 @pytest.mark.parametrize("fields,status", [
     (dict(head_dim=0), 9),         # a problem that makes no sense is refused as the other entry points refuse it
     (dict(page_size=0), 9),
