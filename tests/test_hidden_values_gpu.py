@@ -1,6 +1,7 @@
 """An infinity or a NaN among the values of a key: it reaches the rows that see the key and no others, also where a matrix
 product weighs the values of hidden keys by zero.  The ops whose reference walks only a row's own keys: packed 16-bit
-prefill and dense f32 attention.
+prefill and dense f32 attention.  And of paged attention what cache places that belong to no key hold, and keys that other
+sequences and kv heads see.
 
 The reference is float64 over each row's visible keys; where it is finite the output is, within the type's rounding of
 values up to about 4 (bf16 2^-9, f16 2^-12, f32 sums), and elsewhere the same infinity or NaN."""
@@ -107,3 +108,66 @@ def test_dense_f32_of_the_tensor_surface(dim, lengths, bad):
         end = [i + 1 if lengths is None else lengths[b] for i in range(length)]
         rows = [t[b].transpose(0, 1) for t in (q, k, v)]
         same(out[b].transpose(0, 1), visible_only(*rows, first, end, dim ** -0.5), torch.float32)
+
+
+def paged(values, dtype, heads, kv_heads, dim, page, sequences, splits, window, key_values=None):
+    """The paged op over a cache whose places without a key hold `values` and whose keys are the same whatever that is."""
+    counts = [-(-keys // page) for _, keys in sequences]
+    pages, tokens = sum(counts), sum(queries for queries, _ in sequences)
+    caches = []
+    for seed in (1, 2):
+        cache, at = torch.full((pages + 1, page, kv_heads, dim), values), 0
+        for s, ((_, keys), count) in enumerate(zip(sequences, counts)):
+            rows = draw(10 * s + seed, keys, kv_heads, dim)
+            hidden = 0 if window is None else max(0, keys - sequences[s][0] + 1 - window) // 64 * 64  # whole tiles that no row sees
+            rows[:hidden] = values
+            cache[at:at + count].view(count * page, kv_heads, dim)[:keys] = rows
+            at += count
+        caches.append(cache.to(dtype))
+    for where, value in (key_values or {}).items():
+        cache, sequence, key, kv_head = where
+        place = sum(counts[:sequence]) * page + key
+        caches[cache].view(-1, kv_heads, dim)[place, kv_head, dim // 2] = value
+    index = lambda numbers: torch.tensor(numbers, dtype=torch.int32, device="cuda")
+    sums = lambda numbers: [sum(numbers[:i]) for i in range(len(numbers) + 1)]
+    paging = neural.Paging(index(sums([queries for queries, _ in sequences])), index(sums(counts)), index(list(range(pages))),
+                           index([keys - (count - 1) * page for (_, keys), count in zip(sequences, counts)]))
+    neural._native.lib().singe_hip_set_paged_attention_splits(splits)
+    try:
+        return neural.paged_attention(draw(3, tokens, heads, dim).to(dtype).cuda(), caches[0].cuda(), caches[1].cuda(), paging,
+                                      neural.AttentionOptions(causal=True, window=window))
+    finally:
+        neural._native.lib().singe_hip_set_paged_attention_splits(0)
+
+
+# (one to sixteen rows a kv head, which have a loop of their own from pages of sixteen keys up, beside row tiles)
+PAGED = [(1, 5), (2, 130), (1, 16), (40, 77), (1, 700), (2, 333), (1, 81)]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("heads,kv_heads,dim,page", [(8, 2, 128, 16), (16, 2, 64, 32), (6, 3, 96, 64), (4, 1, 32, 16), (8, 2, 128, 12), (8, 2, 80, 16)])
+@pytest.mark.parametrize("splits", [0, 3])
+@pytest.mark.parametrize("window", [None, 70])
+def test_paged_places_that_belong_to_no_key(dtype, heads, kv_heads, dim, page, splits, window):
+    clean, clean_lse = paged(0.0, dtype, heads, kv_heads, dim, page, PAGED, splits, window)
+    out, lse = paged(NAN, dtype, heads, kv_heads, dim, page, PAGED, splits, window)
+    assert torch.equal(out, clean) and torch.equal(lse, clean_lse) and out.isfinite().all() and lse.isfinite().all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("heads,kv_heads,dim", [(8, 2, 128), (16, 2, 64), (4, 1, 32)])
+@pytest.mark.parametrize("splits,cache,bad", [(0, 0, NAN), (0, 1, NAN), (0, 1, INF), (0, 1, -INF), (3, 1, NAN), (3, 1, INF)])
+def test_paged_keys_reach_the_rows_that_see_them(dtype, heads, kv_heads, dim, splits, cache, bad):
+    # (a share whose sum is a NaN has a log-sum-exp of -inf and is left out by the merge: scores without shares only)
+    # keys that every row of their sequence sees: of the last sequences' first and last groups, and of one with row tiles
+    places = {(cache, 4, 3, 0): bad, (cache, 6, 79, kv_head := kv_heads - 1): bad, (cache, 3, 20, kv_head): bad}
+    clean, _ = paged(0.0, dtype, heads, kv_heads, dim, 16, PAGED, splits, None)
+    out, _ = paged(0.0, dtype, heads, kv_heads, dim, 16, PAGED, splits, None, places)
+    reached = torch.zeros_like(out, dtype=torch.bool)
+    group, start = heads // kv_heads, [sum(queries for queries, _ in PAGED[:s]) for s in range(len(PAGED))]
+    for (_, sequence, _, head) in places:
+        rows = slice(start[sequence], start[sequence] + PAGED[sequence][0])
+        of = slice(head * group, (head + 1) * group)
+        reached[rows, of, dim // 2 if cache == 1 else slice(None)] = True
+    assert torch.equal(out[~reached], clean[~reached])
+    assert (out[reached].isnan() if math.isnan(bad) else out[reached] == bad).all()

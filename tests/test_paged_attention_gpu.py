@@ -27,14 +27,14 @@ def layout(sequences, page_size, extra_pages=3):
     return query_offsets, page_offsets, table, last, page_count
 
 
-def run_case(sequences, heads, kv_heads, page_size, options, index_dtype=torch.int32, seed=0, dim=128):
+def run_case(sequences, heads, kv_heads, page_size, options, index_dtype=torch.int32, seed=0, dim=128, dtype=torch.bfloat16):
     query_offsets, page_offsets, table, last, page_count = layout(sequences, page_size)
     tokens = query_offsets[-1]
     gen = torch.Generator(device="cuda")
     gen.manual_seed(seed)
-    q = torch.randn((tokens, heads, dim), generator=gen, device="cuda").to(torch.bfloat16)
-    kc = torch.randn((page_count, page_size, kv_heads, dim), generator=gen, device="cuda").to(torch.bfloat16)
-    vc = torch.randn((page_count, page_size, kv_heads, dim), generator=gen, device="cuda").to(torch.bfloat16)
+    q = torch.randn((tokens, heads, dim), generator=gen, device="cuda").to(dtype)
+    kc = torch.randn((page_count, page_size, kv_heads, dim), generator=gen, device="cuda").to(dtype)
+    vc = torch.randn((page_count, page_size, kv_heads, dim), generator=gen, device="cuda").to(dtype)
     index = lambda values: torch.tensor(values, dtype=index_dtype, device="cuda")
     paging = neural.Paging(index(query_offsets), index(page_offsets), index(table), index(last))
     out, lse = neural.paged_attention(q, kc, vc, paging, options)
@@ -501,6 +501,12 @@ def test_sequences_of_at_most_sixteen_rows_beside_a_chunk(heads, kv_heads, page_
     run_case(NARROW + [(150, 400)], heads, kv_heads, page_size, options, index_dtype=index_dtype, seed=dim + heads, dim=dim)
 
 
+@pytest.mark.parametrize("options", [OPTIONS[1], OPTIONS[2], OPTIONS[4]])
+@pytest.mark.parametrize("heads,kv_heads,page_size,dim", [(8, 1, 16, 128), (12, 3, 32, 64), (16, 2, 16, 32)])
+def test_f16_sequences_of_at_most_sixteen_rows_beside_a_chunk(heads, kv_heads, page_size, dim, options):
+    run_case(NARROW + [(150, 400)], heads, kv_heads, page_size, options, seed=dim, dim=dim, dtype=torch.float16)
+
+
 @pytest.mark.parametrize("heads,kv_heads,splits", [(8, 1, 0), (8, 1, 3), (4, 2, 1)])
 def test_sequences_of_at_most_sixteen_rows_over_many_keys(heads, kv_heads, splits):
     # a wave looks 64 groups' page ids up at a time: 64 turns are 4096 keys
@@ -684,4 +690,36 @@ def test_tokens_no_sequence_owns_are_zero_with_a_log_sum_exp_of_minus_infinity(c
         _native.lib().singe_hip_set_paged_attention_rows_per_wave(0)
     assert not out[~mine].any() and torch.isneginf(lse[~mine]).all()
     assert torch.isfinite(out[mine].float()).all() and torch.isfinite(lse[mine]).all()
+    assert (out[mine].float().abs().amax(dim=-1) > 0).all()
+
+
+@pytest.mark.parametrize("dim,dtype", [(16, torch.bfloat16), (32, torch.float16), (48, torch.bfloat16), (64, torch.float16), (80, torch.bfloat16),
+                                       (96, torch.float16), (112, torch.bfloat16), (128, torch.float16)])
+@pytest.mark.parametrize("case", ["row tiles", "shares", "two tiles a wave", "decode", "decode of one sequence", "decode of many sequences"])
+def test_rows_no_sequence_owns_at_every_width(case, dim, dtype):
+    """(queries, keys) of the sequences, unowned tokens before the first and after the last: also the decode kernels' merges of
+    a row's shares, for few of them (more sequences than workers), some, and many (a lone long sequence)."""
+    before, after, sequences = {"decode": (3, 4, [(1, 700)] * 3 + [(0, 9)] * 20), "decode of one sequence": (2, 1, [(1, 40000)] + [(0, 1)] * 3),
+                                "decode of many sequences": (5, 6, [(1, 60)] * 600 + [(0, 3)] * 11)}.get(case, (3, 300, [(7, 40), (255, 300), (1, 90)]))
+    heads, kv_heads, page_size = 8, 2, 16
+    query_offsets, page_offsets, table, last, page_count = layout(sequences, page_size)
+    tokens = before + query_offsets[-1] + after
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(dim)
+    rand = lambda *shape: torch.randn(shape, generator=gen, device="cuda").to(dtype)
+    index = lambda values: torch.tensor([int(v) for v in values], dtype=torch.int32, device="cuda")
+    paging = neural.Paging(index([before + offset for offset in query_offsets]), index(page_offsets), index(table), index(last))
+    q, kc, vc = rand(tokens, heads, dim), rand(page_count, page_size, kv_heads, dim), rand(page_count, page_size, kv_heads, dim)
+    _native.lib().singe_hip_set_paged_attention_splits(3 if case == "shares" else 0)
+    _native.lib().singe_hip_set_paged_attention_rows_per_wave(64 if case == "two tiles a wave" else 32 if case == "row tiles" else 0)
+    try:
+        poison(((tokens, heads, dim), dtype), ((tokens, heads), torch.float32))
+        out, lse = neural.paged_attention(q, kc, vc, paging, neural.AttentionOptions(causal=True))
+    finally:
+        _native.lib().singe_hip_set_paged_attention_splits(0)
+        _native.lib().singe_hip_set_paged_attention_rows_per_wave(0)
+    mine = torch.zeros(tokens, dtype=torch.bool, device="cuda")
+    mine[before:tokens - after] = True
+    assert not out[~mine].any() and torch.isneginf(lse[~mine]).all()
+    assert torch.isfinite(out.float()).all() and torch.isfinite(lse[mine]).all()
     assert (out[mine].float().abs().amax(dim=-1) > 0).all()
