@@ -313,7 +313,6 @@ struct GeneralPagedArgs {
     double scale_wide;              // the scale for f64 tensors: the default 1 / sqrt(head_dim) is taken in f64 there
 };
 
-// singe_paged_mla_attention_general_*: contiguous operands of one element type.
 // What the matrix-core latent kernel leaves for the merge about a unit (128 rows of a sequence at most).
 struct alignas(16) LatentUnit {
     uint64_t first_row;   // its first row of [tokens, heads]
@@ -323,6 +322,7 @@ struct alignas(16) LatentUnit {
     uint32_t shares;
 };
 
+// singe_paged_mla_attention_general_*: contiguous operands of one element type.
 struct LatentAttentionArgs {
     const void* latent_queries;      // [tokens, heads, latent_dim]
     const void* positional_queries;  // [tokens, heads, position_dim]
