@@ -237,8 +237,9 @@ namespace {
 //     head_dim 64           1024 x 256 x 2048 (1024) 263 / 206    512 x 256 x 1024 (512) 55 / 55      1024 x 256 x 512 (1024) 64 / 67
 //     head_dim 80           512 x 256 x 1024 (512) 89 / 67        1024 x 160 x 512 (1024) 92 / 79     1024 x 256 x 1024, causal 55 / 67
 // Narrow heads without the mask in two rounds: 64 x 3500 (448) 279 / 256 at head_dim 64, 272 / 251 at 48; of short rows, whose last
-// tiles are not whole, 256 x 700 x 3000 (512) 172 / 226.  What the lines cost: 6 % for 128 x 2048 (512) there (172 / 162, on the
-// 32-row kernel), 5 % and less for the other shapes timed either side of them.
+// tiles are not whole, 256 x 700 x 3000 (512) 172 / 226.  What the lines cost against the faster kernel, of 520 shapes: up to 11 %
+// for narrow heads without the mask in many rounds (head_dim 48, 256 x 4096 (2048) 1154 / 1281, on the two-tile kernel), 9 % under it
+// at head_dim 48 (32 x 8192 (512) 331 / 305, on the 32-row one), 7 % for 128 x 2048 (512) at 64 without it (174 / 162) and from 80 up.
 bool two_tiles_a_wave(const SingeFmhaPrefillConfig& c) {
     const uint32_t wanted = g_rows_per_wave.load(std::memory_order_relaxed);
     if (wanted == 32 || !has_pair_build(static_cast<long long>(c.head_dim)) || c.key_len == 0 || !(c.scale > 0.0f) || dense_prefill_packs_heads(c))
