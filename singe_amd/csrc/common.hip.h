@@ -77,6 +77,10 @@ SINGE_DEVICE uint4 stream_load_16(const void* address) {
     return make_uint4(bits.x, bits.y, bits.z, bits.w);
 }
 
+SINGE_DEVICE void stream_store_16(void* address, uint4 bits) {
+    __builtin_nontemporal_store(u32x4_t{bits.x, bits.y, bits.z, bits.w}, reinterpret_cast<u32x4_t*>(address));
+}
+
 typedef unsigned int u32x2_t __attribute__((ext_vector_type(2)));
 SINGE_DEVICE uint2 stream_load_8(const void* address) {
     const u32x2_t bits = __builtin_nontemporal_load(reinterpret_cast<const u32x2_t*>(address));

@@ -264,6 +264,48 @@ bool two_tiles_a_wave(const SingeFmhaPrefillConfig& c) {
     return seen >= 3072 || (seen >= 2048 && share >= 70) || (seen >= 1536 && (rounds == 1 || share >= 95));
 }
 
+// Short causal windows over grouped heads, where a workgroup of eight waves walks along a run of rows with the keys its windows
+// reach kept in LDS (fmha_window.hip.h): how many blocks of 32 keys it holds, how many runs a (batch, kv head) pair's rows are
+// cut into and how many steps of 256 rows a run has; no runs where the call is not for that kernel, which are windows whose
+// blocks do not fit LDS (half of it where rows are 128 bytes, since a compute unit must hold two workgroups there: one took
+// 0.97 to 1.3 x the row tiles' time), and launches that do not give a compute unit its step (129 steps and up; at most 1.13 x
+// below).  Row tiles / runs, us (heads x head_dim, batch x length, window; steps of all pairs):
+//   64 / 8 x 64    1 x 8192, 16 (2048)  48 / 31     128   58 / 41     256   70 / 55     512   98 / 100 (left on row tiles)
+//                  4 x 8192, 128 (8192) 224 / 173   1 x 1500, 128 (376) 12.5 / 11.9, 256 15.5 / 16.2 (a second step on some
+//                  compute units only, and ten blocks to bring in first: left on row tiles)   1 x 512, 128 (128) 9.7 / 9.7
+//   64 / 8 x 128   1 x 8192, 128 (2048) 125 / 75    256  151 / 98     1 x 2048, 128 (512) 31 / 21   1 x 512, 128 (128) 11.4 / 11.9
+//   32 / 8 x 128   2 x 4096, 128 (1024) 59 / 39     160   61 / 42
+//   28 / 4 x 128   1 x 3000, 128 (332)  26 / 21     64 / 8 x 96, 1 x 4096, 128 (1024) 47 / 34
+struct WindowRuns {
+    uint32_t ring_blocks, runs, run_steps;
+};
+
+WindowRuns window_runs(const SingeFmhaPrefillConfig& c, uint64_t window) {
+    constexpr uint64_t kStepRows = 32 * kWindowPrefillWaves, kLdsBytes = 160 * 1024;
+    const uint64_t group = c.heads / c.kv_heads, row_bytes = c.head_dim <= 64 ? 128 : 256;
+    // The kernel counts a batch entry's queries and output rows in 32 bits of bytes.
+    const uint64_t query_reach = (c.query_len - 1) * c.query_sequence_stride + (c.heads - 1) * c.query_head_stride + c.head_dim;
+    const uint64_t output_reach = (c.query_len - 1) * c.output_sequence_stride + (c.heads - 1) * c.output_head_stride + c.head_dim;
+    if (query_reach > 0x7fffffffull || output_reach > 0x7fffffffull) return {0, 0, 0};
+    // The keys from the first one that a step's first row sees to the last one that the next step's last row does, in blocks
+    // of 32; where every step starts with a query that is a multiple of 32 the first key's place in its block is known.
+    const bool whole = kStepRows % group == 0 && kStepRows / group % 32 == 0;
+    const uint64_t keys = window + (whole ? 2 * kStepRows / group - 1 : (2 * kStepRows - 1 + group - 1) / group);
+    const uint64_t ring = ((whole ? (32 - (window + 31) % 32) % 32 : 31) + keys - 1) / 32 + 1, bytes = ring * 64 * row_bytes;
+    if (bytes > (c.head_dim <= 64 ? kLdsBytes / 2 : kLdsBytes)) return {0, 0, 0};
+    const uint64_t units = compute_units(), places = units * (c.head_dim <= 64 ? 2 : 1);
+    const uint64_t pairs = static_cast<uint64_t>(c.batch) * c.kv_heads, steps = (c.query_len * group + kStepRows - 1) / kStepRows, all = pairs * steps;
+    if (2 * all <= units || (c.head_dim <= 64 && ring > 8 && all > units && 2 * all < 3 * units)) return {0, 0, 0};
+    // Runs of one length that fill the chip's places in whole rounds, a run's first keys counted as a step.
+    uint64_t best = ~0ull, best_steps = steps;
+    for (uint64_t runs = 1; runs <= steps && (runs - 1) * pairs <= 4 * places; ++runs) {
+        const uint64_t run_steps = (steps + runs - 1) / runs, rounds = (pairs * ((steps + run_steps - 1) / run_steps) + places - 1) / places;
+        const uint64_t cost = rounds * (run_steps + 1);
+        if (cost < best) best = cost, best_steps = run_steps;
+    }
+    return {static_cast<uint32_t>(ring), static_cast<uint32_t>((steps + best_steps - 1) / best_steps), static_cast<uint32_t>(best_steps)};
+}
+
 int32_t prefill(void* stream, uint16_t* out, size_t out_len, float* lse, size_t lse_len, bool with_lse,
                 const uint16_t* query, size_t query_len, const uint16_t* key, size_t key_len, const uint16_t* value,
                 size_t value_len, const SingeFmhaPrefillConfig* config, bool f16 = false, const DenseOptions& options = DenseOptions()) {
@@ -401,6 +443,16 @@ int32_t prefill(void* stream, uint16_t* out, size_t out_len, float* lse, size_t 
     const uint64_t group = c.heads / c.kv_heads, packed_rows = static_cast<uint64_t>(c.query_len) * group;
     if (c.causal && window >= 0 && options.mask == nullptr && splits == 1 && group > 1 && args.packed_heads == 0 && packed_rows <= 0x7fffff00ull &&
         (group > 2 || 4 * static_cast<uint64_t>(window) < 3 * static_cast<uint64_t>(c.query_len))) {
+        const WindowRuns run = options.softcap == 0.0f ? window_runs(c, static_cast<uint64_t>(window)) : WindowRuns{0, 0, 0};
+        if (run.runs != 0) {
+            args.ring_blocks = run.ring_blocks;
+            args.query_tiles = run.runs;
+            args.run_steps = run.run_steps;
+            const uint64_t workgroups = (static_cast<uint64_t>(c.batch) * c.kv_heads * run.runs + 7) / 8 * 8;
+            if (workgroups > 0x7fffffffull) return fail(SINGE_HIP_UNSUPPORTED_CONFIGURATION, "too many workgroups");
+            return launch(static_cast<KernelId>(prefill_window_at(head_dim) + (f16 ? 1 : 0)), static_cast<unsigned>(workgroups), 1, 1,
+                          64 * kWindowPrefillWaves, stream, args, run.ring_blocks * 64 * (c.head_dim <= 64 ? 128 : 256));
+        }
         // (runs of eight tiles, whole rounds of the XCDs: see fmha_prefill_body)
         const uint64_t tiles = (packed_rows + kTileRows - 1) / kTileRows, runs = static_cast<uint64_t>(c.batch) * c.kv_heads * ((tiles + 7) / 8);
         if (runs <= 0x7fffff0ull) {

@@ -24,6 +24,7 @@
 #define SINGE_PREFILL_ROW_BYTES 128
 #endif
 #include "prefill_blocks.hip.h"
+#include "fmha_window.hip.h"
 
 namespace {
 
@@ -596,6 +597,13 @@ SINGE_DEVICE void fmha_prefill_combine_body(const PrefillArgs& a) {
         fmha_prefill_body<CAUSAL, prefill::HALF, kDenseWaves, false, 2>(args, prefill_lds);         \
     }
 
+// Short causal windows over grouped heads (fmha_window.hip.h), in as much LDS as the launch asks for.
+#define SINGE_FMHA_WINDOW_KERNEL(NAME, HALF)                                                       \
+    extern "C" __global__ __launch_bounds__(64 * kWindowPrefillWaves, SINGE_HEAD_DIM <= 64 ? 4 : 2) void NAME(PrefillArgs args) { \
+        extern __shared__ __attribute__((aligned(1024))) unsigned char window_lds[];                 \
+        fmha_window_body<prefill::HALF>(args, window_lds);                                          \
+    }
+
 // Names carry the head dimension of the build: singe_fmha_prefill_bf16_d128_causal, ..._d64_causal.
 #define SINGE_PASTE3_(a, b, c) a##b##c
 #define SINGE_PASTE3(a, b, c) SINGE_PASTE3_(a, b, c)
@@ -613,5 +621,7 @@ SINGE_FMHA_PREFILL_HALVES_KERNEL(SINGE_PREFILL_NAME(bf16, _causal_halves), true,
 SINGE_FMHA_PREFILL_HALVES_KERNEL(SINGE_PREFILL_NAME(bf16, _full_halves), false, Bf16)
 SINGE_FMHA_PREFILL_HALVES_KERNEL(SINGE_PREFILL_NAME(f16, _causal_halves), true, F16)
 SINGE_FMHA_PREFILL_HALVES_KERNEL(SINGE_PREFILL_NAME(f16, _full_halves), false, F16)
+SINGE_FMHA_WINDOW_KERNEL(SINGE_PREFILL_NAME(bf16, _causal_window), Bf16)
+SINGE_FMHA_WINDOW_KERNEL(SINGE_PREFILL_NAME(f16, _causal_window), F16)
 extern "C" __global__ __launch_bounds__(256) void SINGE_PREFILL_NAME(bf16, _combine)(PrefillArgs args) { fmha_prefill_combine_body<prefill::Bf16>(args); }
 extern "C" __global__ __launch_bounds__(256) void SINGE_PREFILL_NAME(f16, _combine)(PrefillArgs args) { fmha_prefill_combine_body<prefill::F16>(args); }

@@ -56,6 +56,8 @@ struct CombineArgs {
 // it through this constant.  4 (two workgroups per compute unit) and 8 (one, whose K and V tiles serve 256 rows)
 // both pass the tests and measure the same; 4 is what the committed profiles were taken with.
 constexpr int kDensePrefillWaves = 4;
+// Waves of a workgroup of the kernel for short causal windows, 32 (query, head) rows of a step each.
+constexpr int kWindowPrefillWaves = 8;
 
 struct PrefillArgs {
     const uint16_t* query;          // [batch, query_len, heads, 128] bf16, element strides below
@@ -103,6 +105,9 @@ struct PrefillArgs {
     uint32_t packed_heads = 0;
     // With single_tiles != 0 a workgroup takes one query tile instead of two (32-row kernels).
     uint32_t single_tiles = 0;
+    // The *_window kernels: a workgroup takes run_steps steps of 32 * kWindowPrefillWaves (query, head) rows of a (batch, kv
+    // head) pair, query_tiles such runs to a pair, with ring_blocks blocks of 32 keys in LDS.
+    uint32_t run_steps = 0, ring_blocks = 0;
 };
 
 struct PrefillF32Args {

@@ -403,6 +403,14 @@ const char* const kKernelNames[kKernelCount] = {
     "singe_fmha_prefill_f16_d80_causal_halves", "singe_fmha_prefill_f16_d80_full_halves",
     "singe_fmha_prefill_bf16_d112_causal_halves", "singe_fmha_prefill_bf16_d112_full_halves",
     "singe_fmha_prefill_f16_d112_causal_halves", "singe_fmha_prefill_f16_d112_full_halves",
+    "singe_fmha_prefill_bf16_d128_causal_window", "singe_fmha_prefill_f16_d128_causal_window",
+    "singe_fmha_prefill_bf16_d64_causal_window", "singe_fmha_prefill_f16_d64_causal_window",
+    "singe_fmha_prefill_bf16_d32_causal_window", "singe_fmha_prefill_f16_d32_causal_window",
+    "singe_fmha_prefill_bf16_d96_causal_window", "singe_fmha_prefill_f16_d96_causal_window",
+    "singe_fmha_prefill_bf16_d16_causal_window", "singe_fmha_prefill_f16_d16_causal_window",
+    "singe_fmha_prefill_bf16_d48_causal_window", "singe_fmha_prefill_f16_d48_causal_window",
+    "singe_fmha_prefill_bf16_d80_causal_window", "singe_fmha_prefill_f16_d80_causal_window",
+    "singe_fmha_prefill_bf16_d112_causal_window", "singe_fmha_prefill_f16_d112_causal_window",
 };
 
 // The code object is built in parts, one per kernel source (so they compile side by side and a process loads only
@@ -459,6 +467,7 @@ constexpr PartRun kPartRuns[] = {
     {3, 2}, {15, 2}, {19, 2}, {21, 2}, {23, 2}, {25, 2}, {27, 2}, {29, 2},    // packed sequences
     {52, 7},                      // dense f32 attention on the matrix cores
     {1, 4}, {14, 4}, {18, 4}, {20, 4}, {22, 4}, {24, 4}, {26, 4}, {28, 4},    // the dense prefill with two sets of waves to a tile
+    {1, 2}, {14, 2}, {18, 2}, {20, 2}, {22, 2}, {24, 2}, {26, 2}, {28, 2},    // the dense prefill of short causal windows
 };
 constexpr int runs_total() {
     int total = 0;

@@ -105,7 +105,9 @@ enum KernelId : int {
     // the dense prefill with two sets of waves to a tile (no options), four to a head dimension in kRaggedPrefill's order:
     // + (no causal mask) + 2 * f16
     kPrefillHalves = kAttentionMfmaF32 + 7,
-    kKernelCount = kPrefillHalves + 4 * 8
+    // the dense prefill of short causal windows over grouped heads: bf16, f16 for each head dimension in kRaggedPrefill's order
+    kPrefillWindow = kPrefillHalves + 4 * 8,
+    kKernelCount = kPrefillWindow + 2 * 8
 };
 
 // The two-tile kernels (fmha_prefill_pair.hip, paged_attention_pair.hip) have a build for every multiple of 16 up to 128.
@@ -182,6 +184,9 @@ inline int head_dim_order(long long head_dim) {
 
 // The dense prefill with two sets of waves to a tile for a head dimension, before 1 without the causal mask and 2 for f16.
 inline int prefill_halves_at(long long head_dim) { return kPrefillHalves + 4 * head_dim_order(head_dim); }
+
+// The dense prefill of short causal windows for a head dimension, before 1 is added for f16.
+inline int prefill_window_at(long long head_dim) { return kPrefillWindow + 2 * head_dim_order(head_dim); }
 
 // The packed-sequences kernel for a head dimension, before 1 is added for f16.
 inline int ragged_prefill_at(long long head_dim) { return kRaggedPrefill + 2 * head_dim_order(head_dim); }

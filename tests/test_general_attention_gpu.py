@@ -451,6 +451,36 @@ def test_causal_windows_over_grouped_heads_share_tiles(batch, heads, kv_heads, q
         close(host(padded[b:b + 1]), want, dtype)
 
 
+@pytest.mark.parametrize("batch,heads,kv_heads,query_len,key_len,dim,dtype,options", [
+    (1, 64, 8, 1100, 1100, 64, torch.bfloat16, dict(window=128, sinks=True)),    # several runs of two steps, a last step that is not whole
+    (2, 64, 8, 777, 777, 128, torch.float16, dict(window=256)),                  # the most blocks that fit, one step after the other in their places
+    (1, 64, 8, 900, 500, 64, torch.bfloat16, dict(window=33, sinks=True)),       # rows past the last key and its window
+    (1, 64, 8, 600, 900, 64, torch.float16, dict(window=1)),                     # keys past the last query
+    (1, 64, 8, 600, 600, 96, torch.bfloat16, dict(window=31, scale=-0.1)),
+    (2, 32, 8, 700, 651, 128, torch.bfloat16, dict(window=160, sinks=True)),     # four heads a kv head: two blocks a step
+    (2, 28, 4, 1000, 1000, 128, torch.float16, dict(window=128)),                # seven: queries that start inside a step
+    (3, 32, 16, 700, 700, 64, torch.bfloat16, dict(window=64)),                  # two
+    (2, 24, 8, 1500, 1500, 48, torch.float16, dict(window=100, sinks=True)),     # three, half a dim block
+    (1, 128, 2, 600, 600, 16, torch.bfloat16, dict(window=70)),                  # a query's heads over two waves
+    (1, 64, 8, 700, 700, 112, torch.bfloat16, dict(window=0)),                   # no key in sight
+])
+def test_short_causal_windows_walk_runs_of_rows(batch, heads, kv_heads, query_len, key_len, dim, dtype, options):
+    options = dict(options)
+    sinks = None
+    q, k, v = tensors((batch, heads, query_len, dim), (batch, kv_heads, key_len, dim), (batch, kv_heads, key_len, dim), dtype, heads + dim)
+    if options.pop("sinks", False):
+        sinks = torch.linspace(-2.0, 2.0, heads, device="cuda").to(dtype)
+    torch.full_like(q, float("nan"))  # (what the output's memory holds before: a row that is not written shows)
+    out = neural.attend(q, k, v, None, sinks, neural.AttentionOptions(causal=True, **options))
+    want = oracle.scaled_dot_product_attention_f32(host(q), host(k), host(v), causal=True, threads=8,
+                                                   sinks=None if sinks is None else host(sinks), **options)
+    close(host(out), want, dtype)
+    lengths = [max(0, key_len - 333 * (b + 1)) if b % 2 == 0 else 0 for b in range(batch)]
+    padded = neural.attend_padded(q, k, v, torch.tensor(lengths, device="cuda", dtype=torch.int32), neural.AttentionOptions(causal=True, **options))
+    want = oracle.scaled_dot_product_attention_f32(host(q), host(k), host(v), causal=True, threads=8, key_lengths=lengths, **options)
+    close(host(padded), want, dtype)
+
+
 @pytest.mark.parametrize("batch,heads,kv_heads,length,window", [
     (1, 32, 8, 256, 40),      # as many pairs as XCDs, one run of eight tiles each
     (2, 16, 4, 257, 200),     # ... and a second run of one tile
