@@ -117,6 +117,40 @@ SINGE_DEVICE float across_groups_sum(float value) {
     return a + b;
 }
 
+// Sum and maximum (any `join` of two) over a wave's 64 lanes, in every lane: four rotations inside the rows of sixteen, two
+// swaps across.
+template <class Value, class Join>
+SINGE_DEVICE Value across_wave(Value value, Join join) {
+    auto turned = [&](auto steps) __attribute__((always_inline)) {
+        return __builtin_bit_cast(Value, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, value), 0x120 + decltype(steps)::value, 0xF, 0xF, false));
+    };
+    value = join(value, turned(std::integral_constant<int, 8>{}));
+    value = join(value, turned(std::integral_constant<int, 4>{}));
+    value = join(value, turned(std::integral_constant<int, 2>{}));
+    value = join(value, turned(std::integral_constant<int, 1>{}));
+    float a, b;
+    swap_with_self<16>(__builtin_bit_cast(float, value), a, b);
+    value = join(__builtin_bit_cast(Value, a), __builtin_bit_cast(Value, b));
+    swap_with_self<32>(__builtin_bit_cast(float, value), a, b);
+    return join(__builtin_bit_cast(Value, a), __builtin_bit_cast(Value, b));
+}
+
+// Inclusive prefix sums over a wave's 64 lanes: shifts inside the rows of sixteen (zeros come in), then each row's last lane
+// to the next row, and that of the second to the upper half.
+SINGE_DEVICE unsigned int sums_through_lane(unsigned int value) {
+    auto shifted = [&](auto control, auto rows) __attribute__((always_inline)) {
+        return static_cast<unsigned int>(__builtin_amdgcn_update_dpp(0, static_cast<int>(value), decltype(control)::value, decltype(rows)::value, 0xF, false));
+    };
+    typedef std::integral_constant<int, 0xF> all;
+    value += shifted(std::integral_constant<int, 0x111>{}, all{});
+    value += shifted(std::integral_constant<int, 0x112>{}, all{});
+    value += shifted(std::integral_constant<int, 0x114>{}, all{});
+    value += shifted(std::integral_constant<int, 0x118>{}, all{});
+    value += shifted(std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xA>{});
+    value += shifted(std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xC>{});
+    return value;
+}
+
 SINGE_DEVICE float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 SINGE_DEVICE float fast_log2(float x) { return __builtin_amdgcn_logf(x); }
 // tanh(x) = 1 - 2 / (e^(2x) + 1): one exponential and one reciprocal; exact at both infinities, absolute error

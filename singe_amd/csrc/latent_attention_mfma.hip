@@ -134,20 +134,6 @@ SINGE_DEVICE bool find_unit(const LatentAttentionArgs& a, unsigned int unit, uns
     return false;
 }
 
-// Sum and maximum over a wave's 64 lanes, in every lane: four rotations inside the rows of sixteen, two swaps across.
-template <class Join>
-SINGE_DEVICE unsigned int across_wave(unsigned int value, Join join) {
-    value = join(value, static_cast<unsigned int>(__builtin_amdgcn_update_dpp(0, static_cast<int>(value), 0x128, 0xF, 0xF, false)));
-    value = join(value, static_cast<unsigned int>(__builtin_amdgcn_update_dpp(0, static_cast<int>(value), 0x124, 0xF, 0xF, false)));
-    value = join(value, static_cast<unsigned int>(__builtin_amdgcn_update_dpp(0, static_cast<int>(value), 0x122, 0xF, 0xF, false)));
-    value = join(value, static_cast<unsigned int>(__builtin_amdgcn_update_dpp(0, static_cast<int>(value), 0x121, 0xF, 0xF, false)));
-    float a, b;
-    swap_with_self<16>(as_float(static_cast<int>(value)), a, b);
-    value = join(static_cast<unsigned int>(as_int(a)), static_cast<unsigned int>(as_int(b)));
-    swap_with_self<32>(as_float(static_cast<int>(value)), a, b);
-    return join(static_cast<unsigned int>(as_int(a)), static_cast<unsigned int>(as_int(b)));
-}
-
 // What of a problem a workgroup takes: share `share` of `shares` of the key tiles of a unit (a row tile of a sequence).
 // Shares are `share_tiles` long, or (0) the unit's tiles over the shares.  Partial rows of a unit start at `first_slot`, its
 // shares one after the other; with a fixed count of shares a row has the slot of its index in each share's [tokens, heads], so

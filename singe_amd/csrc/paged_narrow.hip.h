@@ -90,20 +90,22 @@ SINGE_DEVICE void narrow_wait(unsigned int count) {
 // Until the LDS reads in front of it are done, so that their slot may be loaded into.
 SINGE_DEVICE void narrow_slot_read() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
-// The rows of one (sequence, kv head), keys [key_begin, key_end) of the sequence (multiples of sixteen, but for the end),
-// of which a row sees what its position and the window leave it.  Pages of at least sixteen keys, a power of two of them.
-template <bool SOFTCAP, int FORM, class Half>
-SINGE_DEVICE void narrow_rows(const PagedAttentionArgs& a, unsigned char* lds, const SequenceSpan& span, unsigned int kv_head, unsigned int split,
-                              unsigned int key_begin, unsigned int key_end) {
+// The `packed` packed rows of one (sequence, kv head) from `first_row` on, keys [key_begin, key_end) of the sequence (multiples
+// of sixteen, but for the end), of which a row sees what its position and the window leave it.  Pages of at least sixteen keys,
+// a power of two of them.  finish(row, quad, values, lse2) takes values 4 quad .. of a row, normalised, and its base-two
+// log-sum-exp (a row that sees no key: zeros and -inf).
+template <bool SOFTCAP, int FORM, class Half, class Finish>
+SINGE_DEVICE void narrow_rows(const PagedAttentionArgs& a, unsigned char* lds, const SequenceSpan& span, unsigned int kv_head, unsigned int first_row,
+                              unsigned int packed, unsigned int key_begin, unsigned int key_end, Finish&& finish) {
     const unsigned int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63u;
     const unsigned int column = lane & 15u, g = lane >> 4;
     const unsigned int groups = a.heads / a.kv_heads;
-    const unsigned int queries = span.queries, keys = span.keys, packed = queries * groups;
+    const unsigned int queries = span.queries, keys = span.keys;
     const bool causal = a.causal != 0, windowed = a.window >= 0;
     const unsigned int window = !windowed ? 0u : a.window > 0x7fffffffll ? 0x7fffffffu : static_cast<unsigned int>(a.window);
     const Half half{};
     auto position_of = [&](unsigned int row) __attribute__((always_inline)) {
-        const long long position = static_cast<long long>(keys) - static_cast<long long>(queries) + row / groups;
+        const long long position = static_cast<long long>(keys) - static_cast<long long>(queries) + (first_row + row) / groups;
         return position < 0 ? 0u : static_cast<unsigned int>(position);
     };
     const bool row_valid = column < packed;
@@ -116,7 +118,8 @@ SINGE_DEVICE void narrow_rows(const PagedAttentionArgs& a, unsigned char* lds, c
     const unsigned int flip = (SOFTCAP ? a.softcap_scale : a.scale_log2e) < 0.0f ? 0x80008000u : 0u;
     uint4 q[kNarrowSteps];
     {
-        const size_t flat = (static_cast<size_t>(span.query_start) + my_row / groups) * a.heads + kv_head * groups + my_row % groups;
+        const unsigned int at = first_row + my_row;
+        const size_t flat = (static_cast<size_t>(span.query_start) + at / groups) * a.heads + kv_head * groups + at % groups;
         const uint16_t* row = a.query_rows + flat * kHeadDim + 8u * g;
 #pragma unroll
         for (int s = 0; s < kNarrowSteps; ++s) {
@@ -308,20 +311,9 @@ SINGE_DEVICE void narrow_rows(const PagedAttentionArgs& a, unsigned char* lds, c
             merged.z = fmaf(weight, part.z, merged.z);
             merged.w = fmaf(weight, part.w, merged.w);
         }
-        // (a row that sees no key stays zero and has a log-sum-exp of -inf)
         const float inverse = total > 0.0f ? 1.0f / total : 0.0f;
         merged.x *= inverse; merged.y *= inverse; merged.z *= inverse; merged.w *= inverse;
-        const float lse2 = total > 0.0f ? largest + fast_log2(total) : -INFINITY;
-        const size_t flat = (static_cast<size_t>(span.query_start) + row / groups) * a.heads + kv_head * groups + row % groups;
-        if (a.splits > 1) {
-            const size_t slot = static_cast<size_t>(split) * a.tokens * a.heads + flat;
-            *reinterpret_cast<float4*>(a.partial_out + slot * kHeadDim + 4u * quad) = merged;
-            if (quad == 0) a.partial_lse[slot] = lse2;
-        } else {
-            *reinterpret_cast<uint2*>(a.output + flat * kHeadDim + 4u * quad) =
-                make_uint2(pack_pair(half, merged.x, merged.y), pack_pair(half, merged.z, merged.w));
-            if (a.lse != nullptr && quad == 0) a.lse[flat] = lse2;
-        }
+        finish(row, quad, merged, total > 0.0f ? largest + fast_log2(total) : -INFINITY);
     }
 }
 

@@ -723,3 +723,59 @@ def test_rows_no_sequence_owns_at_every_width(case, dim, dtype):
     assert not out[~mine].any() and torch.isneginf(lse[~mine]).all()
     assert torch.isfinite(out.float()).all() and torch.isfinite(lse[mine]).all()
     assert (out[mine].float().abs().amax(dim=-1) > 0).all()
+
+
+STEPS = [
+    [(1, 100)], [(1, 3000)], [(1, 16)], [(1, 897), (1, 896), (1, 895)],                        # not shared out, shared out, either side of the line
+    [(1, 1), (1, 9000), (1, 0), (1, 33), (0, 500), (1, 64), (1, 65), (1, 4096)],               # one that is far longer, one without keys, one without tokens
+    [(2, 700), (1, 100), (0, 90), (3, 2), (0, 40), (0, 16)],                                   # several tokens of a sequence, more of them than keys
+    [(0, 300)] * 40 + [(40, 2000), (0, 77)],                                                   # all tokens one sequence's, in several units
+    [(1, 37 * i % 700) for i in range(100)],                                                   # more sequences than a wave has lanes
+]
+
+
+@pytest.mark.parametrize("options", [OPTIONS[0], OPTIONS[1], OPTIONS[3], neural.AttentionOptions(causal=True, scale=-0.07, window=1000)])
+@pytest.mark.parametrize("heads,kv_heads,page_size,dim,dtype,index_dtype", [
+    (32, 8, 16, 128, torch.bfloat16, torch.int64), (16, 1, 32, 64, torch.float16, torch.int32), (6, 2, 64, 96, torch.bfloat16, torch.int32),
+    (4, 4, 16, 32, torch.float16, torch.int64), (10, 2, 16, 128, torch.bfloat16, torch.int64)])  # (five heads: threads that merge nothing)
+@pytest.mark.parametrize("step", range(len(STEPS)))
+def test_decode_steps_in_one_launch(step, heads, kv_heads, page_size, dim, dtype, index_dtype, options):
+    run_case(STEPS[step], heads, kv_heads, page_size, options, index_dtype=index_dtype, seed=step, dim=dim, dtype=dtype)
+
+
+def test_a_decode_step_in_one_launch_replays_over_whatever_its_scratch_holds():
+    """Shares tell each other that they are done by words in the scratch: none is taken from an earlier use of it, be that
+    another problem's partial rows, bytes of any kind or the same captured launch's last replay."""
+    lengths = [3000, 9000, 100, 2000]
+    query_offsets, page_offsets, table, last, page_count = layout([(1, n) for n in lengths], 16)
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(3)
+    q = torch.randn((4, 32, 128), generator=gen, device="cuda").bfloat16()
+    kc, vc = (torch.randn((page_count, 16, 8, 128), generator=gen, device="cuda").bfloat16() for _ in range(2))
+    index = lambda values: torch.tensor(values, dtype=torch.int64, device="cuda")
+    paging = neural.Paging(index(query_offsets), index(page_offsets), index(table), index(last))
+    options = neural.AttentionOptions(causal=True)
+    status = torch.zeros(1, device="cuda", dtype=torch.int32)
+    scratch = torch.empty(8 << 20, device="cuda", dtype=torch.uint8)
+    call = lambda: neural.paged_attention(q, kc, vc, paging, options, status=status, check=False, scratch=scratch)
+    want, want_lse = call()
+    code, reference, reference_lse = oracle.paged_attention_f32(q.float().cpu().numpy(), kc.float().cpu().numpy(), vc.float().cpu().numpy(), query_offsets,
+                                                                page_offsets, table, last, scale=None, causal=True, threads=8)
+    assert code == 0 and np.abs(want.float().cpu().numpy() - reference).max() <= MAX_ABS and np.abs(want_lse.cpu().numpy() - reference_lse).max() <= LSE_ABS
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        call()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            out, lse = call()
+        for turn in range(6):
+            if turn % 2 == 1:
+                scratch.copy_(torch.randint(0, 256, scratch.shape, generator=gen, device="cuda", dtype=torch.uint8))
+            if turn % 3 == 2:
+                call()
+            q.copy_(torch.randn(q.shape, generator=gen, device="cuda"))
+            out.fill_(float("nan"))
+            graph.replay()
+            fresh, fresh_lse = call()
+            stream.synchronize()
+            assert torch.equal(out, fresh) and torch.equal(lse, fresh_lse)
