@@ -93,8 +93,9 @@ SINGE_DEVICE void narrow_slot_read() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "
 // The `packed` packed rows of one (sequence, kv head) from `first_row` on, keys [key_begin, key_end) of the sequence (multiples
 // of sixteen, but for the end), of which a row sees what its position and the window leave it.  Pages of at least sixteen keys,
 // a power of two of them.  finish(row, quad, values, lse2) takes values 4 quad .. of a row, normalised, and its base-two
-// log-sum-exp (a row that sees no key: zeros and -inf).
-template <bool SOFTCAP, int FORM, class Half, class Finish>
+// log-sum-exp (a row that sees no key: zeros and -inf).  WIDE: the weights meet the values at f32's precision (split_pair), by a
+// second value product that the memory-bound loop has room for.
+template <bool SOFTCAP, int FORM, bool WIDE, class Half, class Finish>
 SINGE_DEVICE void narrow_rows(const PagedAttentionArgs& a, unsigned char* lds, const SequenceSpan& span, unsigned int kv_head, unsigned int first_row,
                               unsigned int packed, unsigned int key_begin, unsigned int key_end, Finish&& finish) {
     const unsigned int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63u;
@@ -266,9 +267,19 @@ SINGE_DEVICE void narrow_rows(const PagedAttentionArgs& a, unsigned char* lds, c
                 p[r] = fast_exp2(fmaf(x[r], factor, shift));
                 running_sum += p[r];
             }
-            const uint2 weights = make_uint2(pack_pair(half, p[0], p[1]), pack_pair(half, p[2], p[3]));
+            uint2 weights, rest;
+            if constexpr (WIDE) {
+                split_pair(half, p[0], p[1], weights.x, rest.x);
+                split_pair(half, p[2], p[3], weights.y, rest.y);
+            } else {
+                weights = make_uint2(pack_pair(half, p[0], p[1]), pack_pair(half, p[2], p[3]));
+            }
 #pragma unroll
             for (int db = 0; db < kNarrowBlocks; ++db) out[db] = narrow_values(half, value[db], weights, out[db]);
+            if constexpr (WIDE) {
+#pragma unroll
+                for (int db = 0; db < kNarrowBlocks; ++db) out[db] = narrow_values(half, value[db], rest, out[db]);
+            }
             narrow_slot_read();
             if (t + 3u < count) {
                 if (((t + 3u) & 63u) == 0) ids = look_up(t + 3u);
@@ -311,7 +322,7 @@ SINGE_DEVICE void narrow_rows(const PagedAttentionArgs& a, unsigned char* lds, c
             merged.z = fmaf(weight, part.z, merged.z);
             merged.w = fmaf(weight, part.w, merged.w);
         }
-        const float inverse = total > 0.0f ? 1.0f / total : 0.0f;
+        const float inverse = (total > 0.0f ? 1.0f / total : 0.0f) * (WIDE ? 1.0f / kWideScale<Half> : 1.0f);
         merged.x *= inverse; merged.y *= inverse; merged.z *= inverse; merged.w *= inverse;
         finish(row, quad, merged, total > 0.0f ? largest + fast_log2(total) : -INFINITY);
     }

@@ -184,7 +184,7 @@ SINGE_DEVICE void decode_step_body(const PagedAttentionArgs& a, unsigned char* l
             if (a.lse != nullptr && quad == 0) a.lse[flat] = lse2;
         }
     };
-    narrow_rows<false, FORM, Half>(a, lds, span, kv_head, first_row, rows, key_begin, key_end, finish);
+    narrow_rows<false, FORM, true, Half>(a, lds, span, kv_head, first_row, rows, key_begin, key_end, finish);
     if (!shared) return;
 
     // Everything a share leaves is where the others see it before its word says so, and its word before it looks at theirs: of
