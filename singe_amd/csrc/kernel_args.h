@@ -187,7 +187,8 @@ struct PagedAttentionArgs {
     // Workgroups from this one on clear the rows of tokens that no attended sequence owns (clear_unowned_tokens); 0: none do.
     uint32_t clear_from = 0;
     // singe_paged_decode_step_*: row_tiles workgroups a kv head, each with sixteen rows of partial_out and two floats a row of
-    // partial_lse to itself, a word of share_done to say that they are written, and the launch's own number to say it with.
+    // partial_lse to itself, a word of share_done to say that they are written, and the launch's own number to say it with (null: units are not
+    // shared out).
     uint64_t* share_done = nullptr;
     uint64_t launch_number = 0;
 };

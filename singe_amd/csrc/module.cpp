@@ -413,12 +413,20 @@ const char* const kKernelNames[kKernelCount] = {
     "singe_fmha_prefill_bf16_d112_causal_window", "singe_fmha_prefill_f16_d112_causal_window",
     "singe_paged_decode_step_bf16_d128_i32", "singe_paged_decode_step_bf16_d128_i64",
     "singe_paged_decode_step_f16_d128_i32", "singe_paged_decode_step_f16_d128_i64",
+    "singe_paged_decode_step_bf16_d128_i32_w8", "singe_paged_decode_step_bf16_d128_i64_w8",
+    "singe_paged_decode_step_f16_d128_i32_w8", "singe_paged_decode_step_f16_d128_i64_w8",
     "singe_paged_decode_step_bf16_d64_i32", "singe_paged_decode_step_bf16_d64_i64",
     "singe_paged_decode_step_f16_d64_i32", "singe_paged_decode_step_f16_d64_i64",
+    "singe_paged_decode_step_bf16_d64_i32_w8", "singe_paged_decode_step_bf16_d64_i64_w8",
+    "singe_paged_decode_step_f16_d64_i32_w8", "singe_paged_decode_step_f16_d64_i64_w8",
     "singe_paged_decode_step_bf16_d32_i32", "singe_paged_decode_step_bf16_d32_i64",
     "singe_paged_decode_step_f16_d32_i32", "singe_paged_decode_step_f16_d32_i64",
+    "singe_paged_decode_step_bf16_d32_i32_w8", "singe_paged_decode_step_bf16_d32_i64_w8",
+    "singe_paged_decode_step_f16_d32_i32_w8", "singe_paged_decode_step_f16_d32_i64_w8",
     "singe_paged_decode_step_bf16_d96_i32", "singe_paged_decode_step_bf16_d96_i64",
     "singe_paged_decode_step_f16_d96_i32", "singe_paged_decode_step_f16_d96_i64",
+    "singe_paged_decode_step_bf16_d96_i32_w8", "singe_paged_decode_step_bf16_d96_i64_w8",
+    "singe_paged_decode_step_f16_d96_i32_w8", "singe_paged_decode_step_f16_d96_i64_w8",
 };
 
 // The code object is built in parts, one per kernel source (so they compile side by side and a process loads only
@@ -476,7 +484,7 @@ constexpr PartRun kPartRuns[] = {
     {52, 7},                      // dense f32 attention on the matrix cores
     {1, 4}, {14, 4}, {18, 4}, {20, 4}, {22, 4}, {24, 4}, {26, 4}, {28, 4},    // the dense prefill with two sets of waves to a tile
     {1, 2}, {14, 2}, {18, 2}, {20, 2}, {22, 2}, {24, 2}, {26, 2}, {28, 2},    // the dense prefill of short causal windows
-    {3, 4}, {15, 4}, {19, 4}, {21, 4},                                        // a decode step of the paged op in one launch
+    {3, 8}, {15, 8}, {19, 8}, {21, 8},                                        // a decode step of the paged op in one launch
 };
 constexpr int runs_total() {
     int total = 0;

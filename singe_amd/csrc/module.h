@@ -107,9 +107,9 @@ enum KernelId : int {
     kPrefillHalves = kAttentionMfmaF32 + 7,
     // the dense prefill of short causal windows over grouped heads: bf16, f16 for each head dimension in kRaggedPrefill's order
     kPrefillWindow = kPrefillHalves + 4 * 8,
-    // a decode step of the paged op in one launch: (i32, i64) + 2 * f16 for the head dimensions 128, 64, 32, 96
+    // a decode step of the paged op in one launch: (i32, i64) + 2 * f16 + 4 * (eight waves) for the head dimensions 128, 64, 32, 96
     kPagedStep = kPrefillWindow + 2 * 8,
-    kKernelCount = kPagedStep + 4 * 4
+    kKernelCount = kPagedStep + 8 * 4
 };
 
 // The two-tile kernels (fmha_prefill_pair.hip, paged_attention_pair.hip) have a build for every multiple of 16 up to 128.
@@ -187,8 +187,9 @@ inline int head_dim_order(long long head_dim) {
 // The dense prefill with two sets of waves to a tile for a head dimension, before 1 without the causal mask and 2 for f16.
 inline int prefill_halves_at(long long head_dim) { return kPrefillHalves + 4 * head_dim_order(head_dim); }
 
-// The decode-step kernel for a head dimension that is a multiple of 32, before 1 is added for i64 and 2 for f16.
-inline int paged_step_at(long long head_dim) { return kPagedStep + 4 * head_dim_order(head_dim); }
+// The decode-step kernel for a head dimension that is a multiple of 32, before 1 is added for i64, 2 for f16 and 4
+// for eight waves.
+inline int paged_step_at(long long head_dim) { return kPagedStep + 8 * head_dim_order(head_dim); }
 
 // The dense prefill of short causal windows for a head dimension, before 1 is added for f16.
 inline int prefill_window_at(long long head_dim) { return kPrefillWindow + 2 * head_dim_order(head_dim); }

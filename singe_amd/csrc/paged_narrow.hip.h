@@ -95,7 +95,7 @@ SINGE_DEVICE void narrow_slot_read() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "
 // a power of two of them.  finish(row, quad, values, lse2) takes values 4 quad .. of a row, normalised, and its base-two
 // log-sum-exp (a row that sees no key: zeros and -inf).  WIDE: the weights meet the values at f32's precision (split_pair), by a
 // second value product that the memory-bound loop has room for.
-template <bool SOFTCAP, int FORM, bool WIDE, class Half, class Finish>
+template <bool SOFTCAP, int FORM, bool WIDE, unsigned int WAVES, class Half, class Finish>
 SINGE_DEVICE void narrow_rows(const PagedAttentionArgs& a, unsigned char* lds, const SequenceSpan& span, unsigned int kv_head, unsigned int first_row,
                               unsigned int packed, unsigned int key_begin, unsigned int key_end, Finish&& finish) {
     const unsigned int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63u;
@@ -146,10 +146,10 @@ SINGE_DEVICE void narrow_rows(const PagedAttentionArgs& a, unsigned char* lds, c
     const unsigned int lds_start = static_cast<unsigned int>(reinterpret_cast<__UINTPTR_TYPE__>((lds_words_t)lds)) + wave * kNarrowWaveBytes;
     unsigned char* const ring = lds + wave * kNarrowWaveBytes;
 
-    // The wave's groups: key_begin / 16 + wave, and every fourth one from there.
+    // The wave's groups: key_begin / 16 + wave, and every WAVES-th one from there.
     const unsigned int first_group = key_begin / kNarrowKeys + wave, end_group = (key_end + kNarrowKeys - 1u) / kNarrowKeys;
-    const unsigned int count = __builtin_amdgcn_readfirstlane(first_group < end_group ? (end_group - first_group + 3u) / 4u : 0u);
-    auto key_of = [&](unsigned int t) __attribute__((always_inline)) { return (first_group + 4u * t) * kNarrowKeys; };
+    const unsigned int count = __builtin_amdgcn_readfirstlane(first_group < end_group ? (end_group - first_group + WAVES - 1u) / WAVES : 0u);
+    auto key_of = [&](unsigned int t) __attribute__((always_inline)) { return (first_group + WAVES * t) * kNarrowKeys; };
     // Page ids come 64 groups at a time, lane l that of group `first` + l, by a vector load: a scalar load would share its
     // counter with the LDS reads, which would then wait for it in every group.  An id outside the cache is reported and
     // replaced by page 0.
@@ -300,11 +300,11 @@ SINGE_DEVICE void narrow_rows(const PagedAttentionArgs& a, unsigned char* lds, c
         mine[kNarrowRows * kHeadDim + 2u * column + 1u] = sum;
     }
     __syncthreads();
-    for (unsigned int at = threadIdx.x; at < packed * (kHeadDim / 4u); at += 256u) {
+    for (unsigned int at = threadIdx.x; at < packed * (kHeadDim / 4u); at += 64u * WAVES) {
         const unsigned int row = at / (kHeadDim / 4u), quad = at % (kHeadDim / 4u);
-        float references[4], sums[4], largest = -INFINITY;
+        float references[WAVES], sums[WAVES], largest = -INFINITY;
 #pragma unroll
-        for (unsigned int w = 0; w < 4; ++w) {
+        for (unsigned int w = 0; w < WAVES; ++w) {
             const float* from = reinterpret_cast<const float*>(lds + w * kNarrowWaveBytes) + kNarrowRows * kHeadDim + 2u * row;
             references[w] = from[0];
             sums[w] = from[1];
@@ -313,7 +313,7 @@ SINGE_DEVICE void narrow_rows(const PagedAttentionArgs& a, unsigned char* lds, c
         float4 merged = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         float total = 0.0f;
 #pragma unroll
-        for (unsigned int w = 0; w < 4; ++w) {
+        for (unsigned int w = 0; w < WAVES; ++w) {
             const float weight = references[w] == -INFINITY ? 0.0f : fast_exp2(references[w] - largest);
             const float4 part = *reinterpret_cast<const float4*>(reinterpret_cast<const float*>(lds + w * kNarrowWaveBytes) + row * kHeadDim + 4u * quad);
             total = fmaf(weight, sums[w], total);

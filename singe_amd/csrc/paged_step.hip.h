@@ -9,8 +9,9 @@
 //
 // What bounds it is a chain of round trips to memory: the paging vectors, the page ids, the first keys, and where a unit is
 // shared out four more (its rows out, its word out, the words in, the rows in), some 5 us, which is what 8 to 9 tiles of keys take
-// one workgroup.  One token of 32 / 8 heads x 128, device time: 100 keys 6.4 us, 700 11, 3100 14.5, 32000 29 (three launches:
-// 11.3, 11.7, 13.6, 31); sixteen of 16 to 700 keys 13.5 (14.7).  The figures of whole calls stand at `decode_step_entries`.
+// a workgroup of four waves and twice as many one of eight.  One token of 32 / 8 heads x 128, device time: 100 keys 6.7 us, 800 11.4,
+// 3100 14.5, 32000 29 (three launches: 11.3, 11.7, 13.6, 31); sixteen of 16 to 700 keys 12.9 (14.7).  The figures of whole calls
+// stand at `decode_step_entries`.
 #pragma once
 
 #include "paged_locate.hip.h"
@@ -20,8 +21,8 @@ namespace {
 
 constexpr int kStepChunks = 4;                   // of 64 sequences
 constexpr unsigned int kStepMostShares = 64;     // of a unit
-constexpr unsigned int kStepLeastTiles = 4;      // of 64 keys to a share
-constexpr unsigned int kStepWholeTiles = 14;     // a unit of up to so many is not shared out
+// Tiles of 64 keys: the fewest of a share, and as many as a unit may have that is not shared out.
+constexpr unsigned int kStepLeastTiles = 4, kStepWholeTiles = 14;
 
 // A unit's share: rows 16 row_tile .. of the sequence, tiles [first_tile, end_tile) of its keys; `shares` neighbouring entries,
 // this one the `share`-th.
@@ -64,7 +65,7 @@ SINGE_DEVICE bool place_step(const PagedAttentionArgs& a, unsigned int entry, St
         }
     }
     unsigned int length = ~0u;
-    if (!__any(any_bad)) {
+    if (!__any(any_bad) && a.share_done != nullptr) {
         auto add = [](auto x, auto y) { return x + y; };
         const unsigned int all_units = across_wave(mine_units, add), longest = across_wave(mine_longest, [](unsigned int x, unsigned int y) { return x > y ? x : y; });
         const float all_tiles = across_wave(mine_tiles, add);
@@ -127,11 +128,12 @@ SINGE_DEVICE unsigned long long two_floats(float low, float high) {
 // Until this wave's own are where the others see them.
 SINGE_DEVICE void shared_stores_landed() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
-template <int FORM, class Half>
+template <int FORM, class Half, unsigned int WAVES>
 SINGE_DEVICE void decode_step_body(const PagedAttentionArgs& a, unsigned char* lds) {
+    constexpr unsigned int kThreads = 64u * WAVES;
     const unsigned int groups = a.heads / a.kv_heads, tid = threadIdx.x;
     if (blockIdx.x >= a.kv_heads * a.row_tiles) {
-        clear_unowned_tokens<FORM, 256, kNarrowRows>(reinterpret_cast<unsigned int*>(lds), 256u * (blockIdx.x - a.kv_heads * a.row_tiles), a.query_offsets,
+        clear_unowned_tokens<FORM, kThreads, kNarrowRows>(reinterpret_cast<unsigned int*>(lds), kThreads * (blockIdx.x - a.kv_heads * a.row_tiles), a.query_offsets,
                                                      a.page_offsets, a.last_page_lengths, a.tokens, a.sequences, a.page_table, a.page_size, groups,
                                                      a.row_tiles, a.output, a.heads * kHeadDim * 2u, a.lse, a.heads, a.status);
         return;
@@ -184,7 +186,7 @@ SINGE_DEVICE void decode_step_body(const PagedAttentionArgs& a, unsigned char* l
             if (a.lse != nullptr && quad == 0) a.lse[flat] = lse2;
         }
     };
-    narrow_rows<false, FORM, true, Half>(a, lds, span, kv_head, first_row, rows, key_begin, key_end, finish);
+    narrow_rows<false, FORM, true, WAVES, Half>(a, lds, span, kv_head, first_row, rows, key_begin, key_end, finish);
     if (!shared) return;
 
     // Everything a share leaves is where the others see it before its word says so, and its word before it looks at theirs: of
@@ -209,9 +211,9 @@ SINGE_DEVICE void decode_step_body(const PagedAttentionArgs& a, unsigned char* l
     constexpr unsigned int kQuads = kHeadDim / 4u, kAtOnce = 16;
     float* const weights = reinterpret_cast<float*>(lds) + 4;               // [rows][kStepMostShares]
     float* const row_lse = weights + kNarrowRows * kStepMostShares;         // [rows]
-    float4* const sums = reinterpret_cast<float4*>(row_lse + kNarrowRows);  // [256]
+    float4* const sums = reinterpret_cast<float4*>(row_lse + kNarrowRows);  // [kThreads]
     const unsigned int wave = tid >> 6, lane = tid & 63u, shares = place.shares, items = rows * kQuads;
-    const unsigned int turns = items >= 256u ? 1u : 256u / items, turn = items >= 256u ? 0u : tid / items;
+    const unsigned int turns = items >= kThreads ? 1u : kThreads / items, turn = items >= kThreads ? 0u : tid / items;
     const size_t stride = static_cast<size_t>(a.kv_heads) * kShareFloats;
     const float* const first_partial = a.partial_out + static_cast<size_t>(first_block) * kShareFloats;
     unsigned long long low[kAtOnce], high[kAtOnce];
@@ -239,9 +241,9 @@ SINGE_DEVICE void decode_step_body(const PagedAttentionArgs& a, unsigned char* l
         }
     };
     const bool working = turn < turns;
-    const unsigned int first_item = items >= 256u ? tid : tid - turn * items;
+    const unsigned int first_item = items >= kThreads ? tid : tid - turn * items;
     if (working) ask(first_item, turn);
-    for (unsigned int row = wave; row < rows; row += 4u) {
+    for (unsigned int row = wave; row < rows; row += WAVES) {
         const float mine = lane < shares ? __builtin_bit_cast(float, static_cast<unsigned int>(shared_load(
                                                a.partial_lse + static_cast<size_t>(first_block + lane * a.kv_heads) * (2u * kNarrowRows) + 2u * row)))
                                          : -INFINITY;
@@ -252,7 +254,7 @@ SINGE_DEVICE void decode_step_body(const PagedAttentionArgs& a, unsigned char* l
         if (lane == 0) row_lse[row] = total > 0.0f ? largest + fast_log2(total) : -INFINITY;
     }
     __syncthreads();
-    for (unsigned int item = first_item; item < items; item += 256u) {
+    for (unsigned int item = first_item; item < items; item += kThreads) {
         float4 merged = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         if (working) {
             if (item != first_item) ask(item, turn);
