@@ -509,6 +509,30 @@ SINGE_HIP_API int32_t singe_hip_paged_attention_every_row(
     void* scratch,
     size_t scratch_bytes,
     const SingePagedAttentionProblem* problem);
+
+/* The same call as one record, for callers to whom every argument across the boundary costs a conversion.  With
+ * `asks_scratch` set the scratch is what singe_hip_paged_attention_scratch_bytes asks for, or the call does nothing and returns
+ * SINGE_HIP_LENGTH_TOO_SHORT with that count as the error's minimum; otherwise it is whatever was lent, as above. */
+typedef struct SingePagedAttentionCall {
+    int64_t data_type;
+    void* stream;
+    const void* query_rows;
+    const void* key_cache;
+    const void* value_cache;
+    const void* query_offsets;
+    const void* page_offsets;
+    const void* pages;
+    const void* last_page_lengths;
+    void* output;
+    float* lse;
+    uint32_t* status;
+    void* scratch;
+    uint64_t scratch_bytes;
+    int64_t asks_scratch;
+    SingePagedAttentionProblem problem;
+} SingePagedAttentionCall;
+
+SINGE_HIP_API int32_t singe_hip_paged_attention_every_row_call(const SingePagedAttentionCall* call);
 SINGE_HIP_API int32_t singe_hip_paged_attention_scratch_bf16(
     void* stream,
     const uint16_t* query_rows,
@@ -1076,6 +1100,27 @@ SINGE_HIP_API int32_t singe_hip_rotary_cache_write(
     void* value_cache,
     uint32_t* status,
     const SingeRotaryCacheProblem* problem);
+
+/* The same call as one record. */
+typedef struct SingeRotaryCacheCall {
+    void* stream;
+    const void* query;
+    const void* key;
+    const void* value;
+    const void* cos;
+    const void* sin;
+    const void* page_index;
+    const void* slot_index;
+    const void* query_weight;
+    const void* key_weight;
+    void* query_out;
+    void* key_cache;
+    void* value_cache;
+    uint32_t* status;
+    SingeRotaryCacheProblem problem;
+} SingeRotaryCacheCall;
+
+SINGE_HIP_API int32_t singe_hip_rotary_cache_write_call(const SingeRotaryCacheCall* call);
 
 /* The kernel "paged_cudnn_indices" (kernel_plan/source/paged_attention.rs:325-398): FlashInfer CSR paging
  * -> block-table paging.  Writes packed_offsets [sequences + 1] (first element of each sequence's queries:

@@ -4,6 +4,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import struct
 
 from . import error
 
@@ -93,6 +94,13 @@ class PagedAttentionProblemC(ctypes.Structure):
                 ("causal", ctypes.c_uint8), ("has_scale", ctypes.c_uint8), ("has_window", ctypes.c_uint8),
                 ("has_softcap", ctypes.c_uint8), ("scale", ctypes.c_float), ("softcap", ctypes.c_float),
                 ("window", ctypes.c_int64)]
+
+
+# SingePagedAttentionCall and SingeRotaryCacheCall: packing one takes a third of the time that building the problem and
+# converting the call's other arguments one by one do.
+PAGED_ATTENTION_CALL = struct.Struct("@q12PQq8qi4Bffq")
+ROTARY_CACHE_CALL = struct.Struct("@14P6q3i2Bff")
+LENGTH_TOO_SHORT = 2
 
 
 class AttentionProblemC(ctypes.Structure):
@@ -332,6 +340,10 @@ def bind(path: str) -> ctypes.CDLL:
     handle.singe_hip_paged_attention_scratch_bf16.restype = i32
     handle.singe_hip_paged_attention_every_row.argtypes = [i32] + [c_void] * 12 + [ctypes.c_size_t, ctypes.POINTER(PagedAttentionProblemC)]
     handle.singe_hip_paged_attention_every_row.restype = i32
+    # (a packed record each, as bytes)
+    for name in ("singe_hip_paged_attention_every_row_call", "singe_hip_rotary_cache_write_call"):
+        getattr(handle, name).argtypes = [ctypes.c_char_p]
+        getattr(handle, name).restype = i32
     handle.singe_hip_paged_attention_scratch_bytes.argtypes = [ctypes.POINTER(PagedAttentionProblemC)]
     handle.singe_hip_paged_attention_scratch_bytes.restype = ctypes.c_size_t
     handle.singe_hip_set_paged_attention_splits.argtypes = [ctypes.c_uint32]

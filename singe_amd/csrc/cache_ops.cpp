@@ -90,6 +90,13 @@ extern "C" int32_t singe_hip_rotary_cache_write(void* stream, const void* query,
     return launch(static_cast<KernelId>(kRotaryCacheF32 + type_index), static_cast<unsigned>(blocks), 1, 1, 256, stream, args);
 }
 
+extern "C" int32_t singe_hip_rotary_cache_write_call(const SingeRotaryCacheCall* call) {
+    if (call == nullptr) return fail(SINGE_HIP_NULL_POINTER, "call");
+    const SingeRotaryCacheCall& c = *call;
+    return singe_hip_rotary_cache_write(c.stream, c.query, c.key, c.value, c.cos, c.sin, c.page_index, c.slot_index, c.query_weight, c.key_weight,
+                                        c.query_out, c.key_cache, c.value_cache, c.status, &c.problem);
+}
+
 extern "C" int32_t singe_hip_paging_indices(void* stream, const void* query_offsets, const void* page_offsets, const void* pages,
                                             const void* last_page_lengths, int32_t* packed_offsets, int32_t* query_lengths,
                                             int32_t* key_lengths, int32_t* page_table, uint32_t* status,

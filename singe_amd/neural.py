@@ -52,33 +52,44 @@ class Paging:
     last_page_lengths: torch.Tensor
 
 
-def _problem(query, key_cache, value_cache, paging: Paging, options: AttentionOptions):
-    """spec::paged_attention_problem (singe/src/backend/spec/neural/attention.rs:337-438)."""
-    if query.dim() != 3 or key_cache.dim() != 4:
+def _problem_fields(query, key_cache, value_cache, paging: Paging, options: AttentionOptions) -> tuple:
+    """spec::paged_attention_problem (singe/src/backend/spec/neural/attention.rs:337-438): the fields of the C record."""
+    shape, cache_shape = query.shape, key_cache.shape
+    if len(shape) != 3 or len(cache_shape) != 4:
         raise error.InvalidArgument("paged attention query or cache rank")
-    if key_cache.shape != value_cache.shape:
+    if cache_shape != value_cache.shape:
         raise error.InvalidArgument("paged attention value cache shape")
-    tokens, heads, head_dim = query.shape
-    cache_pages, page_size, kv_heads, key_dim = key_cache.shape
+    tokens, heads, head_dim = shape
+    cache_pages, page_size, kv_heads, key_dim = cache_shape
     if key_dim != head_dim or kv_heads <= 0 or heads % kv_heads != 0 or page_size <= 0:
         raise error.InvalidArgument("paged attention heads, head dimension, or page size")
-    indices = (paging.query_offsets, paging.page_offsets, paging.pages, paging.last_page_lengths)
-    kinds = {t.dtype for t in indices}
-    if not kinds <= {torch.int32, torch.int64}:
-        raise error.InvalidArgument("paged attention index type")
-    if len(kinds) != 1:
+    query_offsets, page_offsets, pages, last = paging.query_offsets, paging.page_offsets, paging.pages, paging.last_page_lengths
+    kind = pages.dtype
+    if not (kind is torch.int64 or kind is torch.int32) or query_offsets.dtype is not kind or page_offsets.dtype is not kind or last.dtype is not kind:
+        if not {t.dtype for t in (query_offsets, page_offsets, pages, last)} <= {torch.int32, torch.int64}:
+            raise error.InvalidArgument("paged attention index type")
         raise error.InvalidArgument("paged attention index tensors must share one type")
-    if any(t.dim() != 1 for t in indices):
+    if query_offsets.dim() != 1 or page_offsets.dim() != 1 or pages.dim() != 1 or last.dim() != 1:
         raise error.InvalidArgument("paged attention index rank")
-    sequences = paging.last_page_lengths.numel()
-    if paging.query_offsets.numel() != sequences + 1 or paging.page_offsets.numel() != sequences + 1:
+    sequences = last.shape[0]
+    if query_offsets.shape[0] != sequences + 1 or page_offsets.shape[0] != sequences + 1:
         raise error.InvalidArgument("paged attention offset count")
-    return _native.PagedAttentionProblemC(
-        tokens, heads, kv_heads, head_dim, page_size, sequences, cache_pages, paging.pages.numel(),
-        1 if paging.pages.dtype == torch.int64 else 0, 1 if options.causal else 0,
-        1 if options.scale is not None else 0, 1 if options.window is not None else 0,
-        1 if options.softcap is not None else 0, options.scale if options.scale is not None else 0.0,
-        options.softcap if options.softcap is not None else 0.0, options.window if options.window is not None else 0)
+    scale, window, softcap = options.scale, options.window, options.softcap
+    return (tokens, heads, kv_heads, head_dim, page_size, sequences, cache_pages, pages.shape[0], 1 if kind is torch.int64 else 0,
+            1 if options.causal else 0, 0 if scale is None else 1, 0 if window is None else 1, 0 if softcap is None else 1,
+            0.0 if scale is None else ctypes.c_float(scale).value, 0.0 if softcap is None else ctypes.c_float(softcap).value,
+            0 if window is None else ctypes.c_int64(window).value)
+
+
+def _problem(query, key_cache, value_cache, paging: Paging, options: AttentionOptions):
+    return _native.PagedAttentionProblemC(*_problem_fields(query, key_cache, value_cache, paging, options))
+
+
+def _same_device_tensors(kind, *tensors) -> bool:
+    for tensor in tensors:
+        if not tensor.is_cuda or tensor.dtype is not kind or not tensor.is_contiguous():
+            return False
+    return True
 
 
 _DATA_TYPES = {torch.float32: _native.DATA_TYPE_F32, torch.bfloat16: _native.DATA_TYPE_BF16,
@@ -260,47 +271,53 @@ def paged_attention(query: torch.Tensor, key_cache: torch.Tensor, value_cache: t
     back: a paging value outside its buffers raises IndexOutOfBounds.  ``check=False`` skips the
     read-back (and the synchronisation it implies); pass ``status`` to inspect the word yourself.
     """
-    for tensor, name in ((query, "query"), (key_cache, "key_cache"), (value_cache, "value_cache")):
-        if not tensor.is_cuda or tensor.dtype != query.dtype or not tensor.is_contiguous():
-            raise error.InvalidArgument(f"paged attention {name} must be a contiguous device tensor of the query's type")
-    if query.dtype not in _ATTENTION_TYPES:
-        raise error.InvalidArgument(f"paged attention data type {query.dtype}")
-    for tensor in (paging.query_offsets, paging.page_offsets, paging.pages, paging.last_page_lengths):
+    kind = query.dtype
+    if not _same_device_tensors(kind, query, key_cache, value_cache):
+        for tensor, name in ((query, "query"), (key_cache, "key_cache"), (value_cache, "value_cache")):
+            if not _same_device_tensors(kind, tensor):
+                raise error.InvalidArgument(f"paged attention {name} must be a contiguous device tensor of the query's type")
+    if kind not in _ATTENTION_TYPES:
+        raise error.InvalidArgument(f"paged attention data type {kind}")
+    query_offsets, page_offsets, pages, last = paging.query_offsets, paging.page_offsets, paging.pages, paging.last_page_lengths
+    for tensor in (query_offsets, page_offsets, pages, last):
         if not tensor.is_cuda or not tensor.is_contiguous():
             raise error.InvalidArgument("paged attention index tensors must be contiguous device tensors")
-    problem = _problem(query, key_cache, value_cache, paging, options)
+    fields = _problem_fields(query, key_cache, value_cache, paging, options)
+    tokens, heads, _, head_dim, _, sequences = fields[:6]
     # The matrix-core kernels write every row, those of tokens that no sequence owns included; the others leave such rows
     # alone, so their outputs are filled first.
-    sixteen_bit = query.dtype in (torch.bfloat16, torch.float16)
-    every_row = sixteen_bit and query.shape[2] % 16 == 0 and query.shape[2] <= 128 and problem.sequences > 0
+    every_row = (kind is torch.bfloat16 or kind is torch.float16) and head_dim % 16 == 0 and head_dim <= 128 and sequences > 0
     if every_row:
         output = torch.empty_like(query)
-        lse = torch.empty(query.shape[:2], device=query.device, dtype=torch.float32)
+        lse = torch.empty((tokens, heads), device=query.device, dtype=torch.float32)
     else:
         output = torch.zeros_like(query)
-        lse = torch.full(query.shape[:2], float("-inf"), device=query.device, dtype=torch.float32)
+        lse = torch.full((tokens, heads), float("-inf"), device=query.device, dtype=torch.float32)
     if status is None:
         status = torch.zeros(1, device=query.device, dtype=torch.int32)
-    handle = _stream_handle(stream)
-    # 16-bit calls with few query rows (decoding) share a row tile's keys out over several workgroups, given
-    # scratch: ``scratch`` is a uint8 device tensor, True for this module's own per-device buffer (calls on
-    # different streams must then not overlap), or False for none.
-    wanted = 0
-    if sixteen_bit and scratch is not False:
-        wanted = int(_native.lib().singe_hip_paged_attention_scratch_bytes(ctypes.byref(problem)))
-    lent = None if wanted == 0 else _scratch_for(query.device, wanted) if scratch is True else scratch
-    operands = (handle, query.data_ptr(), key_cache.data_ptr(), value_cache.data_ptr(), paging.query_offsets.data_ptr(),
-                paging.page_offsets.data_ptr(), paging.pages.data_ptr(), paging.last_page_lengths.data_ptr(), output.data_ptr(),
-                lse.data_ptr(), status.data_ptr())
-    scratch_operands = (0, 0) if lent is None else (lent.data_ptr(), lent.numel())
+    operands = (_stream_handle(stream), query.data_ptr(), key_cache.data_ptr(), value_cache.data_ptr(), query_offsets.data_ptr(), page_offsets.data_ptr(),
+                pages.data_ptr(), last.data_ptr(), output.data_ptr(), lse.data_ptr(), status.data_ptr())
     if every_row:
-        code = _native.lib().singe_hip_paged_attention_every_row(_ATTENTION_TYPES[query.dtype], *operands, *scratch_operands, ctypes.byref(problem))
+        # Calls with few query rows (decoding) share a row tile's keys out over several workgroups, given scratch: ``scratch`` is a
+        # uint8 device tensor, True for this module's own per-device buffer (calls on different streams must then not
+        # overlap), or False for none.
+        asks = scratch is True
+        lent = _scratch.get(query.device) if asks else None if scratch is False else scratch
+        while True:
+            code = _native.lib().singe_hip_paged_attention_every_row_call(_native.PAGED_ATTENTION_CALL.pack(
+                _ATTENTION_TYPES[kind], *operands, 0 if lent is None else lent.data_ptr(), 0 if lent is None else lent.numel(), 1 if asks else 0, *fields))
+            if code != _native.LENGTH_TOO_SHORT or not asks:
+                break
+            wanted = int(_native.lib().singe_hip_paged_attention_scratch_bytes(ctypes.byref(_native.PagedAttentionProblemC(*fields))))
+            if lent is not None and lent.numel() >= wanted:
+                break
+            lent = _scratch_for(query.device, wanted)
     else:
         entry = {torch.bfloat16: _native.lib().singe_hip_paged_attention_bf16,
                  torch.float32: _native.lib().singe_hip_paged_attention_f32,
                  torch.float64: _native.lib().singe_hip_paged_attention_f64,
-                 torch.float16: _native.lib().singe_hip_paged_attention_f16}[query.dtype]
-        code = entry(*operands, ctypes.byref(problem))
+                 torch.float16: _native.lib().singe_hip_paged_attention_f16}[kind]
+        code = entry(*operands, ctypes.byref(_native.PagedAttentionProblemC(*fields)))
     _native.check(code, "paged_attention")
     if check and int(status.item()) == STATUS_INDEX_OUT_OF_BOUNDS:
         raise error.IndexOutOfBounds("paged attention paging value outside its buffers")
@@ -438,45 +455,47 @@ def rotary_cache_write(query, key, value, cos, sin, pages, slots, key_cache, val
     and ``key`` [T, G, D] by the angles ``cos`` / ``sin`` [T, D/2] (half-split pairs), and writes the rotated
     keys and ``value`` [T, G, D] into the caches [P, S, G, D] at (pages[t], slots[t]), in place.  Returns the
     rotated queries (None without a query).  A page or slot outside the cache raises IndexOutOfBounds."""
-    tensors = [(key, "key"), (value, "value"), (key_cache, "key_cache"), (value_cache, "value_cache")]
-    if query is not None:
-        tensors.append((query, "query"))
-    for tensor, name in tensors:
-        if not tensor.is_cuda or tensor.dtype != key.dtype or not tensor.is_contiguous():
-            raise error.InvalidArgument(f"rotary cache {name} must be a contiguous device tensor of the key's type")
-    if key.dtype not in _DATA_TYPES or cos.dtype not in _DATA_TYPES or sin.dtype != cos.dtype:
+    kind = key.dtype
+    if not _same_device_tensors(kind, key, value, key_cache, value_cache) or not (query is None or _same_device_tensors(kind, query)):
+        for tensor, name in ((key, "key"), (value, "value"), (key_cache, "key_cache"), (value_cache, "value_cache"), (query, "query")):
+            if tensor is not None and not _same_device_tensors(kind, tensor):
+                raise error.InvalidArgument(f"rotary cache {name} must be a contiguous device tensor of the key's type")
+    if kind not in _DATA_TYPES or cos.dtype not in _DATA_TYPES or sin.dtype != cos.dtype:
         raise error.InvalidArgument("rotary cache data type")
-    tokens, cache_heads, head_dim = key.shape
-    if value.shape != key.shape or key_cache.shape != value_cache.shape or key_cache.dim() != 4:
+    tokens, cache_heads, head_dim = shape = key.shape
+    cache_shape = key_cache.shape
+    if value.shape != shape or cache_shape != value_cache.shape or len(cache_shape) != 4:
         raise error.InvalidArgument("rotary cache value or cache shape")
-    cache_pages, page_slots = key_cache.shape[:2]
-    if tuple(key_cache.shape[2:]) != (cache_heads, head_dim):
+    cache_pages, page_slots, cached_heads, cached_dim = cache_shape
+    if cached_heads != cache_heads or cached_dim != head_dim:
         raise error.InvalidArgument("rotary cache heads or head dimension")
     cos, sin = cos.contiguous(), sin.contiguous()
     if cos.numel() != tokens * (head_dim // 2) or sin.numel() != cos.numel():
         raise error.InvalidArgument("rotary cache angles must be [tokens, 1, head_dim / 2]")
     if pages.dtype != slots.dtype or pages.dtype not in (torch.int32, torch.int64) or pages.numel() != tokens or slots.numel() != tokens:
         raise error.InvalidArgument("rotary cache pages and slots must be [tokens] of one integer type")
-    query_heads = 0 if query is None else query.shape[1]
+    pages, slots = pages.contiguous(), slots.contiguous()
     query_out = None if query is None else torch.empty_like(query)
     weights = []
     for norm in (query_norm, key_norm):
-        weight = None if norm is None or norm.weight is None else norm.weight.to(key.dtype).contiguous()
-        if weight is not None and weight.numel() != head_dim:
-            raise error.InvalidArgument("rotary cache norm weight must hold head_dim values")
+        weight = None if norm is None else norm.weight
+        if weight is not None:
+            if weight.dtype is not kind:
+                weight = weight.to(kind)
+            weight = weight.contiguous()
+            if weight.numel() != head_dim:
+                raise error.InvalidArgument("rotary cache norm weight must hold head_dim values")
         weights.append(weight)
-    problem = _native.RotaryCacheProblemC(
-        tokens, query_heads, cache_heads, head_dim, cache_pages, page_slots, _DATA_TYPES[key.dtype], _DATA_TYPES[cos.dtype],
-        1 if pages.dtype == torch.int64 else 0, 1 if query_norm is not None else 0, 1 if key_norm is not None else 0,
-        query_norm.eps if query_norm is not None else 0.0, key_norm.eps if key_norm is not None else 0.0)
     if status is None:
         status = torch.zeros(1, device=key.device, dtype=torch.int32)
-    pointer = lambda tensor: tensor.data_ptr() if tensor is not None else None
-    handle = _stream_handle(stream)
-    code = _native.lib().singe_hip_rotary_cache_write(
-        handle, pointer(query), key.data_ptr(), value.data_ptr(), cos.data_ptr(), sin.data_ptr(), pages.contiguous().data_ptr(),
-        slots.contiguous().data_ptr(), pointer(weights[0]), pointer(weights[1]), pointer(query_out), key_cache.data_ptr(),
-        value_cache.data_ptr(), status.data_ptr(), ctypes.byref(problem))
+    query_weight, key_weight = weights
+    code = _native.lib().singe_hip_rotary_cache_write_call(_native.ROTARY_CACHE_CALL.pack(
+        _stream_handle(stream), 0 if query is None else query.data_ptr(), key.data_ptr(), value.data_ptr(), cos.data_ptr(), sin.data_ptr(),
+        pages.data_ptr(), slots.data_ptr(), 0 if query_weight is None else query_weight.data_ptr(), 0 if key_weight is None else key_weight.data_ptr(),
+        0 if query is None else query_out.data_ptr(), key_cache.data_ptr(), value_cache.data_ptr(), status.data_ptr(),
+        tokens, 0 if query is None else query.shape[1], cache_heads, head_dim, cache_pages, page_slots, _DATA_TYPES[kind], _DATA_TYPES[cos.dtype],
+        1 if pages.dtype is torch.int64 else 0, 0 if query_norm is None else 1, 0 if key_norm is None else 1,
+        0.0 if query_norm is None else ctypes.c_float(query_norm.eps).value, 0.0 if key_norm is None else ctypes.c_float(key_norm.eps).value))
     _native.check(code, "rotary_cache_write")
     if check and int(status.item()) == STATUS_INDEX_OUT_OF_BOUNDS:
         raise error.IndexOutOfBounds("rotary cache page or slot outside the cache")
