@@ -389,10 +389,26 @@ int32_t prefill(void* stream, uint16_t* out, size_t out_len, float* lse, size_t 
     // A decode step through the dense op (few query rows, grouped heads, no causal mask): the query heads of a kv head
     // share one tile, so its keys and values are fetched once.
     args.packed_heads = dense_prefill_packs_heads(c) ? 1u : 0u;
-    const uint64_t rows = (static_cast<uint64_t>(c.batch) * (args.packed_heads ? c.kv_heads : c.heads) + 7) / 8 * 8;
+    const uint64_t rows = static_cast<uint64_t>(c.batch) * (args.packed_heads ? c.kv_heads : c.heads);
     const DenseShares shares = dense_prefill_shares(c);
     args.single_tiles = shares.single_tiles ? 1u : 0u;
-    uint64_t groups = rows * (shares.single_tiles ? args.query_tiles : (args.query_tiles + 1) / 2);
+    // Whole (batch, head)s to an XCD leave some of them with one more than others where those are no multiple of eight, and such an
+    // XCD's compute units with a workgroup more: so every XCD gets an eighth of the tiles.  Batch entries of their own key counts
+    // are dealt so only up to a tile a compute unit; up to three, long ones go by their lengths, and the rest by whole (batch,
+    // head)s as they come (by length 16 x 8 heads x 300 takes 11.6 us, as they come 10.2; 16 x 12 x 1500 122 and 118).  us, whole
+    // (batch, head)s / now, head_dim 64 where not said:
+    //   no lengths   1 x 6 heads x 1500  20.4 / 18.0   3 x 6  36 / 19.4   7 x 6  42 / 32.7   8 x 6  42.6 / 42.8
+    //                causal 1 x 28 / 4 x 4096 x 128 (two tiles a wave)  124 / 114   1 x 28 / 4 x 4096 x 96  104 / 100   3 x 28 / 4 x 1500 x 96,
+    //                no mask  114 / 85   causal 2 x 32 / 8 x 2048 x 128  76 / 71 (query heads that share keys share an XCD's L2)
+    //   lengths of half the keys to all of them   1 x 6 x 1500  16.8 / 14.9   3 x 6  29.4 / 19.5   4 x 6  28.7 / 25.8   5 x 6  29.2 / 26.4
+    //                7 x 6  36.4 / 31.4   8 x 6  37.4 / 32.1   9 x 6  38.8 / 34.7   10 x 6  40.8 / 39.1   5 x 12 x 700  17.1 / 15.9
+    const uint64_t units = rows * (shares.single_tiles ? args.query_tiles : (args.query_tiles + 1) / 2);
+    args.deal = kDealEvenly;
+    if (options.key_lengths != nullptr && units > compute_units())
+        args.deal = !c.causal && args.single_tiles != 0 && args.packed_heads == 0 && c.batch <= 64 && c.key_len >= 512 && units <= 3 * compute_units()
+                        ? kDealByLength : kDealWhole;
+    auto dealt = [&](uint64_t each) { return args.deal == kDealEvenly ? (rows * each + 7) / 8 * 8 : (rows + 7) / 8 * 8 * each; };  // workgroups, `each` to a row
+    uint64_t groups = dealt(shares.single_tiles ? args.query_tiles : (args.query_tiles + 1) / 2);
     if (groups > 0x7fffffffull) return fail(SINGE_HIP_UNSUPPORTED_CONFIGURATION, "too many workgroups");
     // Key splits, when the caller lent scratch for them and the launch is too small to fill the chip.
     uint32_t splits = options.scratch != nullptr ? shares.splits : 1;
@@ -423,8 +439,9 @@ int32_t prefill(void* stream, uint16_t* out, size_t out_len, float* lse, size_t 
     // key tile is not whole.
     if (!with_options && splits == 1 && two_tiles_a_wave(c)) {
         const uint32_t pair_tiles = static_cast<uint32_t>((c.query_len + 255) / 256);
-        const uint64_t pair_groups = rows * ((pair_tiles + 1) / 2);
         args.query_tiles = pair_tiles;
+        args.deal = options.key_lengths != nullptr ? kDealWhole : kDealEvenly;
+        const uint64_t pair_groups = dealt((pair_tiles + 1) / 2);
         // (the builds that take a last tile that is not whole also take a key count of their own for every batch entry)
         const bool ragged = c.key_len % 64 != 0 || options.key_lengths != nullptr;
         const KernelId pair = static_cast<KernelId>(pair_kernels_at(static_cast<long long>(c.head_dim), false) + (c.causal ? 0 : 1) + (f16 ? 2 : 0) + (ragged ? 4 : 0));

@@ -484,6 +484,45 @@ SINGE_DEVICE void fmha_prefill_tile(const PrefillArgs& a, unsigned char* lds, un
     }
 }
 
+// The `within`-th workgroup of an XCD -> (batch, head) `bh` and which of its `pairs` of query tiles (see kDeal...); false: none.
+// By length: the dispatcher fills an XCD's 32 compute units one after the other, round after round, and those at the front of an
+// incomplete last round take one workgroup more than the rest.  They get the shortest, the others the longest, and both change
+// direction from round to round so that a compute unit's sum is about the same.
+SINGE_DEVICE bool deal_units(const PrefillArgs& a, unsigned int heads, unsigned int pairs, unsigned int xcd, unsigned int& within, unsigned int& bh) {
+    constexpr unsigned int kUnitsOfXcd = 32;
+    const unsigned int all = a.batch * heads;
+    if (a.deal == kDealEvenly) {
+        const unsigned int units = pairs * all, per_xcd = (units + 7u) / 8u, unit = xcd * per_xcd + within;
+        if (within >= per_xcd || unit >= units) return false;
+        bh = unit / pairs;
+        within = unit - bh * pairs;
+        if (a.key_lengths != nullptr) bh = bh % a.batch * heads + bh / a.batch;
+        return true;
+    }
+    const unsigned int count = (all + 7u - xcd) / 8u * pairs;
+    if (within >= count) return false;
+    if (a.deal == kDealWhole) {
+        bh = within / pairs * 8u + xcd;
+        within %= pairs;
+        return true;
+    }
+    const unsigned int lane = threadIdx.x & 63u;
+    const int keys = lane < a.batch ? a.key_lengths[lane] : 0;
+    unsigned int longer = lane < a.batch ? 0u : ~0u;  // batch entries before the lane's, by length
+    for (unsigned int b = 0; b < a.batch; ++b) {
+        const int others = __builtin_amdgcn_readlane(keys, b);
+        if (lane < a.batch && (others > keys || (others == keys && b < lane))) ++longer;
+    }
+    const unsigned int rounds = count / kUnitsOfXcd, first = count % kUnitsOfXcd, unit = within % kUnitsOfXcd, round = within / kUnitsOfXcd;
+    unsigned int rank = within;
+    if (rounds > 0 && unit < first) rank = count - first * (rounds + 1u) + round * first + (round % 2u != 0 ? first - 1u - unit : unit);
+    else if (rounds > 0) rank = round * (kUnitsOfXcd - first) + (round % 2u != 0 ? kUnitsOfXcd - 1u - unit : unit - first);
+    const unsigned int position = rank / pairs * 8u + xcd, batch = position / heads;
+    within = rank % pairs;
+    bh = static_cast<unsigned int>(__builtin_ctzll(__ballot(longer == batch))) * heads + position % heads;
+    return true;
+}
+
 // Workgroup id -> (batch * heads + head, pair of query tiles): see the header comment.
 template <bool CAUSAL, class Half, int WAVES, bool OPTIONS = false, int HALVES = 1>
 SINGE_DEVICE void fmha_prefill_body(const PrefillArgs& a, unsigned char* lds) {
@@ -505,10 +544,9 @@ SINGE_DEVICE void fmha_prefill_body(const PrefillArgs& a, unsigned char* lds) {
         split = within % a.splits;  // the shares of a query tile are neighbours
         within /= a.splits;
         const unsigned int pairs = a.single_tiles != 0 ? a.query_tiles : (a.query_tiles + 1u) / 2u;
-        bh = (within / pairs) * 8u + xcd;
-        if (bh >= a.batch * (a.packed_heads != 0 ? a.kv_heads : a.heads)) return;
-        heavy = a.query_tiles - 1u - within % pairs;
-        light = a.single_tiles != 0 ? heavy : within % pairs;
+        if (!deal_units(a, a.packed_heads != 0 ? a.kv_heads : a.heads, pairs, xcd, within, bh)) return;
+        heavy = a.query_tiles - 1u - within;
+        light = a.single_tiles != 0 ? heavy : within;
     }
     fmha_prefill_tile<CAUSAL, Half, WAVES, OPTIONS, HALVES>(a, lds, bh, heavy, split);
     if (HALVES == 1 && light != heavy) fmha_prefill_tile<CAUSAL, Half, WAVES, OPTIONS, HALVES>(a, lds, bh, light, split);

@@ -307,10 +307,19 @@ SINGE_DEVICE void fmha_prefill_pair_tile(const PrefillArgs& a, unsigned char* ld
 template <bool CAUSAL, bool RAGGED, class Half>
 SINGE_DEVICE void fmha_prefill_pair_body(const PrefillArgs& a, unsigned char* lds) {
     const unsigned int xcd = blockIdx.x & 7u, within = blockIdx.x >> 3;
-    const unsigned int pairs = (a.query_tiles + 1u) / 2u;
-    const unsigned int bh = (within / pairs) * 8u + xcd;
-    if (bh >= a.batch * a.heads) return;
-    const unsigned int light = within % pairs, heavy = a.query_tiles - 1u - light;
+    const unsigned int pairs = (a.query_tiles + 1u) / 2u, all = a.batch * a.heads;
+    unsigned int bh, light;
+    if (a.deal == kDealEvenly) {
+        const unsigned int units = pairs * all, per_xcd = (units + 7u) / 8u, unit = xcd * per_xcd + within;
+        if (within >= per_xcd || unit >= units) return;
+        bh = unit / pairs;
+        light = unit - bh * pairs;
+    } else {
+        bh = within / pairs * 8u + xcd;
+        light = within % pairs;
+        if (bh >= all) return;
+    }
+    const unsigned int heavy = a.query_tiles - 1u - light;
     // (one copy of the tile's code for both tiles: written out per stage it is long, and two copies of it would not fit
     // the instruction cache)
 #pragma nounroll

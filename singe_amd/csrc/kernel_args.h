@@ -59,6 +59,13 @@ constexpr int kDensePrefillWaves = 4;
 // Waves of a workgroup of the kernel for short causal windows, 32 (query, head) rows of a step each.
 constexpr int kWindowPrefillWaves = 8;
 
+// How the dense kernels deal the (batch, head)s' query tiles, `units` of them (pairs without single_tiles), to the XCDs:
+//   kDealEvenly     an eighth of all units to each, side by side; batch entries of their own key counts take turns
+//   kDealWhole      every eighth (batch, head)
+//   kDealByLength   every eighth (batch, head), the batch entries with the most keys first, and inside an XCD so that a compute
+//                   unit that takes a workgroup more than others takes short ones (32-row kernels, 64 batch entries at most)
+enum : uint32_t { kDealEvenly = 0, kDealWhole = 1, kDealByLength = 2 };
+
 struct PrefillArgs {
     const uint16_t* query;          // [batch, query_len, heads, 128] bf16, element strides below
     const uint16_t* key;            // [batch, key_len, kv_heads, 128]
@@ -105,6 +112,8 @@ struct PrefillArgs {
     uint32_t packed_heads = 0;
     // With single_tiles != 0 a workgroup takes one query tile instead of two (32-row kernels).
     uint32_t single_tiles = 0;
+    // How workgroups go to the XCDs (kDeal...).
+    uint32_t deal = 0;
     // The *_window kernels: a workgroup takes run_steps steps of 32 * kWindowPrefillWaves (query, head) rows of a (batch, kv
     // head) pair, query_tiles such runs to a pair, with ring_blocks blocks of 32 keys in LDS.
     uint32_t run_steps = 0, ring_blocks = 0;

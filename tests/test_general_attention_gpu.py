@@ -510,3 +510,24 @@ def test_scores_that_outgrow_a_share_s_reference_point(heads, length, causal, dt
     out = neural.scaled_dot_product_attention(q, k, v, causal=causal)
     want = oracle.scaled_dot_product_attention_f32(host(q), host(k), host(v), causal=causal, threads=8)
     close(host(out), want, dtype)
+
+
+@pytest.mark.parametrize("batch,heads,kv_heads,length,dim,lengths", [
+    (9, 6, 6, 640, 64, [640, 0, 5, 320, 320, 639, 1, 64, 500]),     # by length: 270 tiles, of entries without keys and of equal lengths too
+    (3, 43, 43, 300, 32, [300, 299, 20]),                           # as many tiles, short keys: whole (batch, head)s
+    (64, 3, 1, 520, 16, [(37 * b) % 521 for b in range(64)]),       # as many entries as a wave has lanes: 960 tiles, past three a compute unit
+    (64, 2, 2, 515, 48, [(37 * b) % 516 for b in range(64)]),       # ... and 640
+    (3, 6, 2, 777, 64, [777, 100, 400]),                            # a tile a compute unit at most: an eighth of them to an XCD
+    (5, 7, 7, 260, 128, None),                                      # 105 tiles over eight XCDs
+])
+@pytest.mark.parametrize("causal", [False, True])
+def test_query_tiles_dealt_to_the_xcds_cover_every_row(batch, heads, kv_heads, length, dim, lengths, causal):
+    q, k, v = tensors((batch, heads, length, dim), (batch, kv_heads, length, dim), (batch, kv_heads, length, dim), torch.bfloat16, length)
+    options = neural.AttentionOptions(causal=causal)
+    torch.full_like(q, float("nan"))  # (what the output's memory holds before: a row that is not written shows)
+    if lengths is None:
+        out = neural.attend(q, k, v, options=options)
+    else:
+        out = neural.attend_padded(q, k, v, torch.tensor(lengths, device="cuda", dtype=torch.int32), options)
+    want = oracle.scaled_dot_product_attention_f32(host(q), host(k), host(v), causal=causal, key_lengths=lengths, threads=8)
+    close(host(out), want, torch.bfloat16)
