@@ -94,7 +94,8 @@ SINGE_DEVICE void narrow_slot_read() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "
 // of sixteen, but for the end), of which a row sees what its position and the window leave it.  Pages of at least sixteen keys,
 // a power of two of them.  finish(row, quad, values, lse2) takes values 4 quad .. of a row, normalised, and its base-two
 // log-sum-exp (a row that sees no key: zeros and -inf).  WIDE: the weights meet the values at f32's precision (split_pair), by a
-// second value product that the memory-bound loop has room for.
+// second value product that the memory-bound loop has room for, and a row with a score that is NaN or +inf has a log-sum-exp of
+// NaN beside its values, so that whoever merges it with others can tell it from a row that sees no key.
 template <bool SOFTCAP, int FORM, bool WIDE, unsigned int WAVES, class Half, class Finish>
 SINGE_DEVICE void narrow_rows(const PagedAttentionArgs& a, unsigned char* lds, const SequenceSpan& span, unsigned int kv_head, unsigned int first_row,
                               unsigned int packed, unsigned int key_begin, unsigned int key_end, Finish&& finish) {
@@ -324,7 +325,9 @@ SINGE_DEVICE void narrow_rows(const PagedAttentionArgs& a, unsigned char* lds, c
         }
         const float inverse = (total > 0.0f ? 1.0f / total : 0.0f) * (WIDE ? 1.0f / kWideScale<Half> : 1.0f);
         merged.x *= inverse; merged.y *= inverse; merged.z *= inverse; merged.w *= inverse;
-        finish(row, quad, merged, total > 0.0f ? largest + fast_log2(total) : -INFINITY);
+        float lse2 = total > 0.0f ? largest + fast_log2(total) : -INFINITY;
+        if (WIDE && total != total) lse2 = total;
+        finish(row, quad, merged, lse2);
     }
 }
 

@@ -206,9 +206,11 @@ SINGE_DEVICE void decode_step_body(const PagedAttentionArgs& a, unsigned char* l
     __syncthreads();
     if (reinterpret_cast<unsigned int*>(lds)[0] == 0u) return;
     // Each share's rows weigh 2^(lse - largest) over the sum of those.  A row's values are asked for before the weights are
-    // worked out, sixteen shares a thread, and where the rows leave threads over, several take turns at a row's shares; past the
-    // last share it stands in with a weight of zero, and what a share that weighs nothing holds is not used.
+    // worked out, sixteen shares a thread, and where the rows leave threads over, several take turns at a row's shares.  What a
+    // share that sees no key of the row holds is not used (its weight is kNoWeight, and past the last share too); a log-sum-exp
+    // that is NaN makes the row NaN.
     constexpr unsigned int kQuads = kHeadDim / 4u, kAtOnce = 16;
+    constexpr float kNoWeight = -1.0f;
     float* const weights = reinterpret_cast<float*>(lds) + 4;               // [rows][kStepMostShares]
     float* const row_lse = weights + kNarrowRows * kStepMostShares;         // [rows]
     float4* const sums = reinterpret_cast<float4*>(row_lse + kNarrowRows);  // [kThreads]
@@ -232,12 +234,12 @@ SINGE_DEVICE void decode_step_body(const PagedAttentionArgs& a, unsigned char* l
 #pragma unroll
         for (unsigned int i = 0; i < kAtOnce; ++i) {
             const unsigned int s = from_share + i * turns;
-            const float w = s < shares ? weights[(item / kQuads) * kStepMostShares + s] : 0.0f;
+            const float w = s < shares ? weights[(item / kQuads) * kStepMostShares + s] : kNoWeight;
             auto part = [&](unsigned long long bits) __attribute__((always_inline)) { return __builtin_bit_cast(float, static_cast<unsigned int>(bits)); };
-            merged.x = w == 0.0f ? merged.x : fmaf(w, part(low[i]), merged.x);
-            merged.y = w == 0.0f ? merged.y : fmaf(w, part(low[i] >> 32), merged.y);
-            merged.z = w == 0.0f ? merged.z : fmaf(w, part(high[i]), merged.z);
-            merged.w = w == 0.0f ? merged.w : fmaf(w, part(high[i] >> 32), merged.w);
+            merged.x = w == kNoWeight ? merged.x : fmaf(w, part(low[i]), merged.x);
+            merged.y = w == kNoWeight ? merged.y : fmaf(w, part(low[i] >> 32), merged.y);
+            merged.z = w == kNoWeight ? merged.z : fmaf(w, part(high[i]), merged.z);
+            merged.w = w == kNoWeight ? merged.w : fmaf(w, part(high[i] >> 32), merged.w);
         }
     };
     const bool working = turn < turns;
@@ -248,10 +250,10 @@ SINGE_DEVICE void decode_step_body(const PagedAttentionArgs& a, unsigned char* l
                                                a.partial_lse + static_cast<size_t>(first_block + lane * a.kv_heads) * (2u * kNarrowRows) + 2u * row)))
                                          : -INFINITY;
         const float largest = across_wave(mine, [](float x, float y) { return fmaxf(x, y); });
-        const float weight = mine == -INFINITY ? 0.0f : fast_exp2(mine - largest);  // an empty share weighs nothing
+        const float weight = mine == -INFINITY ? 0.0f : fast_exp2(mine - largest);
         const float total = across_wave(weight, [](float x, float y) { return x + y; });
-        weights[row * kStepMostShares + lane] = weight * (total > 0.0f ? 1.0f / total : 0.0f);
-        if (lane == 0) row_lse[row] = total > 0.0f ? largest + fast_log2(total) : -INFINITY;
+        weights[row * kStepMostShares + lane] = mine == -INFINITY ? kNoWeight : weight * (1.0f / total);
+        if (lane == 0) row_lse[row] = total == 0.0f ? -INFINITY : largest + fast_log2(total);
     }
     __syncthreads();
     for (unsigned int item = first_item; item < items; item += kThreads) {

@@ -171,3 +171,46 @@ def test_paged_keys_reach_the_rows_that_see_them(dtype, heads, kv_heads, dim, sp
         reached[rows, of, dim // 2 if cache == 1 else slice(None)] = True
     assert torch.equal(out[~reached], clean[~reached])
     assert (out[reached].isnan() if math.isnan(bad) else out[reached] == bad).all()
+
+
+# (queries, keys) of a decode step that runs in one launch: sequences that are shared out over several workgroups and ones that
+# are not, one without tokens, and one of two tokens, whose first does not see the last key
+STEP = [(1, 3100), (1, 50), (0, 20), (2, 1000), (1, 700)]
+
+
+def decode_step(dtype, heads, kv_heads, dim, scratch, bad):
+    """The paged op over STEP with `bad` = {(cache, sequence, key, kv head): value of one element}: what it gives, and what
+    float64 gives over the keys that each row sees."""
+    page, scale = 16, dim ** -0.5
+    counts = [-(-keys // page) for _, keys in STEP]
+    tokens, starts = sum(queries for queries, _ in STEP), [sum(counts[:s]) * page for s in range(len(STEP))]
+    q = draw(1, tokens, heads, dim).to(dtype)
+    caches = [draw(seed, sum(counts) * page, kv_heads, dim).to(dtype) for seed in (2, 3)]
+    for (cache, sequence, key, kv_head), value in bad.items():
+        caches[cache][starts[sequence] + key, kv_head, dim // 2] = value
+    index = lambda numbers: torch.tensor(numbers, dtype=torch.int32, device="cuda")
+    sums = lambda numbers: [sum(numbers[:i]) for i in range(len(numbers) + 1)]
+    paging = neural.Paging(index(sums([queries for queries, _ in STEP])), index(sums(counts)), index(list(range(sum(counts)))),
+                           index([keys - (count - 1) * page for (_, keys), count in zip(STEP, counts)]))
+    out, lse = neural.paged_attention(q.cuda(), *(cache.view(-1, page, kv_heads, dim).cuda() for cache in caches), paging,
+                                      neural.AttentionOptions(causal=True, scale=scale), scratch=scratch)
+    first = [start for (queries, _), start in zip(STEP, starts) for _ in range(queries)]
+    end = [start + keys - queries + 1 + i for (queries, keys), start in zip(STEP, starts) for i in range(queries)]
+    scores = [torch.einsum("hd,khd->hk", q[t].double(), caches[0][f:e].double().repeat_interleave(heads // kv_heads, 1)) * scale
+              for t, (f, e) in enumerate(zip(first, end))]
+    want_lse = torch.stack([torch.logsumexp(s, -1) / math.log(2.0) for s in scores])
+    # (torch's logsumexp of scores with an infinity is that infinity; the softmax over them is not a number)
+    want_lse[torch.stack([(s == INF).any(-1) for s in scores])] = NAN
+    return out, lse.double().cpu(), visible_only(q, *caches, first, end, scale), want_lse
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("heads,kv_heads,dim", [(32, 8, 128), (16, 1, 64), (8, 2, 96), (6, 2, 32)])
+@pytest.mark.parametrize("scratch", [True, False])
+@pytest.mark.parametrize("cache,bad", [(0, NAN), (0, INF), (0, -INF), (1, NAN)])
+def test_a_decode_step_gives_every_row_what_its_keys_hold(dtype, heads, kv_heads, dim, scratch, cache, bad):
+    # in the first and in a middle share of a sequence, at its last key, in ones that are not shared out
+    places = {(cache, 0, 3, 0): bad, (cache, 0, 1700, kv_heads - 1): bad, (cache, 1, 49, 0): bad, (cache, 3, 998, 0): bad, (cache, 4, 64, kv_heads - 1): bad}
+    out, lse, want, want_lse = decode_step(dtype, heads, kv_heads, dim, scratch, places)
+    same(out, want, dtype)
+    assert (lse.isnan() == want_lse.isnan()).all() and ((lse - want_lse).abs()[~want_lse.isnan()] <= 2e-3).all()
