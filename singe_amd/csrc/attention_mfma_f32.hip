@@ -138,6 +138,7 @@ struct DenseF32Row {
     const float* values;
     size_t key_stride, value_stride;
     float* out_row;
+    SINGE_DEVICE unsigned int place(unsigned int k) const { return k; }
     SINGE_DEVICE float query(unsigned int d) const { return query_row[d]; }
     SINGE_DEVICE float key(unsigned int k, unsigned int d) const { return keys[k * key_stride + d]; }
     SINGE_DEVICE float value(unsigned int k, unsigned int d) const { return values[k * value_stride + d]; }

@@ -90,6 +90,8 @@ SINGE_DEVICE unsigned int pack_pair(F16, float lo, float hi) {
     return __builtin_bit_cast(unsigned int, __builtin_convertvector(both, f16x2v_t));
 }
 SINGE_DEVICE unsigned int pack_pair(float lo, float hi) { return pack_pair(Bf16{}, lo, hi); }
+SINGE_DEVICE float widen(Bf16, uint16_t bits) { return __builtin_bit_cast(float, static_cast<unsigned int>(bits) << 16); }
+SINGE_DEVICE float widen(F16, uint16_t bits) { return static_cast<float>(__builtin_bit_cast(_Float16, bits)); }
 
 // Two weights as two 16-bit values each: `rounded`, and in `rest` what the rounding left out, rounded in turn.  Together
 // they are within 2^-18 of a bf16 weight and 2^-22 of an f16 one.  An f16 weight is first scaled by kWideScale (no weight

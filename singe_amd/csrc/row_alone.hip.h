@@ -21,7 +21,8 @@ SINGE_DEVICE bool not_finite(int count, Values&& value) {
     return sum != sum;
 }
 
-//   row.query(d), row.key(k, d), row.value(k, d)   the operands as f32
+//   row.place(k)                                   where key k lies, as the next two take it
+//   row.query(d), row.key(at, d), row.value(at, d) the operands as f32
 //   row.store(d, value)                            takes the output
 // The row sees keys begin .. end - 1.  Called by all 64 lanes with the same arguments.
 template <int D, class Row>
@@ -36,9 +37,10 @@ SINGE_DEVICE void row_alone(const Row& row, unsigned int begin, unsigned int end
     for (unsigned int first = begin; first < end; first += 64u) {  // a key a lane for the scores
         float score = -INFINITY;
         if (first + lane < end) {
+            const auto at = row.place(first + lane);
             float dot = 0.0f;
 #pragma unroll 4
-            for (int d = 0; d < D; ++d) dot = fmaf(row.query(d), row.key(first + lane, d), dot);
+            for (int d = 0; d < D; ++d) dot = fmaf(row.query(d), row.key(at, d), dot);
             score = dot * scale_log2e;
         }
         float most = score;
@@ -56,9 +58,10 @@ SINGE_DEVICE void row_alone(const Row& row, unsigned int begin, unsigned int end
         for (unsigned int k = 0; k < count; ++k) {
             if (__shfl(score, k, 64) == -INFINITY) continue;
             const float w = __shfl(weight, k, 64);
+            const auto at = row.place(first + k);
 #pragma unroll
             for (int h = 0; h < kHeld; ++h)
-                if (lane + 64u * h < D) out[h] = fmaf(w, row.value(first + k, lane + 64u * h), out[h]);
+                if (lane + 64u * h < D) out[h] = fmaf(w, row.value(at, lane + 64u * h), out[h]);
         }
     }
     const float inverse = total > 0.0f ? 1.0f / total : 0.0f;

@@ -207,10 +207,11 @@ def decode_step(dtype, heads, kv_heads, dim, scratch, bad):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("heads,kv_heads,dim", [(32, 8, 128), (16, 1, 64), (8, 2, 96), (6, 2, 32)])
 @pytest.mark.parametrize("scratch", [True, False])
-@pytest.mark.parametrize("cache,bad", [(0, NAN), (0, INF), (0, -INF), (1, NAN)])
+@pytest.mark.parametrize("cache,bad", [(0, NAN), (0, INF), (0, -INF), (1, NAN), (1, INF), (1, -INF)])
 def test_a_decode_step_gives_every_row_what_its_keys_hold(dtype, heads, kv_heads, dim, scratch, cache, bad):
     # in the first and in a middle share of a sequence, at its last key, in ones that are not shared out
-    places = {(cache, 0, 3, 0): bad, (cache, 0, 1700, kv_heads - 1): bad, (cache, 1, 49, 0): bad, (cache, 3, 998, 0): bad, (cache, 4, 64, kv_heads - 1): bad}
+    # (and at a key that the second of two tokens sees, not the first)
+    places = {(cache, 0, 3, 0): bad, (cache, 0, 1700, kv_heads - 1): bad, (cache, 1, 49, 0): bad, (cache, 3, 999, 0): bad, (cache, 4, 64, kv_heads - 1): bad}
     out, lse, want, want_lse = decode_step(dtype, heads, kv_heads, dim, scratch, places)
     same(out, want, dtype)
     assert (lse.isnan() == want_lse.isnan()).all() and ((lse - want_lse).abs()[~want_lse.isnan()] <= 2e-3).all()
