@@ -31,10 +31,9 @@ constexpr unsigned int kNarrowSlots = 5;                    // of a wave's ring
 constexpr unsigned int kNarrowSlotBytes = kNarrowKeys * kRowBytes;
 constexpr unsigned int kNarrowWaveBytes = kNarrowSlots * kNarrowSlotBytes;
 static_assert(4 * kNarrowWaveBytes <= kStagedLdsBytes, "the rings take the place of the tiles' stages");
-// What a wave leaves in the place of its ring, in floats: sixteen rows of sums, two words a row, a word of rows that are worked
-// out by themselves, and such a row.
-constexpr unsigned int kNarrowWordsAt = kNarrowRows * kHeadDim, kNarrowAloneAt = kNarrowWordsAt + 2u * kNarrowRows, kNarrowRowAt = kNarrowAloneAt + 4u;
-static_assert((kNarrowRowAt + kHeadDim) * 4 <= kNarrowWaveBytes, "and a wave's sums that of its ring");
+// (behind a wave's sums in its ring's place, in floats: a row that is worked out by itself)
+constexpr unsigned int kNarrowRowAt = kNarrowRows * (kHeadDim + 2);
+static_assert((kNarrowRowAt + kHeadDim) * 4 <= kNarrowWaveBytes, "a wave's sums take the place of its ring");
 // A score product takes 32 dims and needs all of them.
 constexpr bool kNarrowBuild = kHeadDim % 32 == 0;
 
@@ -117,10 +116,10 @@ struct PagedRow {
 // of sixteen, but for the end), of which a row sees what its position and the window leave it.  Pages of at least sixteen keys,
 // a power of two of them.  finish(row, quad, values, lse2) takes values 4 quad .. of a row, normalised, and its base-two
 // log-sum-exp (a row that sees no key: zeros and -inf).  WIDE: the weights meet the values at f32's precision (split_pair), by a
-// second value product that the memory-bound loop has room for.  An infinity among the values is a NaN to that product, so a row
-// whose sums are not finite is worked out by itself there, from the keys it sees and no others (row_alone); and a row with a
-// score that is NaN or +inf has a log-sum-exp of NaN beside its values, so that whoever merges it with others can tell it from a
-// row that sees no key.
+// second value product that the memory-bound loop has room for.  An infinity among the values is a NaN to that product, so
+// values that come out not finite are worked out again there, from the keys the row sees and no others (row_alone); and a row
+// with a score that is NaN or +inf has a log-sum-exp of NaN beside its values, so that whoever merges it with others can tell it
+// from a row that sees no key.
 template <bool SOFTCAP, int FORM, bool WIDE, unsigned int WAVES, class Half, class Finish>
 SINGE_DEVICE void narrow_rows(const PagedAttentionArgs& a, unsigned char* lds, const SequenceSpan& span, unsigned int kv_head, unsigned int first_row,
                               unsigned int packed, unsigned int key_begin, unsigned int key_end, Finish&& finish) {
@@ -322,78 +321,55 @@ SINGE_DEVICE void narrow_rows(const PagedAttentionArgs& a, unsigned char* lds, c
     for (int db = 0; db < kNarrowBlocks; ++db)
         *reinterpret_cast<float4*>(mine + column * kHeadDim + 16 * db + 4 * g) = make_float4(out[db][0], out[db][1], out[db][2], out[db][3]);
     if (g == 0) {
-        mine[kNarrowWordsAt + 2u * column] = reference;
-        mine[kNarrowWordsAt + 2u * column + 1u] = sum;
-    }
-    unsigned int alone = 0;  // rows (bit r: row r) with a sum that is not finite in some wave, though their scores are
-    if constexpr (WIDE) {
-        const unsigned long long spoiled = __builtin_amdgcn_ballot_w64(sum == sum && not_finite(4 * kNarrowBlocks, [&](int i) { return out[i / 4][i % 4]; }));
-        const unsigned int halves = static_cast<unsigned int>(spoiled) | static_cast<unsigned int>(spoiled >> 32);
-        if (lane == 0) reinterpret_cast<unsigned int*>(mine)[kNarrowAloneAt] = halves | halves >> 16;
+        mine[kNarrowRows * kHeadDim + 2u * column] = reference;
+        mine[kNarrowRows * kHeadDim + 2u * column + 1u] = sum;
     }
     __syncthreads();
-    if constexpr (WIDE) {
-#pragma unroll
-        for (unsigned int w = 0; w < WAVES; ++w) alone |= reinterpret_cast<const unsigned int*>(lds + w * kNarrowWaveBytes)[kNarrowAloneAt];
-        alone = __builtin_amdgcn_readfirstlane(alone) & ((1u << packed) - 1u);
-    }
-    // The waves' weights in a row's sum, the sum, and the reference point they are scaled by.
-    auto meet = [&](unsigned int row, float (&weights)[WAVES], float& total) __attribute__((always_inline)) {
+    const unsigned int items = packed * (kHeadDim / 4u);
+    for (unsigned int first = 64u * wave; first < items; first += 64u * WAVES) {  // (with all of a wave's lanes)
+        const unsigned int item = first + lane, at = item < items ? item : items - 1u, row = at / (kHeadDim / 4u), quad = at % (kHeadDim / 4u);
         float references[WAVES], sums[WAVES], largest = -INFINITY;
 #pragma unroll
         for (unsigned int w = 0; w < WAVES; ++w) {
-            const float* from = reinterpret_cast<const float*>(lds + w * kNarrowWaveBytes) + kNarrowWordsAt + 2u * row;
+            const float* from = reinterpret_cast<const float*>(lds + w * kNarrowWaveBytes) + kNarrowRows * kHeadDim + 2u * row;
             references[w] = from[0];
             sums[w] = from[1];
             largest = fmaxf(largest, references[w]);
         }
-        total = 0.0f;
-#pragma unroll
-        for (unsigned int w = 0; w < WAVES; ++w) {
-            weights[w] = references[w] == -INFINITY ? 0.0f : fast_exp2(references[w] - largest);
-            total = fmaf(weights[w], sums[w], total);
-        }
-        return largest;
-    };
-    auto log_sum = [](float largest, float total) __attribute__((always_inline)) {
-        const float lse2 = total > 0.0f ? largest + fast_log2(total) : -INFINITY;
-        return WIDE && total != total ? total : lse2;
-    };
-    for (unsigned int at = threadIdx.x; at < packed * (kHeadDim / 4u); at += 64u * WAVES) {
-        const unsigned int row = at / (kHeadDim / 4u), quad = at % (kHeadDim / 4u);
-        if (WIDE && (alone >> row & 1u) != 0) continue;
-        float weights[WAVES], total;
-        const float largest = meet(row, weights, total);
         float4 merged = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        float total = 0.0f;
 #pragma unroll
         for (unsigned int w = 0; w < WAVES; ++w) {
+            const float weight = references[w] == -INFINITY ? 0.0f : fast_exp2(references[w] - largest);
             const float4 part = *reinterpret_cast<const float4*>(reinterpret_cast<const float*>(lds + w * kNarrowWaveBytes) + row * kHeadDim + 4u * quad);
-            merged.x = fmaf(weights[w], part.x, merged.x);
-            merged.y = fmaf(weights[w], part.y, merged.y);
-            merged.z = fmaf(weights[w], part.z, merged.z);
-            merged.w = fmaf(weights[w], part.w, merged.w);
+            total = fmaf(weight, sums[w], total);
+            merged.x = fmaf(weight, part.x, merged.x);
+            merged.y = fmaf(weight, part.y, merged.y);
+            merged.z = fmaf(weight, part.z, merged.z);
+            merged.w = fmaf(weight, part.w, merged.w);
         }
         const float inverse = (total > 0.0f ? 1.0f / total : 0.0f) * (WIDE ? 1.0f / kWideScale<Half> : 1.0f);
         merged.x *= inverse; merged.y *= inverse; merged.z *= inverse; merged.w *= inverse;
-        finish(row, quad, merged, log_sum(largest, total));
-    }
-    if constexpr (WIDE) {
-        static_assert(!SOFTCAP, "row_alone takes the scores as they are");
-        for (; alone != 0; alone &= alone - 1u) {
-            const unsigned int row = static_cast<unsigned int>(__builtin_ctz(alone));
-            if (row % WAVES != wave) continue;
-            const unsigned int at = first_row + row, position = position_of(row);
-            const size_t flat = (static_cast<size_t>(span.query_start) + at / groups) * a.heads + kv_head * groups + at % groups;
-            const unsigned int seen = windowed && position >= window ? position - window + 1u : 0u, reach = causal && position < key_end ? position + 1u : key_end;
-            float* const values = mine + kNarrowRowAt;
-            row_alone<kHeadDim>(PagedRow<FORM, Half>{a.query_rows + flat * kHeadDim, a, static_cast<size_t>(span.page_start), kv_head * kHeadDim, values},
-                                key_begin > seen ? key_begin : seen, reach, a.scale_log2e);
-            narrow_slot_read();  // (and written: the lanes that take a quad each find what others stored)
-            float weights[WAVES], total;
-            const float largest = meet(row, weights, total);
-            if (lane < kHeadDim / 4u) finish(row, lane, *reinterpret_cast<const float4*>(values + 4u * lane), log_sum(largest, total));
-            narrow_slot_read();
+        float lse2 = total > 0.0f ? largest + fast_log2(total) : -INFINITY;
+        if constexpr (WIDE) {
+            static_assert(!SOFTCAP, "row_alone takes the scores as they are");
+            if (total != total) lse2 = total;  // (and so are all of the row's values)
+            const float values[4] = {merged.x, merged.y, merged.z, merged.w};
+            const bool bad = total == total && not_finite(4, [&](int i) { return values[i]; });
+            for (unsigned long long left = __builtin_amdgcn_ballot_w64(bad); left != 0;) {
+                const unsigned int r = __builtin_amdgcn_readlane(row, __builtin_ctzll(left)), packed_row = first_row + r, position = position_of(r);
+                const size_t flat = (static_cast<size_t>(span.query_start) + packed_row / groups) * a.heads + kv_head * groups + packed_row % groups;
+                const unsigned int seen = windowed && position >= window ? position - window + 1u : 0u, reach = causal && position < key_end ? position + 1u : key_end;
+                float* const apart = mine + kNarrowRowAt;
+                row_alone<kHeadDim>(PagedRow<FORM, Half>{a.query_rows + flat * kHeadDim, a, static_cast<size_t>(span.page_start), kv_head * kHeadDim, apart},
+                                    key_begin > seen ? key_begin : seen, reach, a.scale_log2e);
+                narrow_slot_read();  // (and written: a lane's values are other lanes' stores)
+                if (bad && row == r) merged = *reinterpret_cast<const float4*>(apart + 4u * quad);
+                narrow_slot_read();
+                left &= ~__builtin_amdgcn_ballot_w64(row == r);
+            }
         }
+        if (item < items) finish(row, quad, merged, lse2);
     }
 }
 
