@@ -487,6 +487,12 @@ SINGE_HIP_API void singe_hip_set_paged_attention_rows_per_wave(uint32_t rows);
 /* What a bf16 / f16 call of this problem takes when it is given scratch: 32 or 64 rows a wave,
  * 0 when the head dimension has no matrix-core build. */
 SINGE_HIP_API uint32_t singe_hip_paged_attention_rows_per_wave(const SingePagedAttentionProblem* problem);
+/* Which kernels a bf16 / f16 call of this problem without a fused query rotation runs on when it is lent `scratch_bytes` of
+ * scratch at `scratch` (null: none; only its alignment is looked at). */
+#define SINGE_HIP_PAGED_ROW_TILES 0u
+#define SINGE_HIP_PAGED_DECODE_KERNELS 1u
+#define SINGE_HIP_PAGED_ONE_LAUNCH 2u
+SINGE_HIP_API uint32_t singe_hip_paged_attention_route(const SingePagedAttentionProblem* problem, const void* scratch, size_t scratch_bytes);
 /* singe_hip_paged_attention_scratch_* for an output that holds nothing yet: the rows of tokens that no valid sequence owns
  * are written too, zeros with a log-sum-exp of -inf, where the others leave them as they are.  Sequences before the first whose
  * query offsets make no sense are attended as ever, those after it whole or not at all; rows of tokens that two of them claim

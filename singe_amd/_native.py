@@ -346,6 +346,8 @@ def bind(path: str) -> ctypes.CDLL:
         getattr(handle, name).restype = i32
     handle.singe_hip_paged_attention_scratch_bytes.argtypes = [ctypes.POINTER(PagedAttentionProblemC)]
     handle.singe_hip_paged_attention_scratch_bytes.restype = ctypes.c_size_t
+    handle.singe_hip_paged_attention_route.argtypes = [ctypes.POINTER(PagedAttentionProblemC), c_void, ctypes.c_size_t]
+    handle.singe_hip_paged_attention_route.restype = ctypes.c_uint32
     handle.singe_hip_set_paged_attention_splits.argtypes = [ctypes.c_uint32]
     handle.singe_hip_set_paged_attention_splits.restype = None
     handle.singe_hip_paged_mla_attention.argtypes = [c_void] * 12 + [ctypes.POINTER(PagedMlaAttentionProblemC)]

@@ -21,8 +21,11 @@ namespace {
 
 constexpr int kStepChunks = 4;                   // of 64 sequences
 constexpr unsigned int kStepMostShares = 64;     // of a unit
-// Tiles of 64 keys: the fewest of a share, and as many as a unit may have that is not shared out.
-constexpr unsigned int kStepLeastTiles = 4, kStepWholeTiles = 14;
+constexpr unsigned int kStepLeastTiles = 4;      // of 64 keys, to a share
+// As many tiles as a unit may have that is not shared out.  Eleven or fourteen on eight waves, many steps in turn over 700 MB of
+// caches: 32 / 8 heads x 128, one sequence of 800 keys 13.8 / 15.5 us, eight of 700 to 900 16.1 / 17.8; x 64 11.8 / 11.2, 13.8 / 13.8.
+template <unsigned int WAVES>
+constexpr unsigned int kStepWholeTiles = WAVES == 8 && kHeadDim > 64 ? 11 : 14;
 
 // A unit's share: rows 16 row_tile .. of the sequence, tiles [first_tile, end_tile) of its keys; `shares` neighbouring entries,
 // this one the `share`-th.
@@ -31,7 +34,7 @@ struct StepPlace {
     unsigned int row_tile, share, shares, first_tile, end_tile;
 };
 
-template <int FORM>
+template <int FORM, unsigned int WAVES>
 SINGE_DEVICE bool place_step(const PagedAttentionArgs& a, unsigned int entry, StepPlace& place) {
     const unsigned int lane = threadIdx.x & 63u, groups = a.heads / a.kv_heads;
     const bool windowed = a.window >= 0;
@@ -82,7 +85,7 @@ SINGE_DEVICE bool place_step(const PagedAttentionArgs& a, unsigned int entry, St
 #pragma unroll
     for (int c = 0; c < kStepChunks; ++c) {
         if (64u * c >= a.sequences) break;
-        const unsigned int shares = tiles[c] <= (length > kStepWholeTiles ? length : kStepWholeTiles) ? 1u : (tiles[c] - 1u) / length + 1u;
+        const unsigned int shares = tiles[c] <= (length > kStepWholeTiles<WAVES> ? length : kStepWholeTiles<WAVES>) ? 1u : (tiles[c] - 1u) / length + 1u;
         const unsigned int mine = units[c] * shares, through = sums_through_lane(mine), total = __builtin_amdgcn_readlane(through, 63);
         if (entry >= total) {
             entry -= total;
@@ -107,8 +110,10 @@ SINGE_DEVICE bool place_step(const PagedAttentionArgs& a, unsigned int entry, St
         place.span.keys = owners(spans[c].keys);
         place.span.valid = owners(spans[c].valid ? 1u : 0u) != 0u;
         const unsigned int first = owners(first_tile[c]), end = first + owners(tiles[c]);
-        place.first_tile = place.shares == 1u ? first : first + place.share * length;
-        place.end_tile = place.shares == 1u || end - place.first_tile < length ? end : place.first_tile + length;
+        // (cut evenly: a unit of fifteen tiles takes eight and seven, not fourteen and one with a merge behind them)
+        const unsigned int each = (end - first + place.shares - 1u) / place.shares;
+        place.first_tile = first + place.share * each;
+        place.end_tile = end - place.first_tile < each ? end : place.first_tile + each;
         return true;
     }
     return false;
@@ -140,7 +145,7 @@ SINGE_DEVICE void decode_step_body(const PagedAttentionArgs& a, unsigned char* l
     }
     const unsigned int entry = blockIdx.x / a.kv_heads, kv_head = blockIdx.x - entry * a.kv_heads;
     StepPlace place;
-    if (!place_step<FORM>(a, entry, place)) return;
+    if (!place_step<FORM, WAVES>(a, entry, place)) return;
     const SequenceSpan& span = place.span;
     if (!span.valid) {
         if (tid == 0) report_index_error(a.status);

@@ -628,3 +628,47 @@ def test_every_row_refuses_what_makes_no_sense_before_what_it_has_no_build_for(f
         latent = _native.PagedMlaAttentionProblemC(fields.get("tokens", 4), 8, fields.get("head_dim", 512), 64, fields.get("page_size", 16),
                                                    fields.get("sequences", 2), 4, 4, 1, 0, 1, 0, 0.0)
         assert lib.singe_hip_paged_mla_attention_every_row(None, *[0x1000] * 11, None, 0, ctypes.byref(latent)) == status
+
+
+ROW_TILES, DECODE_KERNELS, ONE_LAUNCH = 0, 1, 2
+
+
+def paged_route(heads, kv_heads, head_dim, sequences, keys, scratch="asked for", page_size=16, **fields):
+    """The route of a step of a token a sequence, `keys` each on average, with no scratch, as much as it asks for, or (address, bytes)."""
+    lib = _native.lib()
+    known = dict(tokens=sequences, heads=heads, kv_heads=kv_heads, head_dim=head_dim, page_size=page_size, sequences=sequences,
+                 cache_pages=1 << 20, page_table=sequences * keys // page_size, index_type=1, causal=1, has_scale=0, has_window=0, has_softcap=0,
+                 scale=0.0, softcap=0.0, window=0)
+    problem = _native.PagedAttentionProblemC(*{**known, **fields}.values())
+    wanted = lib.singe_hip_paged_attention_scratch_bytes(ctypes.byref(problem))
+    address, count = (0x1000, wanted) if scratch == "asked for" else (None, 0) if scratch is None else scratch(wanted)
+    return lib.singe_hip_paged_attention_route(ctypes.byref(problem), address, count)
+
+
+@pytest.mark.parametrize("heads,kv_heads,head_dim,sequences,keys,route", [
+    (32, 8, 128, 1, 32000, ONE_LAUNCH),        # few units: 2^18 keys between them
+    (32, 8, 128, 1, 32784, DECODE_KERNELS),
+    (32, 8, 64, 1, 7168, ONE_LAUNCH),          # ... of up to four narrow rows, and of fewer than four: 7 * 2^13
+    (32, 8, 64, 1, 7184, DECODE_KERNELS),
+    (32, 32, 128, 1, 1792, ONE_LAUNCH),
+    (32, 32, 128, 1, 2000, DECODE_KERNELS),
+    (32, 8, 128, 16, 896, ONE_LAUNCH),         # up to 128 units of 896 keys
+    (32, 8, 128, 16, 912, DECODE_KERNELS),
+    (32, 8, 128, 24, 704, ONE_LAUNCH),         # ... 192 of 704
+    (32, 8, 128, 24, 720, DECODE_KERNELS),
+    (32, 8, 128, 24, 864, DECODE_KERNELS),
+    (32, 8, 128, 64, 384, ONE_LAUNCH),         # more: 576 of more than four rows, else 384
+    (32, 8, 128, 64, 400, DECODE_KERNELS),
+    (64, 8, 128, 64, 576, ONE_LAUNCH),
+    (64, 8, 128, 64, 592, DECODE_KERNELS),
+    (32, 8, 128, 128, 96, ONE_LAUNCH),         # up to 1024 units, 512 of four narrower rows and of fewer
+    (32, 8, 96, 64, 96, ONE_LAUNCH),
+    (32, 8, 96, 80, 96, DECODE_KERNELS),
+    (64, 8, 64, 128, 96, ONE_LAUNCH),
+    (32, 32, 128, 16, 96, ONE_LAUNCH),
+    (32, 32, 128, 24, 96, DECODE_KERNELS),
+    (64, 8, 128, 129, 96, DECODE_KERNELS),
+])
+def test_decode_steps_in_one_launch_are_those_that_gain_by_it_whatever_their_lengths(heads, kv_heads, head_dim, sequences, keys, route):
+    # (200 to 1500 keys on 24 sequences of 32 / 8 heads x 128 took 30 us in one launch and 26 in three)
+    assert paged_route(heads, kv_heads, head_dim, sequences, keys) == route
