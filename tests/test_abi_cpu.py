@@ -672,3 +672,16 @@ def paged_route(heads, kv_heads, head_dim, sequences, keys, scratch="asked for",
 def test_decode_steps_in_one_launch_are_those_that_gain_by_it_whatever_their_lengths(heads, kv_heads, head_dim, sequences, keys, route):
     # (200 to 1500 keys on 24 sequences of 32 / 8 heads x 128 took 30 us in one launch and 26 in three)
     assert paged_route(heads, kv_heads, head_dim, sequences, keys) == route
+
+
+@pytest.mark.parametrize("sequences,keys,scratch,route", [
+    (1, 32000, lambda wanted: (0x1000, wanted), ONE_LAUNCH),
+    (1, 32000, lambda wanted: (0x1010, wanted), ROW_TILES),                       # not on a 256-byte boundary: key shares of the row tiles
+    (1, 32000, lambda wanted: (0x1010, 63 * 32 * 129 * 4), ROW_TILES),            # ... which 63 shares of 32 rows need
+    (1, 32000, lambda wanted: (0x1010, 63 * 32 * 129 * 4 - 1), ONE_LAUNCH),
+    (1, 32000, lambda wanted: (None, 0), ONE_LAUNCH),
+    (1, 32000, lambda wanted: (0x1000, 16), ONE_LAUNCH),
+    (1, 400, lambda wanted: (0x1010, wanted), ONE_LAUNCH),                        # too few keys for shares
+])
+def test_scratch_that_the_one_launch_has_no_use_for_goes_to_key_shares(sequences, keys, scratch, route):
+    assert paged_route(32, 8, 128, sequences, keys, scratch) == route

@@ -779,3 +779,23 @@ def test_a_decode_step_in_one_launch_replays_over_whatever_its_scratch_holds():
             fresh, fresh_lse = call()
             stream.synchronize()
             assert torch.equal(out, fresh) and torch.equal(lse, fresh_lse)
+
+
+@pytest.mark.parametrize("first,count", [(16, 8 << 20), (0, 1 << 18), (16, 100)])
+def test_scratch_that_starts_anywhere_or_is_short_serves_a_decode_step(first, count):
+    """Off a 256-byte boundary the keys are shared out by the row tiles, as they are where the scratch is too short for the one launch;
+    with too little for either the call goes without."""
+    query_offsets, page_offsets, table, last, page_count = layout([(1, 3000), (1, 50)], 16)
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(5)
+    rand = lambda *shape: torch.randn(shape, generator=gen, device="cuda").bfloat16()
+    q, kc, vc = rand(2, 32, 128), rand(page_count, 16, 8, 128), rand(page_count, 16, 8, 128)
+    index = lambda values: torch.tensor(values, dtype=torch.int32, device="cuda")
+    paging = neural.Paging(index(query_offsets), index(page_offsets), index(table), index(last))
+    scratch = torch.empty(first + count, device="cuda", dtype=torch.uint8)[first:]
+    out, lse = neural.paged_attention(q, kc, vc, paging, neural.AttentionOptions(causal=True), scratch=scratch)
+    status, want, want_lse = oracle.paged_attention_f32(q.float().cpu().numpy(), kc.float().cpu().numpy(), vc.float().cpu().numpy(), query_offsets,
+                                                        page_offsets, table, last, causal=True, threads=8)
+    assert status == 0
+    gap = np.abs(out.float().cpu().numpy() - want)
+    assert gap.max() <= MAX_ABS and gap.mean() <= MEAN_ABS and np.abs(lse.cpu().numpy() - want_lse).max() <= LSE_ABS
