@@ -7,6 +7,7 @@
 #include "module.h"
 #include "singe_hip_attention.h"
 #include "validate.h"
+#include "window_runs.h"
 
 using namespace singe_hip;
 
@@ -296,14 +297,8 @@ WindowRuns window_runs(const SingeFmhaPrefillConfig& c, uint64_t window) {
     const uint64_t units = compute_units(), places = units * (c.head_dim <= 64 ? 2 : 1);
     const uint64_t pairs = static_cast<uint64_t>(c.batch) * c.kv_heads, steps = (c.query_len * group + kStepRows - 1) / kStepRows, all = pairs * steps;
     if (2 * all <= units || (c.head_dim <= 64 && ring > 8 && all > units && 2 * all < 3 * units)) return {0, 0, 0};
-    // Runs of one length that fill the chip's places in whole rounds, a run's first keys counted as a step.
-    uint64_t best = ~0ull, best_steps = steps;
-    for (uint64_t runs = 1; runs <= steps && (runs - 1) * pairs <= 4 * places; ++runs) {
-        const uint64_t run_steps = (steps + runs - 1) / runs, rounds = (pairs * ((steps + run_steps - 1) / run_steps) + places - 1) / places;
-        const uint64_t cost = rounds * (run_steps + 1);
-        if (cost < best) best = cost, best_steps = run_steps;
-    }
-    return {static_cast<uint32_t>(ring), static_cast<uint32_t>((steps + best_steps - 1) / best_steps), static_cast<uint32_t>(best_steps)};
+    const uint64_t run_steps = window_run_steps(steps, pairs, places);
+    return {static_cast<uint32_t>(ring), static_cast<uint32_t>((steps + run_steps - 1) / run_steps), static_cast<uint32_t>(run_steps)};
 }
 
 int32_t prefill(void* stream, uint16_t* out, size_t out_len, float* lse, size_t lse_len, bool with_lse,
