@@ -241,6 +241,9 @@ namespace {
 // tiles are not whole, 256 x 700 x 3000 (512) 172 / 226.  What the lines cost against the faster kernel, of 520 shapes: up to 11 %
 // for narrow heads without the mask in many rounds (head_dim 48, 256 x 4096 (2048) 1154 / 1281, on the two-tile kernel), 9 % under it
 // at head_dim 48 (32 x 8192 (512) 331 / 305, on the 32-row one), 7 % for 128 x 2048 (512) at 64 without it (174 / 162) and from 80 up.
+// (Workgroups are counted with (batch, head)s rounded up to a multiple of eight, as the lines were drawn, though the launch deals
+// them out evenly: counted as dealt, 28 x 2560, 18 x 4096 and 12 x 6000 without the mask would go to the 32-row kernel, 132, 205 and
+// 296 us in place of 113, 171 and 246.)
 bool two_tiles_a_wave(const SingeFmhaPrefillConfig& c) {
     const uint32_t wanted = g_rows_per_wave.load(std::memory_order_relaxed);
     if (wanted == 32 || !has_pair_build(static_cast<long long>(c.head_dim)) || c.key_len == 0 || !(c.scale > 0.0f) || dense_prefill_packs_heads(c))
@@ -398,7 +401,11 @@ int32_t prefill(void* stream, uint16_t* out, size_t out_len, float* lse, size_t 
     //   lengths of half the keys to all of them   1 x 6 x 1500  16.8 / 14.9   3 x 6  29.4 / 19.5   4 x 6  28.7 / 25.8   5 x 6  29.2 / 26.4
     //                7 x 6  36.4 / 31.4   8 x 6  37.4 / 32.1   9 x 6  38.8 / 34.7   10 x 6  40.8 / 39.1   5 x 12 x 700  17.1 / 15.9
     const uint64_t units = rows * (shares.single_tiles ? args.query_tiles : (args.query_tiles + 1) / 2);
-    args.deal = kDealEvenly;
+    // Single tiles under the causal mask, more of them than the compute units hold at once, go by whole (batch, head)s too: an eighth that
+    // ends inside one ends on its first tiles, which are its longest and run on by themselves.  Whole / evenly
+    //   45 heads x 1500 x 128  48.5 / 56.3   30 x 2560  73 / 81   20 x 6000 x 64  137 / 148   (all at once: 36 x 2560 x 64  53.6 / 51.8)
+    const uint64_t at_once = compute_units() * (c.head_dim > 64 ? 2 : c.head_dim > 32 ? 3 : 4);
+    args.deal = c.causal && args.single_tiles != 0 && units > at_once ? kDealWhole : kDealEvenly;
     if (options.key_lengths != nullptr && units > compute_units())
         args.deal = !c.causal && args.single_tiles != 0 && args.packed_heads == 0 && c.batch <= 64 && c.key_len >= 512 && units <= 3 * compute_units()
                         ? kDealByLength : kDealWhole;

@@ -519,6 +519,7 @@ def test_scores_that_outgrow_a_share_s_reference_point(heads, length, causal, dt
     (64, 2, 2, 515, 48, [(37 * b) % 516 for b in range(64)]),       # ... and 640
     (3, 6, 2, 777, 64, [777, 100, 400]),                            # a tile a compute unit at most: an eighth of them to an XCD
     (5, 7, 7, 260, 128, None),                                      # 105 tiles over eight XCDs
+    (5, 27, 9, 512, 128, None),                                     # 540 single tiles, more than two a compute unit
 ])
 @pytest.mark.parametrize("causal", [False, True])
 def test_query_tiles_dealt_to_the_xcds_cover_every_row(batch, heads, kv_heads, length, dim, lengths, causal):
