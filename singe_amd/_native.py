@@ -96,8 +96,8 @@ class PagedAttentionProblemC(ctypes.Structure):
                 ("window", ctypes.c_int64)]
 
 
-# SingePagedAttentionCall and SingeRotaryCacheCall: packing one takes a third of the time that building the problem and
-# converting the call's other arguments one by one do.
+# SingePagedAttentionCall and SingeRotaryCacheCall, field by field as the header has them (tests/test_call_records_cpu.py compares
+# them): packing one takes a third of the time that building the problem and converting the call's other arguments one by one do.
 PAGED_ATTENTION_CALL = struct.Struct("@q12PQq8qi4Bffq")
 ROTARY_CACHE_CALL = struct.Struct("@14P6q3i2Bff")
 LENGTH_TOO_SHORT = 2
