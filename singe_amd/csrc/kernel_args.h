@@ -151,6 +151,10 @@ struct PrefillF32Args {
     uint32_t row_waves = 1;         // row tiles of a workgroup, which has key_waves * row_waves waves
 };
 
+// Limits of the decode step in one launch, which the host keeps to and the kernel counts on (paged_step.hip.h): sequences, and rows
+// of a workgroup.
+constexpr uint32_t kStepMostSequences = 256, kStepRows = 16;
+
 struct PagedAttentionArgs {
     const uint16_t* query_rows;     // [tokens, heads, 128] bf16
     const uint16_t* key_cache;      // [cache_pages, page_size, kv_heads, 128] bf16
@@ -195,9 +199,9 @@ struct PagedAttentionArgs {
     float query_eps = 0.0f;
     // Workgroups from this one on clear the rows of tokens that no attended sequence owns (clear_unowned_tokens); 0: none do.
     uint32_t clear_from = 0;
-    // singe_paged_decode_step_*: row_tiles workgroups a kv head, each with sixteen rows of partial_out and two floats a row of
-    // partial_lse to itself, a word of share_done to say that they are written, and the launch's own number to say it with (null: units are not
-    // shared out).
+    // singe_paged_decode_step_*: row_tiles workgroups a kv head, each with kStepRows rows of partial_out and two floats a row of
+    // partial_lse to itself, a word of share_done to say that they are written, and the launch's own number to say it with
+    // (share_done null: units are not shared out).
     uint64_t* share_done = nullptr;
     uint64_t launch_number = 0;
 };

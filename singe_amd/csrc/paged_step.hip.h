@@ -19,7 +19,8 @@
 
 namespace {
 
-constexpr int kStepChunks = 4;                   // of 64 sequences
+constexpr int kStepChunks = kStepMostSequences / 64;
+static_assert(kStepMostSequences % 64 == 0 && kStepRows == kNarrowRows, "limits");
 constexpr unsigned int kStepMostShares = 64;     // of a unit
 constexpr unsigned int kStepLeastTiles = 4;      // of 64 keys, to a share
 // As many tiles as a unit may have that is not shared out.  Eleven or fourteen on eight waves, many steps in turn over 700 MB of
