@@ -18,8 +18,10 @@ BUILDS = [
     ("latent_attention_mfma.hip", [], [r"singe_paged_mla_attention_(bf16|f16)_(l512_p64|any)"]),
     ("fmha_prefill_pair.hip", [], [r"singe_fmha_prefill_pair_.*"]),
     ("paged_attention_pair.hip", [], [r"singe_(rotary_)?paged_attention_pair_.*"]),
-    ("fmha_prefill.hip", [], [r"singe_fmha_prefill_(bf16|f16)_d128_(causal|full)(_options)?"]),
-    ("paged_attention.hip", [], [r"singe_ragged_prefill_(bf16|f16)_d128"]),
+    ("fmha_prefill.hip", [], [r"singe_fmha_prefill_(bf16|f16)_d128_(causal|full)(_options)?", r"singe_fmha_prefill_(bf16|f16)_d128_causal_window"]),
+    ("fmha_prefill.hip", ["-DSINGE_HEAD_DIM=64"], [r"singe_fmha_prefill_(bf16|f16)_d64_causal_window"]),
+    ("paged_attention.hip", [], [r"singe_ragged_prefill_(bf16|f16)_d128", r"singe_paged_decode_step_(bf16|f16)_d128_i(32|64)", r"singe_paged_decode_step_(bf16|f16)_d128_i(32|64)_w8"]),
+    ("paged_attention.hip", ["-DSINGE_HEAD_DIM=96"], [r"singe_paged_decode_step_(bf16|f16)_d96_i(32|64)(_w8)?"]),
     ("attention_mfma_f32.hip", [], [r"singe_attention_mfma_f32_d\d+_r\d+"]),
     ("paged_decode.hip", [], [r"singe_paged_decode_(bf16|f16)_d128_g1_b16", r"singe_paged_decode_f8kv_wide(_relaxed)?_d128_b16",
                               r"singe_paged_decode_(bf16|f16)_wide_d128_b16"]),
@@ -38,14 +40,14 @@ def remarks_of(name, flags):
 def remarks():
     with ThreadPoolExecutor(max_workers=min(4, os.cpu_count() or 1)) as pool:
         texts = list(pool.map(lambda item: remarks_of(item[0], item[1]), BUILDS))
-    return {name: text for (name, _, _), text in zip(BUILDS, texts)}
+    return {(name, *flags): text for (name, flags, _), text in zip(BUILDS, texts)}
 
 
-@pytest.mark.parametrize("name,flags,patterns", BUILDS, ids=[item[0] for item in BUILDS])
+@pytest.mark.parametrize("name,flags,patterns", BUILDS, ids=[" ".join([item[0], *item[1]]) for item in BUILDS])
 def test_no_scratch_memory_in_the_kernels_that_cannot_afford_it(remarks, name, flags, patterns):
     scratch = {}
     kernel = None
-    for line in remarks[name].splitlines():
+    for line in remarks[(name, *flags)].splitlines():
         found = re.search(r"Function Name: (\S+)", line)
         if found:
             kernel = found.group(1)
