@@ -4,6 +4,7 @@ error without touching a device."""
 import ctypes
 import os
 import re
+import subprocess
 
 import pytest
 
@@ -685,3 +686,9 @@ def test_decode_steps_in_one_launch_are_those_that_gain_by_it_whatever_their_len
 ])
 def test_scratch_that_the_one_launch_has_no_use_for_goes_to_key_shares(sequences, keys, scratch, route):
     assert paged_route(32, 8, 128, sequences, keys, scratch) == route
+
+
+def test_no_entry_point_draws_random_numbers_that_may_throw():
+    # (std::random_device throws where the system has no source of them, through a C entry: the process ends)
+    symbols = subprocess.run(["nm", "-D", "--undefined-only", "-C", _native.LIBRARY_PATH], check=True, capture_output=True, text=True).stdout
+    assert "std::random_device" not in symbols
