@@ -465,16 +465,24 @@ SINGE_HIP_API int32_t singe_hip_paged_attention_bf16(
  * partial and its log-sum-exp, and a second kernel merges them (the scheme of the reference's own split
  * kernels, which declare such scratch in their plan: kernel_plan/source/mla.rs:232-241, 497-560).
  * singe_hip_paged_attention_scratch_bytes says how much this problem wants (0: it would not split);
- * with a null or smaller buffer the call runs unsplit, exactly as singe_hip_paged_attention_bf16.  The scratch
- * holds nothing between calls; calls that share it must not overlap.  Results equal the unsplit ones up to
+ * with a null buffer, or one too small for any of its routes, the call runs exactly as singe_hip_paged_attention_bf16.
+ * The scratch holds nothing between calls; calls that share it must not overlap.  Results equal the unsplit ones up to
  * the order of summation.  singe_hip_set_paged_attention_splits fixes the number of shares (0 = chosen by
  * problem size, the default), the counterpart of TuningChoice::Explicit
  * (singe-kernel/src/cuda/attention/mod.rs:2364-2380); it changes what ..._scratch_bytes returns.
- * A decode step (no more tokens than sequences, head_dim a multiple of 16 up to 128, no softcap, no window below 2048 keys) given
- * scratch on a 256-byte boundary runs on the block-table decode kernels instead, which cut the keys of all
- * sequences into equal ranges: a first kernel checks the paging vectors (same status word) and gives each token
- * its page list and key count, and the scratch then also holds those and the decode kernels' partial rows.  The
- * result is the same up to the order of summation; a fixed number of shares keeps such a call on the row-tile kernel. */
+ *
+ * A decode step (no more tokens than sequences, no softcap; singe_hip_paged_attention_route says which way one goes) has two
+ * routes of its own, unless a number of shares is fixed.  Either reports the same status word, and its results are those of
+ * the row tiles up to the order of summation and the rounding of the weights.
+ *   One launch, with any window: head_dim a multiple of 32 up to 128, pages of a power of two of sixteen keys and up, 256
+ *   sequences and sixteen query heads a kv head at most, few enough keys (decode_step_entries in csrc/paged_attention.cpp says
+ *   how many).  Given scratch on a 256-byte boundary workgroups that share a sequence's keys meet in it, inside the launch;
+ *   without scratch, or with less than any route has a use for, every sixteen rows have one workgroup.  Scratch off that
+ *   boundary, or too little of it, that is enough for the row tiles' shares goes to those.
+ *   The block-table decode kernels, where that one is not taken and no window is below 2048 keys: head_dim a multiple of 16 up to
+ *   128, scratch on a 256-byte boundary.  They cut the keys of all sequences into equal ranges: a first kernel checks the paging
+ *   vectors and gives each token its page list and key count, and the scratch also holds those and the decode kernels' partial
+ *   rows. */
 SINGE_HIP_API size_t singe_hip_paged_attention_scratch_bytes(const SingePagedAttentionProblem* problem);
 SINGE_HIP_API void singe_hip_set_paged_attention_splits(uint32_t splits);
 /* Packed rows a wave of the bf16 / f16 paged attention kernels takes, as singe_hip_set_dense_prefill_rows_per_wave: 32,

@@ -12,10 +12,11 @@
 // (prefill_blocks.hip.h), which keeps the matrix core fed while the vector unit works.
 //
 // Grid: one workgroup per (batch, head, pair of 128-row query tiles): tile i from the end and tile i from
-// the start, so under the causal mask every workgroup has the same amount of work.  Workgroup i lands on
-// XCD i % 8; ids are laid out so the workgroups of one (batch, head) are neighbours on one XCD and walk
-// its keys side by side, which keeps its K/V in that XCD's L2.  Small launches take one tile to a workgroup
-// instead, the longest first (`single_tiles`).
+// the start, so under the causal mask every workgroup has the same amount of work.  Small launches take one
+// tile to a workgroup instead, the longest first (`single_tiles`).  Workgroup i lands on XCD i % 8; ids are laid
+// out so the workgroups of one (batch, head) are neighbours on one XCD and walk its keys side by side, which keeps
+// its K/V in that XCD's L2: whole (batch, head)s to an XCD, or an eighth of all tiles, whose ends may lie inside
+// one (`deal`).
 #include "kernel_args.h"
 // Up to head_dim 64 an LDS row is 128 bytes: 40 KiB a workgroup, so a compute unit holds as many as its registers allow
 // instead of two (four at head_dim 16 and 32, three at 48 and 64, with or without the options), and every lane of a tile's
@@ -487,7 +488,8 @@ SINGE_DEVICE void fmha_prefill_tile(const PrefillArgs& a, unsigned char* lds, un
 // The `within`-th workgroup of an XCD -> (batch, head) `bh` and which of its `pairs` of query tiles (see kDeal...); false: none.
 // By length: the dispatcher fills an XCD's 32 compute units one after the other, round after round, and those at the front of an
 // incomplete last round take one workgroup more than the rest.  They get the shortest, the others the longest, and both change
-// direction from round to round so that a compute unit's sum is about the same.
+// direction from round to round so that a compute unit's sum is about the same.  (Any other placement gives the same tiles in
+// another order: only the time rests on it.)
 SINGE_DEVICE bool deal_units(const PrefillArgs& a, unsigned int heads, unsigned int pairs, unsigned int xcd, unsigned int& within, unsigned int& bh) {
     constexpr unsigned int kUnitsOfXcd = 32;
     const unsigned int all = a.batch * heads;
