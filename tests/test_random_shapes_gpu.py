@@ -1,6 +1,8 @@
 """Seeded random shapes for the bf16 matrix-core kernels against the CPU oracle: what a hand-picked list of cases
 misses (odd groupings, page sizes on both sides of the scalar page path, sequences of any mix of query and key
 counts, key splits on and off, every option at once).  Same tolerances as the hand-picked cases."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -133,19 +135,33 @@ def dense_prefill_random_shape(seed, rng, dim, stretch):
 @pytest.mark.parametrize("seed", range(32))
 def test_decode_steps_through_the_op_random_shapes(seed):
     """Random decode steps (no more tokens than sequences: mostly a token a sequence, some sequences with none, a few
-    with two or three) through the paged attention op, which runs them on the block-table decode kernels: against the
-    oracle, both head dimensions, both index types, bf16 and f16, causal or not, with and without a window, up to 16 query
+    with two or three) through the paged attention op, which runs them in one launch or on the block-table decode kernels: against
+    the oracle, both head dimensions, both index types, bf16 and f16, causal or not, with and without a window, up to 16 query
     heads a kv head."""
-    rng = np.random.default_rng(5000 + seed)
+    check_random_decode_step(seed, np.random.default_rng(5000 + seed))
+
+
+@pytest.mark.parametrize("seed", range(16))
+def test_decode_steps_past_the_one_launch_random_shapes(seed):
+    """The same with the page sizes that one launch takes, of more and longer sequences than it does."""
+    check_random_decode_step(seed, np.random.default_rng(7000 + seed), past_one_launch=True)
+
+
+def check_random_decode_step(seed, rng, past_one_launch=False):
     kv_heads = int(rng.choice([1, 2, 4, 8]))
     heads = kv_heads * int(rng.choice([1, 2, 3, 4, 5, 8, 12, 16]))
     dim = int(rng.choice([128, 128, 64]))
     page_size = int(rng.choice([1, 3, 8, 16, 16, 32, 64, 24]))
     dtype = torch.bfloat16 if rng.integers(0, 3) else torch.float16
     count = int(rng.choice([1, 2, 5, 17, 70, 130]))
+    windows = [1, 100, 2048, 2300, 2999, 5000]
+    if past_one_launch:
+        page_size, count, windows = int(rng.choice([16, 32, 64])), 160 // kv_heads + int(rng.integers(0, 7)), windows[2:]
     sequences, spare = [], 0
     for _ in range(count):
         keys = int(rng.choice([0, 1, int(rng.integers(1, 64)), int(rng.integers(64, 700)), int(rng.integers(700, 3000)), int(rng.integers(2048, 4500))]))
+        if past_one_launch and rng.integers(0, 4):
+            keys = int(rng.integers(900, 3500))
         queries = int(rng.choice([1, 1, 1, 1, 0, 2, 3]))
         if queries > 1 and spare < queries - 1:
             queries = 1
@@ -154,7 +170,7 @@ def test_decode_steps_through_the_op_random_shapes(seed):
     if sum(q for q, _ in sequences) == 0:
         sequences[0] = (1, sequences[0][1])
     options = neural.AttentionOptions(causal=bool(rng.integers(0, 2)), scale=None if rng.integers(0, 2) else float(rng.uniform(0.02, 0.2)),
-                                      window=None if rng.integers(0, 2) else int(rng.choice([1, 100, 2048, 2300, 2999, 5000])))
+                                      window=None if rng.integers(0, 2) else int(rng.choice(windows)))
     index_dtype = torch.int64 if rng.integers(0, 2) else torch.int32
     query_offsets, page_offsets, last = [0], [0], []
     for queries, keys in sequences:
@@ -173,6 +189,9 @@ def test_decode_steps_through_the_op_random_shapes(seed):
     q, kc, vc = rand(tokens, heads, dim), rand(page_count, page_size, kv_heads, dim), rand(page_count, page_size, kv_heads, dim)
     index = lambda values: torch.tensor(values, dtype=index_dtype, device="cuda")
     paging = neural.Paging(index(query_offsets), index(page_offsets), index(table), index(last))
+    if past_one_launch:
+        problem = ctypes.byref(neural._problem(q, kc, vc, paging, options))
+        assert _native.lib().singe_hip_paged_attention_route(problem, 256, _native.lib().singe_hip_paged_attention_scratch_bytes(problem)) == 1
     out, lse = neural.paged_attention(q, kc, vc, paging, options)
     torch.cuda.synchronize()
     status, want, want_lse = oracle.paged_attention_f32(q.float().cpu().numpy(), kc.float().cpu().numpy(), vc.float().cpu().numpy(), query_offsets,
