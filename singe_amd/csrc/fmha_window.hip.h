@@ -13,10 +13,12 @@
 // What bounds it is the queries' way in and the outputs' way out (64 / 8 heads x 8192 x 64, bf16: 151 MB, 31 us at the 4.8 TB/s
 // of a copy) with the folding beside them: window 16 31 us, 128 41 us, 256 55 us, where tiles of 128 rows in workgroups of their
 // own, each with round trips of its own at either end and a barrier to 64 keys, take 48, 58 and 70 us; at head_dim 128 62, 75
-// and 98 us against 96, 125 and 151.  The outputs leave as 64 contiguous bytes a row, past the caches: as 32 bytes a row and
-// through them they cost 11 us more at head_dim 128; 32 bytes a row past the caches 11 us more at head_dim 64 too.  The queries
-// come through the caches (past them +8 us at 64, +30 us at 128), 64 bytes a row at a time or 32 alike.  Up to head_dim 64 a
-// compute unit holds two workgroups of at most 128 registers, which is why lane offsets are worked out again from step to step.
+// and 98 us against 96, 125 and 151.  (One call's buffers over and over; many calls in turn over 600 MB: 40, 51 and 65 us
+// against 50, 62 and 74; window 128 at head_dim 128 95 against 121.)  The outputs leave as 64 contiguous bytes a row, past the
+// caches (see store_row_16): as 32 bytes a row and through them they cost 11 us more at head_dim 128; 32 bytes a row past the
+// caches 11 us more at head_dim 64 too.  The queries come through the caches (past them +8 us at 64, +30 us at 128), 64 bytes a
+// row at a time or 32 alike.  Up to head_dim 64 a compute unit holds two workgroups of at most 128 registers, which is why lane
+// offsets are worked out again from step to step.
 #pragma once
 
 #include "prefill_blocks.hip.h"
@@ -24,6 +26,14 @@
 namespace prefill {
 
 constexpr unsigned int kWindowStepRows = 32u * kWindowPrefillWaves;
+
+// Rows of whole 64-byte pieces leave past the caches; the others end inside pieces, which past them go out in parts.  Past /
+// through the caches (tiles of 128 rows), us, many calls in turn over 600 MB:
+//   28 / 4 heads x 112, 4 x 9401, window 16  219 / 120 (153)   40 / 8 x 80, 4 x 3764, 20  92 / 56 (78)   64 / 8 x 48, 4 x 2325, 16  49 / 33 (46)
+SINGE_DEVICE void store_row_16(unsigned char* address, uint4 bits) {
+    if constexpr (kHeadDim % 32 == 0) stream_store_16(address, bits);
+    else *reinterpret_cast<uint4*>(address) = bits;
+}
 
 template <class Half>
 SINGE_DEVICE void fmha_window_body(const PrefillArgs& a, unsigned char* lds) {
@@ -225,8 +235,8 @@ SINGE_DEVICE void fmha_window_body(const PrefillArgs& a, unsigned char* lds) {
             unsigned char* const to = out_bytes + 16u * hi;
 #pragma unroll
             for (int p = 0; p + 1 < kPieces; p += 2) {
-                if (at != ~0u) stream_store_16(to + 2u * (lane & 16u) + at + 32 * p, packed[p]);
-                if (other != ~0u) stream_store_16(to + 2u * (lane & 16u) + other + 32 * p, packed[p + 1]);
+                if (at != ~0u) store_row_16(to + 2u * (lane & 16u) + at + 32 * p, packed[p]);
+                if (other != ~0u) store_row_16(to + 2u * (lane & 16u) + other + 32 * p, packed[p + 1]);
             }
             if (kPieces % 2 != 0 && mine != ~0u) *reinterpret_cast<uint4*>(to + mine + 32 * (kPieces - 1)) = packed[kPieces - 1];
             if (my_query < a.query_len) {

@@ -58,3 +58,18 @@ def test_no_scratch_memory_in_the_kernels_that_cannot_afford_it(remarks, name, f
         named = {kernel: size for kernel, size in scratch.items() if re.fullmatch(pattern, kernel)}
         assert named, f"no kernel of {name} matches {pattern}"
         assert all(size == 0 for size in named.values()), {kernel: size for kernel, size in named.items() if size}
+
+
+@pytest.mark.parametrize("head_dim,past_the_caches", [(32, True), (48, False)])
+def test_rows_that_end_inside_64_byte_pieces_leave_through_the_caches(head_dim, past_the_caches):
+    # (past them such rows of a causal window's call go out in parts: 4 x 28 / 4 heads x 9401 x 112, window 16, 219 us and 120)
+    source, flags = os.path.join(CSRC, "fmha_prefill.hip"), [flag for flag in build.HIPCC_FLAGS if flag != "--genco"]
+    with tempfile.TemporaryDirectory() as scratch:
+        listing = os.path.join(scratch, "out.s")
+        subprocess.run([build.hipcc(), *flags, f"-DSINGE_HEAD_DIM={head_dim}", "--cuda-device-only", "-S", "-I", CSRC, source, "-o", listing],
+                       check=True, capture_output=True)
+        text = open(listing).read()
+    for name in ("bf16", "f16"):
+        kernel = f"singe_fmha_prefill_{name}_d{head_dim}_causal_window"
+        stores = re.findall(r"global_store_dwordx4 .*", re.search(rf"^{kernel}:(.*?)s_endpgm", text, re.S | re.M).group(1))
+        assert stores and any(store.endswith(" nt") for store in stores) == past_the_caches
