@@ -8,10 +8,9 @@
 // (and the gaps around them) were most of a step.
 //
 // What bounds it is a chain of round trips to memory: the paging vectors, the page ids, the first keys, and where a unit is
-// shared out four more (its rows out, its word out, the words in, the rows in), some 5 us, which is what 8 to 9 tiles of keys take
-// a workgroup of four waves and twice as many one of eight.  One token of 32 / 8 heads x 128, device time: 100 keys 6.7 us, 800 11.4,
-// 3100 14.5, 32000 29 (three launches: 11.3, 11.7, 13.6, 31); sixteen of 16 to 700 keys 12.9 (14.7).  The figures of whole calls
-// stand at `decode_step_entries`.
+// shared out four more (its rows out, its word out, the words in, the rows in), which is why a unit of up to kStepWholeTiles is not.
+// One token of 32 / 8 heads x 128, device time over 700 MB of caches: 100 keys 7.7 us, 800 13.5, 2000 14.5, 32000 31 (three launches:
+// 12.4, 12.9, 13.6, 34); sixteen of 16 to 700 keys 14.7 (16.7).  The figures of whole calls stand at `decode_step_entries`.
 #pragma once
 
 #include "paged_locate.hip.h"
